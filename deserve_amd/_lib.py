@@ -30,6 +30,15 @@ class MixedPlanInfo(ctypes.Structure):
                 ("decode_workspace_bytes", c_int64)]
 
 
+class DecodeStep(ctypes.Structure):
+    """dskv_decode_step_t of include/dskv.h."""
+    _fields_ = [("kv_page_indices", c_void_p), ("plan_dev", c_void_p), ("workspace", c_void_p),
+                ("workspace_bytes", c_int64), ("merge_counters", c_void_p), ("n_merge_counters", c_int64),
+                ("rope_table", c_void_p), ("n_items", c_int32), ("n_workgroups", c_int32), ("batch", c_int32),
+                ("n_qo_heads", c_int32), ("n_kv_heads", c_int32), ("head_dim", c_int32), ("page_size", c_int32),
+                ("dtype", c_int32), ("sm_scale", c_float)]
+
+
 _lib: Optional[ctypes.CDLL] = None
 
 # name -> (restype, argtypes); mirrors include/dskv.h one to one
@@ -68,6 +77,7 @@ _SIGNATURES = {
                                                c_void_p, c_void_p, c_int32, c_int32, c_void_p,
                                                c_int64, c_int32, c_int32, c_int32, c_int32, c_int32,
                                                c_float, c_int32, c_void_p, c_int32, c_void_p]),
+    "dskv_decode_step": (c_int32, [POINTER(DecodeStep)] + [c_void_p] * 6),
     "dskv_prefill_plan_bound": (c_int64, [c_int32, c_int64]),
     "dskv_prefill_plan": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32, c_int32,
                                     c_void_p, c_int64, POINTER(c_int32), POINTER(c_int32),

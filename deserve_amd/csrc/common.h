@@ -42,6 +42,7 @@ void set_error(const char *fmt, ...) __attribute__((format(printf, 1, 2)));
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -67,8 +68,8 @@ struct DecodeRow {
     int64_t len;
     int32_t page_begin, row;
 };
-int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, int32_t head_dim,
-                     int32_t target_workgroups, int32_t *plan_host, int64_t plan_capacity_words,
+int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, int32_t n_kv_heads,
+                     int32_t head_dim, int32_t target_workgroups, int32_t *plan_host, int64_t plan_capacity_words,
                      int32_t *n_items_out, int32_t *n_workgroups_out, int64_t *plan_words_out,
                      int64_t *workspace_bytes_out);
 int decode_rows_attn(void *out, const void *q, const void *pages_layer,

@@ -20,6 +20,9 @@
 //   inside a workgroup.  Items are padded to a multiple of kStages tiles; the
 //   padding tiles fetch nothing (empty buffer descriptor) and contribute zero.
 //
+//   Batches too small for that (the planner's rule) run with a workgroup per (share,
+//   kv head) instead: decode_split_kernel.h.
+//
 // Per 16-token tile and wave (D = 128, 16-bit elements):
 //   S^T[token, qhead] = K_tile (16x128) . Q^T (128x16): four 16x16x32 MFMAs.
 //     The A operand wants lane (g = lane/16, c = lane%16) to hold 8 consecutive
@@ -33,6 +36,7 @@
 //     needs 4 tokens of ONE dim per lane - the transpose of how it lies in
 //     memory - so the V tile goes through a wave-private LDS tile.
 #include "decode_kernel.h"
+#include "decode_split_kernel.h"
 #include "merge_kernel.h"
 
 #include <algorithm>
@@ -421,6 +425,14 @@ static int default_workgroups()
     return cached;
 }
 
+// Whether a plan's shares are so few that the attention runs as one workgroup per (share, kv
+// head) (decode_split_kernel.h) instead of one per share: when that still gives every compute
+// unit at most one.
+static bool decode_splits_tokens(int n_workgroups, int n_qo_heads, int n_kv_heads)
+{
+    return n_qo_heads / n_kv_heads <= kSplitMaxGroup && (int64_t)n_workgroups * n_kv_heads <= default_workgroups();
+}
+
 }  // namespace dskv
 
 // ---------------------------------------------------------------------------
@@ -438,8 +450,8 @@ namespace dskv {
 
 // The planner proper.  reqs[i]: tokens, start of the block table and q / output row of
 // request i (row i itself for a decode batch).
-int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, int32_t head_dim,
-                     int32_t target_workgroups, int32_t *plan_host, int64_t plan_capacity_words,
+int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, int32_t n_kv_heads,
+                     int32_t head_dim, int32_t target_workgroups, int32_t *plan_host, int64_t plan_capacity_words,
                      int32_t *n_items_out, int32_t *n_workgroups_out, int64_t *plan_words_out,
                      int64_t *workspace_bytes_out)
 {
@@ -450,9 +462,20 @@ int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, i
         tiles[b] = (reqs[b].len + kTile - 1) / kTile;
         total_tiles += tiles[b];
     }
-    // Workgroup count: one per CU unless told otherwise, fewer when there is so
-    // little work that a share would drop below a few tiles.
-    int64_t wgs = target_workgroups > 0 ? target_workgroups : default_workgroups();
+    // Share count: one per CU unless told otherwise, fewer when there is so little work that a
+    // share would drop below a few tiles.  Small batches get so few that the attention runs as
+    // one workgroup per (share, kv head): measured (bf16, 8 kv heads, attention and merge in a
+    // replayed graph, us) with 32 shares against 256 or the four-tile shares of before: 318 tiles
+    // 15 / 24, 1024 tiles 21 / 26, 2048 tiles 31-33 / 33-41, 3255 tiles 51 / 48, 4096 tiles
+    // 56 / 52.  A share of six tiles: one request of 112 tiles takes 13.1 us in 18 shares (14.0 in
+    // 28), three of 13 tiles take 10.7 us in 9 shares (13.0 in 4).
+    int64_t wgs = target_workgroups;
+    if (wgs <= 0) {
+        wgs = default_workgroups();
+        const int64_t few = wgs / n_kv_heads;
+        if (head_dim == kHeadDim && few > 0 && n_qo_heads / n_kv_heads <= kSplitMaxGroup && total_tiles <= kSplitMaxTiles)
+            wgs = std::min<int64_t>(few, std::max<int64_t>(1, total_tiles / kSplitTilesPerShare));
+    }
     wgs = std::min<int64_t>(wgs, kMaxWorkgroups);
     wgs = std::min<int64_t>(wgs, std::max<int64_t>(1, total_tiles / kMinTilesPerWorkgroup));
 
@@ -462,12 +485,12 @@ int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, i
     std::vector<Item> items;
     std::vector<int32_t> wg_ptr(1, 0), req(2 * (size_t)batch, 0);
     int32_t n_slots = 0;
-    int64_t w = 0, g0 = 0;                        // current workgroup, global tile index
+    int64_t w = 0, g0 = 0, share_begin = 0;       // current workgroup, global tile index, its share's first
     auto share_end = [&](int64_t wg) { return (wg + 1) * total_tiles / wgs; };
     for (int b = 0; b < batch; b++) {
         const int64_t len = reqs[b].len;
         if (tiles[b] == 0) {
-            items.push_back(Item{reqs[b].row, 0, 0, -1, reqs[b].page_begin, 0, {0, 0}});
+            items.push_back(Item{reqs[b].row, 0, 0, -1, reqs[b].page_begin, 0, 0, (int32_t)(g0 - share_begin)});
             continue;
         }
         const size_t first_item = items.size();
@@ -476,12 +499,13 @@ int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, i
             while (w + 1 < wgs && g0 >= share_end(w)) {     // this workgroup's share is full
                 wg_ptr.push_back((int32_t)items.size());
                 w++;
+                share_begin = g0;
             }
             const int64_t room = (w + 1 < wgs) ? share_end(w) - g0 : tiles[b] - done;
             const int64_t take = std::min(room, tiles[b] - done);
             items.push_back(Item{reqs[b].row, (int32_t)(done * kTile),
                                  (int32_t)std::min<int64_t>((done + take) * kTile, len), -1,
-                                 reqs[b].page_begin, done + take == tiles[b], {0, 0}});
+                                 reqs[b].page_begin, done + take == tiles[b], 0, (int32_t)(g0 - share_begin)});
             done += take;
             g0 += take;
         }
@@ -489,7 +513,10 @@ int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, i
         if (parts > 1) {
             req[2 * b] = n_slots;
             req[2 * b + 1] = (int32_t)parts;
-            for (size_t i = first_item; i < items.size(); i++) items[i].slot = n_slots++;
+            for (size_t i = first_item; i < items.size(); i++) {
+                items[i].slot = n_slots++;
+                items[i].parts = req[2 * b] << kPartsBits | (int32_t)parts;
+            }
         }
     }
     while ((int64_t)wg_ptr.size() < wgs + 1) wg_ptr.push_back((int32_t)items.size());
@@ -555,7 +582,7 @@ extern "C" int dskv_decode_plan(const int32_t *kv_page_indptr_host,
                      "decode_plan: kv_last_page_len[%d] = %d outside [1, %d]", b, last, page_size);
         reqs[b] = DecodeRow{np > 0 ? (np - 1) * page_size + last : 0, kv_page_indptr_host[b], b};
     }
-    return plan_decode_rows(reqs.data(), batch, n_qo_heads, head_dim, target_workgroups, plan_host,
+    return plan_decode_rows(reqs.data(), batch, n_qo_heads, n_kv_heads, head_dim, target_workgroups, plan_host,
                             plan_capacity_words, n_items_out, n_workgroups_out, plan_words_out,
                             workspace_bytes_out);
 }
@@ -571,7 +598,8 @@ static int decode_attn_impl(void *out, const void *q, const void *pages_layer,
                             int32_t n_kv_heads, int32_t head_dim, int32_t page_size,
                             float sm_scale, int32_t dtype, int32_t phases, void *stream,
                             const void *k_new, const void *v_new, const float *rope_table,
-                            const int32_t *row_map = nullptr)
+                            const int32_t *row_map = nullptr, uint32_t *merge_counters = nullptr,
+                            int64_t n_merge_counters = 0)
 {
     DSKV_REQUIRE(phases >= 1 && phases <= 3, "decode_attn: phases must be 1, 2 or 3");
     DSKV_REQUIRE(batch >= 0 && n_items >= 0 && n_workgroups >= 0,
@@ -615,6 +643,7 @@ static int decode_attn_impl(void *out, const void *q, const void *pages_layer,
     DSKV_REQUIRE(!k_new || (mfma_path(dtype, head_dim, n_qo_heads, n_kv_heads) && (phases & 1)),
                  "decode_append_attn: shape or dtype outside the fused kernel (see "
                  "dskv_decode_append_attn_supported); append and attend separately");
+    bool merged = false;   // the attention launch merges the parts itself
     if (!(phases & 1)) {
         // merge only: the split-KV pass of this plan has already been enqueued
     } else if (mfma_path(dtype, head_dim, n_qo_heads, n_kv_heads)) {
@@ -624,25 +653,53 @@ static int decode_attn_impl(void *out, const void *q, const void *pages_layer,
                      page_size);
         DSKV_REQUIRE((int64_t)2 * page_size * n_kv_heads * head_dim * 2 < (int64_t(1) << 31),
                      "decode_attn: a page must be smaller than 2 GiB");
-        const int waves = std::min(n_kv_heads, kMaxWaves);
-        dim3 grid((unsigned)n_workgroups, (unsigned)((n_kv_heads + kMaxWaves - 1) / kMaxWaves));
-        dim3 block(64 * waves);
         const int shift = ilog2(page_size);
+        if (decode_splits_tokens(n_workgroups, n_qo_heads, n_kv_heads)) {
+            // every cut adds an item, and a request cut c times owns c + 1 slots
+            const int64_t slots = std::min<int64_t>(n_items, 2 * ((int64_t)n_items - batch));
+            DSKV_REQUIRE(!merge_counters || n_merge_counters >= slots * n_kv_heads,
+                         "decode_attn: %lld merge counters, the plan needs %lld", (long long)n_merge_counters,
+                         (long long)(slots * n_kv_heads));
+            merged = merge_counters && phases == 3;
+            const int share_stride = (n_workgroups + 7) / 8 * 8;
+            const SplitArgs args = {(uint16_t *)out, (const uint16_t *)q, (const char *)pages_layer, kv_page_indices,
+                                    items, wg_ptr, part_o, part_ml, (int)max_slots, n_qo_heads, n_kv_heads, shift,
+                                    scale_log2, (const uint16_t *)k_new, (const uint16_t *)v_new, rope_table,
+                                    merged && n_items > batch ? merge_counters : nullptr,
+                                    (int)std::min<int64_t>(n_merge_counters, 1 << 30), n_workgroups, share_stride};
+            const dim3 grid((unsigned)(share_stride * n_kv_heads)), block(64 * kSplitWaves);
+#define DSKV_LAUNCH_SPLIT(DT, COVER) \
+    hipLaunchKernelGGL((decode_attn_split_kernel<DT, COVER>), grid, block, 0, s, args)
+            if (dtype == DSKV_BF16) {
+                if (page_size >= kTile) DSKV_LAUNCH_SPLIT(DSKV_BF16, 1);
+                else if (page_size == 8) DSKV_LAUNCH_SPLIT(DSKV_BF16, 2);
+                else DSKV_LAUNCH_SPLIT(DSKV_BF16, 0);
+            } else {
+                if (page_size >= kTile) DSKV_LAUNCH_SPLIT(DSKV_F16, 1);
+                else if (page_size == 8) DSKV_LAUNCH_SPLIT(DSKV_F16, 2);
+                else DSKV_LAUNCH_SPLIT(DSKV_F16, 0);
+            }
+#undef DSKV_LAUNCH_SPLIT
+        } else {
+            const int waves = std::min(n_kv_heads, kMaxWaves);
+            const dim3 grid((unsigned)n_workgroups, (unsigned)((n_kv_heads + kMaxWaves - 1) / kMaxWaves));
+            const dim3 block(64 * waves);
 #define DSKV_LAUNCH_MFMA(DT, COVER)                                                              \
     hipLaunchKernelGGL((decode_attn_mfma_kernel<DT, COVER>), grid, block, 0, s, (uint16_t *)out, \
                        (const uint16_t *)q, (const char *)pages_layer, kv_page_indices, items,   \
                        wg_ptr, part_o, part_ml, (int)max_slots, n_qo_heads, n_kv_heads, shift,   \
                        scale_log2, (const uint16_t *)k_new, (const uint16_t *)v_new, rope_table)
-        if (dtype == DSKV_BF16) {
-            if (page_size >= kTile) DSKV_LAUNCH_MFMA(DSKV_BF16, 1);
-            else if (page_size == 8) DSKV_LAUNCH_MFMA(DSKV_BF16, 2);
-            else DSKV_LAUNCH_MFMA(DSKV_BF16, 0);
-        } else {
-            if (page_size >= kTile) DSKV_LAUNCH_MFMA(DSKV_F16, 1);
-            else if (page_size == 8) DSKV_LAUNCH_MFMA(DSKV_F16, 2);
-            else DSKV_LAUNCH_MFMA(DSKV_F16, 0);
-        }
+            if (dtype == DSKV_BF16) {
+                if (page_size >= kTile) DSKV_LAUNCH_MFMA(DSKV_BF16, 1);
+                else if (page_size == 8) DSKV_LAUNCH_MFMA(DSKV_BF16, 2);
+                else DSKV_LAUNCH_MFMA(DSKV_BF16, 0);
+            } else {
+                if (page_size >= kTile) DSKV_LAUNCH_MFMA(DSKV_F16, 1);
+                else if (page_size == 8) DSKV_LAUNCH_MFMA(DSKV_F16, 2);
+                else DSKV_LAUNCH_MFMA(DSKV_F16, 0);
+            }
 #undef DSKV_LAUNCH_MFMA
+        }
         DSKV_LAUNCH_CHECK("decode_attn_mfma_kernel");
     } else if (n_qo_heads / n_kv_heads <= 8 && head_dim % 8 == 0 && head_dim <= 128 &&
                ((uintptr_t)pages_layer % 16 == 0) && ((int64_t)n_kv_heads * head_dim * (dtype == DSKV_F32 ? 4 : 2)) % 16 == 0) {
@@ -678,7 +735,7 @@ static int decode_attn_impl(void *out, const void *q, const void *pages_layer,
 #undef DSKV_LAUNCH_GEN
         DSKV_LAUNCH_CHECK("decode_attn_generic_kernel");
     }
-    if ((phases & 2) && n_items > batch) {
+    if (!merged && (phases & 2) && n_items > batch) {
         // many parts per request (long requests, small batch): eight waves share a merge.
         // One wave needs a round trip per 8 parts, eight waves a barrier and a second pass
         // through LDS: they break even at about 32 parts.
@@ -800,6 +857,25 @@ extern "C" int dskv_decode_rope_append_attn(void *out, const void *q, const void
     return decode_attn_impl(out, q, pages_layer, kv_page_indices, plan_dev, n_items, n_workgroups,
                             workspace, workspace_bytes, batch, n_qo_heads, n_kv_heads, head_dim,
                             page_size, sm_scale, dtype, phases, stream, k_new, v_new, rope_table);
+}
+
+extern "C" int dskv_decode_step(const dskv_decode_step_t *step, void *out, const void *q, const void *k_new,
+                                const void *v_new, void *pages_layer, void *stream)
+{
+    using namespace dskv;
+    DSKV_REQUIRE(step, "decode_step: null step");
+    if (step->batch == 0 || step->n_items == 0) return 0;
+    DSKV_REQUIRE(!k_new == !v_new, "decode_step: k_new and v_new go together");
+    DSKV_REQUIRE(k_new || !step->rope_table, "decode_step: the rotation needs k_new / v_new");
+    DSKV_REQUIRE(((uintptr_t)k_new | (uintptr_t)v_new | (uintptr_t)step->rope_table) % 16 == 0,
+                 "decode_step: k_new / v_new / table must be 16-byte aligned");
+    DSKV_REQUIRE(step->n_merge_counters >= 0 && (step->merge_counters || step->n_merge_counters == 0),
+                 "decode_step: bad merge counters");
+    return decode_attn_impl(out, q, pages_layer, step->kv_page_indices, step->plan_dev, step->n_items,
+                            step->n_workgroups, step->workspace, step->workspace_bytes, step->batch,
+                            step->n_qo_heads, step->n_kv_heads, step->head_dim, step->page_size,
+                            step->sm_scale, step->dtype, 3, stream, k_new, v_new, step->rope_table, nullptr,
+                            step->merge_counters, step->n_merge_counters);
 }
 
 // ---------------------------------------------------------------------------

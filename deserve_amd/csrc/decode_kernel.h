@@ -18,6 +18,9 @@ constexpr int kStages = DSKV_DECODE_STAGES;   // tiles in flight per wave (one c
 constexpr int kPlanHeaderWords = 4;  // n_items, n_workgroups, n_slots, batch
 constexpr int kItemWords = 8;
 constexpr int kMaxWorkgroups = 4096;
+constexpr int kPartsBits = 13;       // a request has at most one part per workgroup
+static_assert(kMaxWorkgroups < (1 << kPartsBits) && 2L * kMaxWorkgroups < (1L << (31 - kPartsBits)),
+              "first slot and number of parts share a word");
 #ifndef DSKV_DECODE_MIN_TILES
 #define DSKV_DECODE_MIN_TILES 4
 #endif
@@ -30,7 +33,8 @@ struct Item {
     int32_t tok_begin, tok_end, slot;
     int32_t page_begin;   // kv_page_indptr[b]: start of the request's block table
     int32_t tail;         // 1: tok_end is the request's length (the item holds its newest token)
-    int32_t reserved[2];
+    int32_t parts;        // of a cut request: its first partial slot << kPartsBits | number of parts
+    int32_t tile_at;      // tiles of the same share in front of the item
 };
 static_assert(sizeof(Item) == kItemWords * 4, "plan item layout");
 
@@ -84,7 +88,7 @@ __device__ __forceinline__ void decode_attn_body(
     const const_i32_ptr item_words = as_const(reinterpret_cast<const int32_t *>(items));
     auto load_item = [&](int idx) {
         const const_i32_ptr w = item_words + (long)idx * kItemWords;
-        return Item{w[0], w[1], w[2], w[3], w[4], w[5], {0, 0}};
+        return Item{w[0], w[1], w[2], w[3], w[4], w[5], 0, 0};
     };
     const const_i32_ptr indices_c = as_const(kv_indices);
     const int item_begin = as_const(wg_ptr)[share];

@@ -95,6 +95,7 @@ class _PagedWrapper:
         self._workspace = workspace_buffer
         self._planned = False
         self._rope_table, self._rope_key = None, None
+        self._counters = None
         self._max_page_id = -1
         self._empty_requests = []
 
@@ -188,6 +189,19 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
             plan_buffers.upload(max(words, 1))
         else:
             self._plan = staging.to_device(block, max(words, 1), indices.device)
+        self._bind_step()
+
+    def _bind_step(self) -> None:
+        """What all layers of the planned step share, for dskv_decode_step."""
+        ws_bytes = self._workspace.numel() * self._workspace.element_size()
+        if self._counters is None:
+            # one word per (partial slot, kv head) for as many slots as the workspace can hold;
+            # kept for good: captured launches hold its address, and every launch leaves it zero
+            self._counters = torch.zeros((max(ws_bytes // 256, 1),), dtype=torch.int32, device=self._plan.device)
+        self._step = _lib.DecodeStep(
+            self._indices.data_ptr(), self._plan.data_ptr(), self._workspace.data_ptr(), ws_bytes,
+            self._counters.data_ptr(), self._counters.numel(), None, self._n_items, self._n_workgroups, self._batch,
+            self._hq, self._hkv, self._d, self._p)
         self._planned = True
 
     @staticmethod
@@ -243,7 +257,7 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
         self._indptr = dev[indptr_at: indptr_at + batch + 1]
         used = int(h_indptr[-1]) if batch > 0 else 0
         self._indices = dev[indices_at: indices_at + used]
-        self._planned = True
+        self._bind_step()
         return dev[:meta_words]
 
     def fused_append_supported(self, dtype: torch.dtype) -> bool:
@@ -277,6 +291,7 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
             out = torch.empty_like(q)
         scale = 1.0 / math.sqrt(self._d) if sm_scale is None else sm_scale
         ws_bytes = self._workspace.numel() * self._workspace.element_size()
+        table = None
         if k_append is not None or v_append is not None:
             if k_append is None or v_append is None or phases not in (1, 3):
                 raise ValueError("the fused form takes both k_append and v_append, with the attention pass")
@@ -300,28 +315,26 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
                                                           self._batch, self._d, rope_theta,
                                                           _lib.current_stream()), "rope table")
                     self._rope_table, self._rope_key = table, key
-                rc = _lib.lib().dskv_decode_rope_append_attn(
-                    out.data_ptr(), q.data_ptr(), k_append.data_ptr(), v_append.data_ptr(),
-                    paged_kv_data.data_ptr(), self._indices.data_ptr(), self._plan.data_ptr(),
-                    self._n_items, self._n_workgroups, self._workspace.data_ptr(), ws_bytes,
-                    self._batch, self._hq, self._hkv, self._d, self._p, scale,
-                    _lib.dtype_code(q.dtype), self._rope_table.data_ptr(), phases,
-                    _lib.current_stream())
-                _lib.check(rc, "decode rope + append + forward")
-                return out
-            rc = _lib.lib().dskv_decode_append_attn(
-                out.data_ptr(), q.data_ptr(), k_append.data_ptr(), v_append.data_ptr(),
-                paged_kv_data.data_ptr(), self._indices.data_ptr(), self._plan.data_ptr(),
-                self._n_items, self._n_workgroups, self._workspace.data_ptr(), ws_bytes, self._batch,
-                self._hq, self._hkv, self._d, self._p, scale, _lib.dtype_code(q.dtype), phases,
-                _lib.current_stream())
-            _lib.check(rc, "decode append + forward")
+                table = self._rope_table.data_ptr()
+        if phases == 3:
+            step = self._step
+            step.rope_table, step.dtype, step.sm_scale = table, _lib.dtype_code(q.dtype), scale
+            rc = _lib.lib().dskv_decode_step(ctypes.byref(step), out.data_ptr(), q.data_ptr(), _lib.ptr(k_append),
+                                             _lib.ptr(v_append), paged_kv_data.data_ptr(), _lib.current_stream())
+            _lib.check(rc, "decode forward")
             return out
-        rc = _lib.lib().dskv_decode_attn_phases(
-            out.data_ptr(), q.data_ptr(), paged_kv_data.data_ptr(), self._indices.data_ptr(),
-            self._plan.data_ptr(), self._n_items, self._n_workgroups, self._workspace.data_ptr(),
-            ws_bytes, self._batch, self._hq, self._hkv, self._d, self._p, scale,
-            _lib.dtype_code(q.dtype), phases, _lib.current_stream())
+        args = (paged_kv_data.data_ptr(), self._indices.data_ptr(), self._plan.data_ptr(), self._n_items,
+                self._n_workgroups, self._workspace.data_ptr(), ws_bytes, self._batch, self._hq, self._hkv,
+                self._d, self._p, scale, _lib.dtype_code(q.dtype))
+        if k_append is None:
+            rc = _lib.lib().dskv_decode_attn_phases(out.data_ptr(), q.data_ptr(), *args, phases, _lib.current_stream())
+        elif table is None:
+            rc = _lib.lib().dskv_decode_append_attn(out.data_ptr(), q.data_ptr(), k_append.data_ptr(),
+                                                    v_append.data_ptr(), *args, phases, _lib.current_stream())
+        else:
+            rc = _lib.lib().dskv_decode_rope_append_attn(out.data_ptr(), q.data_ptr(), k_append.data_ptr(),
+                                                         v_append.data_ptr(), *args, table, phases,
+                                                         _lib.current_stream())
         _lib.check(rc, "decode forward")
         return out
 

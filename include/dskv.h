@@ -194,6 +194,29 @@ int dskv_decode_rope_append_attn(void *out, const void *q, const void *k_new, co
                                  const float *rope_table, int32_t phases, void *stream);
 
 /*
+ * A decode step's attention, one call per layer, with everything that is the same for all layers
+ * of the step in one struct (the fields are those of the calls above).  k_new / v_new null: the
+ * tokens are in the pages already; rope_table (with k_new / v_new) null: no rotation.
+ * merge_counters (device, may be null): words that are zero before the first call that is given
+ * them and are used by one launch at a time, like the workspace; every launch leaves them zero.
+ * At least 2 * (n_items - batch) * n_kv_heads of them (n_items * n_kv_heads always suffice).  With
+ * them the attention launch merges the parts of cut requests itself instead of in a launch of its
+ * own (16-bit head_dim-128 kernels; other shapes leave them alone).
+ */
+typedef struct dskv_decode_step {
+    const int32_t *kv_page_indices, *plan_dev;
+    void *workspace;
+    int64_t workspace_bytes;
+    uint32_t *merge_counters;
+    int64_t n_merge_counters;
+    const float *rope_table;
+    int32_t n_items, n_workgroups, batch, n_qo_heads, n_kv_heads, head_dim, page_size, dtype;
+    float sm_scale;
+} dskv_decode_step_t;
+int dskv_decode_step(const dskv_decode_step_t *step, void *out, const void *q, const void *k_new,
+                     const void *v_new, void *pages_layer, void *stream);
+
+/*
  * Paged prefill attention with the end-aligned causal mask.  Replaces
  * BatchPrefillWithPagedKVCacheWrapper.forward(q, pages, causal=True)
  * (model/layer/attention.py:188-192, execution/exec.py:227-236).
