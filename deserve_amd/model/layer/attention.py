@@ -5,6 +5,8 @@ around it are dense GEMMs of the model proper and are not part of this package;
 in ragged (nnz, Hq * D) form, as the reference's method does before ``wo``."""
 from __future__ import annotations
 
+from typing import Optional
+
 import torch
 
 from deserve_amd.model.context.flash import FlashDecodeCtx, FlashForwardCtx, FlashPrefillCtx
@@ -24,7 +26,11 @@ class PagedAttentionCore:
 
     @torch.inference_mode()
     def paged_forward(self, xq: torch.Tensor, xk: torch.Tensor, xv: torch.Tensor,
-                      ctx: FlashForwardCtx) -> torch.Tensor:
+                      ctx: FlashForwardCtx, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """out: where the result goes (contiguous, one row of Hq * D per token); None: a tensor of
+        its own."""
+        if out is not None:
+            out = out.view(-1, self.n_local_heads, self.head_dim)
         xq = xq.view(-1, self.n_local_heads, self.head_dim)
         xk = xk.view(-1, self.n_local_kv_heads, self.head_dim)
         xv = xv.view(-1, self.n_local_kv_heads, self.head_dim)
@@ -34,7 +40,7 @@ class PagedAttentionCore:
             # a decode step: the attention launch rotates q and the new k and writes the new
             # token into its page slot itself
             rope = dict(rope_offsets=ctx.offsets, rope_theta=self.rope_theta) if self.use_rope else {}
-            out = ctx.decode_wrapper.forward(xq, pages, k_append=xk, v_append=xv, **rope)
+            out = ctx.decode_wrapper.forward(xq, pages, k_append=xk, v_append=xv, out=out, **rope)
             return out.view(-1, self.dim)
         if self.use_rope and self.fuse_rope_append:
             # one kernel: rotated q comes back, rotated k and v go straight into their slots
@@ -48,9 +54,9 @@ class PagedAttentionCore:
             append_paged_kv_cache(xk, xv, ctx.indptr, pages, ctx.kv_page_indices,
                                   ctx.kv_page_indptr, ctx.kv_last_page_lens)
         if isinstance(ctx, FlashDecodeCtx):
-            out = ctx.decode_wrapper.forward(xq, pages)
+            out = ctx.decode_wrapper.forward(xq, pages, out=out)
         elif isinstance(ctx, FlashPrefillCtx):
-            out = ctx.prefill_wrapper.forward(xq, pages, causal=True)
+            out = ctx.prefill_wrapper.forward(xq, pages, causal=True, out=out)
         else:
             raise TypeError(f"unsupported forward context {type(ctx).__name__}")
         return out.view(-1, self.dim)
