@@ -39,6 +39,16 @@ class DecodeStep(ctypes.Structure):
                 ("dtype", c_int32), ("sm_scale", c_float)]
 
 
+class MixedStep(ctypes.Structure):
+    """dskv_mixed_step_t of include/dskv.h."""
+    _fields_ = [("qo_indptr", c_void_p), ("kv_page_indices", c_void_p), ("kv_page_indptr", c_void_p),
+                ("kv_last_page_len", c_void_p), ("plan_dev", c_void_p), ("info", POINTER(MixedPlanInfo)),
+                ("workspace", c_void_p), ("workspace_bytes", c_int64), ("rope_table", c_void_p),
+                ("num_pages", c_int32), ("batch", c_int32), ("nnz", c_int32), ("n_qo_heads", c_int32),
+                ("n_kv_heads", c_int32), ("head_dim", c_int32), ("page_size", c_int32), ("causal", c_int32),
+                ("dtype", c_int32), ("sm_scale", c_float)]
+
+
 _lib: Optional[ctypes.CDLL] = None
 
 # name -> (restype, argtypes); mirrors include/dskv.h one to one
@@ -73,6 +83,8 @@ _SIGNATURES = {
                                           c_int32, c_int32, c_int32, c_int32, c_float, c_int32,
                                           c_int32, c_void_p]),
     "dskv_rope_table": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_float, c_void_p]),
+    "dskv_rope_table_ragged": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32, c_float,
+                                         c_void_p]),
     "dskv_decode_rope_append_attn": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                                c_void_p, c_void_p, c_int32, c_int32, c_void_p,
                                                c_int64, c_int32, c_int32, c_int32, c_int32, c_int32,
@@ -93,6 +105,8 @@ _SIGNATURES = {
                                   c_void_p, c_void_p, POINTER(MixedPlanInfo), c_void_p, c_int64,
                                   c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_float,
                                   c_int32, c_int32, c_void_p]),
+    "dskv_mixed_step_supported": (c_int32, [c_int32, c_int32, c_int32, c_int32, c_float, c_int32]),
+    "dskv_mixed_step": (c_int32, [POINTER(MixedStep)] + [c_void_p] * 6),
     "dskv_apply_rope": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                   c_int32, c_int32, c_int32, c_int32, c_int32, c_float, c_int32,
                                   c_void_p]),

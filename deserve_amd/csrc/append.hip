@@ -16,18 +16,24 @@
 // dependent loads, with kv_page_indptr and kv_last_page_len fetched by the same
 // lanes at the same time; the page id is the second link.  Batches over 63
 // requests take the binary search.
-#include "common.h"
+#include "rope_math.h"
 
 namespace dskv {
 
 constexpr int kAppendWaves = 4;
 constexpr int kAppendMaxChunks = 4;   // 16-byte chunks per lane and row set held in registers (row sets <= 4 KiB)
 
+// kRotate: K rows are rotated on their way (16-bit elements DT, head_dim 128).  `table` holds the
+// token's 64 cosines and 64 sines; a lane's chunks lie 64 apart, so all of them are chunk lane % 16
+// of a head and need the same four pairs.  Evaluating the angles here instead, as the stand-alone
+// RoPE kernel does, is work and a barrier in every layer for values that are the same in all.
+constexpr int kAppendRotatePairs = 64;   // dim pairs of a head
+template <int DT, bool kRotate>
 __global__ __launch_bounds__(64 * kAppendWaves) void append_kernel(
     char *__restrict__ pages, const char *__restrict__ k, const char *__restrict__ v,
     const int32_t *__restrict__ qo_indptr, const int32_t *__restrict__ kv_indices,
     const int32_t *__restrict__ kv_indptr, const int32_t *__restrict__ kv_last, int batch, int nnz,
-    int page_size, int row_bytes, int num_pages)
+    int page_size, int row_bytes, int num_pages, const float *__restrict__ table)
 {
     const int lane = threadIdx.x & 63;
     const int t = blockIdx.x * kAppendWaves + (threadIdx.x >> 6);
@@ -48,6 +54,25 @@ __global__ __launch_bounds__(64 * kAppendWaves) void append_kernel(
             }
         }
     }
+
+    float cs[4], sn[4];
+    if (kRotate) {
+        const float *tab = table + (long)t * (2 * kAppendRotatePairs) + (lane & 15) * 4;
+        const f32x4 c4 = *reinterpret_cast<const f32x4 *>(tab);
+        const f32x4 s4 = *reinterpret_cast<const f32x4 *>(tab + kAppendRotatePairs);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            cs[j] = c4[j];
+            sn[j] = s4[j];
+        }
+    }
+    auto k_chunk = [&](const u32x4 &raw) {
+        if (!kRotate) return raw;
+        float f[Chunk<DT>::kElems];
+        Chunk<DT>::unpack(raw, f);
+        rope_rotate<4>(f, cs, sn);
+        return Chunk<DT>::pack(f);
+    };
 
     // link 1: request that owns token t = largest b with qo_indptr[b] <= t
     int b, n_b, first, page_begin, n_pages, last;
@@ -97,7 +122,7 @@ __global__ __launch_bounds__(64 * kAppendWaves) void append_kernel(
         for (int i = 0; i < kAppendMaxChunks; i++) {
             const int off = (i * 64 + lane) * 16;
             if (off < row_bytes) {
-                __builtin_nontemporal_store(rk[i], reinterpret_cast<u32x4 *>(dst_k + off));
+                __builtin_nontemporal_store(k_chunk(rk[i]), reinterpret_cast<u32x4 *>(dst_k + off));
                 __builtin_nontemporal_store(rv[i], reinterpret_cast<u32x4 *>(dst_v + off));
             }
         }
@@ -105,22 +130,19 @@ __global__ __launch_bounds__(64 * kAppendWaves) void append_kernel(
         for (int off = lane * 16; off < row_bytes; off += 64 * 16) {
             u32x4 a = *reinterpret_cast<const u32x4 *>(src_k + off);
             u32x4 c = *reinterpret_cast<const u32x4 *>(src_v + off);
-            *reinterpret_cast<u32x4 *>(dst_k + off) = a;
+            *reinterpret_cast<u32x4 *>(dst_k + off) = k_chunk(a);
             *reinterpret_cast<u32x4 *>(dst_v + off) = c;
         }
     }
 }
 
-}  // namespace dskv
-
-extern "C" int dskv_append_paged_kv(void *pages_layer, int32_t num_pages, const void *k, const void *v,
-                                    const int32_t *qo_indptr, const int32_t *kv_page_indices,
-                                    const int32_t *kv_page_indptr, const int32_t *kv_last_page_len,
-                                    int32_t batch, int32_t nnz, int32_t page_size,
-                                    int32_t n_kv_heads, int32_t head_dim, int32_t elt_bytes,
-                                    void *stream)
+// rope_table null: the rows are copied as they are (elements of elt_bytes); else dtype is 16-bit.
+int launch_append(void *pages_layer, int32_t num_pages, const void *k, const void *v,
+                  const int32_t *qo_indptr, const int32_t *kv_page_indices, const int32_t *kv_page_indptr,
+                  const int32_t *kv_last_page_len, int32_t batch, int32_t nnz, int32_t page_size,
+                  int32_t n_kv_heads, int32_t head_dim, int32_t elt_bytes, const float *rope_table,
+                  int32_t dtype, hipStream_t stream)
 {
-    using namespace dskv;
     DSKV_REQUIRE(batch >= 0 && nnz >= 0, "append: negative batch/nnz (%d, %d)", batch, nnz);
     if (batch == 0 || nnz == 0) return 0;
     DSKV_REQUIRE(pages_layer && k && v && qo_indptr && kv_page_indices && kv_page_indptr &&
@@ -133,13 +155,35 @@ extern "C" int dskv_append_paged_kv(void *pages_layer, int32_t num_pages, const 
     DSKV_REQUIRE(row_bytes % 16 == 0 && row_bytes < (1 << 30),
                  "append: a token's row set (%lld bytes) must be a multiple of 16 bytes",
                  (long long)row_bytes);
-    DSKV_REQUIRE(((uintptr_t)pages_layer | (uintptr_t)k | (uintptr_t)v) % 16 == 0,
-                 "append: pages/k/v must be 16-byte aligned");
+    DSKV_REQUIRE(((uintptr_t)pages_layer | (uintptr_t)k | (uintptr_t)v | (uintptr_t)rope_table) % 16 == 0,
+                 "append: pages/k/v/table must be 16-byte aligned");
+    DSKV_REQUIRE(!rope_table || (elt_bytes == 2 && head_dim == 2 * kAppendRotatePairs &&
+                                 (dtype == DSKV_BF16 || dtype == DSKV_F16)),
+                 "append: rotation by a table takes 16-bit rows of head_dim %d", 2 * kAppendRotatePairs);
     const unsigned grid = (unsigned)((nnz + kAppendWaves - 1) / kAppendWaves);
-    hipLaunchKernelGGL(append_kernel, dim3(grid), dim3(64 * kAppendWaves), 0, (hipStream_t)stream,
-                       (char *)pages_layer, (const char *)k, (const char *)v, qo_indptr,
-                       kv_page_indices, kv_page_indptr, kv_last_page_len, batch, nnz, page_size,
-                       (int)row_bytes, num_pages);
+#define DSKV_LAUNCH_APPEND(DT, ROTATE)                                                                  \
+    hipLaunchKernelGGL((append_kernel<DT, ROTATE>), dim3(grid), dim3(64 * kAppendWaves), 0, stream,     \
+                       (char *)pages_layer, (const char *)k, (const char *)v, qo_indptr,                \
+                       kv_page_indices, kv_page_indptr, kv_last_page_len, batch, nnz, page_size,        \
+                       (int)row_bytes, num_pages, rope_table)
+    if (!rope_table) DSKV_LAUNCH_APPEND(DSKV_BF16, false);
+    else if (dtype == DSKV_BF16) DSKV_LAUNCH_APPEND(DSKV_BF16, true);
+    else DSKV_LAUNCH_APPEND(DSKV_F16, true);
+#undef DSKV_LAUNCH_APPEND
     DSKV_LAUNCH_CHECK("append_kernel");
     return 0;
+}
+
+}  // namespace dskv
+
+extern "C" int dskv_append_paged_kv(void *pages_layer, int32_t num_pages, const void *k, const void *v,
+                                    const int32_t *qo_indptr, const int32_t *kv_page_indices,
+                                    const int32_t *kv_page_indptr, const int32_t *kv_last_page_len,
+                                    int32_t batch, int32_t nnz, int32_t page_size,
+                                    int32_t n_kv_heads, int32_t head_dim, int32_t elt_bytes,
+                                    void *stream)
+{
+    return dskv::launch_append(pages_layer, num_pages, k, v, qo_indptr, kv_page_indices, kv_page_indptr,
+                               kv_last_page_len, batch, nnz, page_size, n_kv_heads, head_dim, elt_bytes,
+                               nullptr, DSKV_BF16, (hipStream_t)stream);
 }

@@ -62,7 +62,8 @@ int launch_partials_merge(void *out, const float *part_o, const float *part_ml,
 // entry `page_begin` of the table array, and its query and output are row `row` of q and out.
 // plan_decode_rows is dskv_decode_plan over such a list (same plan layout, the items name the
 // rows); decode_rows_attn is dskv_decode_attn over that plan, with row_map[i] = reqs[i].row on
-// the device for the merge pass.  decode_mfma_shape: whether the 16-bit decode kernel takes
+// the device for the merge pass; rope_table (may be null): the rows' angles, by query row, and q
+// is rotated as it is loaded.  decode_mfma_shape: whether the 16-bit decode kernel takes
 // the shape (the routing is only worth it then).
 struct DecodeRow {
     int64_t len;
@@ -77,8 +78,16 @@ int decode_rows_attn(void *out, const void *q, const void *pages_layer,
                      int32_t n_workgroups, void *workspace, int64_t workspace_bytes, int32_t n_rows,
                      const int32_t *row_map, int32_t n_qo_heads, int32_t n_kv_heads,
                      int32_t head_dim, int32_t page_size, float sm_scale, int32_t dtype,
-                     hipStream_t stream);
+                     const float *rope_table, hipStream_t stream);
 bool decode_mfma_shape(int head_dim, int n_qo_heads, int n_kv_heads, int page_size);
+
+// dskv_append_paged_kv, with K rotated on its way by rope_table (cosines | sines by token; may be
+// null) where the rows are 16-bit (dtype) and head_dim is 128.
+int launch_append(void *pages_layer, int32_t num_pages, const void *k, const void *v,
+                  const int32_t *qo_indptr, const int32_t *kv_page_indices, const int32_t *kv_page_indptr,
+                  const int32_t *kv_last_page_len, int32_t batch, int32_t nnz, int32_t page_size,
+                  int32_t n_kv_heads, int32_t head_dim, int32_t elt_bytes, const float *rope_table,
+                  int32_t dtype, hipStream_t stream);
 
 static inline bool is_pow2(int64_t x) { return x > 0 && (x & (x - 1)) == 0; }
 static inline int ilog2(int64_t x) {

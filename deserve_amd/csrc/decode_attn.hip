@@ -751,11 +751,11 @@ int decode_rows_attn(void *out, const void *q, const void *pages_layer,
                      int32_t n_workgroups, void *workspace, int64_t workspace_bytes, int32_t n_rows,
                      const int32_t *row_map, int32_t n_qo_heads, int32_t n_kv_heads,
                      int32_t head_dim, int32_t page_size, float sm_scale, int32_t dtype,
-                     hipStream_t stream)
+                     const float *rope_table, hipStream_t stream)
 {
     return decode_attn_impl(out, q, pages_layer, kv_page_indices, plan_dev, n_items, n_workgroups,
                             workspace, workspace_bytes, n_rows, n_qo_heads, n_kv_heads, head_dim,
-                            page_size, sm_scale, dtype, 3, stream, nullptr, nullptr, nullptr, row_map);
+                            page_size, sm_scale, dtype, 3, stream, nullptr, nullptr, rope_table, row_map);
 }
 
 int launch_partials_merge(void *out, const float *part_o, const float *part_ml,

@@ -181,6 +181,7 @@ struct MixedArgs {
     const int32_t *qo_indptr, *kv_indptr, *kv_last, *tile_info;
     float *tile_part_o, *tile_part_ml;
     int tile_max_slots, causal;
+    const float *rope;   // cos | sin by query row (q is rotated as it is loaded), or null
 };
 
 template <int DT, int kPagesPerTile>
@@ -194,13 +195,13 @@ __global__ __launch_bounds__(64 * kSharedWaves, 2) void mixed_attn_kernel(const 
         decode_attn_body<DT, kPagesPerTile, kSharedWaves, kSharedRing>(
             lds, wg / a.head_groups, wg % a.head_groups, a.out, a.q, a.pages, a.kv_indices, a.items, a.wg_ptr,
             a.dec_part_o, a.dec_part_ml, a.dec_max_slots, a.n_qo_heads, a.n_kv_heads, a.page_shift,
-            a.scale_log2, nullptr, nullptr, nullptr);
+            a.scale_log2, nullptr, nullptr, a.rope);
     else {
         __builtin_amdgcn_s_setprio(kSharedTilePriority);
         prefill_attn_body<DT, true, kPrefillWavesShared>(
             lds, wg - a.n_decode_wgs, a.out, a.q, a.qo_indptr, a.pages, a.kv_indices, a.kv_indptr, a.kv_last,
             a.tile_info, a.n_qo_heads, a.n_kv_heads, a.page_shift, a.scale_log2, a.causal,
-            a.tile_part_o, a.tile_part_ml, a.tile_max_slots);
+            a.tile_part_o, a.tile_part_ml, a.tile_max_slots, a.rope);
     }
 }
 
@@ -577,7 +578,7 @@ static int prefill_attn_impl(void *out, const void *q, const int32_t *qo_indptr,
                              void *workspace, int64_t workspace_bytes, int32_t batch, int32_t nnz,
                              int32_t n_qo_heads, int32_t n_kv_heads, int32_t head_dim,
                              int32_t page_size, float sm_scale, int32_t causal, int32_t dtype,
-                             void *stream, bool some_rows_elsewhere)
+                             void *stream, bool some_rows_elsewhere, const float *rope_table = nullptr)
 {
     DSKV_REQUIRE(batch >= 0 && nnz >= 0 && n_tiles >= 0, "prefill_attn: negative sizes");
     if (batch == 0 || nnz == 0) return 0;
@@ -627,7 +628,7 @@ static int prefill_attn_impl(void *out, const void *q, const int32_t *qo_indptr,
                        (const uint16_t *)q, qo_indptr, (const char *)pages_layer,               \
                        kv_page_indices, kv_page_indptr, kv_last_page_len, plan_dev,             \
                        n_qo_heads, n_kv_heads, shift, scale_log2, causal, part_o, part_ml,     \
-                       (int)max_slots)
+                       (int)max_slots, rope_table)
         if (dtype == DSKV_BF16) {
             if (page_size >= 4) DSKV_LAUNCH_PREFILL(DSKV_BF16, true);
             else DSKV_LAUNCH_PREFILL(DSKV_BF16, false);
@@ -641,6 +642,7 @@ static int prefill_attn_impl(void *out, const void *q, const int32_t *qo_indptr,
             return launch_parts_merge(out, part_o, part_ml, plan_dev + (int64_t)n_tiles * kTileWords, nnz,
                                       max_slots, n_qo_heads, dtype, s);
     } else {
+        DSKV_REQUIRE(!rope_table, "prefill_attn: only the 16-bit kernel rotates q");
         dim3 grid((unsigned)nnz, (unsigned)n_qo_heads);
 #define DSKV_LAUNCH_GEN(DT)                                                                      \
     hipLaunchKernelGGL((prefill_attn_generic_kernel<DT>), grid, dim3(64), 0, s, out, q, qo_indptr, \
@@ -675,7 +677,7 @@ static int mixed_shared_launch(void *out, const void *q, const int32_t *qo_indpt
                                const dskv_mixed_plan_t *info, void *workspace, int64_t workspace_bytes,
                                int32_t batch, int32_t nnz, int32_t n_qo_heads, int32_t n_kv_heads,
                                int32_t head_dim, int32_t page_size, float sm_scale, int32_t causal,
-                               int32_t dtype, hipStream_t s)
+                               int32_t dtype, const float *rope_table, hipStream_t s)
 {
     DSKV_REQUIRE(out && q && qo_indptr && pages_layer && kv_page_indices && kv_page_indptr && kv_last_page_len,
                  "mixed_attn: null pointer argument");
@@ -735,6 +737,7 @@ static int mixed_shared_launch(void *out, const void *q, const int32_t *qo_indpt
     a.kv_last = kv_last_page_len;
     a.tile_info = plan_dev;
     a.causal = causal;
+    a.rope = rope_table;
     const int64_t grid = (int64_t)a.n_decode_wgs + (int64_t)info->n_tiles * n_kv_heads;
     DSKV_REQUIRE(grid < (int64_t(1) << 31), "mixed_attn: too many workgroups");
     const dim3 g((unsigned)grid), b(64 * kSharedWaves);
@@ -786,16 +789,16 @@ extern "C" int dskv_prefill_attn(void *out, const void *q, const int32_t *qo_ind
                                    page_size, sm_scale, causal, dtype, stream, false);
 }
 
-extern "C" int dskv_mixed_attn(void *out, const void *q, const int32_t *qo_indptr,
-                               const void *pages_layer, const int32_t *kv_page_indices,
-                               const int32_t *kv_page_indptr, const int32_t *kv_last_page_len,
-                               const int32_t *plan_dev, const dskv_mixed_plan_t *info,
-                               void *workspace, int64_t workspace_bytes, int32_t batch, int32_t nnz,
-                               int32_t n_qo_heads, int32_t n_kv_heads, int32_t head_dim,
-                               int32_t page_size, float sm_scale, int32_t causal, int32_t dtype,
-                               void *stream)
+namespace dskv {
+
+static int mixed_attn_impl(void *out, const void *q, const int32_t *qo_indptr, const void *pages_layer,
+                           const int32_t *kv_page_indices, const int32_t *kv_page_indptr,
+                           const int32_t *kv_last_page_len, const int32_t *plan_dev,
+                           const dskv_mixed_plan_t *info, void *workspace, int64_t workspace_bytes,
+                           int32_t batch, int32_t nnz, int32_t n_qo_heads, int32_t n_kv_heads,
+                           int32_t head_dim, int32_t page_size, float sm_scale, int32_t causal,
+                           int32_t dtype, const float *rope_table, void *stream)
 {
-    using namespace dskv;
     DSKV_REQUIRE(info, "mixed_attn: null plan info");
     DSKV_REQUIRE(info->n_decode_rows >= 0 && info->n_tile_rows >= 0 && info->n_tiles >= 0 &&
                      info->tile_workspace_bytes >= 0 && info->decode_workspace_bytes >= 0,
@@ -810,7 +813,7 @@ extern "C" int dskv_mixed_attn(void *out, const void *q, const int32_t *qo_indpt
         return prefill_attn_impl(out, q, qo_indptr, pages_layer, kv_page_indices, kv_page_indptr,
                                  kv_last_page_len, plan_dev, info->n_tiles, info->n_splits, workspace,
                                  workspace_bytes, batch, nnz, n_qo_heads, n_kv_heads, head_dim,
-                                 page_size, sm_scale, causal, dtype, stream, false);
+                                 page_size, sm_scale, causal, dtype, stream, false, rope_table);
     DSKV_REQUIRE(plan_dev, "mixed_attn: missing plan");
     DSKV_REQUIRE(info->n_decode_rows + info->n_tile_rows == nnz && info->n_decode_rows <= batch,
                  "mixed_attn: the plan covers %d + %d rows, the batch has %d", info->n_decode_rows,
@@ -824,7 +827,7 @@ extern "C" int dskv_mixed_attn(void *out, const void *q, const int32_t *qo_indpt
         return mixed_shared_launch(out, q, qo_indptr, pages_layer, kv_page_indices, kv_page_indptr,
                                    kv_last_page_len, plan_dev, info, workspace, workspace_bytes, batch, nnz,
                                    n_qo_heads, n_kv_heads, head_dim, page_size, sm_scale, causal, dtype,
-                                   (hipStream_t)stream);
+                                   rope_table, (hipStream_t)stream);
     // The one-row requests: the split-KV decode pass (each K/V byte read once, at the speed
     // of memory) and its merge; their partials lie behind those of the tile parts.
     int rc = decode_rows_attn(out, q, pages_layer, kv_page_indices, plan_dev + info->decode_plan_at,
@@ -832,11 +835,56 @@ extern "C" int dskv_mixed_attn(void *out, const void *q, const int32_t *qo_indpt
                               workspace ? (char *)workspace + info->tile_workspace_bytes : nullptr,
                               workspace ? workspace_bytes - info->tile_workspace_bytes : 0,
                               info->n_decode_rows, plan_dev + info->row_map_at, n_qo_heads, n_kv_heads,
-                              head_dim, page_size, sm_scale, dtype, (hipStream_t)stream);
+                              head_dim, page_size, sm_scale, dtype, rope_table, (hipStream_t)stream);
     if (rc) return rc;
     // The others: query tiles (and the merge of their parts, over the tiled rows only).
     return prefill_attn_impl(out, q, qo_indptr, pages_layer, kv_page_indices, kv_page_indptr,
                              kv_last_page_len, plan_dev, info->n_tiles, info->n_splits, workspace,
                              info->tile_workspace_bytes, batch, nnz, n_qo_heads, n_kv_heads, head_dim,
-                             page_size, sm_scale, causal, dtype, stream, true);
+                             page_size, sm_scale, causal, dtype, stream, true, rope_table);
+}
+
+}  // namespace dskv
+
+extern "C" int dskv_mixed_attn(void *out, const void *q, const int32_t *qo_indptr,
+                               const void *pages_layer, const int32_t *kv_page_indices,
+                               const int32_t *kv_page_indptr, const int32_t *kv_last_page_len,
+                               const int32_t *plan_dev, const dskv_mixed_plan_t *info,
+                               void *workspace, int64_t workspace_bytes, int32_t batch, int32_t nnz,
+                               int32_t n_qo_heads, int32_t n_kv_heads, int32_t head_dim,
+                               int32_t page_size, float sm_scale, int32_t causal, int32_t dtype,
+                               void *stream)
+{
+    return dskv::mixed_attn_impl(out, q, qo_indptr, pages_layer, kv_page_indices, kv_page_indptr,
+                                 kv_last_page_len, plan_dev, info, workspace, workspace_bytes, batch, nnz,
+                                 n_qo_heads, n_kv_heads, head_dim, page_size, sm_scale, causal, dtype, nullptr,
+                                 stream);
+}
+
+extern "C" int dskv_mixed_step_supported(int32_t n_qo_heads, int32_t n_kv_heads, int32_t head_dim,
+                                         int32_t page_size, float sm_scale, int32_t dtype)
+{
+    using namespace dskv;
+    return n_qo_heads > 0 && n_kv_heads > 0 && n_qo_heads % n_kv_heads == 0 && page_size > 0 &&
+           is_pow2(page_size) &&
+           prefill_mfma_path(dtype, head_dim, n_qo_heads, n_kv_heads, sm_scale * 1.4426950408889634f);
+}
+
+extern "C" int dskv_mixed_step(const dskv_mixed_step_t *step, void *out, const void *q, const void *k_new,
+                               const void *v_new, void *pages_layer, void *stream)
+{
+    using namespace dskv;
+    DSKV_REQUIRE(step, "mixed_step: null step");
+    const dskv_mixed_step_t &s = *step;
+    DSKV_REQUIRE(dskv_mixed_step_supported(s.n_qo_heads, s.n_kv_heads, s.head_dim, s.page_size, s.sm_scale, s.dtype),
+                 "mixed_step: shape, scale or type outside the 16-bit kernels (see dskv_mixed_step_supported)");
+    DSKV_REQUIRE(s.info, "mixed_step: null plan info");
+    DSKV_REQUIRE((uintptr_t)s.rope_table % 16 == 0, "mixed_step: the table must be 16-byte aligned");
+    int rc = launch_append(pages_layer, s.num_pages, k_new, v_new, s.qo_indptr, s.kv_page_indices, s.kv_page_indptr,
+                           s.kv_last_page_len, s.batch, s.nnz, s.page_size, s.n_kv_heads, s.head_dim, 2,
+                           s.rope_table, s.dtype, (hipStream_t)stream);
+    if (rc) return rc;
+    return mixed_attn_impl(out, q, s.qo_indptr, pages_layer, s.kv_page_indices, s.kv_page_indptr, s.kv_last_page_len,
+                           s.plan_dev, s.info, s.workspace, s.workspace_bytes, s.batch, s.nnz, s.n_qo_heads,
+                           s.n_kv_heads, s.head_dim, s.page_size, s.sm_scale, s.causal, s.dtype, s.rope_table, stream);
 }

@@ -171,6 +171,36 @@ __global__ __launch_bounds__(256) void rope_table_kernel(float *__restrict__ tab
     table[(long)b * head_dim + pairs + pair] = sn;
 }
 
+// The same for the tokens of a ragged batch: row t holds the angles of token t's position,
+// offsets[b] + (t - qo_indptr[b]) for the request b that owns it.  A wave per token, a lane per pair.
+__global__ __launch_bounds__(256) void rope_table_ragged_kernel(float *__restrict__ table,
+                                                                const int32_t *__restrict__ qo_indptr,
+                                                                const int32_t *__restrict__ offsets,
+                                                                int batch, int nnz, int head_dim,
+                                                                float theta, RopeFreqs freqs)
+{
+    const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (t >= nnz) return;
+    int lo = 0, hi = batch;   // largest b with qo_indptr[b] <= t
+    if (batch < 64) {
+        const unsigned long long le = __ballot(lane <= batch && qo_indptr[min(lane, batch)] <= t);
+        lo = max(min(__popcll(le) - 1, batch - 1), 0);
+    } else {
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (qo_indptr[mid] <= t) lo = mid; else hi = mid;
+        }
+    }
+    const float pos = (float)(offsets[lo] + (t - qo_indptr[lo]));
+    const int pairs = head_dim / 2;
+    for (int pair = lane; pair < pairs; pair += 64) {
+        float cs, sn;
+        rope_angle(pos, pair, head_dim, theta, freqs, cs, sn);
+        table[(long)t * head_dim + pair] = cs;
+        table[(long)t * head_dim + pairs + pair] = sn;
+    }
+}
+
 static int launch_rope(void *q_out, void *k_out, const void *q, const void *k,
                        const int32_t *qo_indptr, const int32_t *offsets, int32_t batch, int32_t nnz,
                        int32_t n_qo_heads, int32_t n_kv_heads, int32_t head_dim, float rope_theta,
@@ -223,6 +253,25 @@ extern "C" int dskv_rope_table(float *table, const int32_t *positions, int32_t b
                        (hipStream_t)stream, table, positions, batch, head_dim, rope_theta,
                        rope_freqs(rope_theta, head_dim));
     DSKV_LAUNCH_CHECK("rope_table_kernel");
+    return 0;
+}
+
+extern "C" int dskv_rope_table_ragged(float *table, const int32_t *qo_indptr, const int32_t *offsets,
+                                      int32_t batch, int32_t nnz, int32_t head_dim, float rope_theta,
+                                      void *stream)
+{
+    using namespace dskv;
+    DSKV_REQUIRE(batch >= 0 && nnz >= 0, "rope_table: negative batch/nnz");
+    if (batch == 0 || nnz == 0) return 0;
+    DSKV_REQUIRE(table && qo_indptr && offsets, "rope_table: null pointer argument");
+    DSKV_REQUIRE(head_dim > 0 && head_dim % 8 == 0, "rope_table: head_dim %d must be a multiple of 8",
+                 head_dim);
+    DSKV_REQUIRE(rope_theta > 0.f, "rope_table: rope_theta must be positive");
+    DSKV_REQUIRE((uintptr_t)table % 16 == 0, "rope_table: the table must be 16-byte aligned");
+    hipLaunchKernelGGL(rope_table_ragged_kernel, dim3((unsigned)((nnz + 3) / 4)), dim3(256), 0,
+                       (hipStream_t)stream, table, qo_indptr, offsets, batch, nnz, head_dim, rope_theta,
+                       rope_freqs(rope_theta, head_dim));
+    DSKV_LAUNCH_CHECK("rope_table_ragged_kernel");
     return 0;
 }
 

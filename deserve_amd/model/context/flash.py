@@ -25,7 +25,7 @@ from deserve_amd.kvcache.paged.kvcache import PagedKVCache
 from deserve_amd.kvcache.paged.page_pool import GpuPagePool
 from deserve_amd.model.context.forward import PagedForwardCtx
 from deserve_amd.paged_ops import (BatchDecodeWithPagedKVCacheWrapper,
-                                   BatchPrefillWithPagedKVCacheWrapper)
+                                   BatchPrefillWithPagedKVCacheWrapper, rope_table)
 from deserve_amd.task import TaskData
 
 _FIELDS = ("indptr", "kv_page_indptr", "kv_last_page_lens", "offsets", "seqlens",
@@ -211,6 +211,14 @@ class FlashDecodeCtx(FlashForwardCtx):
 @dataclass
 class FlashPrefillCtx(FlashForwardCtx):
     prefill_wrapper: BatchPrefillWithPagedKVCacheWrapper = None   # type: ignore[assignment]
+    rope_tables: Dict[tuple, torch.Tensor] = field(default_factory=dict, repr=False)
+
+    def rope_table(self, nnz: int, head_dim: int, theta: float) -> torch.Tensor:
+        """The step's cosines and sines (paged_ops.rope_table), built for the first layer that asks."""
+        key = (nnz, head_dim, theta)
+        if key not in self.rope_tables:
+            self.rope_tables[key] = rope_table(self.indptr, self.offsets, nnz, head_dim, theta)
+        return self.rope_tables[key]
 
     @classmethod
     def init_paged_prefill_ctx(cls, task_datas: List[TaskData],

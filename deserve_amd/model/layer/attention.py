@@ -42,6 +42,13 @@ class PagedAttentionCore:
             rope = dict(rope_offsets=ctx.offsets, rope_theta=self.rope_theta) if self.use_rope else {}
             out = ctx.decode_wrapper.forward(xq, pages, k_append=xk, v_append=xv, out=out, **rope)
             return out.view(-1, self.dim)
+        if (isinstance(ctx, FlashPrefillCtx) and (self.fuse_rope_append or not self.use_rope)
+                and ctx.prefill_wrapper.fused_append_supported(xq.dtype)):
+            # k is rotated on its way into its slots, q as the attention loads it
+            table = ctx.rope_table(xq.shape[0], self.head_dim, self.rope_theta) if self.use_rope else None
+            out = ctx.prefill_wrapper.forward(xq, pages, causal=True, out=out, k_append=xk, v_append=xv,
+                                              rope_table=table)
+            return out.view(-1, self.dim)
         if self.use_rope and self.fuse_rope_append:
             # one kernel: rotated q comes back, rotated k and v go straight into their slots
             xq = rope_append_paged_kv_cache(xq, xk, xv, ctx.indptr, ctx.offsets, pages,

@@ -62,6 +62,18 @@ def apply_rope(q: torch.Tensor, k: torch.Tensor, indptr: torch.Tensor, offsets: 
     return q_out, k_out
 
 
+def rope_table(indptr: torch.Tensor, offsets: torch.Tensor, nnz: int, head_dim: int,
+               rope_theta: float = 1e4) -> torch.Tensor:
+    """(nnz, head_dim) floats, row t = cosines | sines of the angles apply_rope rotates token t by:
+    the same for every layer of a step."""
+    table = torch.empty((nnz, head_dim), dtype=torch.float32, device=indptr.device)
+    rc = _lib.lib().dskv_rope_table_ragged(
+        table.data_ptr(), _i32(indptr).data_ptr(), _i32(offsets).data_ptr(), indptr.shape[0] - 1, nnz, head_dim,
+        float(rope_theta), _lib.current_stream())
+    _lib.check(rc, "rope_table")
+    return table
+
+
 def rope_append_paged_kv_cache(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                                indptr: torch.Tensor, offsets: torch.Tensor,
                                paged_kv_data: torch.Tensor, kv_indices: torch.Tensor,
@@ -449,10 +461,24 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
         self._planned = True
         return dev[:meta_words]
 
+    def fused_append_supported(self, dtype: torch.dtype, sm_scale: Optional[float] = None) -> bool:
+        """Whether forward(..., k_append=, v_append=) takes the shape given to begin_forward."""
+        if dtype not in (torch.bfloat16, torch.float16):
+            return False
+        scale = 1.0 / math.sqrt(self._d) if sm_scale is None else sm_scale
+        return bool(_lib.lib().dskv_mixed_step_supported(self._hq, self._hkv, self._d, self._p, scale,
+                                                         _lib.dtype_code(dtype)))
+
     def forward(self, q: torch.Tensor, paged_kv_data: torch.Tensor, causal: bool = True,
                 sm_scale: Optional[float] = None, *, out: Optional[torch.Tensor] = None,
-                **_ignored) -> torch.Tensor:
-        """out: optional result tensor (contiguous, q's shape and dtype); every row is written."""
+                k_append: Optional[torch.Tensor] = None, v_append: Optional[torch.Tensor] = None,
+                rope_table: Optional[torch.Tensor] = None, **_ignored) -> torch.Tensor:
+        """out: optional result tensor (contiguous, q's shape and dtype); every row is written.
+        k_append, v_append (nnz, Hkv, D): the step's tokens, not yet in the pages - the call
+        appends them first (see fused_append_supported).
+        rope_table (with k_append / v_append): rope_table() of their positions; q and k_append are
+        then taken unrotated, k_append is rotated on its way into the pages and q as the attention
+        loads it."""
         if not self._planned:
             raise RuntimeError("prefill forward called before begin_forward")
         q = q.contiguous()
@@ -464,6 +490,27 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
         elif out.shape != q.shape or out.dtype != q.dtype or not out.is_contiguous():
             raise ValueError("out must be contiguous and of q's shape and dtype")
         scale = 1.0 / math.sqrt(self._d) if sm_scale is None else sm_scale
+        if k_append is not None or v_append is not None or rope_table is not None:
+            if k_append is None or v_append is None:
+                raise ValueError("the fused form takes both k_append and v_append")
+            k_append, v_append = k_append.contiguous(), v_append.contiguous()
+            want = (self._nnz, self._hkv, self._d)
+            if tuple(k_append.shape) != want or tuple(v_append.shape) != want or \
+                    k_append.dtype != q.dtype or v_append.dtype != q.dtype:
+                raise ValueError(f"k_append / v_append must be {want} of q's dtype")
+            if rope_table is not None and (tuple(rope_table.shape) != (self._nnz, self._d) or
+                                           rope_table.dtype != torch.float32 or not rope_table.is_contiguous()):
+                raise ValueError(f"rope_table must be a contiguous float32 ({self._nnz}, {self._d}) tensor")
+            step = _lib.MixedStep(
+                self._qo_indptr.data_ptr(), self._indices.data_ptr(), self._indptr.data_ptr(), self._last.data_ptr(),
+                self._tiles.data_ptr(), ctypes.pointer(self._info), self._workspace.data_ptr(),
+                self._workspace.numel() * self._workspace.element_size(), _lib.ptr(rope_table),
+                paged_kv_data.shape[0], self._batch, self._nnz, self._hq, self._hkv, self._d, self._p, int(causal),
+                _lib.dtype_code(q.dtype), scale)
+            rc = _lib.lib().dskv_mixed_step(ctypes.byref(step), out.data_ptr(), q.data_ptr(), k_append.data_ptr(),
+                                            v_append.data_ptr(), paged_kv_data.data_ptr(), _lib.current_stream())
+            _lib.check(rc, "prefill forward")
+            return out
         rc = _lib.lib().dskv_mixed_attn(
             out.data_ptr(), q.data_ptr(), self._qo_indptr.data_ptr(), paged_kv_data.data_ptr(),
             self._indices.data_ptr(), self._indptr.data_ptr(), self._last.data_ptr(),

@@ -185,6 +185,10 @@ int dskv_decode_append_attn(void *out, const void *q, const void *k_new, const v
  */
 int dskv_rope_table(float *table, const int32_t *positions, int32_t batch, int32_t head_dim,
                     float rope_theta, void *stream);
+/* The same for the tokens of a ragged batch: row t of (nnz, head_dim) holds the angles of position
+ * offsets[b] + (t - qo_indptr[b]), b the request that owns token t. */
+int dskv_rope_table_ragged(float *table, const int32_t *qo_indptr, const int32_t *offsets,
+                           int32_t batch, int32_t nnz, int32_t head_dim, float rope_theta, void *stream);
 int dskv_decode_rope_append_attn(void *out, const void *q, const void *k_new, const void *v_new,
                                  void *pages_layer, const int32_t *kv_page_indices,
                                  const int32_t *plan_dev, int32_t n_items, int32_t n_workgroups,
@@ -324,6 +328,29 @@ int dskv_mixed_attn(void *out, const void *q, const int32_t *qo_indptr, const vo
                     int32_t batch, int32_t nnz, int32_t n_qo_heads, int32_t n_kv_heads,
                     int32_t head_dim, int32_t page_size, float sm_scale, int32_t causal,
                     int32_t dtype, void *stream);
+
+/*
+ * A prefill or mixed step of a layer in one call: the append of the new tokens (k_new, v_new:
+ * (nnz, n_kv_heads, head_dim)) and dskv_mixed_attn, with everything that is the same for all layers
+ * of the step in one struct.  rope_table (dskv_rope_table_ragged; null: no rotation): k_new is rotated
+ * on its way into the pages and q as the attention loads it, with the arithmetic of dskv_apply_rope,
+ * so that no launch reads and writes q for the rotation alone.  For the shapes, scales and types that
+ * dskv_mixed_step_supported accepts (16-bit, head_dim 128, group <= 32, power-of-two page); others
+ * return DSKV_E_INVAL before anything is written.
+ */
+typedef struct dskv_mixed_step {
+    const int32_t *qo_indptr, *kv_page_indices, *kv_page_indptr, *kv_last_page_len, *plan_dev;
+    const dskv_mixed_plan_t *info;
+    void *workspace;
+    int64_t workspace_bytes;
+    const float *rope_table;
+    int32_t num_pages, batch, nnz, n_qo_heads, n_kv_heads, head_dim, page_size, causal, dtype;
+    float sm_scale;
+} dskv_mixed_step_t;
+int dskv_mixed_step_supported(int32_t n_qo_heads, int32_t n_kv_heads, int32_t head_dim,
+                              int32_t page_size, float sm_scale, int32_t dtype);
+int dskv_mixed_step(const dskv_mixed_step_t *step, void *out, const void *q, const void *k_new,
+                    const void *v_new, void *pages_layer, void *stream);
 
 /*
  * Rotary embedding, adjacent-pair convention.  Replaces the call site
