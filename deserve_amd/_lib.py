@@ -124,6 +124,7 @@ _SIGNATURES = {
     "dskv_swap_exchange_async": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                            c_int32, c_int32, c_int64, c_int64, c_void_p]),
     "dskv_swap_wait": (c_int32, [c_void_p]),
+    "dskv_swap_fence_pages": (c_int32, [c_void_p, c_void_p]),
     "dskv_swap_fence": (c_int32, [c_void_p, c_void_p]),
     "dskv_swap_query": (c_int32, [c_void_p, POINTER(c_int32)]),
     "dskv_swap_streams": (c_int32, [c_void_p, POINTER(c_void_p), POINTER(c_void_p)]),

@@ -156,6 +156,12 @@ class SwapEngine:
         """Make the current torch stream wait for everything enqueued so far."""
         _lib.check(_lib.lib().dskv_swap_fence(self._h, _lib.current_stream()), "swap_fence")
 
+    def fence_pages(self) -> None:
+        """Make the current torch stream wait until the pool is as the calls so far leave it: pages
+        swapped out have been packed, pages swapped in have arrived.  Host memory may still be
+        written; wait() and fence() wait for that too."""
+        _lib.check(_lib.lib().dskv_swap_fence_pages(self._h, _lib.current_stream()), "swap_fence_pages")
+
 
 def swap_slice(pool, page_begin: int, page_end: int, host_to: Optional[torch.Tensor],
                host_from: Optional[torch.Tensor], stream0: int, stream1: int) -> None:

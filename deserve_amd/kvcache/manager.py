@@ -7,8 +7,9 @@ layout (L * n, 2, P, Hkv, D) - layer major, then block-table order - and reload
 does the reverse into freshly allocated pages.  Both are enqueued on the swap
 engine's side streams (gather/scatter kernel + one large copy per staging
 chunk) instead of the reference's blocking advanced-index copy; ``synchronize``
-blocks the host until they are done, and the compute stream is fenced behind
-them so a caller that keeps the reference's call order sees the same results.
+blocks the host until they are done - a chunk holds its request's pages from
+then on - and the compute stream is fenced behind what the copies do to the pool,
+so a caller that keeps the reference's call order sees the same results.
 """
 from __future__ import annotations
 
@@ -41,8 +42,9 @@ class KVCacheManager:
         handle = self.cpu_chunk_pool.alloc(n)
         rows = n * self.cpu_chunk_pool.num_layers
         self.engine.swap_out(handle.retrieve()[:rows], self.virtual_page_pool, table.retrieve())
-        # pages may be handed to another request right after this returns
-        self.engine.fence()
+        # pages may be handed to another request right after this returns: they have been packed
+        # by the time the current stream goes on, and travel while it does
+        self.engine.fence_pages()
         return handle
 
     def copy_cpu_to_gpu(self, chunk_handle: ChunkHandle, task_id: str) -> VirtualPagedKVCache:
@@ -56,7 +58,7 @@ class KVCacheManager:
         table.extend(ids)
         rows = n * self.cpu_chunk_pool.num_layers
         self.engine.swap_in(pool, chunk_handle.retrieve()[:rows], ids)
-        self.engine.fence()   # attention on the current stream must see the pages
+        self.engine.fence_pages()   # attention on the current stream must see the pages
         isswap = torch.zeros((self.page_table_allocator.max_context_len,), dtype=torch.bool)
         isswap[:n] = ids >= pool.num_pages_main
         return VirtualPagedKVCache(page_table=table, isswap=isswap, pool=pool)

@@ -400,7 +400,10 @@ int dskv_swap_slice(void *slice_base, int64_t layer_stride_bytes, int64_t slice_
  * time, into a ring of 2^20 ids that in-flight calls hold until they have run: a call that
  * finds the ring full is refused with DSKV_E_STATE - nothing in these calls waits); ids
  * outside a layer are refused with DSKV_E_INVAL.  after_stream: work already enqueued
- * there is waited for (on the device) before the pool is touched.  dskv_swap_wait blocks
+ * there is waited for (on the device) before the pool is touched.  The calls' accesses to the
+ * pool, and to host memory that two calls share, keep the order of the calls; beyond that a
+ * swap-in's trip over the link runs beside those of the swap-outs before it.  Out staging is
+ * four chunks of staging_bytes, at most 512 MiB (or one chunk).  dskv_swap_wait blocks
  * the host until everything enqueued on the handle is done; dskv_swap_fence makes `stream`
  * wait for it instead.
  */
@@ -426,6 +429,12 @@ int dskv_swap_exchange_async(dskv_swap_t *handle, void *host_dst, const void *ho
                              int64_t layer_stride_bytes, int64_t page_bytes, void *after_stream);
 int dskv_swap_wait(dskv_swap_t *handle);
 int dskv_swap_fence(dskv_swap_t *handle, void *stream);
+/*
+ * As dskv_swap_fence, but only until the pool is as the calls so far leave it: pages swapped out
+ * have been packed (and may be overwritten), pages swapped in have arrived.  The packed pages may
+ * still be on their way to host memory; dskv_swap_wait or dskv_swap_fence wait for that.
+ */
+int dskv_swap_fence_pages(dskv_swap_t *handle, void *stream);
 /* Non-blocking: *done_out = 1 if everything enqueued on the handle has finished, else 0. */
 int dskv_swap_query(dskv_swap_t *handle, int32_t *done_out);
 /*

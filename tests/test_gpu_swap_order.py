@@ -1,0 +1,58 @@
+"""Swap-outs and swap-ins travel beside each other but act on the pool, and on host memory they
+share, in the order of the calls: seeded sequences of calls and of kernels that overwrite pages
+behind fence_pages(), against the same sequence on numpy arrays.  Staging of 1 MiB (a ring of 4)
+under transfers of up to 3 MiB: chunks, wraps and stretches that wait for their copy."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import kv_oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("seed", range(4))
+def test_calls_act_in_order(seed):
+    from deserve_amd.kvcache import _native
+    from deserve_amd.kvcache.paged.page_pool import GpuPagePool
+    from deserve_amd.kvcache.pinned.pinned_memory import pinned_empty
+
+    print("[case] swap order", seed, flush=True)
+    L, P, num_pages, most = 3, 16, 40, 16
+    pool = GpuPagePool(L, num_pages, P, "cuda", torch.bfloat16)
+    rng = np.random.default_rng(seed)
+    bits = lambda t: t.view(torch.int16).cpu().numpy()
+    pool.pages.view(torch.int16).random_(0, 1 << 15)
+    model = bits(pool.pages).copy()
+    hosts = [pinned_empty((L * most,) + tuple(pool.pages.shape[2:]), torch.bfloat16) for _ in range(4)]
+    for h in hosts:
+        h.view(torch.int16).copy_(torch.from_numpy(rng.integers(0, 1 << 15, h.shape).astype(np.int16)))
+    images = [bits(h).copy() for h in hosts]
+    eng = _native.SwapEngine(1 << 20)
+    for step in range(60):
+        what = rng.choice(["out", "in", "exchange", "write"], p=[0.42, 0.42, 0.04, 0.12])
+        n, a, b = int(rng.integers(1, most + 1)), int(rng.integers(4)), int(rng.integers(4))
+        ids = rng.permutation(num_pages)[:n].astype(np.int32)
+        tids = torch.from_numpy(ids)
+        if what == "out":
+            eng.swap_out(hosts[a][: L * n], pool, tids)
+            images[a][: L * n] = orc.gather_pages(model, ids)
+        elif what == "in":
+            eng.swap_in(pool, hosts[a][: L * n], tids)
+            orc.scatter_pages(model, ids, images[a][: L * n])
+        elif what == "exchange":
+            eng.exchange(hosts[a][: L * n], hosts[b][: L * n], pool, tids)
+            out = orc.gather_pages(model, ids)
+            if a != b:
+                orc.scatter_pages(model, ids, images[b][: L * n])
+            images[a][: L * n] = out
+        else:
+            eng.fence_pages()      # then the current stream may write pages
+            pool.pages.view(torch.int16)[:, int(ids[0])] = step
+            model[:, int(ids[0])] = step
+    eng.wait()
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(pool.pages), model)
+    for h, image in zip(hosts, images):
+        assert np.array_equal(bits(h), image)
+    eng.close()
