@@ -762,16 +762,17 @@ int launch_partials_merge(void *out, const float *part_o, const float *part_ml,
                           const int32_t *row_parts, const int32_t *row_map, int max_slots, int rows,
                           int n_qo_heads, int head_dim, int dtype, bool wide, hipStream_t s)
 {
-    // rows in a few parts, 16-bit output, head_dim 128: a workgroup per row that requests all
-    // parts at once - half the time of a wave per (row, head) on the 512 rows of a chunk, the
-    // same 4.7 us on a decode batch's 64 requests in 317 parts (about what any launch that
-    // reads what the launch before it wrote takes)
+    // rows in a few parts, 16-bit output, head_dim 128: a workgroup per (row, eight heads) that
+    // requests all parts at once - half the time of a wave per (row, head) on the 512 rows of a
+    // chunk; 4.9 us on a decode batch's 64 requests in 317 parts is about what any launch that
+    // reads what the launch before it wrote takes
     if (!wide && head_dim == kHeadDim && dtype != DSKV_F32) {
+        const dim3 grid((unsigned)rows, (unsigned)((n_qo_heads + kMergeHeads - 1) / kMergeHeads));
         if (dtype == DSKV_BF16)
-            hipLaunchKernelGGL((merge_parts_kernel<DSKV_BF16>), dim3((unsigned)rows), dim3(256), 0, s,
+            hipLaunchKernelGGL((merge_parts_kernel<DSKV_BF16>), grid, dim3(kMergeThreads), 0, s,
                                (uint16_t *)out, part_o, part_ml, row_parts, row_map, max_slots, n_qo_heads);
         else
-            hipLaunchKernelGGL((merge_parts_kernel<DSKV_F16>), dim3((unsigned)rows), dim3(256), 0, s,
+            hipLaunchKernelGGL((merge_parts_kernel<DSKV_F16>), grid, dim3(kMergeThreads), 0, s,
                                (uint16_t *)out, part_o, part_ml, row_parts, row_map, max_slots, n_qo_heads);
         DSKV_LAUNCH_CHECK("merge_parts_kernel");
         return 0;
