@@ -24,16 +24,27 @@ class PagedAttentionCore:
         self.fuse_rope_append = fuse_rope_append
         self.fuse_decode_append = fuse_decode_append
 
-    @torch.inference_mode()
     def paged_forward(self, xq: torch.Tensor, xk: torch.Tensor, xv: torch.Tensor,
                       ctx: FlashForwardCtx, out: Optional[torch.Tensor] = None) -> torch.Tensor:
         """out: where the result goes (contiguous, one row of Hq * D per token); None: a tensor of
         its own."""
+        if torch.is_inference_mode_enabled():      # entering it again costs every layer 3 us
+            return self._paged_forward(xq, xk, xv, ctx, out)
+        with torch.inference_mode():
+            return self._paged_forward(xq, xk, xv, ctx, out)
+
+    def _rows(self, x: torch.Tensor, heads: int) -> torch.Tensor:
+        """x as (tokens, heads, head_dim)."""
+        s = x.shape
+        return x if len(s) == 3 and s[1] == heads and s[2] == self.head_dim else x.view(-1, heads, self.head_dim)
+
+    def _paged_forward(self, xq: torch.Tensor, xk: torch.Tensor, xv: torch.Tensor,
+                       ctx: FlashForwardCtx, out: Optional[torch.Tensor]) -> torch.Tensor:
         if out is not None:
-            out = out.view(-1, self.n_local_heads, self.head_dim)
-        xq = xq.view(-1, self.n_local_heads, self.head_dim)
-        xk = xk.view(-1, self.n_local_kv_heads, self.head_dim)
-        xv = xv.view(-1, self.n_local_kv_heads, self.head_dim)
+            out = self._rows(out, self.n_local_heads)
+        xq = self._rows(xq, self.n_local_heads)
+        xk = self._rows(xk, self.n_local_kv_heads)
+        xv = self._rows(xv, self.n_local_kv_heads)
         pages = ctx.page_pool.get_layered_pages(ctx.layer_id)
         if (isinstance(ctx, FlashDecodeCtx) and self.fuse_decode_append and xk.shape[0] == ctx.bsz
                 and ctx.decode_wrapper.fused_append_supported(xq.dtype)):

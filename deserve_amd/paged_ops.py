@@ -10,12 +10,25 @@ stream.  ``pages`` is one layer of the pool: (num_pages, 2, page_size, Hkv, D).
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 from typing import Optional, Tuple
 
+import numpy as np
 import torch
 
 from deserve_amd import _lib, staging
+
+
+@functools.lru_cache(maxsize=256)
+def _decode_append_supported(n_qo_heads: int, n_kv_heads: int, head_dim: int, page_size: int, dtype: int) -> bool:
+    return bool(_lib.lib().dskv_decode_append_attn_supported(n_qo_heads, n_kv_heads, head_dim, page_size, dtype))
+
+
+@functools.lru_cache(maxsize=256)
+def _mixed_step_supported(n_qo_heads: int, n_kv_heads: int, head_dim: int, page_size: int, scale: float,
+                          dtype: int) -> bool:
+    return bool(_lib.lib().dskv_mixed_step_supported(n_qo_heads, n_kv_heads, head_dim, page_size, scale, dtype))
 
 
 def _i32(t: torch.Tensor) -> torch.Tensor:
@@ -126,21 +139,22 @@ class _PagedWrapper:
         are shorter than indptr says or hold a negative id, last-page lengths that are missing
         or outside [1, page_size], and remember the largest id so that forward() can refuse a
         pool that does not have that page."""
-        batch = h_indptr.shape[0] - 1
-        used = int(h_indptr[-1]) if batch > 0 else 0
-        if batch > 0 and (int(h_indptr[0]) != 0 or bool((h_indptr[1:] < h_indptr[:-1]).any())):
+        ptr = h_indptr.numpy()
+        batch = ptr.shape[0] - 1
+        used = int(ptr[-1]) if batch > 0 else 0
+        if batch > 0 and (ptr[0] != 0 or (ptr[1:] < ptr[:-1]).any()):
             raise ValueError("kv page indptr must start at 0 and not decrease")
         if h_last.numel() < max(batch, 0):
             raise ValueError(f"kv last-page lengths hold {h_last.numel()} entries for {batch} requests")
         if batch > 0:
-            last = h_last[:batch]
-            bad = (h_indptr[1:] > h_indptr[:-1]) & ((last < 1) | (last > self._p))
-            if bool(bad.any()):
-                b = int(bad.nonzero()[0])
+            last = h_last.numpy()[:batch]
+            bad = (ptr[1:] > ptr[:-1]) & ((last < 1) | (last > self._p))
+            if bad.any():
+                b = int(bad.argmax())
                 raise ValueError(f"kv_last_page_len[{b}] = {int(last[b])} outside [1, {self._p}]")
         if indices.numel() < used:
             raise ValueError(f"kv page indices hold {indices.numel()} entries, indptr[-1] is {used}")
-        ids = self._host(indices, indices_host)[:used]
+        ids = self._host(indices, indices_host).numpy()[:used]
         if indices_host is not None and indices_host.numel() < used:
             raise ValueError(f"indices_host holds {indices_host.numel()} entries, indptr[-1] is {used}")
         self._max_page_id = -1
@@ -151,13 +165,13 @@ class _PagedWrapper:
             self._max_page_id = hi
 
     def _check_pool(self, paged_kv_data: torch.Tensor, dtype: torch.dtype) -> None:
-        want = (2, self._p, self._hkv, self._d)
-        if paged_kv_data.dim() != 5 or tuple(paged_kv_data.shape[1:]) != want:
+        want, shape = (2, self._p, self._hkv, self._d), paged_kv_data.shape
+        if len(shape) != 5 or shape[1:] != want:
             raise ValueError(f"paged_kv_data must be (num_pages, {', '.join(map(str, want))}) as given to "
                              f"begin_forward, got {tuple(paged_kv_data.shape)}")
         if not paged_kv_data.is_contiguous() or paged_kv_data.dtype != dtype:
             raise ValueError("paged_kv_data must be contiguous and of q's dtype")
-        if self._max_page_id >= paged_kv_data.shape[0]:
+        if self._max_page_id >= shape[0]:
             raise ValueError(f"the block tables name page {self._max_page_id}, the pool has "
                              f"{paged_kv_data.shape[0]} pages")
 
@@ -238,8 +252,8 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
         self._batch, self._n_items, self._n_workgroups = batch, n_items.value, n_wgs.value
         self._rope_table, self._rope_key = None, None     # positions change with the step
         # requests without a page: the fused append has no slot to write their token to
-        n_pages = h_indptr[1:] - h_indptr[:-1]
-        self._empty_requests = [int(b) for b in (n_pages <= 0).nonzero().flatten()[:4]] if batch > 0 else []
+        ptr = h_indptr.numpy()
+        self._empty_requests = np.flatnonzero(ptr[1:] <= ptr[:-1])[:4].tolist() if batch > 0 else []
         return int(words.value)
 
     def begin_forward_with_metadata(self, meta_words: int, fill_metadata, indptr_at: int, indices_at: int,
@@ -277,8 +291,7 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
         the shape given to begin_forward."""
         if dtype not in (torch.bfloat16, torch.float16):
             return False
-        return bool(_lib.lib().dskv_decode_append_attn_supported(self._hq, self._hkv, self._d, self._p,
-                                                                 _lib.dtype_code(dtype)))
+        return _decode_append_supported(self._hq, self._hkv, self._d, self._p, _lib.dtype_code(dtype))
 
     def forward(self, q: torch.Tensor, paged_kv_data: torch.Tensor,
                 sm_scale: Optional[float] = None, *, phases: int = 3,
@@ -296,7 +309,7 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
         if not self._planned:
             raise RuntimeError("decode forward called before begin_forward")
         q = q.contiguous()
-        if tuple(q.shape) != (self._batch, self._hq, self._d):
+        if q.shape != (self._batch, self._hq, self._d):
             raise ValueError(f"q must be ({self._batch}, {self._hq}, {self._d}), got {tuple(q.shape)}")
         self._check_pool(paged_kv_data, q.dtype)
         if out is None:
@@ -314,7 +327,7 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
                                  "(kv length 0 after the append); extend the caches before begin_forward")
             k_append, v_append = k_append.contiguous(), v_append.contiguous()
             want = (self._batch, self._hkv, self._d)
-            if tuple(k_append.shape) != want or tuple(v_append.shape) != want or \
+            if k_append.shape != want or v_append.shape != want or \
                     k_append.dtype != q.dtype or v_append.dtype != q.dtype:
                 raise ValueError(f"k_append / v_append must be {want} of q's dtype")
             if rope_offsets is not None:
@@ -329,7 +342,7 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
                     self._rope_table, self._rope_key = table, key
                 table = self._rope_table.data_ptr()
         if phases == 3:
-            step = self._step
+            step = _lib.DecodeStep.from_buffer_copy(self._step)    # calls from several threads do not share it
             step.rope_table, step.dtype, step.sm_scale = table, _lib.dtype_code(q.dtype), scale
             rc = _lib.lib().dskv_decode_step(ctypes.byref(step), out.data_ptr(), q.data_ptr(), _lib.ptr(k_append),
                                              _lib.ptr(v_append), paged_kv_data.data_ptr(), _lib.current_stream())
@@ -389,13 +402,22 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
         block = staging.take(max(cap, 4))
         words = self._plan_into(block.tensor, cap, h_qo, h_kv, h_last, target_workgroups, route_one_row_requests)
         self._tiles = staging.to_device(block, max(words, 4), paged_kv_indices.device)
+        self._bind_step()
+
+    def _bind_step(self) -> None:
+        """What all layers of the planned step share, for dskv_mixed_step."""
+        self._step = _lib.MixedStep(
+            self._qo_indptr.data_ptr(), self._indices.data_ptr(), self._indptr.data_ptr(), self._last.data_ptr(),
+            self._tiles.data_ptr(), ctypes.pointer(self._info), self._workspace.data_ptr(),
+            self._workspace.numel() * self._workspace.element_size(), None, 0, self._batch, self._nnz, self._hq,
+            self._hkv, self._d, self._p)
         self._planned = True
 
     def _check_and_bound(self, h_qo: torch.Tensor, h_kv: torch.Tensor, h_last: torch.Tensor,
                          indices: torch.Tensor, indices_host: Optional[torch.Tensor]):
         """Host-side checks of the index arrays; returns the words the plan may need."""
-        batch = h_qo.shape[0] - 1
-        if batch > 0 and (int(h_qo[0]) != 0 or bool((h_qo[1:] < h_qo[:-1]).any())):
+        batch, qo = h_qo.shape[0] - 1, h_qo.numpy()
+        if batch > 0 and (qo[0] != 0 or (qo[1:] < qo[:-1]).any()):
             raise ValueError("qo_indptr must start at 0 and not decrease")
         if h_kv.shape[0] != h_qo.shape[0]:
             raise ValueError("qo_indptr and paged_kv_indptr disagree about the batch")
@@ -458,7 +480,7 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
         self._indptr = dev[starts["kv_page_indptr"]: starts["kv_page_indptr"] + batch + 1]
         self._indices = dev[starts["kv_page_indices"]: starts["kv_page_indices"] + used]
         self._last = dev[starts["kv_last_page_lens"]: starts["kv_last_page_lens"] + batch]
-        self._planned = True
+        self._bind_step()
         return dev[:meta_words]
 
     def fused_append_supported(self, dtype: torch.dtype, sm_scale: Optional[float] = None) -> bool:
@@ -466,8 +488,7 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
         if dtype not in (torch.bfloat16, torch.float16):
             return False
         scale = 1.0 / math.sqrt(self._d) if sm_scale is None else sm_scale
-        return bool(_lib.lib().dskv_mixed_step_supported(self._hq, self._hkv, self._d, self._p, scale,
-                                                         _lib.dtype_code(dtype)))
+        return _mixed_step_supported(self._hq, self._hkv, self._d, self._p, scale, _lib.dtype_code(dtype))
 
     def forward(self, q: torch.Tensor, paged_kv_data: torch.Tensor, causal: bool = True,
                 sm_scale: Optional[float] = None, *, out: Optional[torch.Tensor] = None,
@@ -482,7 +503,7 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
         if not self._planned:
             raise RuntimeError("prefill forward called before begin_forward")
         q = q.contiguous()
-        if tuple(q.shape) != (self._nnz, self._hq, self._d):
+        if q.shape != (self._nnz, self._hq, self._d):
             raise ValueError(f"q must be ({self._nnz}, {self._hq}, {self._d}), got {tuple(q.shape)}")
         self._check_pool(paged_kv_data, q.dtype)
         if out is None:
@@ -495,18 +516,16 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
                 raise ValueError("the fused form takes both k_append and v_append")
             k_append, v_append = k_append.contiguous(), v_append.contiguous()
             want = (self._nnz, self._hkv, self._d)
-            if tuple(k_append.shape) != want or tuple(v_append.shape) != want or \
+            if k_append.shape != want or v_append.shape != want or \
                     k_append.dtype != q.dtype or v_append.dtype != q.dtype:
                 raise ValueError(f"k_append / v_append must be {want} of q's dtype")
-            if rope_table is not None and (tuple(rope_table.shape) != (self._nnz, self._d) or
+            if rope_table is not None and (rope_table.shape != (self._nnz, self._d) or
                                            rope_table.dtype != torch.float32 or not rope_table.is_contiguous()):
                 raise ValueError(f"rope_table must be a contiguous float32 ({self._nnz}, {self._d}) tensor")
-            step = _lib.MixedStep(
-                self._qo_indptr.data_ptr(), self._indices.data_ptr(), self._indptr.data_ptr(), self._last.data_ptr(),
-                self._tiles.data_ptr(), ctypes.pointer(self._info), self._workspace.data_ptr(),
-                self._workspace.numel() * self._workspace.element_size(), _lib.ptr(rope_table),
-                paged_kv_data.shape[0], self._batch, self._nnz, self._hq, self._hkv, self._d, self._p, int(causal),
-                _lib.dtype_code(q.dtype), scale)
+            step = _lib.MixedStep.from_buffer_copy(self._step)
+            step.rope_table = None if rope_table is None else rope_table.data_ptr()
+            step.num_pages, step.causal = paged_kv_data.shape[0], int(causal)
+            step.dtype, step.sm_scale = _lib.dtype_code(q.dtype), scale
             rc = _lib.lib().dskv_mixed_step(ctypes.byref(step), out.data_ptr(), q.data_ptr(), k_append.data_ptr(),
                                             v_append.data_ptr(), paged_kv_data.data_ptr(), _lib.current_stream())
             _lib.check(rc, "prefill forward")
