@@ -47,6 +47,9 @@ constexpr bool kSumOnMfma = DSKV_PREFILL_SUM_ON_MFMA;   // row sums of P by the 
 //   C/D: column r, rows 8i + 4h + j in register 4i + j (i, j = 0..3).
 // LDS of one workgroup: four stages of K rows, then four of V rows.
 constexpr int kPrefillLdsBytes = 8 * kStageBytes;
+// ... and, at the end, 256 bytes of each of a wave's columns (16 bytes of padding between them)
+constexpr int kRowsOutPitch = 256 + 16;
+constexpr int kRowsOutBytes = 32 * kRowsOutPitch;
 struct LdsStages {
     char *base;
     __device__ __forceinline__ char *operator[](int i) const { return base + i * kStageBytes; }
@@ -192,22 +195,11 @@ __device__ __forceinline__ void prefill_attn_body(
     // A tile cut into parts: every part leaves (max, sum, unnormalised O) of its rows in the
     // workspace (O blocks of all slots, then their (max, sum) pairs); a part that sees nothing
     // leaves zeros and a maximum below any real one.
-    auto store_partial = [&](int ct, float m, float l) {
-        const long slot = (long)first_slot + (long)(qrow[ct] - q0) * tile_parts + split;
-        if (slot >= max_slots) return;   // a slot beyond the workspace is never written
-        const long qh = (long)kvh * group + c_head[ct];
-        float *o = part_o + (slot * n_qo_heads + qh) * kHeadDim + 4 * h;
-#pragma unroll
-        for (int dt = 0; dt < 4; dt++)
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                *reinterpret_cast<f32x4 *>(o + dt * 32 + 8 * i) =
-                    f32x4{acc[ct][dt][4 * i], acc[ct][dt][4 * i + 1], acc[ct][dt][4 * i + 2], acc[ct][dt][4 * i + 3]};
-        if (h == 0) {
-            float *ml = part_ml + (slot * n_qo_heads + qh) * 2;
-            ml[0] = m;
-            ml[1] = l;
-        }
+    auto slot_of = [&](int ct) { return (long)first_slot + (long)(qrow[ct] - q0) * tile_parts + split; };
+    auto store_max_sum = [&](int ct, float m, float l) {
+        float *ml = part_ml + (slot_of(ct) * n_qo_heads + (long)kvh * group + c_head[ct]) * 2;
+        ml[0] = m;
+        ml[1] = l;
     };
     // No kv token of this part visible to any row of the tile: the output rows are zero
     // (or the part is empty).  Uniform over the workgroup, and before the first barrier.
@@ -216,7 +208,11 @@ __device__ __forceinline__ void prefill_attn_body(
         for (int ct = 0; ct < kColTiles; ct++) {
             if (!live[ct]) continue;
             if (partial) {
-                store_partial(ct, m_run[ct], 0.f);
+                if (slot_of(ct) >= max_slots) continue;   // a slot beyond the workspace is never written
+                float *o = part_o + (slot_of(ct) * n_qo_heads + (long)kvh * group + c_head[ct]) * kHeadDim + 4 * h;
+#pragma unroll
+                for (int i = 0; i < 16; i++) *reinterpret_cast<f32x4 *>(o + 8 * i) = f32x4{0.f, 0.f, 0.f, 0.f};
+                if (h == 0) store_max_sum(ct, m_run[ct], 0.f);
                 continue;
             }
             uint16_t *o = out + ((long)(q_begin + qrow[ct]) * n_qo_heads + (long)kvh * group + c_head[ct]) * kHeadDim +
@@ -596,6 +592,29 @@ __device__ __forceinline__ void prefill_attn_body(
     if (kRowsSharePage) DSKV_WAIT_VMEM(0);   // nothing of this wave may still be on its way into LDS
 #undef DSKV_WAIT_VMEM
 
+    // The rows leave through LDS, a stretch of the stages per wave: a lane holds four dims here and
+    // four there of one column, and stored from the registers every instruction touched 32 rows,
+    // 16 bytes (of the 16-bit output) or 32 (of a partial) of each.  Laid out by column, 16 lanes
+    // store 256 consecutive bytes: the launch of three short prompts 17.5 -> 15.3 us, the step of a
+    // chunk of 512 tokens in four parts (16 layers) 944 -> 920.
+    __syncthreads();   // the stages have been read by everybody
+    char *const rows_lds = lds_base + wave * kRowsOutBytes;
+    static_assert(kWaves * kRowsOutBytes <= kPrefillLdsBytes, "a stretch per wave");
+    // 256 bytes of every column from rows_lds to base + row * row_bytes + at, `row` being the lane's own
+    // column's row there (negative: none); any lane may hold any column's bytes
+    auto store_columns = [&](char *base, int row, int row_bytes, int at) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int col = 4 * j + g, to = __shfl(row, col);
+            const u32x4 w = *reinterpret_cast<const u32x4 *>(rows_lds + col * kRowsOutPitch + c * 16);
+            if (to < 0) continue;
+            u32x4 *const dst = reinterpret_cast<u32x4 *>(base + (long)to * row_bytes + at + c * 16);
+            *dst = w;
+        }
+        __builtin_amdgcn_wave_barrier();
+    };
 #pragma unroll
     for (int ct = 0; ct < kColTiles; ct++) {
         float l = l_acc[ct][0];   // summed over all tokens by the MFMA (both lane halves)
@@ -604,22 +623,36 @@ __device__ __forceinline__ void prefill_attn_body(
             swap_halves32(l_run[ct], l_other);
             l = l_run[ct] + l_other;
         }
-        if (!live[ct]) continue;
-        if (partial) {
-            store_partial(ct, m_run[ct], l);
+        char *const mine = rows_lds + r * kRowsOutPitch;
+        if (partial) {   // (max, sum, unnormalised O) of the row into its slot, 64 dims at a time
+            const int slot = (qrow[ct] - q0) * tile_parts + split, qh = kvh * group + c_head[ct];   // from first_slot
+            const bool held = live[ct] && first_slot + (long)slot < max_slots;   // never beyond the workspace
+            char *const o = reinterpret_cast<char *>(part_o + (long)first_slot * n_qo_heads * kHeadDim);
+#pragma unroll
+            for (int half = 0; half < 2; half++) {
+#pragma unroll
+                for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const f32x16 &a = acc[ct][2 * half + dt];
+                        *reinterpret_cast<f32x4 *>(mine + (dt * 32 + 8 * i + 4 * h) * 4) =
+                            f32x4{a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3]};
+                    }
+                store_columns(o, held ? slot * n_qo_heads + qh : -1, kHeadDim * 4, half * 256);
+            }
+            if (held && h == 0) store_max_sum(ct, m_run[ct], l);
             continue;
         }
         const float inv = l > 0.f ? 1.f / l : 0.f;
-        uint16_t *o = out + ((long)(q_begin + qrow[ct]) * n_qo_heads + (long)kvh * group + c_head[ct]) * kHeadDim +
-                      4 * h;
 #pragma unroll
         for (int dt = 0; dt < 4; dt++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                u32x2 w = {E::pack2(acc[ct][dt][4 * i] * inv, acc[ct][dt][4 * i + 1] * inv),
-                           E::pack2(acc[ct][dt][4 * i + 2] * inv, acc[ct][dt][4 * i + 3] * inv)};
-                *reinterpret_cast<u32x2 *>(o + dt * 32 + 8 * i) = w;
-            }
+            for (int i = 0; i < 4; i++)
+                *reinterpret_cast<u32x2 *>(mine + (dt * 32 + 8 * i + 4 * h) * 2) =
+                    u32x2{E::pack2(acc[ct][dt][4 * i] * inv, acc[ct][dt][4 * i + 1] * inv),
+                          E::pack2(acc[ct][dt][4 * i + 2] * inv, acc[ct][dt][4 * i + 3] * inv)};
+        store_columns(reinterpret_cast<char *>(out + ((long)(q_begin + q0) * n_qo_heads + (long)kvh * group) * kHeadDim),
+                      live[ct] ? (qrow[ct] - q0) * n_qo_heads + c_head[ct] : -1, kHeadDim * 2, 0);
     }
 }
 
