@@ -198,7 +198,7 @@ __global__ __launch_bounds__(64 * kSharedWaves, 2) void mixed_attn_kernel(const 
             a.scale_log2, nullptr, nullptr, a.rope);
     else {
         __builtin_amdgcn_s_setprio(kSharedTilePriority);
-        prefill_attn_body<DT, true, kPrefillWavesShared>(
+        prefill_attn_body<DT, true, kPrefillWavesShared, true>(
             lds, wg - a.n_decode_wgs, a.out, a.q, a.qo_indptr, a.pages, a.kv_indices, a.kv_indptr, a.kv_last,
             a.tile_info, a.n_qo_heads, a.n_kv_heads, a.page_shift, a.scale_log2, a.causal,
             a.tile_part_o, a.tile_part_ml, a.tile_max_slots, a.rope);

@@ -58,7 +58,12 @@ struct LdsStages {
 // The kernel's body for workgroup `wg` of kWaves waves (a tile of kWaves * 32 / group query
 // rows of one kv head); `lds`: kPrefillLdsBytes of the workgroup's LDS.  A function, so that
 // one launch can hold workgroups of this kind next to workgroups of another.
-template <int DT, bool kRowsSharePage, int kWaves>
+//   kStreamOut: the rows leave past the L2 (non-temporal stores), which is the launch's K/V's.  Beside
+//     decode workgroups, whose own K/V stream past it, the partials of a chunk in two parts (14.5 MB)
+//     pushed the chunk's K/V out of it: 75 decode rows and the chunk 2638 -> 2471 us a step (16
+//     layers), 70B-shaped 1527 -> 1410.  A launch of tiles only loses (a chunk of 512 in four parts 938
+//     -> 955): its merge pass then reads the partials from farther away.
+template <int DT, bool kRowsSharePage, int kWaves, bool kStreamOut>
 __device__ __forceinline__ void prefill_attn_body(
     char *lds_base, int wg, uint16_t *__restrict__ out, const uint16_t *__restrict__ q,
     const int32_t *__restrict__ qo_indptr, const char *__restrict__ pages,
@@ -611,7 +616,8 @@ __device__ __forceinline__ void prefill_attn_body(
             const u32x4 w = *reinterpret_cast<const u32x4 *>(rows_lds + col * kRowsOutPitch + c * 16);
             if (to < 0) continue;
             u32x4 *const dst = reinterpret_cast<u32x4 *>(base + (long)to * row_bytes + at + c * 16);
-            *dst = w;
+            if (kStreamOut) __builtin_nontemporal_store(w, dst);
+            else *dst = w;
         }
         __builtin_amdgcn_wave_barrier();
     };
@@ -669,7 +675,7 @@ __global__ __launch_bounds__(64 * kPrefillWaves, DSKV_PREFILL_MIN_WAVES) void pr
     float *__restrict__ part_o, float *__restrict__ part_ml, int max_slots, const float *__restrict__ rope)
 {
     __shared__ __align__(16) char lds[kPrefillLdsBytes];
-    prefill_attn_body<DT, kRowsSharePage, kPrefillWaves>(
+    prefill_attn_body<DT, kRowsSharePage, kPrefillWaves, false>(
         lds, (int)blockIdx.x, out, q, qo_indptr, pages, kv_indices, kv_indptr, kv_last, tile_info,
         n_qo_heads, n_kv_heads, page_shift, scale_log2, causal, part_o, part_ml, max_slots, rope);
 }
