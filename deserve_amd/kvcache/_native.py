@@ -101,6 +101,10 @@ class SwapEngine:
         _lib.check(_lib.lib().dskv_swap_streams(self._h, ctypes.byref(a), ctypes.byref(b)), "swap_streams")
         return a.value, b.value
 
+    @property
+    def is_open(self) -> bool:
+        return bool(self._h)
+
     def close(self) -> None:
         if self._h:
             _lib.lib().dskv_swap_destroy(self._h)

@@ -9,9 +9,12 @@ engine's side streams (gather/scatter kernel + one large copy per staging
 chunk) instead of the reference's blocking advanced-index copy; ``synchronize``
 blocks the host until they are done - a chunk holds its request's pages from
 then on - and the compute stream is fenced behind what the copies do to the pool,
-so a caller that keeps the reference's call order sees the same results.
+so a caller that keeps the reference's call order sees the same results.  Work of
+that stream on a chunk (a copy of ``handle.retrieve()``) is ordered by ``retrieve``.
 """
 from __future__ import annotations
+
+import functools
 
 import torch
 
@@ -33,6 +36,7 @@ class KVCacheManager:
         shared = getattr(virtual_page_pool, "engine", None)
         self.engine = shared if shared is not None and staging_bytes == shared.staging_bytes \
             else _native.SwapEngine(staging_bytes)
+        self._copies_out, self._finished = 0, 0    # enqueued so far; of these, waited for
 
     def copy_gpu_to_cpu(self, paged_kvcache: PagedKVCache[VirtualPagePool],
                         task_id: str) -> ChunkHandle:
@@ -41,11 +45,18 @@ class KVCacheManager:
         n = table.occupied
         handle = self.cpu_chunk_pool.alloc(n)
         rows = n * self.cpu_chunk_pool.num_layers
-        self.engine.swap_out(handle.retrieve()[:rows], self.virtual_page_pool, table.retrieve())
+        self.engine.swap_out(handle.rows()[:rows], self.virtual_page_pool, table.retrieve())
         # pages may be handed to another request right after this returns: they have been packed
         # by the time the current stream goes on, and travel while it does
         self.engine.fence_pages()
+        # not so work on the chunk: retrieve() waits for the trip
+        self._copies_out += 1
+        handle.fence = functools.partial(self._fence_chunk, self._copies_out)
         return handle
+
+    def _fence_chunk(self, copy: int) -> None:
+        if copy > self._finished and self.engine.is_open:    # closing an engine finishes its copies
+            self.engine.fence()
 
     def copy_cpu_to_gpu(self, chunk_handle: ChunkHandle, task_id: str) -> VirtualPagedKVCache:
         """Only the copy; the caller frees the chunk and owns the new cache."""
@@ -57,11 +68,13 @@ class KVCacheManager:
         table = self.page_table_allocator.alloc()
         table.extend(ids)
         rows = n * self.cpu_chunk_pool.num_layers
-        self.engine.swap_in(pool, chunk_handle.retrieve()[:rows], ids)
+        self.engine.swap_in(pool, chunk_handle.rows()[:rows], ids)
         self.engine.fence_pages()   # attention on the current stream must see the pages
         isswap = torch.zeros((self.page_table_allocator.max_context_len,), dtype=torch.bool)
         isswap[:n] = ids >= pool.num_pages_main
         return VirtualPagedKVCache(page_table=table, isswap=isswap, pool=pool)
 
     def synchronize(self) -> None:
+        enqueued = self._copies_out
         self.engine.wait()
+        self._finished = enqueued

@@ -5,7 +5,8 @@ major - the layout KVCacheManager writes."""
 from __future__ import annotations
 
 import threading
-from dataclasses import dataclass
+from dataclasses import dataclass, field
+from typing import Callable, Optional
 
 import torch
 
@@ -19,11 +20,20 @@ class ChunkHandle:
     level: int
     initial_size: int
     pool: "ChunkPool"
+    # orders the current stream behind the copy that fills the chunk (set by whoever enqueues one)
+    fence: Optional[Callable[[], None]] = field(default=None, repr=False, compare=False)
 
     def free(self) -> None:
         self.pool.free(self.id, self.level)
 
     def retrieve(self) -> torch.Tensor:
+        """The chunk's rows, for work on the current stream: behind the copy that fills them."""
+        if self.fence is not None:
+            self.fence()
+        return self.rows()
+
+    def rows(self) -> torch.Tensor:
+        """The same for a caller that orders its accesses itself."""
         begin, end = BuddyIndex.span(self.id, self.level)
         return self.pool.chunks[begin * self.pool.num_layers: end * self.pool.num_layers]
 

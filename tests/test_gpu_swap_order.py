@@ -56,3 +56,29 @@ def test_calls_act_in_order(seed):
     for h, image in zip(hosts, images):
         assert np.array_equal(bits(h), image)
     eng.close()
+
+
+def test_work_on_an_offloaded_chunk_is_ordered_without_synchronize():
+    """A device copy of handle.retrieve() enqueued right behind copy_gpu_to_cpu sees the pages
+    (256 MB: ~5 ms on the link, the pages are packed long before)."""
+    from deserve_amd.kvcache.manager import KVCacheManager
+    from deserve_amd.kvcache.paged.chunk_pool import CpuChunkPool
+    from deserve_amd.kvcache.paged.page_table import PageTableAllocator
+    from deserve_amd.kvcache.virtual import VirtualPagedKVCache, VirtualPagePool
+
+    print("[case] chunk read behind its offload", flush=True)
+    L, P, n = 16, 16, 256
+    pool = VirtualPagePool(L, n + 8, 8, P, torch.device("cuda"), torch.bfloat16)
+    pool.pages.view(torch.int16).random_(0, 1 << 15)
+    tables = PageTableAllocator(2, n * P, P, torch.device("cuda"))
+    mgr = KVCacheManager(pool, CpuChunkPool(L, 9, P, torch.bfloat16), tables)
+    cache = VirtualPagedKVCache.empty(tables, pool)
+    cache.extend(n * P)
+    want = orc.gather_pages(pool.pages.view(torch.int16).cpu().numpy(), cache.page_table.retrieve().numpy())
+    handle = mgr.copy_gpu_to_cpu(cache, "task")
+    got = handle.retrieve()[: L * n].to("cuda", non_blocking=True)
+    cache.free()
+    torch.cuda.current_stream().synchronize()
+    assert np.array_equal(got.view(torch.int16).cpu().numpy(), want)
+    mgr.synchronize()
+    assert np.array_equal(handle.retrieve()[: L * n].view(torch.int16).numpy(), want)
