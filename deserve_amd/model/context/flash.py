@@ -212,10 +212,16 @@ class FlashDecodeCtx(FlashForwardCtx):
 class FlashPrefillCtx(FlashForwardCtx):
     prefill_wrapper: BatchPrefillWithPagedKVCacheWrapper = None   # type: ignore[assignment]
     rope_tables: Dict[tuple, torch.Tensor] = field(default_factory=dict, repr=False)
+    rope_layer: int = field(default=-1, repr=False)   # that asked last
 
     def rope_table(self, nnz: int, head_dim: int, theta: float) -> torch.Tensor:
-        """The step's cosines and sines (paged_ops.rope_table), built for the first layer that asks."""
+        """The step's cosines and sines (paged_ops.rope_table), built for the first layer that asks:
+        anew in every pass over the layers, since the offsets may have been written in between
+        (and a pass that is captured must hold the launch)."""
         key = (nnz, head_dim, theta)
+        if self.layer_id <= self.rope_layer:
+            self.rope_tables.clear()
+        self.rope_layer = self.layer_id
         if key not in self.rope_tables:
             self.rope_tables[key] = rope_table(self.indptr, self.offsets, nnz, head_dim, theta)
         return self.rope_tables[key]

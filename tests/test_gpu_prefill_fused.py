@@ -56,3 +56,23 @@ def test_fused_rotation_matches_separate_calls(case):
         torch.cuda.synchronize()
         assert torch.equal(bits(pages), bits(want_pages))
         assert bool(torch.isfinite(got.float()).all()) and torch.equal(bits(got), bits(want))
+
+
+def test_a_second_pass_over_the_layers_rotates_by_the_offsets_it_finds():
+    """A context whose offsets are rewritten in place between two passes."""
+    from deserve_amd.model.context.flash import FlashPrefillCtx
+    from deserve_amd.paged_ops import rope_table
+
+    print("[case] offsets rewritten between passes", flush=True)
+    dev = lambda a: torch.tensor(a, dtype=torch.int32, device="cuda")
+    ctx = FlashPrefillCtx(bsz=2, seqlens=dev([3, 4]), layer_id=0, page_pool=None, offsets=dev([0, 9]),
+                          indptr=dev([0, 3, 7]), kv_page_indices=None, kv_page_indptr=None,
+                          kv_last_page_lens=None, host={}, prefill_wrapper=None)
+    first = ctx.rope_table(7, 128, 1e4)
+    ctx.layer_id = 1
+    assert ctx.rope_table(7, 128, 1e4) is first
+    ctx.offsets.copy_(dev([5, 20]))
+    ctx.layer_id = 0
+    got = ctx.rope_table(7, 128, 1e4)
+    assert torch.equal(got, rope_table(ctx.indptr, ctx.offsets, 7, 128, 1e4))
+    assert not torch.equal(got, first)
