@@ -162,6 +162,12 @@ __global__ __launch_bounds__(64) void decode_attn_generic_kernel(
 // the scores are reduced over the 16 lanes of a row with DPP adds, 16 tokens are in flight per
 // iteration, and the per-group partial sums of O are folded across g once, at the end.
 // The block table entries of an iteration are fetched an iteration ahead.
+//
+// What bounds it in small batches is latency: a wave waits for memory once per 16 tokens.  Their
+// plans (up to kSplitMaxTiles tiles) have shares for a workgroup of several waves, so kWaves waves take
+// every kWaves-th 16 tokens of an item and meet in LDS.  fp32, 32 q heads, us: 8 requests of 512
+// tokens 24.9 with a wave alone, 14.4 with four (16.5 with eight), one of 2000 12.3 (14.7); 24 of
+// 50-150 17.9 (26.7: the second eight of a compute unit wait for the first).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float row16_sum(float v)
 {
@@ -186,8 +192,10 @@ __device__ __forceinline__ void load_row8(const char *row, bool live, float (&f)
     }
 }
 
-template <int DT, int kG>   // kG: q heads per kv head the wave carries (group padded to 1, 2, 4, 8)
-__global__ __launch_bounds__(64) void decode_attn_gqa_kernel(
+constexpr int kGqaWaves = 4;
+constexpr int kGqaMaxDim = 128;
+template <int DT, int kG, int kWaves>   // kG: q heads per kv head a wave carries (group padded to 1, 2, 4, 8)
+__global__ __launch_bounds__(64 * kWaves) void decode_attn_gqa_kernel(
     void *__restrict__ out, const void *__restrict__ q, const void *__restrict__ pages,
     const int32_t *__restrict__ kv_indices, const Item *__restrict__ items,
     float *__restrict__ part_o, float *__restrict__ part_ml, int max_slots, int n_qo_heads,
@@ -196,7 +204,9 @@ __global__ __launch_bounds__(64) void decode_attn_gqa_kernel(
     typedef LoadElt<DT> L;
     constexpr int kElt = DT == DSKV_F32 ? 4 : 2;
     constexpr int kSub = 4;                     // sub-steps of 4 tokens per iteration: 16 tokens in flight
-    const int lane = threadIdx.x, g = lane >> 4, c = lane & 15;
+    constexpr int kStep = 4 * kSub * kWaves;    // tokens the workgroup advances by
+    const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+    const int wave = kWaves > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
     const int kvh = blockIdx.y;
     const int group = n_qo_heads / n_kv_heads;
     const Item item = items[blockIdx.x];
@@ -228,8 +238,9 @@ __global__ __launch_bounds__(64) void decode_attn_gqa_kernel(
         for (int j = 0; j < kSub; j++) page[j] = table[min(t0 + 4 * j + g, last_tok) / page_size];
     };
     long page[kSub];
-    if (item.tok_begin < item.tok_end) lookup(item.tok_begin, page);
-    for (int t0 = item.tok_begin; t0 < item.tok_end; t0 += 4 * kSub) {
+    const int first_tok = item.tok_begin + wave * 4 * kSub;
+    if (first_tok < item.tok_end) lookup(first_tok, page);
+    for (int t0 = first_tok; t0 < item.tok_end; t0 += kStep) {
         float kx[kSub][8], vx[kSub][8];
 #pragma unroll
         for (int j = 0; j < kSub; j++) {
@@ -238,7 +249,7 @@ __global__ __launch_bounds__(64) void decode_attn_gqa_kernel(
             load_row8<DT>(row, live, kx[j]);
             load_row8<DT>(row + half_bytes, live, vx[j]);
         }
-        if (t0 + 4 * kSub < item.tok_end) lookup(t0 + 4 * kSub, page);   // for the next turn
+        if (t0 + kStep < item.tok_end) lookup(t0 + kStep, page);   // for the next turn
         float x[kG][kSub], m_new[kG];
 #pragma unroll
         for (int h = 0; h < kG; h++) {
@@ -269,6 +280,8 @@ __global__ __launch_bounds__(64) void decode_attn_gqa_kernel(
             }
         }
     }
+    __shared__ float wave_o[kWaves][kG][kWaves > 1 ? kGqaMaxDim : 1];
+    __shared__ float wave_ml[kWaves][kG][2];
     // fold the four token groups' partial sums; rows of lanes g == 0 then hold the item's result
 #pragma unroll
     for (int h = 0; h < kG; h++) {
@@ -277,6 +290,15 @@ __global__ __launch_bounds__(64) void decode_attn_gqa_kernel(
 #pragma unroll
         for (int i = 0; i < 8; i++) o[i] = quad_rows_sum(acc[h][i]);
         if (g != 0 || !live || h >= group) continue;
+        if (kWaves > 1) {   // a wave without tokens leaves zeros under the lowest maximum
+#pragma unroll
+            for (int i = 0; i < 8; i++) wave_o[wave][h][c * 8 + i] = o[i];
+            if (c == 0) {
+                wave_ml[wave][h][0] = m_run[h];
+                wave_ml[wave][h][1] = l;
+            }
+            continue;
+        }
         const int qh = kvh * group + h;
         if (item.slot < 0) {
             const float inv = l > 0.f ? 1.f / l : 0.f;
@@ -290,6 +312,31 @@ __global__ __launch_bounds__(64) void decode_attn_gqa_kernel(
                 float *ml = part_ml + ((long)item.slot * n_qo_heads + qh) * 2;
                 ml[0] = m_run[h];
                 ml[1] = l;
+            }
+        }
+    }
+    if (kWaves == 1) return;
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < group * head_dim; idx += 64 * kWaves) {
+        const int h = idx / head_dim, d = idx - h * head_dim;
+        const long at = (long)kvh * group + h;   // q head
+        float m = wave_ml[0][h][0];
+#pragma unroll
+        for (int w = 1; w < kWaves; w++) m = fmaxf(m, wave_ml[w][h][0]);
+        float sum = 0.f, l = 0.f;
+#pragma unroll
+        for (int w = 0; w < kWaves; w++) {
+            const float weight = __builtin_amdgcn_exp2f(wave_ml[w][h][0] - m);
+            l += weight * wave_ml[w][h][1];
+            sum += weight * wave_o[w][h][d];
+        }
+        if (item.slot < 0) {
+            L::put(out, ((long)b * n_qo_heads + at) * head_dim + d, l > 0.f ? sum / l : 0.f);
+        } else if (item.slot < max_slots) {
+            part_o[((long)item.slot * n_qo_heads + at) * head_dim + d] = sum;
+            if (d == 0) {
+                part_ml[((long)item.slot * n_qo_heads + at) * 2] = m;
+                part_ml[((long)item.slot * n_qo_heads + at) * 2 + 1] = l;
             }
         }
     }
@@ -703,13 +750,22 @@ static int decode_attn_impl(void *out, const void *q, const void *pages_layer,
         DSKV_LAUNCH_CHECK("decode_attn_mfma_kernel");
     } else if (n_qo_heads / n_kv_heads <= 8 && head_dim % 8 == 0 && head_dim <= 128 &&
                ((uintptr_t)pages_layer % 16 == 0) && ((int64_t)n_kv_heads * head_dim * (dtype == DSKV_F32 ? 4 : 2)) % 16 == 0) {
-        // one wave per (item, kv head) carries the whole GQA group
+        // a wave carries the whole GQA group; four split an item's tokens where the plan has few shares
+        // for the chip and not so many short items instead (then one each is enough: the chip
+        // holds 2048 waves of this kernel)
         const int group = n_qo_heads / n_kv_heads;
+        const bool split = (int64_t)n_workgroups * n_kv_heads <= default_workgroups() &&
+                           (int64_t)n_items * n_kv_heads <= 4 * (int64_t)default_workgroups();
         dim3 grid((unsigned)n_items, (unsigned)n_kv_heads);
+#define DSKV_LAUNCH_GQA_W(DT, G, W)                                                               \
+    hipLaunchKernelGGL((decode_attn_gqa_kernel<DT, G, W>), grid, dim3(64 * W), 0, s, out, q,       \
+                       pages_layer, kv_page_indices, items, part_o, part_ml, (int)max_slots,      \
+                       n_qo_heads, n_kv_heads, head_dim, page_size, scale_log2)
 #define DSKV_LAUNCH_GQA_G(DT, G)                                                                  \
-    hipLaunchKernelGGL((decode_attn_gqa_kernel<DT, G>), grid, dim3(64), 0, s, out, q, pages_layer, \
-                       kv_page_indices, items, part_o, part_ml, (int)max_slots, n_qo_heads,       \
-                       n_kv_heads, head_dim, page_size, scale_log2)
+    do {                                                                                          \
+        if (split) DSKV_LAUNCH_GQA_W(DT, G, kGqaWaves);                                           \
+        else DSKV_LAUNCH_GQA_W(DT, G, 1);                                                         \
+    } while (0)
 #define DSKV_LAUNCH_GQA(DT)                                  \
     do {                                                     \
         if (group <= 1) DSKV_LAUNCH_GQA_G(DT, 1);            \
@@ -722,6 +778,7 @@ static int decode_attn_impl(void *out, const void *q, const void *pages_layer,
         else DSKV_LAUNCH_GQA(DSKV_BF16);
 #undef DSKV_LAUNCH_GQA
 #undef DSKV_LAUNCH_GQA_G
+#undef DSKV_LAUNCH_GQA_W
         DSKV_LAUNCH_CHECK("decode_attn_gqa_kernel");
     } else {
         dim3 grid((unsigned)n_items, (unsigned)n_qo_heads);
