@@ -66,6 +66,7 @@ _SIGNATURES = {
     "dskv_decode_plan": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32, c_int32,
                                    c_int32, c_void_p, c_int64, POINTER(c_int32), POINTER(c_int32),
                                    POINTER(c_int64), POINTER(c_int64)]),
+    "dskv_decode_launch": (c_int64, [c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, POINTER(c_int32)]),
     "dskv_decode_attn": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int32,
                                    c_int32, c_void_p, c_int64, c_int32, c_int32, c_int32, c_int32,
                                    c_int32, c_float, c_int32, c_void_p]),

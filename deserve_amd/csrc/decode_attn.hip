@@ -474,13 +474,46 @@ static int default_workgroups()
 
 // Whether a plan's shares are so few that the attention runs as one workgroup per (share, kv
 // head) (decode_split_kernel.h) instead of one per share: when that still gives every compute
-// unit at most one.
+// unit at most one.  Their ids have no gaps, so the 8 XCDs, which take them in turn, get the same
+// number each.  (Rounded up to a multiple of 8 shares, to keep a share's heads on one XCD, 40 heads
+// filled six XCDs with 40 workgroups each for 32 units: 8 requests of 250 tiles in all 40.8 us,
+// 24.4 this way; 64 heads, 156 tiles 34.7 -> 20.0; 10 heads, 1000 tiles 38.5 -> 23.2; 8 heads as before.)
 static bool decode_splits_tokens(int n_workgroups, int n_qo_heads, int n_kv_heads)
 {
     return n_qo_heads / n_kv_heads <= kSplitMaxGroup && (int64_t)n_workgroups * n_kv_heads <= default_workgroups();
 }
+static int64_t split_launch_workgroups(int n_workgroups, int n_kv_heads) { return (int64_t)n_workgroups * n_kv_heads; }
+
+// The same for the generic kernel, one workgroup per (item, kv head): whether four waves split an
+// item's tokens.
+static bool gqa_splits_tokens(int n_items, int n_workgroups, int n_kv_heads)
+{
+    return (int64_t)n_workgroups * n_kv_heads <= default_workgroups() &&
+           (int64_t)n_items * n_kv_heads <= 4 * (int64_t)default_workgroups();
+}
 
 }  // namespace dskv
+
+extern "C" int64_t dskv_decode_launch(int32_t n_items, int32_t n_workgroups, int32_t n_qo_heads, int32_t n_kv_heads,
+                                      int32_t head_dim, int32_t dtype, int32_t *splits_tokens_out)
+{
+    using namespace dskv;
+    if (n_items <= 0 || n_workgroups <= 0 || n_qo_heads <= 0 || n_kv_heads <= 0 || n_qo_heads % n_kv_heads) return 0;
+    bool splits = false;
+    int64_t launched;
+    if (mfma_path(dtype, head_dim, n_qo_heads, n_kv_heads)) {
+        splits = decode_splits_tokens(n_workgroups, n_qo_heads, n_kv_heads);
+        launched = splits ? split_launch_workgroups(n_workgroups, n_kv_heads)
+                          : (int64_t)n_workgroups * ((n_kv_heads + kMaxWaves - 1) / kMaxWaves);
+    } else if (n_qo_heads / n_kv_heads <= 8 && head_dim % 8 == 0 && head_dim <= kGqaMaxDim) {
+        splits = gqa_splits_tokens(n_items, n_workgroups, n_kv_heads);
+        launched = (int64_t)n_items * n_kv_heads;
+    } else {
+        launched = (int64_t)n_items * n_qo_heads;
+    }
+    if (splits_tokens_out) *splits_tokens_out = splits;
+    return launched;
+}
 
 // ---------------------------------------------------------------------------
 // Host planner
@@ -708,13 +741,12 @@ static int decode_attn_impl(void *out, const void *q, const void *pages_layer,
                          "decode_attn: %lld merge counters, the plan needs %lld", (long long)n_merge_counters,
                          (long long)(slots * n_kv_heads));
             merged = merge_counters && phases == 3;
-            const int share_stride = (n_workgroups + 7) / 8 * 8;
             const SplitArgs args = {(uint16_t *)out, (const uint16_t *)q, (const char *)pages_layer, kv_page_indices,
                                     items, wg_ptr, part_o, part_ml, (int)max_slots, n_qo_heads, n_kv_heads, shift,
                                     scale_log2, (const uint16_t *)k_new, (const uint16_t *)v_new, rope_table,
                                     merged && n_items > batch ? merge_counters : nullptr,
-                                    (int)std::min<int64_t>(n_merge_counters, 1 << 30), n_workgroups, share_stride};
-            const dim3 grid((unsigned)(share_stride * n_kv_heads)), block(64 * kSplitWaves);
+                                    (int)std::min<int64_t>(n_merge_counters, 1 << 30), n_workgroups};
+            const dim3 grid((unsigned)split_launch_workgroups(n_workgroups, n_kv_heads)), block(64 * kSplitWaves);
 #define DSKV_LAUNCH_SPLIT(DT, COVER) \
     hipLaunchKernelGGL((decode_attn_split_kernel<DT, COVER>), grid, block, 0, s, args)
             if (dtype == DSKV_BF16) {
@@ -754,8 +786,7 @@ static int decode_attn_impl(void *out, const void *q, const void *pages_layer,
         // for the chip and not so many short items instead (then one each is enough: the chip
         // holds 2048 waves of this kernel)
         const int group = n_qo_heads / n_kv_heads;
-        const bool split = (int64_t)n_workgroups * n_kv_heads <= default_workgroups() &&
-                           (int64_t)n_items * n_kv_heads <= 4 * (int64_t)default_workgroups();
+        const bool split = gqa_splits_tokens(n_items, n_workgroups, n_kv_heads);
         dim3 grid((unsigned)n_items, (unsigned)n_kv_heads);
 #define DSKV_LAUNCH_GQA_W(DT, G, W)                                                               \
     hipLaunchKernelGGL((decode_attn_gqa_kernel<DT, G, W>), grid, dim3(64 * W), 0, s, out, q,       \

@@ -124,19 +124,19 @@ struct SplitArgs {
     const uint16_t *k_new, *v_new;   // null: the newest tokens are in the pages already
     const float *rope;               // null: q and k_new are not to be rotated
     uint32_t *counters;              // one zeroed word per (partial slot, kv head); null: a merge launch follows
-    int n_counters, n_shares, share_stride;
+    int n_counters, n_shares;
 };
 
-// share = id % share_stride, so that the heads of a share - which read the same pages - sit on one
-// XCD (ids go round the 8 XCDs; share_stride is a multiple of 8).
+// A workgroup fills its compute unit's LDS, so what counts is that the workgroups spread evenly: ids go
+// round the 8 XCDs, and without gaps in them no XCD gets more than its 32, whatever the number of
+// heads.  (The heads of a share need not meet on an XCD: they read other bytes of the same pages.)
 template <int DT, int kPagesPerTile>
 __global__ __launch_bounds__(64 * kSplitWaves) void decode_attn_split_kernel(const SplitArgs a)
 {
     typedef Elt<DT> E;
     constexpr bool kPageCoversTile = kPagesPerTile == 1;
     __shared__ __align__(16) SplitShared sh;
-    const int share = (int)blockIdx.x % a.share_stride, kvh = (int)blockIdx.x / a.share_stride;
-    if (share >= a.n_shares) return;
+    const int share = (int)blockIdx.x % a.n_shares, kvh = (int)blockIdx.x / a.n_shares;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int g = lane >> 4, c = lane & 15;

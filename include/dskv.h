@@ -119,6 +119,13 @@ int dskv_decode_attn(void *out, const void *q, const void *pages_layer,
                      int32_t n_qo_heads, int32_t n_kv_heads, int32_t head_dim, int32_t page_size,
                      float sm_scale, int32_t dtype, void *stream);
 /*
+ * The attention launch of a plan, for tests and measurements: how many workgroups it has, and in
+ * *splits_tokens_out whether the waves of one split the tokens of a kv head (1) or are a kv head each
+ * (0).  Host only; 0 for bad arguments.
+ */
+int64_t dskv_decode_launch(int32_t n_items, int32_t n_workgroups, int32_t n_qo_heads, int32_t n_kv_heads,
+                           int32_t head_dim, int32_t dtype, int32_t *splits_tokens_out);
+/*
  * dskv_decode_attn for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the
  * reference.  Same arguments and result as dskv_decode_attn, bit for bit, minus the

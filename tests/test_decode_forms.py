@@ -1,0 +1,45 @@
+"""Which form of the decode attention a plan gets, and how its workgroups spread over the chip: host
+rules only (256 compute units are assumed where there is no GPU)."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from deserve_amd import _lib
+
+CUS, XCDS = 256, 8
+
+
+def _plan(lens, n_kv, group=4, d=128, page=16, target=0):
+    """(shares, items, most tiles of an item)."""
+    lib = _lib.lib()
+    n = -(-np.asarray(lens, np.int64) // page)
+    indptr = np.concatenate([[0], np.cumsum(n)]).astype(np.int32)
+    last = np.array([(x - 1) % page + 1 if x else 0 for x in lens], np.int32)
+    cap = lib.dskv_decode_plan_bound(len(lens), int(n.sum()) * page)
+    plan = np.zeros(cap, np.int32)
+    items, wgs, words, ws = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int64(), ctypes.c_int64()
+    out = [ctypes.byref(x) for x in (items, wgs, words, ws)]
+    head = (indptr.ctypes.data, last.ctypes.data, len(lens), page, n_kv * group, n_kv, d)
+    rc = lib.dskv_decode_plan(*head, target, plan.ctypes.data, cap, *out)
+    assert rc == 0, _lib.last_error()
+    table = plan[4 + wgs.value + 1 + 2 * len(lens): words.value].reshape(-1, 8)
+    return wgs.value, items.value, int((-(-(table[:, 2] - table[:, 1]) // 16)).max())
+
+
+def _launch(items, shares, n_kv, group=4, d=128, dtype=_lib.BF16):
+    splits = ctypes.c_int32(-1)
+    n = _lib.lib().dskv_decode_launch(items, shares, n_kv * group, n_kv, d, dtype, ctypes.byref(splits))
+    return int(n), bool(splits.value)
+
+
+@pytest.mark.parametrize("n_kv", range(1, 65))
+def test_no_xcd_gets_more_workgroups_than_it_has_units(n_kv):
+    """The split form's workgroups fill a compute unit's LDS: a 33rd on an XCD waits for another to end."""
+    for lens in ([1777], [300, 512, 700, 900], [64] * 32):
+        shares, items, _ = _plan(lens, n_kv)
+        workgroups, splits = _launch(items, shares, n_kv)
+        if splits:
+            assert workgroups == shares * n_kv          # every id has work
+            assert -(-workgroups // XCDS) <= CUS // XCDS
+    assert _launch(3, CUS // n_kv, n_kv) == (CUS // n_kv * n_kv, True)
