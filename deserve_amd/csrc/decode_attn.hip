@@ -472,6 +472,10 @@ static int default_workgroups()
     return cached;
 }
 
+// Parts per request, on average, from which the merge launch gives a (request, head) eight waves: one
+// wave needs a round trip per 8 parts, eight waves a barrier and a second pass through LDS.
+constexpr int64_t kWideMergeParts = 32;
+
 // Whether a plan's shares are so few that the attention runs as one workgroup per (share, kv
 // head) (decode_split_kernel.h) instead of one per share: when that still gives every compute
 // unit at most one.  Their ids have no gaps, so the 8 XCDs, which take them in turn, get the same
@@ -528,6 +532,42 @@ extern "C" int64_t dskv_decode_plan_bound(int32_t batch, int64_t total_tokens)
 
 namespace dskv {
 
+// Whether the 16-bit attention of a batch should run as a workgroup per (share, kv head), on
+// few = CUs / n_kv_heads shares, instead of a workgroup per share whose waves are kv heads (at most
+// eight; more heads, more workgroups per share).  Measured with equal, ragged and lopsided batches
+// of 1 to 64 requests at 1 to 160 kv heads (bf16, attention and merge in a replayed graph, us,
+// workgroup per (share, kv head) / the other form; a range is over the batches):
+//   * Eight heads fill a workgroup of the other form, which then wins as soon as memory is the limit:
+//     1250 tiles 24 / 24-28, 1875 tiles 30-31 / 30-33, 2560 tiles 38 / 36.  The line: 60 tiles a share,
+//     40 for more than 32 requests (64: 1250 tiles 25 / 23, 1750 tiles 30 / 28).
+//   * More heads, or fewer than eight that leave waves of the other form idle, lose there later or
+//     not at all where few * n_kv_heads workgroups leave hardly a unit idle: 5 heads, 2000 tiles 23-26 /
+//     23-27; 12 heads, 1706 tiles 40 / 42-44, 2500 tiles 54 / 53-56; 16 heads, 2500 tiles 64 / 69; 64
+//     heads, 625 tiles 64 / 74-80.  Where they do leave units idle: 20 heads (240 workgroups), 1024 tiles
+//     43 / 44-46, 1500 tiles 59 / 54; 96 heads (192), 104 tiles 27-28 / 30-34, 156 tiles 36 / 34-36.
+//     The line: 80 tiles a share, lower by the share of units that idle.
+//   * Up to four heads a request is cut into many parts (few is 64 and more), and merging them costs
+//     more than the walk saves: 4 heads, 375 tiles 12-13 / 12-16, but one request 16 / 14, and 750 tiles
+//     15-16 / 13-14; 2 heads, 1500 tiles 14-20 / 11-15.
+//   * One head: 256 workgroups of a wave each leave the chip idle: 1500 tiles 14-23 / 11-13, 5000 tiles
+//     17-21 / 18-21, 20480 tiles 36-40 / 47-52.
+//   * Lopsided: one request in dozens of parts beside short ones.  The merge launch gives a row one
+//     workgroup per eight heads: 24 requests, one of 1250 tiles with 8 heads 25 / 58, 2 heads 20 / 48.
+//     (Where requests have more than kWideMergeParts parts on average, that launch gives a row more.)
+static bool splitting_pays(int64_t tiles, int64_t longest, int batch, int n_kv_heads)
+{
+    const int64_t cus = default_workgroups(), few = cus / n_kv_heads, busy = few * n_kv_heads;
+    if (few < 1) return false;
+    if (n_kv_heads == 1 && tiles >= kSplitMinTilesOneHead) return true;
+    if (tiles > kSplitMaxTiles) return false;
+    if (longest * cus > kLopsidedParts * tiles && batch + cus <= kWideMergeParts * (int64_t)batch) return true;
+    int64_t most;
+    if (n_kv_heads <= 4) most = n_kv_heads > 2 && batch > 1 ? 2048 / n_kv_heads : 0;
+    else if (n_kv_heads != kMaxWaves && 32 * busy >= 31 * cus) most = kSplitMaxTiles;
+    else most = (n_kv_heads > kMaxWaves ? 80 : batch > 32 ? 40 : 60) * few * busy / cus;
+    return tiles <= most;
+}
+
 // The planner proper.  reqs[i]: tokens, start of the block table and q / output row of
 // request i (row i itself for a decode batch).
 int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, int32_t n_kv_heads,
@@ -536,28 +576,28 @@ int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, i
                      int64_t *workspace_bytes_out)
 {
     std::vector<int64_t> tiles(batch);
-    int64_t total_tiles = 0;
+    int64_t total_tiles = 0, longest = 0;
     for (int b = 0; b < batch; b++) {
         DSKV_REQUIRE(reqs[b].len >= 0 && reqs[b].len < (int64_t(1) << 30), "decode_plan: request %d too long", b);
         tiles[b] = (reqs[b].len + kTile - 1) / kTile;
         total_tiles += tiles[b];
+        longest = std::max(longest, tiles[b]);
     }
     // Share count: one per CU unless told otherwise, fewer when there is so little work that a
-    // share would drop below a few tiles.  Small batches get so few that the attention runs as
-    // one workgroup per (share, kv head): measured (bf16, 8 kv heads, attention and merge in a
-    // replayed graph, us) with 32 shares against 256 or the four-tile shares of before: 318 tiles
-    // 15 / 24, 1024 tiles 21 / 26, 2048 tiles 31-33 / 33-41, 3255 tiles 51 / 48, 4096 tiles
-    // 56 / 52.  A share of six tiles: one request of 112 tiles takes 13.1 us in 18 shares (14.0 in
-    // 28), three of 13 tiles take 10.7 us in 9 shares (13.0 in 4).
-    int64_t wgs = target_workgroups;
-    if (wgs <= 0) {
-        wgs = default_workgroups();
-        const int64_t few = wgs / n_kv_heads;
-        if (head_dim == kHeadDim && few > 0 && n_qo_heads / n_kv_heads <= kSplitMaxGroup && total_tiles <= kSplitMaxTiles)
-            wgs = std::min<int64_t>(few, std::max<int64_t>(1, total_tiles / kSplitTilesPerShare));
-    }
+    // share would drop below a few tiles.  Batches for which splitting pays get so few that the
+    // attention runs as one workgroup per (share, kv head), shares of six tiles at least: one request
+    // of 112 tiles takes 13.1 us in 18 shares (14.0 in 28), three of 13 tiles 10.7 in 9 (13.0 in 4).
+    // The launcher knows that form by the number of workgroups (decode_splits_tokens), so a plan for
+    // the other one is filled up with workgroups that have nothing to do where it would pass for it.
+    const bool own_rule = target_workgroups <= 0;
+    const bool split_shape = head_dim == kHeadDim && n_qo_heads / n_kv_heads <= kSplitMaxGroup;
+    const bool split = own_rule && split_shape && splitting_pays(total_tiles, longest, batch, n_kv_heads);
+    int64_t wgs = own_rule ? default_workgroups() : target_workgroups;
+    if (split) wgs = std::min<int64_t>(wgs / n_kv_heads, std::max<int64_t>(1, total_tiles / kSplitTilesPerShare));
     wgs = std::min<int64_t>(wgs, kMaxWorkgroups);
     wgs = std::min<int64_t>(wgs, std::max<int64_t>(1, total_tiles / kMinTilesPerWorkgroup));
+    int64_t launched = wgs;
+    if (own_rule && split_shape && !split) launched = std::max<int64_t>(wgs, default_workgroups() / n_kv_heads + 1);
 
     // Lay the requests' tiles end to end; workgroup w owns global tiles
     // [w * T / wgs, (w + 1) * T / wgs).  Requests without tokens ride along as
@@ -599,7 +639,7 @@ int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, i
             }
         }
     }
-    while ((int64_t)wg_ptr.size() < wgs + 1) wg_ptr.push_back((int32_t)items.size());
+    while ((int64_t)wg_ptr.size() < launched + 1) wg_ptr.push_back((int32_t)items.size());
     wg_ptr.back() = (int32_t)items.size();
 
     const int64_t words = kPlanHeaderWords + (int64_t)items.size() * kItemWords +
@@ -611,7 +651,7 @@ int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, i
     }
     int32_t *p = plan_host;
     *p++ = (int32_t)items.size();
-    *p++ = (int32_t)wgs;
+    *p++ = (int32_t)launched;
     *p++ = n_slots;
     *p++ = batch;
     // the variable-length part (the items) goes last, so that where everything lies
@@ -622,7 +662,7 @@ int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, i
     std::copy(reinterpret_cast<const int32_t *>(items.data()),
               reinterpret_cast<const int32_t *>(items.data()) + items.size() * kItemWords, p);
     *n_items_out = (int32_t)items.size();
-    *n_workgroups_out = (int32_t)wgs;
+    *n_workgroups_out = (int32_t)launched;
     *plan_words_out = words;
     *workspace_bytes_out = (int64_t)n_slots * n_qo_heads * (head_dim + 2) * (int64_t)sizeof(float);
     return 0;
@@ -740,7 +780,9 @@ static int decode_attn_impl(void *out, const void *q, const void *pages_layer,
             DSKV_REQUIRE(!merge_counters || n_merge_counters >= slots * n_kv_heads,
                          "decode_attn: %lld merge counters, the plan needs %lld", (long long)n_merge_counters,
                          (long long)(slots * n_kv_heads));
-            merged = merge_counters && phases == 3;
+            // (a request in dozens of parts: one workgroup takes longer over them than the launch of the
+            // eight-wave merge, 35.7 against 16.9 us for 250 parts, 16.0 against 13.0 for 62)
+            merged = merge_counters && phases == 3 && n_items <= kWideMergeParts * (int64_t)batch;
             const SplitArgs args = {(uint16_t *)out, (const uint16_t *)q, (const char *)pages_layer, kv_page_indices,
                                     items, wg_ptr, part_o, part_ml, (int)max_slots, n_qo_heads, n_kv_heads, shift,
                                     scale_log2, (const uint16_t *)k_new, (const uint16_t *)v_new, rope_table,
@@ -824,10 +866,8 @@ static int decode_attn_impl(void *out, const void *q, const void *pages_layer,
         DSKV_LAUNCH_CHECK("decode_attn_generic_kernel");
     }
     if (!merged && (phases & 2) && n_items > batch) {
-        // many parts per request (long requests, small batch): eight waves share a merge.
-        // One wave needs a round trip per 8 parts, eight waves a barrier and a second pass
-        // through LDS: they break even at about 32 parts.
-        const bool wide = (int64_t)n_items > 32 * (int64_t)batch;
+        // many parts per request (long requests, small batch): eight waves share a merge
+        const bool wide = n_items > kWideMergeParts * (int64_t)batch;
         return launch_partials_merge(out, part_o, part_ml, req_parts, row_map, (int)max_slots, batch,
                                      n_qo_heads, head_dim, dtype, wide, s);
     }

@@ -22,8 +22,9 @@ namespace dskv {
 
 constexpr int kSplitWaves = 8;
 constexpr int kSplitRing = 2;        // tiles in flight per wave: a wave rarely has more
-constexpr int kSplitMaxTiles = 2560;       // tiles of a batch, at most, and tiles a share has at least
-constexpr int kSplitTilesPerShare = 6;     // (the planner's rule, measured there)
+// The planner's rule, measured there: tiles of a batch at most (one kv head: at least), tiles of a
+// share at least, and parts of one request that make a batch lopsided.
+constexpr int kSplitMaxTiles = 2560, kSplitMinTilesOneHead = 5000, kSplitTilesPerShare = 6, kLopsidedParts = 64;
 constexpr int kSplitMaxGroup = 8;    // q heads per kv head, at most (LDS for the pieces that meet)
 // LDS: the waves' V tiles; two meeting places per wave ([0] a piece that continues an item of an
 // earlier wave, [1] one that a later wave continues) of O and (m, l) per q head; the new token's
