@@ -554,7 +554,9 @@ namespace dskv {
 //   * Lopsided: one request in dozens of parts beside short ones.  The merge launch gives a row one
 //     workgroup per eight heads: 24 requests, one of 1250 tiles with 8 heads 25 / 58, 2 heads 20 / 48.
 //     (Where requests have more than kWideMergeParts parts on average, that launch gives a row more.)
-static bool splitting_pays(int64_t tiles, int64_t longest, int batch, int n_kv_heads)
+//   * Without counters to merge inside the launch (merges_itself) a request pays for the merge launch
+//     as well: 8 heads, 625 tiles 16-22 / 19-24, 937 tiles 20-25 / 22-27, 1250 tiles 23-28 / 23-26.  A third.
+static bool splitting_pays(int64_t tiles, int64_t longest, int batch, int n_kv_heads, bool merges_itself)
 {
     const int64_t cus = default_workgroups(), few = cus / n_kv_heads, busy = few * n_kv_heads;
     if (few < 1) return false;
@@ -565,15 +567,15 @@ static bool splitting_pays(int64_t tiles, int64_t longest, int batch, int n_kv_h
     if (n_kv_heads <= 4) most = n_kv_heads > 2 && batch > 1 ? 2048 / n_kv_heads : 0;
     else if (n_kv_heads != kMaxWaves && 32 * busy >= 31 * cus) most = kSplitMaxTiles;
     else most = (n_kv_heads > kMaxWaves ? 80 : batch > 32 ? 40 : 60) * few * busy / cus;
-    return tiles <= most;
+    return tiles <= (merges_itself ? most : most / 3);
 }
 
 // The planner proper.  reqs[i]: tokens, start of the block table and q / output row of
 // request i (row i itself for a decode batch).
 int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, int32_t n_kv_heads,
-                     int32_t head_dim, int32_t target_workgroups, int32_t *plan_host, int64_t plan_capacity_words,
-                     int32_t *n_items_out, int32_t *n_workgroups_out, int64_t *plan_words_out,
-                     int64_t *workspace_bytes_out)
+                     int32_t head_dim, bool merges_itself, int32_t target_workgroups, int32_t *plan_host,
+                     int64_t plan_capacity_words, int32_t *n_items_out, int32_t *n_workgroups_out,
+                     int64_t *plan_words_out, int64_t *workspace_bytes_out)
 {
     std::vector<int64_t> tiles(batch);
     int64_t total_tiles = 0, longest = 0;
@@ -591,7 +593,7 @@ int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, i
     // the other one is filled up with workgroups that have nothing to do where it would pass for it.
     const bool own_rule = target_workgroups <= 0;
     const bool split_shape = head_dim == kHeadDim && n_qo_heads / n_kv_heads <= kSplitMaxGroup;
-    const bool split = own_rule && split_shape && splitting_pays(total_tiles, longest, batch, n_kv_heads);
+    const bool split = own_rule && split_shape && splitting_pays(total_tiles, longest, batch, n_kv_heads, merges_itself);
     int64_t wgs = own_rule ? default_workgroups() : target_workgroups;
     if (split) wgs = std::min<int64_t>(wgs / n_kv_heads, std::max<int64_t>(1, total_tiles / kSplitTilesPerShare));
     wgs = std::min<int64_t>(wgs, kMaxWorkgroups);
@@ -702,7 +704,7 @@ extern "C" int dskv_decode_plan(const int32_t *kv_page_indptr_host,
                      "decode_plan: kv_last_page_len[%d] = %d outside [1, %d]", b, last, page_size);
         reqs[b] = DecodeRow{np > 0 ? (np - 1) * page_size + last : 0, kv_page_indptr_host[b], b};
     }
-    return plan_decode_rows(reqs.data(), batch, n_qo_heads, n_kv_heads, head_dim, target_workgroups, plan_host,
+    return plan_decode_rows(reqs.data(), batch, n_qo_heads, n_kv_heads, head_dim, true, target_workgroups, plan_host,
                             plan_capacity_words, n_items_out, n_workgroups_out, plan_words_out,
                             workspace_bytes_out);
 }

@@ -517,12 +517,8 @@ extern "C" int dskv_mixed_plan(const int32_t *qo_indptr_host, const int32_t *kv_
         const int head_groups = (n_kv_heads + kSharedWaves - 1) / kSharedWaves;
         const int cus = target_workgroups > 0 ? std::min<int>(target_workgroups, kMaxWorkgroups) : compute_units();
         decode_target = std::max(1, cus / head_groups);
-    } else if (n_tile_rows > 0 && target_workgroups <= 0) {
-        // a pass of its own in front of the tiles, without the counters that let a launch of few
-        // shares merge its own parts: one share per compute unit
-        decode_target = compute_units();
     }
-    rc = plan_decode_rows(rows.data(), (int32_t)rows.size(), n_qo_heads, n_kv_heads, head_dim, decode_target,
+    rc = plan_decode_rows(rows.data(), (int32_t)rows.size(), n_qo_heads, n_kv_heads, head_dim, false, decode_target,
                           plan_host + at, capacity_words - at, &info->n_decode_items,
                           &info->n_decode_workgroups, &decode_words, &info->decode_workspace_bytes);
     if (rc) return rc;

@@ -62,3 +62,27 @@ def test_which_batches_split_a_head_over_the_waves_of_a_workgroup(n_kv, lens, sp
     total = sum(-(-x // 16) for x in lens)
     if not splits and total >= 1024:      # a share per compute unit, as large plans have
         assert shares == max(CUS, CUS // n_kv + 1)
+
+
+def _mixed(qo_lens, kv_lens, n_kv=8, route=_lib.ROUTE_AUTO, page=16):
+    """(shares, items) of the decode rows of a batch planned as prefill."""
+    lib = _lib.lib()
+    n = -(-np.asarray(kv_lens, np.int64) // page)
+    indptr = np.concatenate([[0], np.cumsum(n)]).astype(np.int32)
+    last = np.array([(x - 1) % page + 1 for x in kv_lens], np.int32)
+    qo = np.concatenate([[0], np.cumsum(qo_lens)]).astype(np.int32)
+    cap = lib.dskv_mixed_plan_bound(len(qo_lens), int(qo[-1]), int(n.sum()) * page)
+    plan, info = np.zeros(cap, np.int32), _lib.MixedPlanInfo()
+    rc = lib.dskv_mixed_plan(qo.ctypes.data, indptr.ctypes.data, last.ctypes.data, len(qo_lens), page, 4 * n_kv,
+                             n_kv, 128, 0, route, plan.ctypes.data, cap, ctypes.byref(info))
+    assert rc == 0 and info.layout == _lib.LAYOUT_SEPARATE, _lib.last_error()
+    return info.n_decode_workgroups, info.n_decode_items
+
+
+@pytest.mark.parametrize("tiles,splits", [(80, True), (81, False)])
+def test_rows_of_a_prefill_batch_have_one_rule_with_and_without_chunks(tiles, splits):
+    """No counters there: parts are merged by a launch of their own, and the line lies lower."""
+    rows = [16 * tiles] * 8
+    alone = _mixed([1] * 8, rows)
+    beside = _mixed([1] * 8 + [100], rows + [100], route=_lib.ROUTE_TWO_LAUNCHES)
+    assert alone == beside and _launch(alone[1], alone[0], 8)[1] == splits
