@@ -66,6 +66,9 @@ _SIGNATURES = {
     "dskv_decode_plan": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32, c_int32,
                                    c_int32, c_void_p, c_int64, POINTER(c_int32), POINTER(c_int32),
                                    POINTER(c_int64), POINTER(c_int64)]),
+    "dskv_decode_plan_typed": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32, c_int32,
+                                         c_int32, c_int32, c_void_p, c_int64, POINTER(c_int32),
+                                         POINTER(c_int32), POINTER(c_int64), POINTER(c_int64)]),
     "dskv_decode_launch": (c_int64, [c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, POINTER(c_int32)]),
     "dskv_decode_attn": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int32,
                                    c_int32, c_void_p, c_int64, c_int32, c_int32, c_int32, c_int32,
@@ -102,6 +105,9 @@ _SIGNATURES = {
     "dskv_mixed_plan_bound": (c_int64, [c_int32, c_int64, c_int64]),
     "dskv_mixed_plan": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32,
                                   c_int32, c_int32, c_int32, c_void_p, c_int64, POINTER(MixedPlanInfo)]),
+    "dskv_mixed_plan_typed": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32,
+                                        c_int32, c_int32, c_int32, c_int32, c_void_p, c_int64,
+                                        POINTER(MixedPlanInfo)]),
     "dskv_mixed_attn": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                   c_void_p, c_void_p, POINTER(MixedPlanInfo), c_void_p, c_int64,
                                   c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_float,

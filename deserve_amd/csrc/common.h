@@ -61,7 +61,7 @@ int launch_partials_merge(void *out, const float *part_o, const float *part_ml,
 // requests of a prefill batch): request i has `len` kv tokens, its block table starts at
 // entry `page_begin` of the table array, and its query and output are row `row` of q and out.
 // plan_decode_rows is dskv_decode_plan over such a list (same plan layout, the items name the
-// rows; merges_itself: the launch has counters to merge cut requests with); decode_rows_attn is dskv_decode_attn over that plan, with row_map[i] = reqs[i].row on
+// rows; dtype: of the pages, which decides the kernel; merges_itself: the launch has counters to merge cut requests with); decode_rows_attn is dskv_decode_attn over that plan, with row_map[i] = reqs[i].row on
 // the device for the merge pass; rope_table (may be null): the rows' angles, by query row, and q
 // is rotated as it is loaded.  decode_mfma_shape: whether the 16-bit decode kernel takes
 // the shape (the routing is only worth it then).
@@ -70,7 +70,7 @@ struct DecodeRow {
     int32_t page_begin, row;
 };
 int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, int32_t n_kv_heads,
-                     int32_t head_dim, bool merges_itself, int32_t target_workgroups, int32_t *plan_host,
+                     int32_t head_dim, int32_t dtype, bool merges_itself, int32_t target_workgroups, int32_t *plan_host,
                      int64_t plan_capacity_words, int32_t *n_items_out, int32_t *n_workgroups_out,
                      int64_t *plan_words_out, int64_t *workspace_bytes_out);
 int decode_rows_attn(void *out, const void *q, const void *pages_layer,

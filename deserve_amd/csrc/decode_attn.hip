@@ -489,7 +489,11 @@ static bool decode_splits_tokens(int n_workgroups, int n_qo_heads, int n_kv_head
 static int64_t split_launch_workgroups(int n_workgroups, int n_kv_heads) { return (int64_t)n_workgroups * n_kv_heads; }
 
 // The same for the generic kernel, one workgroup per (item, kv head): whether four waves split an
-// item's tokens.
+// item's tokens.  (A plan of few shares and more than 1024 items is one of requests of a tile or two.)
+static bool gqa_shape(int head_dim, int n_qo_heads, int n_kv_heads)
+{
+    return n_qo_heads / n_kv_heads <= 8 && head_dim % 8 == 0 && head_dim <= kGqaMaxDim;
+}
 static bool gqa_splits_tokens(int n_items, int n_workgroups, int n_kv_heads)
 {
     return (int64_t)n_workgroups * n_kv_heads <= default_workgroups() &&
@@ -509,7 +513,7 @@ extern "C" int64_t dskv_decode_launch(int32_t n_items, int32_t n_workgroups, int
         splits = decode_splits_tokens(n_workgroups, n_qo_heads, n_kv_heads);
         launched = splits ? split_launch_workgroups(n_workgroups, n_kv_heads)
                           : (int64_t)n_workgroups * ((n_kv_heads + kMaxWaves - 1) / kMaxWaves);
-    } else if (n_qo_heads / n_kv_heads <= 8 && head_dim % 8 == 0 && head_dim <= kGqaMaxDim) {
+    } else if (gqa_shape(head_dim, n_qo_heads, n_kv_heads)) {
         splits = gqa_splits_tokens(n_items, n_workgroups, n_kv_heads);
         launched = (int64_t)n_items * n_kv_heads;
     } else {
@@ -570,10 +574,47 @@ static bool splitting_pays(int64_t tiles, int64_t longest, int batch, int n_kv_h
     return tiles <= (merges_itself ? most : most / 3);
 }
 
+// The same for the generic kernel (four waves split an item / a wave has it alone).  fp32 rows of
+// head_dim 128, where the form comes with few, larger shares; measured as above:
+//   * It wins on small batches only: 8 heads, 8 requests of 94 tiles in all 17 / 21-22, of 187 tiles 22 / 23,
+//     of 625 tiles 38 / 35; 24 requests of 37 tiles 14 / 17, of 87 tiles 21 / 20; 64 of 87 tiles 29 / 18, of 600
+//     tiles 48 / 34; more heads lose later: 16 heads, 16 requests of 87 tiles 13 / 14, 32 heads, 8 of 21 tiles
+//     11 / 12.  The line: 2048 tiles of one head and 128 (request, head) pairs, more of them where the
+//     requests are a tile or two.
+//   * And with eight heads where memory is the limit and requests are few: 2 to 24 requests of 1125 tiles 53-55 /
+//     57-59, of 2000 tiles 75-80 / 79-85 (64: 97 / 80).
+//   * One request: 8 heads, 375 tiles 28 / 30, 937 tiles 46 / 45; 4 heads, 1875 tiles 43 / 47.
+//   * One or two heads: 1500 tiles of two 27-30 / 29-32, 2500 tiles 35-39 / 40-43; 5000 tiles of one 50-80 /
+//     92-94; but not where the items are a few more than the units: one head, 24 requests of 1400 tiles
+//     27 / 39 in 253 items, of 1500 tiles 46 / 39 in 273.
+//   * Lopsided: 24 requests, one of 370 tiles with 8 heads 32 / 37, 1250 tiles 61 / 86.
+// Other head sizes keep their shares: 8 heads of 64, 24 requests of 87 tiles 15 / 25 (f16) and 15 / 19 (fp32), 64
+// requests 23 / 20 and 23 / 17; 16 heads, 24 requests of 43 tiles 10 / 15; 4 heads, 128 of 175 tiles 23 / 20.
+static bool gqa_splitting_pays(int64_t tiles, int64_t longest, int batch, int n_kv_heads, int head_dim)
+{
+    const int64_t cus = default_workgroups(), few = cus / n_kv_heads, work = tiles * n_kv_heads;
+    const int64_t pairs = (int64_t)batch * n_kv_heads;
+    if (few < 1) return false;
+    if (head_dim != kHeadDim) return 2 * pairs <= 3 * cus;
+    if (tiles <= kSplitMaxTiles && longest * cus > kLopsidedParts * tiles &&
+        batch + cus <= kWideMergeParts * (int64_t)batch && pairs + few * n_kv_heads <= 4 * cus)
+        return true;
+    if (n_kv_heads <= 2) {
+        const int64_t shares = std::min(few, std::max<int64_t>(1, tiles / kSplitTilesPerShare));
+        return (n_kv_heads == 1 || tiles <= kSplitMaxTiles) &&
+               !(batch > 16 && work < 2560 && (batch + shares) * n_kv_heads > cus) && !(pairs > cus / 2 && work < 1024);
+    }
+    if (tiles > kSplitMaxTiles) return false;
+    if (batch == 1) return n_kv_heads <= 4 || work <= 5120;
+    if (n_kv_heads == kMaxWaves && work >= 8500 && pairs <= 3 * cus / 4) return true;
+    const int64_t most_pairs = n_kv_heads > kMaxWaves && work <= 1500 ? cus : work <= 512 ? 3 * cus / 4 : cus / 2;
+    return work <= 2048 && pairs <= most_pairs;
+}
+
 // The planner proper.  reqs[i]: tokens, start of the block table and q / output row of
 // request i (row i itself for a decode batch).
 int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, int32_t n_kv_heads,
-                     int32_t head_dim, bool merges_itself, int32_t target_workgroups, int32_t *plan_host,
+                     int32_t head_dim, int32_t dtype, bool merges_itself, int32_t target_workgroups, int32_t *plan_host,
                      int64_t plan_capacity_words, int32_t *n_items_out, int32_t *n_workgroups_out,
                      int64_t *plan_words_out, int64_t *workspace_bytes_out)
 {
@@ -591,15 +632,22 @@ int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, i
     // of 112 tiles takes 13.1 us in 18 shares (14.0 in 28), three of 13 tiles 10.7 in 9 (13.0 in 4).
     // The launcher knows that form by the number of workgroups (decode_splits_tokens), so a plan for
     // the other one is filled up with workgroups that have nothing to do where it would pass for it.
+    // (the generic kernel's forms likewise: gqa_splits_tokens)
     const bool own_rule = target_workgroups <= 0;
-    const bool split_shape = head_dim == kHeadDim && n_qo_heads / n_kv_heads <= kSplitMaxGroup;
-    const bool split = own_rule && split_shape && splitting_pays(total_tiles, longest, batch, n_kv_heads, merges_itself);
+    const bool two_forms = mfma_path(dtype, head_dim, n_qo_heads, n_kv_heads)
+                               ? n_qo_heads / n_kv_heads <= kSplitMaxGroup
+                               : gqa_shape(head_dim, n_qo_heads, n_kv_heads);
+    const bool split = own_rule && two_forms &&
+                       (mfma_path(dtype, head_dim, n_qo_heads, n_kv_heads)
+                            ? splitting_pays(total_tiles, longest, batch, n_kv_heads, merges_itself)
+                            : gqa_splitting_pays(total_tiles, longest, batch, n_kv_heads, head_dim));
     int64_t wgs = own_rule ? default_workgroups() : target_workgroups;
-    if (split) wgs = std::min<int64_t>(wgs / n_kv_heads, std::max<int64_t>(1, total_tiles / kSplitTilesPerShare));
+    if (split && head_dim == kHeadDim)
+        wgs = std::min<int64_t>(wgs / n_kv_heads, std::max<int64_t>(1, total_tiles / kSplitTilesPerShare));
     wgs = std::min<int64_t>(wgs, kMaxWorkgroups);
     wgs = std::min<int64_t>(wgs, std::max<int64_t>(1, total_tiles / kMinTilesPerWorkgroup));
     int64_t launched = wgs;
-    if (own_rule && split_shape && !split) launched = std::max<int64_t>(wgs, default_workgroups() / n_kv_heads + 1);
+    if (own_rule && two_forms && !split) launched = std::max<int64_t>(wgs, default_workgroups() / n_kv_heads + 1);
 
     // Lay the requests' tiles end to end; workgroup w owns global tiles
     // [w * T / wgs, (w + 1) * T / wgs).  Requests without tokens ride along as
@@ -680,8 +728,23 @@ extern "C" int dskv_decode_plan(const int32_t *kv_page_indptr_host,
                                 int32_t *n_workgroups_out, int64_t *plan_words_out,
                                 int64_t *workspace_bytes_out)
 {
+    return dskv_decode_plan_typed(kv_page_indptr_host, kv_last_page_len_host, batch, page_size, n_qo_heads,
+                                  n_kv_heads, head_dim, DSKV_BF16, target_workgroups, plan_host,
+                                  plan_capacity_words, n_items_out, n_workgroups_out, plan_words_out,
+                                  workspace_bytes_out);
+}
+
+extern "C" int dskv_decode_plan_typed(const int32_t *kv_page_indptr_host,
+                                      const int32_t *kv_last_page_len_host, int32_t batch,
+                                      int32_t page_size, int32_t n_qo_heads, int32_t n_kv_heads,
+                                      int32_t head_dim, int32_t dtype, int32_t target_workgroups,
+                                      int32_t *plan_host, int64_t plan_capacity_words,
+                                      int32_t *n_items_out, int32_t *n_workgroups_out,
+                                      int64_t *plan_words_out, int64_t *workspace_bytes_out)
+{
     using namespace dskv;
     DSKV_REQUIRE(batch >= 0, "decode_plan: negative batch");
+    DSKV_REQUIRE(dtype == DSKV_F32 || dtype == DSKV_F16 || dtype == DSKV_BF16, "decode_plan: unknown dtype %d", dtype);
     DSKV_REQUIRE(n_items_out && n_workgroups_out && plan_words_out && workspace_bytes_out,
                  "decode_plan: null output pointer");
     DSKV_REQUIRE(page_size > 0 && n_qo_heads > 0 && n_kv_heads > 0 && head_dim > 0 &&
@@ -704,8 +767,8 @@ extern "C" int dskv_decode_plan(const int32_t *kv_page_indptr_host,
                      "decode_plan: kv_last_page_len[%d] = %d outside [1, %d]", b, last, page_size);
         reqs[b] = DecodeRow{np > 0 ? (np - 1) * page_size + last : 0, kv_page_indptr_host[b], b};
     }
-    return plan_decode_rows(reqs.data(), batch, n_qo_heads, n_kv_heads, head_dim, true, target_workgroups, plan_host,
-                            plan_capacity_words, n_items_out, n_workgroups_out, plan_words_out,
+    return plan_decode_rows(reqs.data(), batch, n_qo_heads, n_kv_heads, head_dim, dtype, true, target_workgroups,
+                            plan_host, plan_capacity_words, n_items_out, n_workgroups_out, plan_words_out,
                             workspace_bytes_out);
 }
 
@@ -824,11 +887,9 @@ static int decode_attn_impl(void *out, const void *q, const void *pages_layer,
 #undef DSKV_LAUNCH_MFMA
         }
         DSKV_LAUNCH_CHECK("decode_attn_mfma_kernel");
-    } else if (n_qo_heads / n_kv_heads <= 8 && head_dim % 8 == 0 && head_dim <= 128 &&
+    } else if (gqa_shape(head_dim, n_qo_heads, n_kv_heads) &&
                ((uintptr_t)pages_layer % 16 == 0) && ((int64_t)n_kv_heads * head_dim * (dtype == DSKV_F32 ? 4 : 2)) % 16 == 0) {
-        // a wave carries the whole GQA group; four split an item's tokens where the plan has few shares
-        // for the chip and not so many short items instead (then one each is enough: the chip
-        // holds 2048 waves of this kernel)
+        // a wave carries the whole GQA group; four split an item's tokens where the plan says so
         const int group = n_qo_heads / n_kv_heads;
         const bool split = gqa_splits_tokens(n_items, n_workgroups, n_kv_heads);
         dim3 grid((unsigned)n_items, (unsigned)n_kv_heads);

@@ -416,11 +416,24 @@ extern "C" int dskv_mixed_plan(const int32_t *qo_indptr_host, const int32_t *kv_
                                int32_t route_one_row_requests, int32_t *plan_host,
                                int64_t capacity_words, dskv_mixed_plan_t *info)
 {
+    return dskv_mixed_plan_typed(qo_indptr_host, kv_page_indptr_host, kv_last_page_len_host, batch, page_size,
+                                 n_qo_heads, n_kv_heads, head_dim, DSKV_BF16, target_workgroups,
+                                 route_one_row_requests, plan_host, capacity_words, info);
+}
+
+extern "C" int dskv_mixed_plan_typed(const int32_t *qo_indptr_host, const int32_t *kv_page_indptr_host,
+                                     const int32_t *kv_last_page_len_host, int32_t batch,
+                                     int32_t page_size, int32_t n_qo_heads, int32_t n_kv_heads,
+                                     int32_t head_dim, int32_t dtype, int32_t target_workgroups,
+                                     int32_t route_one_row_requests, int32_t *plan_host,
+                                     int64_t capacity_words, dskv_mixed_plan_t *info)
+{
     using namespace dskv;
     DSKV_REQUIRE(info, "mixed_plan: null info pointer");
     *info = dskv_mixed_plan_t{};
     info->n_splits = 1;
     DSKV_REQUIRE(batch >= 0, "mixed_plan: negative batch");
+    DSKV_REQUIRE(dtype == DSKV_F32 || dtype == DSKV_F16 || dtype == DSKV_BF16, "mixed_plan: unknown dtype %d", dtype);
     DSKV_REQUIRE(page_size > 0 && n_qo_heads > 0 && n_kv_heads > 0 && head_dim > 0 &&
                      n_qo_heads % n_kv_heads == 0,
                  "mixed_plan: bad shape (page %d, heads %d/%d, dim %d)", page_size, n_qo_heads,
@@ -518,8 +531,8 @@ extern "C" int dskv_mixed_plan(const int32_t *qo_indptr_host, const int32_t *kv_
         const int cus = target_workgroups > 0 ? std::min<int>(target_workgroups, kMaxWorkgroups) : compute_units();
         decode_target = std::max(1, cus / head_groups);
     }
-    rc = plan_decode_rows(rows.data(), (int32_t)rows.size(), n_qo_heads, n_kv_heads, head_dim, false, decode_target,
-                          plan_host + at, capacity_words - at, &info->n_decode_items,
+    rc = plan_decode_rows(rows.data(), (int32_t)rows.size(), n_qo_heads, n_kv_heads, head_dim, dtype, false,
+                          decode_target, plan_host + at, capacity_words - at, &info->n_decode_items,
                           &info->n_decode_workgroups, &decode_words, &info->decode_workspace_bytes);
     if (rc) return rc;
     info->n_decode_rows = (int32_t)rows.size();

@@ -53,6 +53,7 @@ class GraphedDecodeStep:
                                    last_page_len_host=ctx.host["kv_last_page_lens"],
                                    indices_host=ctx.host["kv_page_indices"],
                                    target_workgroups=self.target_workgroups, plan_buffers=self.plan,
+                                   data_type=ctx.page_pool.main_dtype,
                                    **self.shape)
         return ctx
 

@@ -200,7 +200,7 @@ class FlashDecodeCtx(FlashForwardCtx):
         dev = wrapper.begin_forward_with_metadata(
             total, fill, starts["kv_page_indptr"], starts["kv_page_indices"], host["kv_page_indptr"],
             host["kv_last_page_lens"], host["kv_page_indices"], num_qo_heads, num_kv_heads, head_dim,
-            page_size, pool.main_device, target_workgroups)
+            page_size, pool.main_device, target_workgroups, data_type=pool.main_dtype)
         v = {f: dev[starts[f]: starts[f] + meta[f].shape[0]] for f in _FIELDS}
         return cls(bsz=len(task_datas), seqlens=v["seqlens"], layer_id=0, page_pool=pool,
                    offsets=v["offsets"], indptr=v["indptr"], kv_page_indices=v["kv_page_indices"],
@@ -252,7 +252,7 @@ class FlashPrefillCtx(FlashForwardCtx):
         dev = wrapper.begin_forward_with_metadata(
             total, fill, starts, host["indptr"], host["kv_page_indptr"], host["kv_last_page_lens"],
             host["kv_page_indices"], num_qo_heads, num_kv_heads, head_dim, page_size, pool.main_device,
-            target_workgroups)
+            target_workgroups, data_type=pool.main_dtype)
         v = {f: dev[starts[f]: starts[f] + meta[f].shape[0]] for f in _FIELDS}
         return cls(bsz=len(task_datas), seqlens=v["seqlens"], layer_id=0, page_pool=pool,
                    offsets=v["offsets"], indptr=v["indptr"], kv_page_indices=v["kv_page_indices"],

@@ -124,8 +124,12 @@ class _PagedWrapper:
         self._max_page_id = -1
         self._empty_requests = []
 
-    def _shape_args(self, num_qo_heads: int, num_kv_heads: int, head_dim: int, page_size: int) -> None:
+    def _shape_args(self, num_qo_heads: int, num_kv_heads: int, head_dim: int, page_size: int,
+                    data_type=None) -> None:
         self._hq, self._hkv, self._d, self._p = num_qo_heads, num_kv_heads, head_dim, page_size
+        # how many shares are best depends on the kernel, which depends on the type of the pages: fp32
+        # ones have kernels of their own.  Any plan is right for any type.
+        self._plan_dtype = _lib.F32 if data_type in (torch.float32, "float32") else _lib.BF16
 
     @staticmethod
     def _host(t: torch.Tensor, host: Optional[torch.Tensor]) -> torch.Tensor:
@@ -188,14 +192,16 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
                       head_dim: int, page_size: int, *, indptr_host: Optional[torch.Tensor] = None,
                       last_page_len_host: Optional[torch.Tensor] = None,
                       indices_host: Optional[torch.Tensor] = None,
-                      target_workgroups: int = 0, plan_buffers=None, **_ignored) -> None:
-        """The *_host arguments are host copies of the index tensors: the planner and the
+                      target_workgroups: int = 0, plan_buffers=None, data_type=None, **_ignored) -> None:
+        """data_type: element type of the pages, a torch dtype or its name (None: 16 bits), for the
+        planner only: any plan gives the right result for any type.
+        The *_host arguments are host copies of the index tensors: the planner and the
         checks of the block tables run on the host; without them the device tensors are read
         back, which synchronises.
         plan_buffers: optional staged upload (an object with staging() / upload(words) /
         dev, see model.context.flash.StagedUpload) that receives the work list instead of
         fresh tensors, for callers that replay captured launches."""
-        self._shape_args(num_qo_heads, num_kv_heads, head_dim, page_size)
+        self._shape_args(num_qo_heads, num_kv_heads, head_dim, page_size, data_type)
         self._indptr, self._indices = _i32(indptr), _i32(indices)
         h_indptr = self._host(indptr, indptr_host)
         h_last = self._host(last_page_len, last_page_len_host)
@@ -242,10 +248,10 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
         batch = h_indptr.shape[0] - 1
         n_items, n_wgs = ctypes.c_int32(), ctypes.c_int32()
         words, ws = ctypes.c_int64(), ctypes.c_int64()
-        rc = _lib.lib().dskv_decode_plan(h_indptr.data_ptr(), h_last.data_ptr(), batch, self._p,
-                                         self._hq, self._hkv, self._d, target_workgroups,
-                                         plan.data_ptr(), cap, ctypes.byref(n_items), ctypes.byref(n_wgs),
-                                         ctypes.byref(words), ctypes.byref(ws))
+        rc = _lib.lib().dskv_decode_plan_typed(h_indptr.data_ptr(), h_last.data_ptr(), batch, self._p,
+                                               self._hq, self._hkv, self._d, self._plan_dtype, target_workgroups,
+                                               plan.data_ptr(), cap, ctypes.byref(n_items), ctypes.byref(n_wgs),
+                                               ctypes.byref(words), ctypes.byref(ws))
         _lib.check(rc, "decode begin_forward")
         if ws.value > self._workspace.numel() * self._workspace.element_size():
             raise RuntimeError(f"decode workspace too small: need {ws.value} bytes")
@@ -260,7 +266,7 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
                                     indptr_host: torch.Tensor, last_page_len_host: torch.Tensor,
                                     indices_host: torch.Tensor, num_qo_heads: int, num_kv_heads: int,
                                     head_dim: int, page_size: int, device: torch.device,
-                                    target_workgroups: int = 0) -> torch.Tensor:
+                                    target_workgroups: int = 0, data_type=None) -> torch.Tensor:
         """begin_forward for callers that also have the step's other index arrays to upload
         (the forward context): metadata and work list travel in ONE pinned block and ONE
         upload kernel instead of one each.  fill_metadata(view) writes the caller's
@@ -269,7 +275,7 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
         the device tensor that holds the metadata words (the caller slices its views)."""
         if meta_words % 4:
             raise ValueError("meta_words must be a multiple of 4 (16-byte alignment of the work list)")
-        self._shape_args(num_qo_heads, num_kv_heads, head_dim, page_size)
+        self._shape_args(num_qo_heads, num_kv_heads, head_dim, page_size, data_type)
         h_indptr = indptr_host.to(torch.int32).contiguous()
         h_last = last_page_len_host.to(torch.int32).contiguous()
         self._check_block_tables(h_indptr, indices_host, indices_host, h_last)
@@ -378,9 +384,10 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
                       paged_kv_indptr_host: Optional[torch.Tensor] = None,
                       paged_kv_last_page_len_host: Optional[torch.Tensor] = None,
                       paged_kv_indices_host: Optional[torch.Tensor] = None,
-                      target_workgroups: int = 0, route_one_row_requests: bool = True,
+                      target_workgroups: int = 0, route_one_row_requests: bool = True, data_type=None,
                       **_ignored) -> None:
-        """The *_host arguments are host copies of the index tensors (the planner and the
+        """data_type: as in the decode wrapper's begin_forward.
+        The *_host arguments are host copies of the index tensors (the planner and the
         checks of the block tables run on the host; without them the device tensors are read
         back, which synchronises).
         target_workgroups: a batch of few query tiles (a chunk of a few hundred tokens) is
@@ -392,7 +399,7 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
         tiles share the compute units, if the decode rows hold enough kv tokens); False keeps
         them on the tile path (one live row of a 64-row tile each), as a plan of
         dskv_prefill_plan does; _lib.ROUTE_TWO_LAUNCHES / _lib.ROUTE_SHARED_LAUNCH force a form."""
-        self._shape_args(num_qo_heads, num_kv_heads, head_dim, page_size)
+        self._shape_args(num_qo_heads, num_kv_heads, head_dim, page_size, data_type)
         self._qo_indptr, self._indptr = _i32(qo_indptr), _i32(paged_kv_indptr)
         self._indices, self._last = _i32(paged_kv_indices), _i32(paged_kv_last_page_len)
         h_qo = self._host(qo_indptr, qo_indptr_host)
@@ -437,9 +444,9 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
         ws_bytes = self._workspace.numel() * self._workspace.element_size()
         route = int(route)          # True = _lib.ROUTE_AUTO
         for target, routed in ((target_workgroups, route), (-1, route), (-1, _lib.ROUTE_OFF)):
-            rc = _lib.lib().dskv_mixed_plan(h_qo.data_ptr(), h_kv.data_ptr(), h_last.data_ptr(), batch,
-                                            self._p, self._hq, self._hkv, self._d, target, int(routed),
-                                            plan.data_ptr(), cap, ctypes.byref(info))
+            rc = _lib.lib().dskv_mixed_plan_typed(h_qo.data_ptr(), h_kv.data_ptr(), h_last.data_ptr(), batch,
+                                                  self._p, self._hq, self._hkv, self._d, self._plan_dtype, target,
+                                                  int(routed), plan.data_ptr(), cap, ctypes.byref(info))
             _lib.check(rc, "prefill begin_forward")
             if info.tile_workspace_bytes + info.decode_workspace_bytes <= ws_bytes:
                 break
@@ -454,7 +461,8 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
                                     paged_kv_last_page_len_host: torch.Tensor,
                                     paged_kv_indices_host: torch.Tensor, num_qo_heads: int,
                                     num_kv_heads: int, head_dim: int, page_size: int, device: torch.device,
-                                    target_workgroups: int = 0, route_one_row_requests: bool = True) -> torch.Tensor:
+                                    target_workgroups: int = 0, route_one_row_requests: bool = True,
+                                    data_type=None) -> torch.Tensor:
         """begin_forward for callers that also have the step's other index arrays to upload
         (the forward context): metadata and plan travel in ONE pinned block and ONE upload
         kernel.  fill_metadata(view) writes the caller's meta_words int32 words (a multiple of
@@ -463,7 +471,7 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
         device tensor that holds the metadata words (the caller slices its views)."""
         if meta_words % 4:
             raise ValueError("meta_words must be a multiple of 4 (16-byte alignment of the plan)")
-        self._shape_args(num_qo_heads, num_kv_heads, head_dim, page_size)
+        self._shape_args(num_qo_heads, num_kv_heads, head_dim, page_size, data_type)
         h_qo = qo_indptr_host.to(torch.int32).contiguous()
         h_kv = paged_kv_indptr_host.to(torch.int32).contiguous()
         h_last = paged_kv_last_page_len_host.to(torch.int32).contiguous()

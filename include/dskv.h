@@ -95,7 +95,9 @@ int dskv_upload_words(void *dst, const void *src_pinned, int64_t n_words, void *
  * per item - the variable-length part last, so that the layout depends only on
  * the batch and the number of workgroups); the caller copies it to the device
  * once per step and reuses it for every layer.
- *   target_workgroups:   <= 0 = one per compute unit of the current device.
+ *   target_workgroups:   <= 0: the planner's choice, one share per compute unit of the current device
+ *                        or, for small batches, fewer; n_workgroups may then count workgroups
+ *                        that have no share.
  *   plan_capacity_words: size of plan_host; dskv_decode_plan_bound(batch,
  *                        total_tokens) words always suffice.
  *   workspace_bytes_out: device scratch dskv_decode_attn needs for the partial
@@ -107,6 +109,17 @@ int dskv_decode_plan(const int32_t *kv_page_indptr_host, const int32_t *kv_last_
                      int32_t head_dim, int32_t target_workgroups, int32_t *plan_host,
                      int64_t plan_capacity_words, int32_t *n_items_out, int32_t *n_workgroups_out,
                      int64_t *plan_words_out, int64_t *workspace_bytes_out);
+/*
+ * The same with the element type of the pages.  Which kernel computes a batch depends on it, and how many
+ * shares are best on the kernel; any plan gives the right result for any type.  dskv_decode_plan
+ * plans for 16-bit elements.
+ */
+int dskv_decode_plan_typed(const int32_t *kv_page_indptr_host, const int32_t *kv_last_page_len_host,
+                           int32_t batch, int32_t page_size, int32_t n_qo_heads, int32_t n_kv_heads,
+                           int32_t head_dim, int32_t dtype, int32_t target_workgroups,
+                           int32_t *plan_host, int64_t plan_capacity_words, int32_t *n_items_out,
+                           int32_t *n_workgroups_out, int64_t *plan_words_out,
+                           int64_t *workspace_bytes_out);
 
 /*
  * out, q: (batch, n_qo_heads, head_dim) of dtype; pages_layer as for append.
@@ -328,6 +341,12 @@ int dskv_mixed_plan(const int32_t *qo_indptr_host, const int32_t *kv_page_indptr
                     int32_t n_qo_heads, int32_t n_kv_heads, int32_t head_dim,
                     int32_t target_workgroups, int32_t route_one_row_requests,
                     int32_t *plan_host, int64_t capacity_words, dskv_mixed_plan_t *info);
+/* The same with the element type of the pages, as dskv_decode_plan_typed takes it. */
+int dskv_mixed_plan_typed(const int32_t *qo_indptr_host, const int32_t *kv_page_indptr_host,
+                          const int32_t *kv_last_page_len_host, int32_t batch, int32_t page_size,
+                          int32_t n_qo_heads, int32_t n_kv_heads, int32_t head_dim, int32_t dtype,
+                          int32_t target_workgroups, int32_t route_one_row_requests,
+                          int32_t *plan_host, int64_t capacity_words, dskv_mixed_plan_t *info);
 int dskv_mixed_attn(void *out, const void *q, const int32_t *qo_indptr, const void *pages_layer,
                     const int32_t *kv_page_indices, const int32_t *kv_page_indptr,
                     const int32_t *kv_last_page_len, const int32_t *plan_dev,

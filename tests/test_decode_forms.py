@@ -10,7 +10,7 @@ from deserve_amd import _lib
 CUS, XCDS = 256, 8
 
 
-def _plan(lens, n_kv, group=4, d=128, page=16, target=0):
+def _plan(lens, n_kv, group=4, d=128, page=16, target=0, dtype=_lib.BF16):
     """(shares, items, most tiles of an item)."""
     lib = _lib.lib()
     n = -(-np.asarray(lens, np.int64) // page)
@@ -21,7 +21,7 @@ def _plan(lens, n_kv, group=4, d=128, page=16, target=0):
     items, wgs, words, ws = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int64(), ctypes.c_int64()
     out = [ctypes.byref(x) for x in (items, wgs, words, ws)]
     head = (indptr.ctypes.data, last.ctypes.data, len(lens), page, n_kv * group, n_kv, d)
-    rc = lib.dskv_decode_plan(*head, target, plan.ctypes.data, cap, *out)
+    rc = lib.dskv_decode_plan_typed(*head, dtype, target, plan.ctypes.data, cap, *out)
     assert rc == 0, _lib.last_error()
     table = plan[4 + wgs.value + 1 + 2 * len(lens): words.value].reshape(-1, 8)
     return wgs.value, items.value, int((-(-(table[:, 2] - table[:, 1]) // 16)).max())
@@ -86,3 +86,39 @@ def test_rows_of_a_prefill_batch_have_one_rule_with_and_without_chunks(tiles, sp
     alone = _mixed([1] * 8, rows)
     beside = _mixed([1] * 8 + [100], rows + [100], route=_lib.ROUTE_TWO_LAUNCHES)
     assert alone == beside and _launch(alone[1], alone[0], 8)[1] == splits
+
+
+@pytest.mark.parametrize("d", [128, 64])
+@pytest.mark.parametrize("n_kv,lens", [
+    (8, [20000] + [64] * 128), (8, [16000] + [100] * 140), (8, [300] * 130), (8, [50, 150] * 12),
+    (8, [300, 900] * 32), (8, [20000]), (8, [512] * 8), (16, [400] * 40), (4, [64] * 128), (2, [2000] * 3)])
+def test_no_wave_of_an_fp32_batch_walks_longer_than_in_shares_of_a_unit_each(n_kv, lens, d):
+    """Planner and launcher agree: where the plan has few, large shares, four waves have an item each."""
+    shares, items, longest = _plan(lens, n_kv, d=d, dtype=_lib.F32)
+    splits = _launch(items, shares, n_kv, d=d, dtype=_lib.F32)[1]
+    _, _, longest_of_256 = _plan(lens, n_kv, d=d, target=CUS, dtype=_lib.F32)
+    assert -(-longest // (4 if splits else 1)) <= longest_of_256
+
+
+@pytest.mark.parametrize("n_kv,lens,d,splits", [
+    (8, [512] * 8, 128, True), (8, [512] * 17, 128, False), (8, [530] * 8, 128, False),
+    (8, [100] * 24, 128, False), (8, [20] * 64, 128, False), (4, [1000], 128, True), (8, [11000], 128, False),
+    (8, [16 * 1250] + [60] * 23, 128, True), (2, [5000] * 3, 128, True), (1, [100] * 24, 128, True),
+    (1, [1000] * 24, 128, False), (1, [900] * 24, 128, True), (12, [60] * 16, 128, True), (8, [25] * 24, 128, True), (8, [800] * 24, 128, True), (8, [800] * 25, 128, False), (1, [20000], 128, True), (8, [40] * 24, 64, True), (8, [20] * 64, 64, False)])
+def test_which_fp32_batches_split_an_item_over_four_waves(n_kv, lens, d, splits):
+    shares, items, _ = _plan(lens, n_kv, d=d, dtype=_lib.F32)
+    assert _launch(items, shares, n_kv, d=d, dtype=_lib.F32)[1] == splits
+
+
+def test_untyped_plans_are_those_of_16_bit_pages():
+    lib, lens = _lib.lib(), [700, 40, 3]
+    n = -(-np.asarray(lens) // 16)
+    indptr, last = np.concatenate([[0], np.cumsum(n)]).astype(np.int32), np.array([12, 8, 3], np.int32)
+    out = [ctypes.byref(t()) for t in (ctypes.c_int32, ctypes.c_int32, ctypes.c_int64, ctypes.c_int64)]
+    head = (indptr.ctypes.data, last.ctypes.data, 3, 16, 32, 8, 128)
+    cap = lib.dskv_decode_plan_bound(3, 743)
+    a, b = np.zeros(cap, np.int32), np.zeros(cap, np.int32)
+    assert lib.dskv_decode_plan(*head, 0, a.ctypes.data, cap, *out) == 0
+    assert lib.dskv_decode_plan_typed(*head, _lib.F16, 0, b.ctypes.data, cap, *out) == 0
+    assert np.array_equal(a, b)
+    assert lib.dskv_decode_plan_typed(*head, 7, 0, b.ctypes.data, cap, *out) == -1 and "dtype" in _lib.last_error()
