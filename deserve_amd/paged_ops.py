@@ -304,7 +304,10 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
                 out: Optional[torch.Tensor] = None, k_append: Optional[torch.Tensor] = None,
                 v_append: Optional[torch.Tensor] = None, rope_offsets: Optional[torch.Tensor] = None,
                 rope_theta: float = 500000.0, **_ignored) -> torch.Tensor:
-        """phases: 1 = split-KV pass only, 2 = merge pass only, 3 = both (default).
+        """phases: 1 = split-KV pass only, 2 = merge pass only, 3 = both (default).  The two passes one by
+        one add the parts of a cut request in another order than both in one call may: their 16-bit
+        results can differ by one unit in the last place.
+        out: optional result tensor (contiguous, q's dtype, at least q's elements).
         k_append, v_append (batch, Hkv, D): the step's token of every request, not yet in the
         pages - the attention launch writes them into their slots itself (one launch less than
         append_paged_kv_cache + forward; see fused_append_supported).
@@ -320,6 +323,8 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
         self._check_pool(paged_kv_data, q.dtype)
         if out is None:
             out = torch.empty_like(q)
+        elif out.dtype != q.dtype or out.numel() < q.numel() or not out.is_contiguous():
+            raise ValueError("out must be contiguous, of q's dtype, and hold at least q's elements")
         scale = 1.0 / math.sqrt(self._d) if sm_scale is None else sm_scale
         ws_bytes = self._workspace.numel() * self._workspace.element_size()
         table = None

@@ -98,6 +98,21 @@ def test_prefill_begin_forward_refuses_bad_block_tables():
         w.begin_forward(_i32([0, 4, 8]), _i32([0, 1, 2]), _i32([3, 4]), _i32([4]), **shape)
 
 
+def test_decode_forward_refuses_an_out_it_cannot_fill():
+    w = _decode()
+    w._shape_args(32, 8, 128, 16)
+    w._check_block_tables(_i32([0, 1, 2]), _i32([0, 1]), None, _i32([16, 4]))
+    cap = 4096 * 16
+    w._plan_into(torch.zeros(cap, dtype=torch.int32), cap, _i32([0, 1, 2]), _i32([16, 4]), 0)
+    w._planned = True
+    q, pages = torch.zeros((2, 32, 128), dtype=torch.bfloat16), torch.zeros((2, 2, 16, 8, 128), dtype=torch.bfloat16)
+    wide = torch.zeros((2, 32, 256), dtype=torch.bfloat16)
+    for out in (wide[..., :128], torch.zeros_like(q, dtype=torch.float32), torch.zeros_like(q[:1]),
+                torch.zeros((32, 2, 128), dtype=torch.bfloat16).transpose(0, 1)):
+        with pytest.raises(ValueError, match="out must be"):
+            w.forward(q, pages, out=out)
+
+
 def test_gather_and_scatter_refuse_page_ids_outside_the_pool():
     pool = PagePool(2, 8, 4, CPU, torch.float16, n_kv_heads=1, head_dim=8)
     for bad in ([0, 8], [-1, 3]):
