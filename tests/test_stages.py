@@ -177,3 +177,30 @@ def test_step_request_helpers():
     assert r.exec_seqlens == [1, 1] and r.init_tasks == {} and r.offload_task_ids == []
     with pytest.raises(AssertionError):
         r.append_exec("c", toks(0), None)
+
+
+# ------------------------------------------------------------------ KV stage
+def test_a_stage_takes_the_results_of_a_core_of_ones_own():
+    """A core with paged_forward(xq, xk, xv, ctx) that returns a tensor of its own, as a subclass and
+    as a method put in place: the stage stacks what it returns, layer by layer."""
+    from types import SimpleNamespace
+
+    from deserve_amd.model.layer.attention import PagedAttentionCore
+    from deserve_amd.stage import KVStage, StageArgs
+
+    seen = []
+
+    class Own(PagedAttentionCore):
+        def paged_forward(self, xq, xk, xv, ctx):
+            seen.append((ctx.layer_id, xk.shape, xv.shape))
+            return xq.reshape(-1, self.dim) * 2
+
+    q, k = torch.randn(3, 5, 4, 8), torch.randn(3, 5, 2, 8)
+    args = StageArgs(n_heads=4, n_kv_heads=2, dim=32, page_size=16, n_layers=3)
+    stage, ctx = KVStage(args), SimpleNamespace(layer_id=0)
+    stage.core = Own(4, 2, 8)
+    assert torch.equal(stage.forward((q, k, k), ctx), q.reshape(3, 5, 32) * 2)
+    assert [s[0] for s in seen] == [0, 1, 2] and ctx.layer_id == 3
+    stage = KVStage(args)
+    stage.core.paged_forward = lambda xq, xk, xv, ctx: xq.reshape(-1, 32) + 1
+    assert torch.equal(stage.forward((q, k, k), SimpleNamespace(layer_id=0)), q.reshape(3, 5, 32) + 1)
