@@ -43,7 +43,8 @@ struct dskv_swap {
         const char *begin, *end;
     };
     std::vector<HostRange> host_pending;
-    bool in_after_out = false;         // the next swap-in waits for everything on the out stream
+    bool host_overflow = false;        // more ranges than are kept
+    bool out_reads_pool = false;       // an exchange's gathers may still run on the out stream
     // [direction: 0 = out (D2H), 1 = in (H2D)]
     hipStream_t stream[2] = {nullptr, nullptr};
     void *staging[2] = {nullptr, nullptr};
@@ -103,6 +104,13 @@ static void recycle(dskv_swap *h, dskv_swap::IdStretch &st)
         }
 }
 
+// Nothing runs on the out stream.
+static void forget_out(dskv_swap *h)
+{
+    h->host_pending.clear();
+    h->host_overflow = h->out_reads_pool = false;
+}
+
 static int wait_all(dskv_swap *h)
 {
     for (int d = 0; d < 2; d++) DSKV_HIP(hipStreamSynchronize(h->stream[d]));
@@ -112,8 +120,7 @@ static int wait_all(dskv_swap *h)
     for (auto &st : h->out_pending) h->spare_events.push_back(st.copied);
     h->out_pending.clear();
     h->out_head = 0;
-    h->host_pending.clear();
-    h->in_after_out = false;
+    forget_out(h);
     return 0;
 }
 
@@ -165,18 +172,21 @@ static int hold_out_staging(dskv_swap *h, int64_t begin, int64_t bytes)
     return 0;
 }
 
-// Whether copies out that may still run write [host, host + bytes).
-static bool copies_out_write(dskv_swap *h, const void *host, int64_t bytes)
+// Drops what is on record about copies out that have all finished (a query, never a wait).
+static void retire_out(dskv_swap *h)
 {
-    if (h->host_pending.empty() && !h->in_after_out) return false;
+    if (h->host_pending.empty() && !h->host_overflow && !h->out_reads_pool) return;
     const hipError_t q = hipStreamQuery(h->stream[0]);   // also what a call that failed half way left there
     (void)hipGetLastError();
-    if (q == hipSuccess) {
-        h->host_pending.clear();
-        h->in_after_out = false;
-        return false;
-    }
-    if (h->in_after_out) return true;
+    if (q == hipSuccess) forget_out(h);
+}
+
+// Whether a swap-in from [host, host + bytes) has to wait for the out stream: copies out that may
+// still run write there, or an exchange reads the pool.
+static bool waits_for_out(dskv_swap *h, const void *host, int64_t bytes)
+{
+    retire_out(h);
+    if (h->host_overflow || h->out_reads_pool) return true;
     const char *begin = (const char *)host, *end = begin + bytes;
     for (const auto &r : h->host_pending)
         if (r.begin < end && begin < r.end) return true;
@@ -298,10 +308,10 @@ static int check_ids(const char *who, const int32_t *ids, int32_t n, int64_t lay
     return 0;
 }
 
-// The stream of direction `dir` waits for: the caller's stream, the id upload,
-// and everything previously enqueued in the opposite direction (an earlier
-// swap-out may still be reading pages that this swap-in is about to overwrite,
-// and the other way round).
+// For an exchange, which uses both streams in its own order: the stream of direction `dir` waits for
+// the caller's stream, the id upload and everything previously enqueued in the opposite direction (its
+// gathers run on the out stream behind the scatters of earlier swap-ins, its scatters behind the
+// copies of earlier swap-outs into host memory that it may read).
 static int open_direction(dskv_swap *h, int dir, hipStream_t after, hipStream_t ids_stream)
 {
     hipStream_t s = h->stream[dir];
@@ -482,10 +492,11 @@ extern "C" int dskv_swap_out_async(dskv_swap_t *h, void *host_dst, const void *p
     IdsGuard ids_guard{h, true};
     DSKV_HIP(hipEventRecord(h->ready, (hipStream_t)after_stream));
     DSKV_HIP(hipStreamWaitEvent(pages, h->ready, 0));
+    retire_out(h);
     if (h->host_pending.size() < kMaxHostRanges)
         h->host_pending.push_back({(const char *)host_dst, (const char *)host_dst + rows * page_bytes});
     else
-        h->in_after_out = true;
+        h->host_overflow = true;
     for (int64_t r0 = 0; r0 < rows; r0 += rows_per_chunk) {
         const int64_t r1 = std::min(rows, r0 + rows_per_chunk), bytes = (r1 - r0) * page_bytes;
         int64_t at = 0;
@@ -528,7 +539,7 @@ extern "C" int dskv_swap_in_async(dskv_swap_t *h, void *pool, const void *host_s
     IdsGuard ids_guard{h, true};
     DSKV_HIP(hipEventRecord(h->ready, (hipStream_t)after_stream));
     DSKV_HIP(hipStreamWaitEvent(s, h->ready, 0));
-    if (copies_out_write(h, host_src, rows * page_bytes)) {
+    if (waits_for_out(h, host_src, rows * page_bytes)) {
         DSKV_HIP(hipEventRecord(h->dir_done[0], h->stream[0]));
         DSKV_HIP(hipStreamWaitEvent(s, h->dir_done[0], 0));
     }
@@ -576,7 +587,7 @@ extern "C" int dskv_swap_exchange_async(dskv_swap_t *h, void *host_dst, const vo
     const bool same_buffer = host_dst == host_src;
     // its gathers run on the out stream (in front of its own copies, chunk by chunk): whatever
     // touches the pool next waits for that stream
-    h->in_after_out = true;
+    h->out_reads_pool = true;
     int c = 0;
     for (int64_t r0 = 0; r0 < rows; r0 += rows_per_chunk, c ^= 1) {
         const int64_t r1 = std::min(rows, r0 + rows_per_chunk);
@@ -710,7 +721,7 @@ extern "C" int dskv_swap_fence_pages(dskv_swap_t *h, void *stream)
 {
     using namespace dskv;
     DSKV_REQUIRE(h, "swap_fence_pages: null handle");
-    if (h->in_after_out) return dskv_swap_fence(h, stream);   // an exchange also reads the pool on the out stream
+    if (h->out_reads_pool) return dskv_swap_fence(h, stream);
     DSKV_HIP(hipEventRecord(h->fence, h->stream[1]));
     DSKV_HIP(hipStreamWaitEvent((hipStream_t)stream, h->fence, 0));
     return 0;

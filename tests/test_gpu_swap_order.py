@@ -82,3 +82,36 @@ def test_work_on_an_offloaded_chunk_is_ordered_without_synchronize():
     assert np.array_equal(got.view(torch.int16).cpu().numpy(), want)
     mgr.synchronize()
     assert np.array_equal(handle.retrieve()[: L * n].view(torch.int16).numpy(), want)
+
+
+@pytest.mark.parametrize("idle_between", [True, False])
+def test_pages_fence_never_waits_for_the_link_however_many_offloads_went_before(idle_between):
+    """fence_pages behind more offloads than the engine keeps host ranges of (256), all finished or
+    still on their way: the current stream goes on while the last gigabyte (19 ms) travels."""
+    from deserve_amd.kvcache import _native
+    from deserve_amd.kvcache.paged.page_pool import GpuPagePool
+    from deserve_amd.kvcache.pinned.pinned_memory import pinned_empty
+
+    print("[case] pages fence behind 300 offloads", idle_between, flush=True)
+    L, P, n = 16, 16, 1024                       # 1 MiB of all layers per page id
+    pool = GpuPagePool(L, n, P, "cuda", torch.bfloat16)
+    host = pinned_empty((L * n,) + tuple(pool.pages.shape[2:]), torch.bfloat16)
+    every, one = torch.arange(n, dtype=torch.int32), torch.zeros(1, dtype=torch.int32)
+    eng = _native.SwapEngine()
+    assert eng.independent
+    if not idle_between:
+        for _ in range(2):                       # keep the link busy while the calls are made
+            eng.swap_out(host, pool, every)
+    for i in range(300):
+        eng.swap_out(host[i * L: (i + 1) * L], pool, one)
+    if idle_between:
+        torch.cuda.synchronize()                 # the engine is not told
+    eng.swap_out(host, pool, every)
+    eng.fence_pages()
+    event = torch.cuda.Event()
+    event.record()
+    event.synchronize()
+    assert not eng.done()                        # the pages are free again, their copies on the link
+    eng.wait()
+    assert eng.done()
+    eng.close()
