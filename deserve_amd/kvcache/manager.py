@@ -14,8 +14,6 @@ that stream on a chunk (a copy of ``handle.retrieve()``) is ordered by ``retriev
 """
 from __future__ import annotations
 
-import functools
-
 import torch
 
 from deserve_amd.kvcache import _native
@@ -23,6 +21,30 @@ from deserve_amd.kvcache.paged.chunk_pool import ChunkHandle, CpuChunkPool
 from deserve_amd.kvcache.paged.kvcache import PagedKVCache
 from deserve_amd.kvcache.paged.page_table import PageTableAllocator
 from deserve_amd.kvcache.virtual import VirtualPagedKVCache, VirtualPagePool
+
+
+class _Progress:
+    """Copies out of one manager: enqueued so far; of these, waited for."""
+
+    def __init__(self) -> None:
+        self.enqueued = self.finished = 0
+
+
+class _CopyOut:
+    """A request's trip into its chunk (chunk_pool.PendingWrite)."""
+
+    def __init__(self, engine: _native.SwapEngine, progress: _Progress) -> None:
+        progress.enqueued += 1
+        self.engine, self.progress, self.number = engine, progress, progress.enqueued
+
+    def finished(self) -> bool:
+        return self.number <= self.progress.finished or not self.engine.is_open   # closing one finishes its copies
+
+    def poll(self) -> bool:
+        return self.finished() or self.engine.done()
+
+    def fence(self) -> None:
+        self.engine.fence()
 
 
 class KVCacheManager:
@@ -36,7 +58,7 @@ class KVCacheManager:
         shared = getattr(virtual_page_pool, "engine", None)
         self.engine = shared if shared is not None and staging_bytes == shared.staging_bytes \
             else _native.SwapEngine(staging_bytes)
-        self._copies_out, self._finished = 0, 0    # enqueued so far; of these, waited for
+        self._progress = _Progress()
 
     def copy_gpu_to_cpu(self, paged_kvcache: PagedKVCache[VirtualPagePool],
                         task_id: str) -> ChunkHandle:
@@ -45,18 +67,15 @@ class KVCacheManager:
         n = table.occupied
         handle = self.cpu_chunk_pool.alloc(n)
         rows = n * self.cpu_chunk_pool.num_layers
+        # the engine keeps the order of its own copies; another manager's may still write this memory
+        self.cpu_chunk_pool.order_behind_writes(handle, but=self.engine)
         self.engine.swap_out(handle.rows()[:rows], self.virtual_page_pool, table.retrieve())
         # pages may be handed to another request right after this returns: they have been packed
         # by the time the current stream goes on, and travel while it does
         self.engine.fence_pages()
-        # not so work on the chunk: retrieve() waits for the trip
-        self._copies_out += 1
-        handle.fence = functools.partial(self._fence_chunk, self._copies_out)
+        # not so work on the chunk's memory: retrieve() waits for the trip
+        self.cpu_chunk_pool.note_write(handle, _CopyOut(self.engine, self._progress))
         return handle
-
-    def _fence_chunk(self, copy: int) -> None:
-        if copy > self._finished and self.engine.is_open:    # closing an engine finishes its copies
-            self.engine.fence()
 
     def copy_cpu_to_gpu(self, chunk_handle: ChunkHandle, task_id: str) -> VirtualPagedKVCache:
         """Only the copy; the caller frees the chunk and owns the new cache."""
@@ -68,6 +87,7 @@ class KVCacheManager:
         table = self.page_table_allocator.alloc()
         table.extend(ids)
         rows = n * self.cpu_chunk_pool.num_layers
+        self.cpu_chunk_pool.order_behind_writes(chunk_handle, but=self.engine)
         self.engine.swap_in(pool, chunk_handle.rows()[:rows], ids)
         self.engine.fence_pages()   # attention on the current stream must see the pages
         isswap = torch.zeros((self.page_table_allocator.max_context_len,), dtype=torch.bool)
@@ -75,6 +95,6 @@ class KVCacheManager:
         return VirtualPagedKVCache(page_table=table, isswap=isswap, pool=pool)
 
     def synchronize(self) -> None:
-        enqueued = self._copies_out
+        enqueued = self._progress.enqueued
         self.engine.wait()
-        self._finished = enqueued
+        self._progress.finished = enqueued

@@ -5,8 +5,8 @@ major - the layout KVCacheManager writes."""
 from __future__ import annotations
 
 import threading
-from dataclasses import dataclass, field
-from typing import Callable, Optional
+from dataclasses import dataclass
+from typing import List, Protocol, Tuple
 
 import torch
 
@@ -20,22 +20,31 @@ class ChunkHandle:
     level: int
     initial_size: int
     pool: "ChunkPool"
-    # orders the current stream behind the copy that fills the chunk (set by whoever enqueues one)
-    fence: Optional[Callable[[], None]] = field(default=None, repr=False, compare=False)
 
     def free(self) -> None:
         self.pool.free(self.id, self.level)
 
     def retrieve(self) -> torch.Tensor:
-        """The chunk's rows, for work on the current stream: behind the copy that fills them."""
-        if self.fence is not None:
-            self.fence()
+        """The chunk's rows, for work on the current stream: behind the copies that still write them."""
+        self.pool.order_behind_writes(self)
         return self.rows()
 
     def rows(self) -> torch.Tensor:
         """The same for a caller that orders its accesses itself."""
         begin, end = BuddyIndex.span(self.id, self.level)
         return self.pool.chunks[begin * self.pool.num_layers: end * self.pool.num_layers]
+
+
+class PendingWrite(Protocol):
+    """A copy into a chunk that may still be on its way."""
+    engine: object                    # what carries it; its copies keep their order among themselves
+
+    def finished(self) -> bool: ...   # as far as the host knows
+    def poll(self) -> bool: ...       # the same, with a look at the device; never waits
+    def fence(self) -> None: ...      # orders the current stream behind it
+
+
+_MANY_WRITES = 64
 
 
 class ChunkPool:
@@ -48,6 +57,26 @@ class ChunkPool:
         self.chunks = pinned_empty(((1 << (height - 1)) * num_layers,) + self.per_token_shape,
                                    main_dtype)
         self._buddy = BuddyIndex(height)
+        # copies that may still write, by the memory they write (a chunk can be freed and handed out
+        # again while they do): first unit, end, copy
+        self._writes: List[Tuple[int, int, PendingWrite]] = []
+
+    def note_write(self, handle: ChunkHandle, write: PendingWrite) -> None:
+        with self.mutex:
+            self._writes = [w for w in self._writes if not w[2].finished()]
+            if len(self._writes) >= _MANY_WRITES:     # nobody waits for them on the host
+                self._writes = [w for w in self._writes if not w[2].poll()]
+            self._writes.append(BuddyIndex.span(handle.id, handle.level) + (write,))
+
+    def order_behind_writes(self, handle: ChunkHandle, but: object = None) -> None:
+        """Orders the current stream behind the copies that still write the chunk's memory (not those
+        of engine `but`)."""
+        begin, end = BuddyIndex.span(handle.id, handle.level)
+        with self.mutex:
+            writes = [w for lo, hi, w in self._writes if lo < end and begin < hi]
+        for w in writes:
+            if w.engine is not but and not w.finished():
+                w.fence()
 
     @property
     def available_ids(self) -> list:
