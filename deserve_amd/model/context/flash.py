@@ -20,7 +20,7 @@ from typing import Dict, List, Sequence
 import numpy as np
 import torch
 
-from deserve_amd import staging
+from deserve_amd import _lib, staging
 from deserve_amd.kvcache.paged.kvcache import PagedKVCache
 from deserve_amd.kvcache.paged.page_pool import GpuPagePool
 from deserve_amd.model.context.forward import PagedForwardCtx
@@ -216,9 +216,10 @@ class FlashPrefillCtx(FlashForwardCtx):
 
     def rope_table(self, nnz: int, head_dim: int, theta: float) -> torch.Tensor:
         """The step's cosines and sines (paged_ops.rope_table), built for the first layer that asks:
-        anew in every pass over the layers, since the offsets may have been written in between
-        (and a pass that is captured must hold the launch)."""
-        key = (nnz, head_dim, theta)
+        anew in every pass over the layers, since the offsets may have been written in between, on
+        every stream that asks, since nothing orders one behind the other, and in every capture, which
+        must hold the launch."""
+        key = (nnz, head_dim, theta, _lib.current_stream(), torch.cuda.is_current_stream_capturing())
         if self.layer_id <= self.rope_layer:
             self.rope_tables.clear()
         self.rope_layer = self.layer_id

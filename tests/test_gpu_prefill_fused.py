@@ -76,3 +76,38 @@ def test_a_second_pass_over_the_layers_rotates_by_the_offsets_it_finds():
     got = ctx.rope_table(7, 128, 1e4)
     assert torch.equal(got, rope_table(ctx.indptr, ctx.offsets, 7, 128, 1e4))
     assert not torch.equal(got, first)
+
+
+def test_layers_on_another_stream_or_under_capture_have_a_table_of_their_own():
+    """Layer 0 runs eagerly on the current stream.  A later layer on a side stream is not ordered behind
+    it, and one that is captured has to find the offsets of the replay."""
+    from deserve_amd.model.context.flash import FlashPrefillCtx
+    from deserve_amd.paged_ops import rope_table
+
+    print("[case] table per stream and capture", flush=True)
+    dev = lambda a: torch.tensor(a, dtype=torch.int32, device="cuda")
+    ctx = FlashPrefillCtx(bsz=2, seqlens=dev([3, 4]), layer_id=0, page_pool=None, offsets=dev([0, 9]),
+                          indptr=dev([0, 3, 7]), kv_page_indices=None, kv_page_indptr=None,
+                          kv_last_page_lens=None, host={}, prefill_wrapper=None)
+    first = ctx.rope_table(7, 128, 1e4)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        ctx.layer_id = 1
+        other = ctx.rope_table(7, 128, 1e4)
+    torch.cuda.synchronize()
+    assert other is not first and torch.equal(other, first)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ctx.layer_id = 2
+        seen = ctx.rope_table(7, 128, 1e4).clone()
+        ctx.layer_id = 3
+        again = ctx.rope_table(7, 128, 1e4).clone()
+    for offsets in ([5, 20], [0, 9], [700, 3]):
+        ctx.offsets.copy_(dev(offsets))
+        graph.replay()
+        torch.cuda.synchronize()
+        want = rope_table(ctx.indptr, ctx.offsets, 7, 128, 1e4)
+        assert torch.equal(seen, want) and torch.equal(again, want)
+    ctx.layer_id = 4
+    assert ctx.rope_table(7, 128, 1e4) is first
