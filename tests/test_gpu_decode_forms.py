@@ -1,6 +1,9 @@
-"""The two forms of the 16-bit decode attention as the planner's own rule picks them: plans filled up with
-workgroups without work, one head in 256 split shares, requests in so many parts that a merge launch
-follows the split form; plain, with the step's token appended inside the launch and with RoPE inside."""
+"""The two forms of the 16-bit decode attention, plain, with the step's token appended inside the launch
+and with RoPE inside.  As the planner's own rule picks them: plans filled up with workgroups without
+work, one head in 256 split shares, requests in so many parts that a merge launch follows the split
+form, the deployed batch of 75 on 8-token pages.  And the form whose waves are kv heads on every kind
+of page and with more than one workgroup per share, in explicit shares: small batches of these shapes
+have the split form by themselves."""
 import ctypes
 
 import numpy as np
@@ -20,6 +23,16 @@ CASES = [
     ("two_heads_lopsided", [16 * 700 + 3] + [40 + i for i in range(9)], 16, 8, 2, "bf16", 0, True),
     ("one_head_256_shares", [16 * 1700, 16 * 3310 + 5], 16, 4, 1, "f16", 0, True),
     ("parts_in_the_dozens", [16 * 500 + 1], 16, 10, 5, "bf16", 0, True),
+    ("75_on_page8", [200 + 7 * i for i in range(75)], 8, 16, 8, "f16", 0, False),
+    ("page8_bf16", [3000, 700, 9, 8, 1, 600], 8, 32, 8, "bf16", 64, False),
+    ("page8_f16_group8", [2100, 1999, 16, 7], 8, 64, 8, "f16", 64, False),
+    ("page4", [3001, 1200, 5, 4], 4, 32, 8, "bf16", 64, False),
+    ("page2", [2500, 1700, 2, 1], 2, 16, 8, "f16", 64, False),
+    ("page32", [2500, 1700, 31, 33], 32, 16, 8, "bf16", 64, False),
+    ("kv12_page8", [1500, 700, 33], 8, 24, 12, "bf16", 32, False),
+    ("kv16", [1500, 700, 33], 16, 32, 16, "f16", 32, False),
+    ("kv17_one_wave_in_the_last_workgroup", [1500, 700, 33], 16, 17, 17, "bf16", 32, False),
+    ("eight_wave_merge", [33000], 16, 8, 8, "bf16", 256, False),
 ]
 
 
