@@ -71,6 +71,8 @@ class ChunkPool:
     def order_behind_writes(self, handle: ChunkHandle, but: object = None) -> None:
         """Orders the current stream behind the copies that still write the chunk's memory (not those
         of engine `but`)."""
+        if not self._writes:
+            return
         begin, end = BuddyIndex.span(handle.id, handle.level)
         with self.mutex:
             writes = [w for lo, hi, w in self._writes if lo < end and begin < hi]

@@ -20,7 +20,7 @@ from typing import Dict, List, Sequence
 import numpy as np
 import torch
 
-from deserve_amd import _lib, staging
+from deserve_amd import staging
 from deserve_amd.kvcache.paged.kvcache import PagedKVCache
 from deserve_amd.kvcache.paged.page_pool import GpuPagePool
 from deserve_amd.model.context.forward import PagedForwardCtx
@@ -213,19 +213,24 @@ class FlashPrefillCtx(FlashForwardCtx):
     prefill_wrapper: BatchPrefillWithPagedKVCacheWrapper = None   # type: ignore[assignment]
     rope_tables: Dict[tuple, torch.Tensor] = field(default_factory=dict, repr=False)
     rope_layer: int = field(default=-1, repr=False)   # that asked last
+    rope_device: int = field(default=-1, repr=False)
 
     def rope_table(self, nnz: int, head_dim: int, theta: float) -> torch.Tensor:
         """The step's cosines and sines (paged_ops.rope_table), built for the first layer that asks:
         anew in every pass over the layers, since the offsets may have been written in between, on
         every stream that asks, since nothing orders one behind the other, and in every capture, which
         must hold the launch."""
-        key = (nnz, head_dim, theta, _lib.current_stream(), torch.cuda.is_current_stream_capturing())
+        if self.rope_device < 0:
+            self.rope_device = self.indptr.get_device()
+        stream = torch._C._cuda_getCurrentRawStream(self.rope_device)     # 0: the default one, never captured
+        key = (nnz, head_dim, theta, stream, stream != 0 and torch.cuda.is_current_stream_capturing())
         if self.layer_id <= self.rope_layer:
             self.rope_tables.clear()
         self.rope_layer = self.layer_id
-        if key not in self.rope_tables:
-            self.rope_tables[key] = rope_table(self.indptr, self.offsets, nnz, head_dim, theta)
-        return self.rope_tables[key]
+        table = self.rope_tables.get(key)
+        if table is None:
+            table = self.rope_tables[key] = rope_table(self.indptr, self.offsets, nnz, head_dim, theta)
+        return table
 
     @classmethod
     def init_paged_prefill_ctx(cls, task_datas: List[TaskData],

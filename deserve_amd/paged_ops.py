@@ -320,13 +320,13 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
         q = q.contiguous()
         if q.shape != (self._batch, self._hq, self._d):
             raise ValueError(f"q must be ({self._batch}, {self._hq}, {self._d}), got {tuple(q.shape)}")
-        self._check_pool(paged_kv_data, q.dtype)
+        dtype = q.dtype
+        self._check_pool(paged_kv_data, dtype)
         if out is None:
             out = torch.empty_like(q)
-        elif out.dtype != q.dtype or out.numel() < q.numel() or not out.is_contiguous():
+        elif out.dtype != dtype or out.numel() < q.numel() or not out.is_contiguous():
             raise ValueError("out must be contiguous, of q's dtype, and hold at least q's elements")
         scale = 1.0 / math.sqrt(self._d) if sm_scale is None else sm_scale
-        ws_bytes = self._workspace.numel() * self._workspace.element_size()
         table = None
         if k_append is not None or v_append is not None:
             if k_append is None or v_append is None or phases not in (1, 3):
@@ -339,7 +339,7 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
             k_append, v_append = k_append.contiguous(), v_append.contiguous()
             want = (self._batch, self._hkv, self._d)
             if k_append.shape != want or v_append.shape != want or \
-                    k_append.dtype != q.dtype or v_append.dtype != q.dtype:
+                    k_append.dtype != dtype or v_append.dtype != dtype:
                 raise ValueError(f"k_append / v_append must be {want} of q's dtype")
             if rope_offsets is not None:
                 key = (rope_offsets.data_ptr(), float(rope_theta))
@@ -354,14 +354,15 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
                 table = self._rope_table.data_ptr()
         if phases == 3:
             step = _lib.DecodeStep.from_buffer_copy(self._step)    # calls from several threads do not share it
-            step.rope_table, step.dtype, step.sm_scale = table, _lib.dtype_code(q.dtype), scale
+            step.rope_table, step.dtype, step.sm_scale = table, _lib.dtype_code(dtype), scale
             rc = _lib.lib().dskv_decode_step(ctypes.byref(step), out.data_ptr(), q.data_ptr(), _lib.ptr(k_append),
                                              _lib.ptr(v_append), paged_kv_data.data_ptr(), _lib.current_stream())
             _lib.check(rc, "decode forward")
             return out
         args = (paged_kv_data.data_ptr(), self._indices.data_ptr(), self._plan.data_ptr(), self._n_items,
-                self._n_workgroups, self._workspace.data_ptr(), ws_bytes, self._batch, self._hq, self._hkv,
-                self._d, self._p, scale, _lib.dtype_code(q.dtype))
+                self._n_workgroups, self._workspace.data_ptr(),
+                self._workspace.numel() * self._workspace.element_size(), self._batch, self._hq, self._hkv,
+                self._d, self._p, scale, _lib.dtype_code(dtype))
         if k_append is None:
             rc = _lib.lib().dskv_decode_attn_phases(out.data_ptr(), q.data_ptr(), *args, phases, _lib.current_stream())
         elif table is None:
@@ -518,10 +519,11 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
         q = q.contiguous()
         if q.shape != (self._nnz, self._hq, self._d):
             raise ValueError(f"q must be ({self._nnz}, {self._hq}, {self._d}), got {tuple(q.shape)}")
-        self._check_pool(paged_kv_data, q.dtype)
+        dtype = q.dtype
+        self._check_pool(paged_kv_data, dtype)
         if out is None:
             out = torch.empty_like(q)
-        elif out.shape != q.shape or out.dtype != q.dtype or not out.is_contiguous():
+        elif out.shape != q.shape or out.dtype != dtype or not out.is_contiguous():
             raise ValueError("out must be contiguous and of q's shape and dtype")
         scale = 1.0 / math.sqrt(self._d) if sm_scale is None else sm_scale
         if k_append is not None or v_append is not None or rope_table is not None:
@@ -530,7 +532,7 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
             k_append, v_append = k_append.contiguous(), v_append.contiguous()
             want = (self._nnz, self._hkv, self._d)
             if k_append.shape != want or v_append.shape != want or \
-                    k_append.dtype != q.dtype or v_append.dtype != q.dtype:
+                    k_append.dtype != dtype or v_append.dtype != dtype:
                 raise ValueError(f"k_append / v_append must be {want} of q's dtype")
             if rope_table is not None and (rope_table.shape != (self._nnz, self._d) or
                                            rope_table.dtype != torch.float32 or not rope_table.is_contiguous()):
@@ -538,7 +540,7 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
             step = _lib.MixedStep.from_buffer_copy(self._step)
             step.rope_table = None if rope_table is None else rope_table.data_ptr()
             step.num_pages, step.causal = paged_kv_data.shape[0], int(causal)
-            step.dtype, step.sm_scale = _lib.dtype_code(q.dtype), scale
+            step.dtype, step.sm_scale = _lib.dtype_code(dtype), scale
             rc = _lib.lib().dskv_mixed_step(ctypes.byref(step), out.data_ptr(), q.data_ptr(), k_append.data_ptr(),
                                             v_append.data_ptr(), paged_kv_data.data_ptr(), _lib.current_stream())
             _lib.check(rc, "prefill forward")
@@ -548,7 +550,7 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
             self._indices.data_ptr(), self._indptr.data_ptr(), self._last.data_ptr(),
             self._tiles.data_ptr(), ctypes.byref(self._info), self._workspace.data_ptr(),
             self._workspace.numel() * self._workspace.element_size(), self._batch, self._nnz, self._hq,
-            self._hkv, self._d, self._p, scale, int(causal), _lib.dtype_code(q.dtype),
+            self._hkv, self._d, self._p, scale, int(causal), _lib.dtype_code(dtype),
             _lib.current_stream())
         _lib.check(rc, "prefill forward")
         return out
