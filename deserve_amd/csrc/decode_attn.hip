@@ -163,11 +163,10 @@ __global__ __launch_bounds__(64) void decode_attn_generic_kernel(
 // iteration, and the per-group partial sums of O are folded across g once, at the end.
 // The block table entries of an iteration are fetched an iteration ahead.
 //
-// What bounds it in small batches is latency: a wave waits for memory once per 16 tokens.  Their
-// plans (up to kSplitMaxTiles tiles) have shares for a workgroup of several waves, so kWaves waves take
-// every kWaves-th 16 tokens of an item and meet in LDS.  fp32, 32 q heads, us: 8 requests of 512
-// tokens 24.9 with a wave alone, 14.4 with four (16.5 with eight), one of 2000 12.3 (14.7); 24 of
-// 50-150 17.9 (26.7: the second eight of a compute unit wait for the first).
+// What bounds it in small batches is latency: a wave waits for memory once per 16 tokens.  Where the
+// planner finds that it pays (gqa_splitting_pays, with the figures), kWaves waves take every kWaves-th 16
+// tokens of an item and meet in LDS: fp32, 32 q heads, 8 requests of 512 tokens 17.1 us with a wave alone
+// in 64 shares, 14.4-15.3 with four in 32 (16.5 with eight), one of 2000 12.3 (14.7).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float row16_sum(float v)
 {

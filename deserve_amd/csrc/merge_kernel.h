@@ -52,8 +52,8 @@ __device__ __forceinline__ void merge_dims(uint16_t *__restrict__ dst, const flo
 // A workgroup per (row, kMergeHeads heads); a thread owns four dims of one head.  What bounds it is
 // the memory path of a compute unit (~36 GB/s) on the row with the most parts: one workgroup
 // per row (a thread per 16 dims) took 16 us for 128 requests of 64 heads, the longest in 15-20 parts
-// of 33 KB, and now 11.7 (10 layers 2426 -> 2380 us); 64 requests of 32 heads in 4-5 parts, 16 layers
-// 1648 -> 1624 us.  Four or two heads per workgroup take the same time.
+// of 33 KB, and now 11.7; 64 requests of 32 heads in 4-5 parts take 4.9.  Four or two heads per
+// workgroup take the same time.
 constexpr int kMergeHeads = 8;
 constexpr int kMergeThreads = kMergeHeads * (kHeadDim / 4);
 template <int DT>

@@ -78,7 +78,8 @@ namespace dskv {
 constexpr int64_t kIdsCapacity = int64_t(1) << 20;
 // Out staging: this many chunks, in at most this many bytes (or one chunk, if that is more).  It
 // holds what a step's requests leave with, a few hundred MB: with one chunk of 128 MiB the
-// packing of the last of 387 MB waits for two thirds of the trip.
+// packing of the last of 387 MB waits for two thirds of the trip.  What leaves beyond that in one
+// go is packed as the link frees the ring, and the swap-ins behind it wait as long.
 constexpr int kOutChunks = 4;
 constexpr int64_t kOutRingBytes = int64_t(512) << 20;
 constexpr size_t kMaxHostRanges = 256;   // beyond that swap-ins wait for all copies out

@@ -61,13 +61,14 @@ class GraphedDecodeStep:
     def graph_key(batch: int, n_workgroups: int, n_items: int, tensors: Sequence[torch.Tensor],
                   persistent_kernel: bool) -> tuple:
         """What decides which launches a captured step holds.  Always: batch, workgroup
-        count, whether anything is merged and with which of the two merge kernels (the
-        launcher takes the wide one from 32 parts per request on), input shapes.  The
-        attention kernel of the 16-bit head_dim-128 path is launched with one workgroup per
-        planned workgroup and reads its items from the plan, so the item count is not part
-        of its launch; the generic kernel (fp32 pools, other head dims, groups over 16) is
-        launched with one workgroup per item, so there the item count is part of the key -
-        a replay with another count would skip items or run on stale plan words."""
+        count, whether anything is merged and whether in the attention launch or how (from
+        32 parts per request on by the merge launch of eight waves), input shapes.  The
+        16-bit head_dim-128 attention has two forms, a workgroup per planned workgroup or per
+        (planned workgroup, kv head), told apart by the workgroup count; both read their
+        items from the plan, so the item count is not part of the launch.  The generic
+        kernel (fp32 pools, other head dims, groups over 16) is launched per item, so there
+        the item count is part of the key - a replay with another count would skip items or
+        run on stale plan words."""
         key = (batch, n_workgroups, n_items > batch, n_items > 32 * batch,
                tuple((tuple(t.shape), t.dtype) for t in tensors))
         return key if persistent_kernel else key + (n_items,)

@@ -224,8 +224,10 @@ int dskv_decode_rope_append_attn(void *out, const void *q, const void *k_new, co
  * merge_counters (device, may be null): words that are zero before the first call that is given
  * them and are used by one launch at a time, like the workspace; every launch leaves them zero.
  * At least 2 * (n_items - batch) * n_kv_heads of them (n_items * n_kv_heads always suffice).  With
- * them the attention launch merges the parts of cut requests itself instead of in a launch of its
- * own (16-bit head_dim-128 kernels; other shapes leave them alone).
+ * them the attention launch of a small batch merges the parts of cut requests itself instead of in a
+ * launch of its own (16-bit head_dim-128 kernels; other shapes leave them alone).  The two ways add the
+ * parts in different orders: 16-bit results can differ by one unit in the last place between them,
+ * and so between this call with counters and the other decode calls.  Each repeats its own bits.
  */
 typedef struct dskv_decode_step {
     const int32_t *kv_page_indices, *plan_dev;

@@ -135,8 +135,8 @@ DECODE_CASES = [
     ("mha", [300, 40], 16, 8, 8, 128, "bf16", 0),
     ("group16", [300, 40], 16, 32, 2, 128, "bf16", 8),
     ("kv4", [300, 40, 1], 16, 16, 4, 128, "bf16", 0),
-    ("kv16", [300, 40, 17, 1000], 16, 32, 16, 128, "bf16", 12),    # two groups of 8 kv heads per workgroup id
-    ("kv12", [200, 33], 16, 24, 12, 128, "f16", 0),                # the second group half full
+    ("kv16", [300, 40, 17, 1000], 16, 32, 16, 128, "bf16", 12),    # twelve shares of sixteen kv heads
+    ("kv12", [200, 33], 16, 24, 12, 128, "f16", 0),
     ("f32", [512, 100, 1, 33], 16, 32, 8, 128, "f32", 8),
     ("f32_d64", [200, 17], 8, 8, 2, 64, "f32", 0),
     ("bf16_d64_generic", [200, 17], 16, 8, 2, 64, "bf16", 4),
@@ -152,7 +152,7 @@ DECODE_CASES = [
     ("empty_request", [0, 50], 16, 32, 8, 128, "bf16", 0),
     ("long_single", [33000], 16, 32, 8, 128, "bf16", 0),          # 256 parts: the wide merge
     ("long_and_short", [9000, 50, 1], 16, 32, 8, 128, "f16", 128),
-    # more than 8 parts of one request among short ones: the row merge's loop, four parts at a time
+    # more than 16 parts of one request among short ones: the row merge's loop, sixteen parts at a time
     ("one_long_among_short", [9000, 50, 1, 300, 17, 64, 5, 700], 16, 32, 8, 128, "bf16", 64),
     ("ten_parts", [2600, 40], 16, 32, 8, 128, "f16", 10),
 ]
