@@ -254,6 +254,8 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
                                                ctypes.byref(words), ctypes.byref(ws))
         _lib.check(rc, "decode begin_forward")
         if ws.value > self._workspace.numel() * self._workspace.element_size():
+            if target_workgroups <= 0 and self._few_shares_apply(h_indptr, h_last):
+                return self._plan_into(plan, cap, h_indptr, h_last, max(1, n_wgs.value // self._hkv))
             raise RuntimeError(f"decode workspace too small: need {ws.value} bytes")
         self._batch, self._n_items, self._n_workgroups = batch, n_items.value, n_wgs.value
         self._rope_table, self._rope_key = None, None     # positions change with the step
@@ -261,6 +263,13 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
         ptr = h_indptr.numpy()
         self._empty_requests = np.flatnonzero(ptr[1:] <= ptr[:-1])[:4].tolist() if batch > 0 else []
         return int(words.value)
+
+    def _few_shares_apply(self, h_indptr: torch.Tensor, h_last: torch.Tensor) -> bool:
+        """Whether a batch whose plan does not fit the workspace runs in the few shares of the form for
+        small batches (up to 2560 tiles of 16 tokens), which need a fraction of it, if not as fast."""
+        pages = np.diff(h_indptr.numpy()).astype(np.int64)
+        lens = np.where(pages > 0, (pages - 1) * self._p + h_last.numpy()[: pages.shape[0]], 0)
+        return self._d == 128 and self._hq // self._hkv <= 8 and int((-(-lens // 16)).sum()) <= 2560
 
     def begin_forward_with_metadata(self, meta_words: int, fill_metadata, indptr_at: int, indices_at: int,
                                     indptr_host: torch.Tensor, last_page_len_host: torch.Tensor,

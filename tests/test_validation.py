@@ -113,6 +113,28 @@ def test_decode_forward_refuses_an_out_it_cannot_fill():
             w.forward(q, pages, out=out)
 
 
+def test_decode_plan_falls_back_to_few_shares_when_the_workspace_cannot_hold_the_partials():
+    """Eight requests of 313 tiles: in 256 shares they leave 4.4 MB of partials, in 32 half a MB."""
+    lens = [16 * 313] * 8
+    indptr, last = _i32([313 * i for i in range(9)]), _i32([16] * 8)
+    cap = 1 << 17
+
+    def plan(ws_bytes, n_kv=8, target=0, lens_factor=1):
+        w = BatchDecodeWithPagedKVCacheWrapper(torch.empty(ws_bytes, dtype=torch.uint8))
+        w._shape_args(4 * n_kv, n_kv, 128, 16)
+        w._plan_into(torch.zeros(cap, dtype=torch.int32), cap, indptr * lens_factor, last, target)
+        return w._n_workgroups
+
+    assert sum(lens) // 16 <= 2560
+    assert plan(64 << 20) == 256 and plan(2 << 20) == 32
+    with pytest.raises(RuntimeError, match="workspace too small"):
+        plan(16)                                            # not even those
+    with pytest.raises(RuntimeError, match="workspace too small"):
+        plan(2 << 20, target=256)                           # asked for
+    with pytest.raises(RuntimeError, match="workspace too small"):
+        plan(2 << 20, lens_factor=2)                        # a large batch
+
+
 def test_gather_and_scatter_refuse_page_ids_outside_the_pool():
     pool = PagePool(2, 8, 4, CPU, torch.float16, n_kv_heads=1, head_dim=8)
     for bad in ([0, 8], [-1, 3]):
