@@ -541,17 +541,21 @@ namespace dskv {
 // of 1 to 64 requests at 1 to 160 kv heads (bf16, attention and merge in a replayed graph, us,
 // workgroup per (share, kv head) / the other form; a range is over the batches):
 //   * Eight heads fill a workgroup of the other form, which then wins as soon as memory is the limit:
-//     1250 tiles 24 / 24-28, 1875 tiles 30-31 / 30-33, 2560 tiles 38 / 36.  The line: 60 tiles a share,
-//     40 for more than 32 requests (64: 1250 tiles 25 / 23, 1750 tiles 30 / 28).
+//     1200 tiles 23-24 / 24-27, 1800 tiles 30-31 / 30-32, 2550 tiles 38-39 / 36-39 for 1 to 48 requests; 64 and more
+//     from 1200 tiles on 24-25 / 23.  9 to 24 requests are in ten parts and more each, which the merge launch
+//     adds up in two trips: 10 requests of 2550 tiles 38 / 42, 16 39 / 40-42; one of 2000 tiles 33-35 / 35-38, 2250
+//     tiles 36 / 36.  The line: 60 tiles a share, 40 for more than 48 requests, 80 for 9 to 24, 70 for one or two.
 //   * More heads, or fewer than eight that leave waves of the other form idle, lose there later or
 //     not at all where few * n_kv_heads workgroups leave hardly a unit idle: 5 heads, 2000 tiles 23-26 /
 //     23-27; 12 heads, 1706 tiles 40 / 42-44, 2500 tiles 54 / 53-56; 16 heads, 2500 tiles 64 / 69; 64
 //     heads, 625 tiles 64 / 74-80.  Where they do leave units idle: 20 heads (240 workgroups), 1024 tiles
 //     43 / 44-46, 1500 tiles 59 / 54; 96 heads (192), 104 tiles 27-28 / 30-34, 156 tiles 36 / 34-36.
 //     The line: 80 tiles a share, lower by the share of units that idle.
+//   * Groups under four q heads have small partials to merge: up to 15 heads the lines lie a quarter lower
+//     (8 heads in groups of one, 1400 tiles 24 / 22-27, 2000 tiles 31 / 27-34; 12 heads, 2083 tiles 46 / 43-48).
 //   * Up to four heads a request is cut into many parts (few is 64 and more), and merging them costs
-//     more than the walk saves: 4 heads, 375 tiles 12-13 / 12-16, but one request 16 / 14, and 750 tiles
-//     15-16 / 13-14; 2 heads, 1500 tiles 14-20 / 11-15.
+//     more than the walk saves: 4 heads, 375 tiles 12-13 / 12-16, but one request 16 / 14 (87 tiles, which are
+//     no more than 32 parts, 11 / 15), and 750 tiles 15-16 / 13-14; 2 heads, 1500 tiles 14-20 / 11-15.
 //   * One head: 256 workgroups of a wave each leave the chip idle: 1500 tiles 14-23 / 11-13, 5000 tiles
 //     17-21 / 18-21, 20480 tiles 36-40 / 47-52.
 //   * Lopsided: one request in dozens of parts beside short ones.  The merge launch gives a row one
@@ -559,7 +563,7 @@ namespace dskv {
 //     (Where requests have more than kWideMergeParts parts on average, that launch gives a row more.)
 //   * Without counters to merge inside the launch (merges_itself) a request pays for the merge launch
 //     as well: 8 heads, 625 tiles 16-22 / 19-24, 937 tiles 20-25 / 22-27, 1250 tiles 23-28 / 23-26.  A third.
-static bool splitting_pays(int64_t tiles, int64_t longest, int batch, int n_kv_heads, bool merges_itself)
+static bool splitting_pays(int64_t tiles, int64_t longest, int batch, int n_kv_heads, int group, bool merges_itself)
 {
     const int64_t cus = default_workgroups(), few = cus / n_kv_heads, busy = few * n_kv_heads;
     if (few < 1) return false;
@@ -567,9 +571,12 @@ static bool splitting_pays(int64_t tiles, int64_t longest, int batch, int n_kv_h
     if (tiles > kSplitMaxTiles) return false;
     if (longest * cus > kLopsidedParts * tiles && batch + cus <= kWideMergeParts * (int64_t)batch) return true;
     int64_t most;
-    if (n_kv_heads <= 4) most = n_kv_heads > 2 && batch > 1 ? 2048 / n_kv_heads : 0;
+    if (n_kv_heads <= 2) most = 0;
+    else if (n_kv_heads <= 4) most = batch > 1 ? 2048 / n_kv_heads : kWideMergeParts * kSplitTilesPerShare;
     else if (n_kv_heads != kMaxWaves && 32 * busy >= 31 * cus) most = kSplitMaxTiles;
-    else most = (n_kv_heads > kMaxWaves ? 80 : batch > 32 ? 40 : 60) * few * busy / cus;
+    else most = (n_kv_heads > kMaxWaves || (batch >= 9 && batch <= 24) ? 80 : batch > 48 ? 40 : batch <= 2 ? 70 : 60) *
+                few * busy / cus;
+    if (group < 4 && n_kv_heads < 2 * kMaxWaves) most = most * 3 / 4;
     return tiles <= (merges_itself ? most : most / 3);
 }
 
@@ -638,7 +645,7 @@ int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, i
                                : gqa_shape(head_dim, n_qo_heads, n_kv_heads);
     const bool split = own_rule && two_forms &&
                        (mfma_path(dtype, head_dim, n_qo_heads, n_kv_heads)
-                            ? splitting_pays(total_tiles, longest, batch, n_kv_heads, merges_itself)
+                            ? splitting_pays(total_tiles, longest, batch, n_kv_heads, n_qo_heads / n_kv_heads, merges_itself)
                             : gqa_splitting_pays(total_tiles, longest, batch, n_kv_heads, head_dim));
     int64_t wgs = own_rule ? default_workgroups() : target_workgroups;
     if (split && head_dim == kHeadDim)

@@ -45,20 +45,23 @@ def test_no_xcd_gets_more_workgroups_than_it_has_units(n_kv):
     assert _launch(3, CUS // n_kv, n_kv) == (CUS // n_kv * n_kv, True)
 
 
-@pytest.mark.parametrize("n_kv,lens,splits", [
-    (8, [16 * 240] * 8, True), (8, [16 * 245] * 8, False),            # 1920 tiles: 60 a share
-    (8, [16 * 20] * 64, True), (8, [16 * 21] * 64, False),            # many requests: 40 a share
-    (24, [16 * 93] * 8, True), (24, [16 * 95] * 8, False),            # 240 of 256 units busy: 750 tiles
-    (40, [16 * 56] * 8, True), (40, [16 * 57] * 8, False),
-    (16, [16 * 320] * 8, True), (64, [16 * 320] * 8, True),           # every unit busy: 2560 tiles
-    (12, [16 * 320] * 8, True), (12, [16 * 321] * 8, False),
-    (4, [16 * 64] * 8, True), (4, [16 * 65] * 8, False), (4, [16 * 64], False),
-    (2, [16 * 20] * 8, False), (2, [16 * 1200] + [100] * 23, True),   # lopsided
-    (1, [16 * 200] * 8, False), (1, [16 * 630] * 8, True),
+@pytest.mark.parametrize("n_kv,group,lens,splits", [
+    (8, 4, [16 * 240] * 8, True), (8, 4, [16 * 245] * 8, False),            # 1920 tiles: 60 a share
+    (8, 4, [16 * 40] * 48, True), (8, 4, [16 * 41] * 48, False),
+    (8, 8, [16 * 20] * 64, True), (8, 8, [16 * 21] * 64, False),            # many requests: 40 a share
+    (8, 4, [16 * 160] * 16, True), (8, 4, [16 * 161] * 16, False),          # requests in many parts: 80 a share
+    (8, 1, [16 * 180] * 8, True), (8, 1, [16 * 185] * 8, False),            # small groups: three quarters
+    (24, 1, [16 * 93] * 8, True), (24, 1, [16 * 95] * 8, False),            # 240 of 256 units busy: 750 tiles
+    (40, 1, [16 * 56] * 8, True), (40, 1, [16 * 57] * 8, False),
+    (16, 1, [16 * 320] * 8, True), (64, 1, [16 * 320] * 8, True),           # every unit busy: 2560 tiles
+    (12, 4, [16 * 320] * 8, True), (12, 4, [16 * 321] * 8, False), (12, 1, [16 * 241] * 8, False),
+    (4, 4, [16 * 64] * 8, True), (4, 4, [16 * 65] * 8, False), (4, 4, [16 * 192], True), (4, 4, [16 * 193], False), (8, 4, [16 * 2240], True), (8, 4, [16 * 2241], False),
+    (2, 4, [16 * 20] * 8, False), (2, 4, [16 * 1200] + [100] * 23, True),   # lopsided
+    (1, 8, [16 * 200] * 8, False), (1, 8, [16 * 630] * 8, True),
 ])
-def test_which_batches_split_a_head_over_the_waves_of_a_workgroup(n_kv, lens, splits):
-    shares, items, _ = _plan(lens, n_kv, group=4 if n_kv < 16 else 1)
-    assert _launch(items, shares, n_kv, 4 if n_kv < 16 else 1)[1] == splits
+def test_which_batches_split_a_head_over_the_waves_of_a_workgroup(n_kv, group, lens, splits):
+    shares, items, _ = _plan(lens, n_kv, group=group)
+    assert _launch(items, shares, n_kv, group)[1] == splits
     total = sum(-(-x // 16) for x in lens)
     if not splits and total >= 1024:      # a share per compute unit, as large plans have
         assert shares == max(CUS, CUS // n_kv + 1)

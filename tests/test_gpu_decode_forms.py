@@ -19,7 +19,7 @@ CASES = [
     # (name, kv_lens, P, Hq, Hkv, dtype, target, splits a head over waves)
     ("two_heads_filled_up", [700, 1, 33, 16], 16, 8, 2, "bf16", 0, False),
     ("one_head_filled_up", [40, 300, 17], 8, 8, 1, "f16", 0, False),
-    ("four_heads_one_request", [1000], 16, 16, 4, "bf16", 0, False),
+    ("four_heads_one_request", [4000], 16, 16, 4, "bf16", 0, False),
     ("two_heads_lopsided", [16 * 700 + 3] + [40 + i for i in range(9)], 16, 8, 2, "bf16", 0, True),
     ("one_head_256_shares", [16 * 1700, 16 * 3310 + 5], 16, 4, 1, "f16", 0, True),
     ("parts_in_the_dozens", [16 * 500 + 1], 16, 10, 5, "bf16", 0, True),

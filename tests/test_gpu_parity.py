@@ -150,7 +150,7 @@ DECODE_CASES = [
     ("f16_d256_per_head", [50, 7], 16, 4, 2, 256, "f16", 0),
     ("f32_d100_per_head", [50, 7], 16, 4, 2, 100, "f32", 0),
     ("empty_request", [0, 50], 16, 32, 8, 128, "bf16", 0),
-    ("long_single", [33000], 16, 32, 8, 128, "bf16", 0),          # 256 parts: the wide merge
+    ("long_single", [33000], 16, 32, 8, 128, "bf16", 0),          # 32 parts, merged in the launch
     ("long_and_short", [9000, 50, 1], 16, 32, 8, 128, "f16", 128),
     # more than 16 parts of one request among short ones: the row merge's loop, sixteen parts at a time
     ("one_long_among_short", [9000, 50, 1, 300, 17, 64, 5, 700], 16, 32, 8, 128, "bf16", 64),
