@@ -587,9 +587,10 @@ static bool splitting_pays(int64_t tiles, int64_t longest, int batch, int n_kv_h
 //     tiles 48 / 34; more heads lose later: 16 heads, 16 requests of 87 tiles 13 / 14, 32 heads, 8 of 21 tiles
 //     11 / 12.  The line: 2048 tiles of one head and 128 (request, head) pairs, more of them where the
 //     requests are a tile or two.
-//   * And with eight heads where memory is the limit and requests are few: 2 to 24 requests of 1125 tiles 53-55 /
-//     57-59, of 2000 tiles 75-80 / 79-85 (64: 97 / 80).
-//   * One request: 8 heads, 375 tiles 28 / 30, 937 tiles 46 / 45; 4 heads, 1875 tiles 43 / 47.
+//     Beyond it a wave walks longer than in the other form, and adds up more in one chain: 16 requests of 2512
+//     tiles are off from 64 bits by 2.33e-7 / 2.10e-7, one of 625 tiles by 2.16e-7 / 2.08e-7 (8 x 512 tokens 1.55e-7 /
+//     1.63e-7), so what it would win there (2 to 24 requests of 1125 tiles 53-55 us / 57-59) is left.
+//   * One request with three or four heads, where no wave walks longer: 4 heads, 1875 tiles 43 / 47.
 //   * One or two heads: 1500 tiles of two 27-30 / 29-32, 2500 tiles 35-39 / 40-43; 5000 tiles of one 50-80 /
 //     92-94; but not where the items are a few more than the units: one head, 24 requests of 1400 tiles
 //     27 / 39 in 253 items, of 1500 tiles 46 / 39 in 273.
@@ -611,8 +612,7 @@ static bool gqa_splitting_pays(int64_t tiles, int64_t longest, int batch, int n_
                !(batch > 16 && work < 2560 && (batch + shares) * n_kv_heads > cus) && !(pairs > cus / 2 && work < 1024);
     }
     if (tiles > kSplitMaxTiles) return false;
-    if (batch == 1) return n_kv_heads <= 4 || work <= 5120;
-    if (n_kv_heads == kMaxWaves && work >= 8500 && pairs <= 3 * cus / 4) return true;
+    if (batch == 1 && n_kv_heads <= 4) return true;
     const int64_t most_pairs = n_kv_heads > kMaxWaves && work <= 1500 ? cus : work <= 512 ? 3 * cus / 4 : cus / 2;
     return work <= 2048 && pairs <= most_pairs;
 }

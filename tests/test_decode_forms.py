@@ -107,7 +107,7 @@ def test_no_wave_of_an_fp32_batch_walks_longer_than_in_shares_of_a_unit_each(n_k
     (8, [512] * 8, 128, True), (8, [512] * 17, 128, False), (8, [530] * 8, 128, False),
     (8, [100] * 24, 128, False), (8, [20] * 64, 128, False), (4, [1000], 128, True), (8, [11000], 128, False),
     (8, [16 * 1250] + [60] * 23, 128, True), (2, [5000] * 3, 128, True), (1, [100] * 24, 128, True),
-    (1, [1000] * 24, 128, False), (1, [900] * 24, 128, True), (12, [60] * 16, 128, True), (8, [25] * 24, 128, True), (8, [800] * 24, 128, True), (8, [800] * 25, 128, False), (1, [20000], 128, True), (8, [40] * 24, 64, True), (8, [20] * 64, 64, False)])
+    (1, [1000] * 24, 128, False), (1, [900] * 24, 128, True), (12, [60] * 16, 128, True), (8, [25] * 24, 128, True), (8, [4096], 128, True), (8, [4097], 128, False), (1, [20000], 128, True), (8, [40] * 24, 64, True), (8, [20] * 64, 64, False)])
 def test_which_fp32_batches_split_an_item_over_four_waves(n_kv, lens, d, splits):
     shares, items, _ = _plan(lens, n_kv, d=d, dtype=_lib.F32)
     assert _launch(items, shares, n_kv, d=d, dtype=_lib.F32)[1] == splits
