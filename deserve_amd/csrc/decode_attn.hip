@@ -554,8 +554,9 @@ namespace dskv {
 //   * Groups under four q heads have small partials to merge: up to 15 heads the lines lie a quarter lower
 //     (8 heads in groups of one, 1400 tiles 24 / 22-27, 2000 tiles 31 / 27-34; 12 heads, 2083 tiles 46 / 43-48).
 //   * Up to four heads a request is cut into many parts (few is 64 and more), and merging them costs
-//     more than the walk saves: 4 heads, 375 tiles 12-13 / 12-16, but one request 16 / 14 (87 tiles, which are
-//     no more than 32 parts, 11 / 15), and 750 tiles 15-16 / 13-14; 2 heads, 1500 tiles 14-20 / 11-15.
+//     more than the walk saves: 4 heads, 375 tiles 12-15 / 12-20, but one request 16 / 14 (87 tiles, which are
+//     no more than 32 parts, 11 / 15), and 750 tiles 15-18 / 13-16 (8 requests, just under the 32 parts of the wide
+//     merge, 15 / 20); 2 heads, 1500 tiles 14-20 / 11-15.
 //   * One head: 256 workgroups of a wave each leave the chip idle: 1500 tiles 14-23 / 11-13, 5000 tiles
 //     17-21 / 18-21, 20480 tiles 36-40 / 47-52.
 //   * Lopsided: one request in dozens of parts beside short ones.  The merge launch gives a row one
