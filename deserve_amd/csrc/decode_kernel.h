@@ -58,14 +58,19 @@ struct LoadCursor {
 #define DSKV_DECODE_MIN_WAVES 1
 #endif
 // The kernel's body for one workgroup: share `share` of the plan, kv heads head_group *
-// kWaves .. + kWaves (one per wave); `lds_base`: kWaves * kVTileBytes of the workgroup's LDS.
+// kWaves .. + kWaves (one per wave); `lds_base`: kWaves * tile_lds_bytes(kWholeRows) of the workgroup's LDS.
 // A function, so that one launch can hold workgroups of this kind next to others.
 //   kPagesPerTile: pages a 16-token tile spans - 1 (pages of 16 tokens or more: one buffer
 //     descriptor per tile), 2 (pages of 8 tokens: the two page ids as scalars, selected per
 //     lane), 0 (smaller pages: every lane looks its page up itself; with four scalar ids and
 //     a four-way selection pages of 4 tokens were slower than that, 130 against 113 us).
 //   kRing: tiles in flight per wave (one consumed, the rest loading).
-template <int DT, int kPagesPerTile, int kWaves, int kRing = kStages>
+//   kWholeRows: K is read by whole rows (TileRegs).  Beside query tiles, which share the compute unit's
+//     memory path, that and two tiles in flight instead of three take the step of 75 rows and a chunk
+//     from 2540 to 2364 us (16 layers), 70B-shaped from 1415 to 1327.  Workgroups of eight waves, alone on
+//     their units, do not gain: 64 requests 1636 -> 1645 us, 128 long ones 2386 -> 2437 (their younger waves
+//     only run once the older ones have finished: half of a unit's waves are reading at any time).
+template <int DT, int kPagesPerTile, int kWaves, int kRing, bool kWholeRows>
 __device__ __forceinline__ void decode_attn_body(
     char *lds_base, int share, int head_group, uint16_t *__restrict__ out,
     const uint16_t *__restrict__ q, const char *pages, const int32_t *__restrict__ kv_indices,
@@ -103,7 +108,7 @@ __device__ __forceinline__ void decode_attn_body(
     kv.half_bytes = kv.row_bytes << page_shift;
     kv.page_bytes = 2L * kv.half_bytes;
     kv.head_off = kvh * (kHeadDim * 2);
-    char *lds = lds_base + wave * kVTileBytes;
+    char *lds = lds_base + wave * tile_lds_bytes(kWholeRows);
 
     // Fused append (k_new != null): the newest token of a request has not been written
     // to its page yet.  The wave that will read it - kv head `kvh` of the item that ends
@@ -216,15 +221,15 @@ __device__ __forceinline__ void decode_attn_body(
     auto load_next = [&](TileRegs &r) {
         kv.page_ids = cur.page_ids;
         if (kPageCoversTile) {
-            load_kv_tile_in_page<kLoadStreaming>(kv, cur.page[0], cur.t, cur.t_end, g, c, r);
+            load_kv_tile_in_page<kLoadStreaming, kWholeRows>(kv, cur.page[0], cur.t, cur.t_end, g, c, r);
         } else if (kPagesPerTile > 1) {
             long pages_of_tile[kPagesPerTile > 1 ? kPagesPerTile : 1];
 #pragma unroll
             for (int j = 0; j < kPagesPerTile; j++) pages_of_tile[j] = cur.page[j];
-            load_kv_tile_small_pages<(kPagesPerTile > 1 ? kPagesPerTile : 1), kLoadStreaming>(
+            load_kv_tile_small_pages<(kPagesPerTile > 1 ? kPagesPerTile : 1), kLoadStreaming, kWholeRows>(
                 kv, pages_of_tile, cur.t, cur.t_end, g, c, r);
         } else {
-            load_kv_tile<false, kLoadStreaming>(kv, cur.t, cur.t_end, g, c, r);
+            load_kv_tile<false, kLoadStreaming, kWholeRows>(kv, cur.t, cur.t_end, g, c, r);
         }
         cur.t += kTile;
         settle();
@@ -274,10 +279,12 @@ __device__ __forceinline__ void decode_attn_body(
         float l_run = 0.f;
 
         auto compute_tile = [&](int t, const TileRegs &r) {
+            if (kWholeRows) stage_k_tile(lds, r, g, c);
             // scores: S^T = K . Q^T ; lane holds tokens t + 4g + j of q column c
             f32x4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int kk = 0; kk < 4; kk++) s = E::mfma_k32(r.k[kk], qreg[kk], s);
+            for (int kk = 0; kk < 4; kk++)
+                s = E::mfma_k32(kWholeRows ? read_k_operand(lds, kk, g, c) : r.k[kk], qreg[kk], s);
             const bool ragged = t + kTile > t_end;   // wave-uniform: last and padding tiles
             float x[4];
 #pragma unroll
@@ -363,8 +370,8 @@ __global__ __launch_bounds__(64 * kMaxWaves, DSKV_DECODE_MIN_WAVES) void decode_
     const uint16_t *__restrict__ k_new, const uint16_t *__restrict__ v_new,
     const float *__restrict__ rope)
 {
-    __shared__ __align__(16) char v_lds[kMaxWaves * kVTileBytes];
-    decode_attn_body<DT, kPagesPerTile, kMaxWaves>(v_lds, (int)blockIdx.x, (int)blockIdx.y, out, q, pages,
+    __shared__ __align__(16) char v_lds[kMaxWaves * tile_lds_bytes(false)];
+    decode_attn_body<DT, kPagesPerTile, kMaxWaves, kStages, false>(v_lds, (int)blockIdx.x, (int)blockIdx.y, out, q, pages,
                                                    kv_indices, items, wg_ptr, part_o, part_ml, max_slots,
                                                    n_qo_heads, n_kv_heads, page_shift, scale_log2, k_new,
                                                    v_new, rope);

@@ -4,7 +4,8 @@
 // Lane roles, with g = lane / 16 and c = lane % 16:
 //   K: lane holds dims kk*32 + g*8 .. +8 (kk = 0..3) of tile token c - the A
 //      operand of the 16x16x32 MFMA, so S^T = K.Q^T has tokens 4g..4g+3 of query
-//      column c in lane (g, c).
+//      column c in lane (g, c).  With kWholeRows it is loaded as V is, written to LDS row-major
+//      and read back as that operand.
 //   V: lane loads the 16-byte chunk c of tile tokens g, g+4, g+8, g+12; the tile
 //      is written to LDS row-major (one token per 288-byte row) and read back
 //      with the transposing LDS read, which hands lane (g, c) tokens 4g..4g+3 of
@@ -19,6 +20,9 @@ constexpr int kTile = 16;                 // tokens per MFMA tile
 constexpr int kHeadDim = 128;             // the MFMA kernels are specialised for D = 128
 constexpr int kVPitch = 288;              // bytes per V row in LDS (256 + 32 pad)
 constexpr int kVTileBytes = kTile * kVPitch;
+constexpr int kKPitch = 272;              // bytes per K row in LDS (256 + 16: 16 rows' chunks at one offset meet no bank twice)
+// LDS of a wave: its V tile, then (kWholeRows) its K tile.
+constexpr int tile_lds_bytes(bool whole_rows) { return kVTileBytes + (whole_rows ? kTile * kKPitch : 0); }
 constexpr int kBufferFlags = 0x00020000;  // raw buffer descriptor word 3 for 32-bit data
 // Cache-policy bits of the K/V loads.  Decode uses every K/V byte once, so its
 // loads carry the streaming hint (bit 1): measured on MI355X, a 607 MB read with
@@ -34,6 +38,10 @@ constexpr int kLoadCached = 0;
 typedef const __attribute__((address_space(4))) int32_t *const_i32_ptr;
 __device__ __forceinline__ const_i32_ptr as_const(const int32_t *p) { return (const_i32_ptr)p; }
 
+// How a wave reads the K rows of a tile.  As the score MFMA's operand a load instruction takes 64 bytes
+// of each of 16 rows; whole rows (kWholeRows) are 256 consecutive bytes of each of four, as V's, for a
+// trip through LDS.  Reading alone, 512 workgroups over 604 MB take 99.4 us in the first pattern and 93.4 in
+// the second, 256 workgroups 94.0 and 91.6.
 struct TileRegs {
     u32x4 k[4];
     u32x4 v[4];
@@ -56,7 +64,7 @@ struct KvView {
 // row: lanes that hold later rows (or a whole tile past the end) read zero and
 // generate no memory traffic, and the per-lane offsets never change.  Always
 // issues exactly 8 loads.
-template <int kAux>
+template <int kAux, bool kWholeRows>
 __device__ __forceinline__ void load_kv_tile_in_page(const KvView &kv, long page, int t, int t_end,
                                                      int g, int c, TileRegs &r)
 {
@@ -72,7 +80,8 @@ __device__ __forceinline__ void load_kv_tile_in_page(const KvView &kv, long page
     const int ko = c * kv.row_bytes + kv.head_off + g * 16;
 #pragma unroll
     for (int kk = 0; kk < 4; kk++)
-        r.k[kk] = __builtin_amdgcn_raw_buffer_load_b128(k_rows, ko + kk * 64, 0, kAux);
+        r.k[kk] = __builtin_amdgcn_raw_buffer_load_b128(
+            k_rows, kWholeRows ? (g + 4 * kk) * kv.row_bytes + kv.head_off + c * 16 : ko + kk * 64, 0, kAux);
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const int vo = (g + 4 * i) * kv.row_bytes + kv.head_off + c * 16;
@@ -91,32 +100,34 @@ __device__ __forceinline__ int page_slot_of(const KvView &kv, int t, int t_end)
 // Loads tile [t, t + 16) of a request whose valid tokens end at t_end.  Issued
 // unconditionally (so the count of loads in flight is static); nothing past
 // t_end is fetched.
-template <bool kPageCoversTile, int kAux>
+template <bool kPageCoversTile, int kAux, bool kWholeRows>
 __device__ __forceinline__ void load_kv_tile(const KvView &kv, int t, int t_end, int g, int c,
                                              TileRegs &r)
 {
     if (kPageCoversTile) {
-        load_kv_tile_in_page<kAux>(kv, kv.page_ids[page_slot_of(kv, t, t_end)], t, t_end, g, c, r);
+        load_kv_tile_in_page<kAux, kWholeRows>(kv, kv.page_ids[page_slot_of(kv, t, t_end)], t, t_end, g, c, r);
     } else {
         // Pages smaller than a tile: every lane resolves its own page.  Tokens
         // past the end are clamped to the last valid one; the consumer masks
         // their scores and zeroes their V rows.
-        const int k_tok = c;
         const int page_mask = (1 << kv.page_shift) - 1;
         const int t_last = max(t_end - 1, 0);
-        const int tk = min(t + k_tok, t_last);
-        const long kpage = kv.page_ids[tk >> kv.page_shift];
-        const char *kp = kv.pages + kpage * kv.page_bytes + (long)(tk & page_mask) * kv.row_bytes +
-                         kv.head_off + g * 16;
+        if (!kWholeRows) {
+            const int tk = min(t + c, t_last);
+            const long kpage = kv.page_ids[tk >> kv.page_shift];
+            const char *kp = kv.pages + kpage * kv.page_bytes + (long)(tk & page_mask) * kv.row_bytes +
+                             kv.head_off + g * 16;
 #pragma unroll
-        for (int kk = 0; kk < 4; kk++) r.k[kk] = *reinterpret_cast<const u32x4 *>(kp + kk * 64);
+            for (int kk = 0; kk < 4; kk++) r.k[kk] = *reinterpret_cast<const u32x4 *>(kp + kk * 64);
+        }
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int tv = min(t + g + 4 * i, t_last);
             const long vpage = kv.page_ids[tv >> kv.page_shift];
-            const char *vp = kv.pages + vpage * kv.page_bytes + kv.half_bytes +
-                             (long)(tv & page_mask) * kv.row_bytes + kv.head_off + c * 16;
-            r.v[i] = *reinterpret_cast<const u32x4 *>(vp);
+            const char *row = kv.pages + vpage * kv.page_bytes + (long)(tv & page_mask) * kv.row_bytes +
+                              kv.head_off + c * 16;
+            if (kWholeRows) r.k[i] = *reinterpret_cast<const u32x4 *>(row);
+            r.v[i] = *reinterpret_cast<const u32x4 *>(row + kv.half_bytes);
         }
     }
 }
@@ -130,7 +141,7 @@ __device__ __forceinline__ void load_kv_tile(const KvView &kv, int t, int t_end,
 // tokens the pass took 114 us; this way 100 (98 with pages of 16).  Tokens past the end are clamped to the last
 // valid one, as in the per-lane path; page[0] is a valid page of the request also for a tile
 // that lies wholly past the end.
-template <int kPages, int kAux>
+template <int kPages, int kAux, bool kWholeRows>
 __device__ __forceinline__ void load_kv_tile_small_pages(const KvView &kv, const long (&page)[kPages],
                                                          int t, int t_end, int g, int c, TileRegs &r)
 {
@@ -148,11 +159,14 @@ __device__ __forceinline__ void load_kv_tile_small_pages(const KvView &kv, const
         const u32x4 *q = reinterpret_cast<const u32x4 *>(p);
         return kAux == kLoadStreaming ? __builtin_nontemporal_load(q) : *q;
     };
-    const char *kp = row_of(t + c) + g * 16;
+    const char *rows[4];
 #pragma unroll
-    for (int kk = 0; kk < 4; kk++) r.k[kk] = load16(kp + kk * 64);
+    for (int i = 0; i < 4; i++) rows[i] = row_of(t + g + 4 * i) + c * 16;
+    const char *const kp = row_of(t + c) + g * 16;
 #pragma unroll
-    for (int i = 0; i < 4; i++) r.v[i] = load16(row_of(t + g + 4 * i) + kv.half_bytes + c * 16);
+    for (int i = 0; i < 4; i++) r.k[i] = load16(kWholeRows ? rows[i] : kp + i * 64);
+#pragma unroll
+    for (int i = 0; i < 4; i++) r.v[i] = load16(rows[i] + kv.half_bytes);
 }
 
 // V tile -> this wave's LDS tile.  Rows at or past t_end must be zero (their
@@ -173,6 +187,22 @@ __device__ __forceinline__ void stage_v_tile(char *lds, const TileRegs &r, int t
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
+}
+
+// kWholeRows: K tile -> this wave's LDS, behind the V tile; then the A operand of the 16x16x32 score
+// MFMA, dims kk*32 + 8g .. +7 of token c.  Rows past the end may hold anything: their scores are masked.
+__device__ __forceinline__ void stage_k_tile(char *lds, const TileRegs &r, int g, int c)
+{
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        *reinterpret_cast<u32x4 *>(lds + kVTileBytes + (g + 4 * i) * kKPitch + c * 16) = r.k[i];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+__device__ __forceinline__ u32x4 read_k_operand(const char *lds, int kk, int g, int c)
+{
+    return *reinterpret_cast<const u32x4 *>(lds + kVTileBytes + c * kKPitch + kk * 64 + g * 16);
 }
 
 // The transposing LDS read works on blocks of 16 lanes: lane i of a block

@@ -158,8 +158,10 @@ static int prefill_rows_per_tile(int n_qo_heads, int n_kv_heads, int waves)
 // behind 8000 tokens): the tile workgroups finish within 66 us, the decode workgroups, which
 // share the CU's memory path with them meanwhile, after 145 us instead of 113 us alone.
 // ---------------------------------------------------------------------------
-// Tiles in flight per decode wave of the mixed launch (2, 4 and 5 measured the same).
-constexpr int kSharedRing = kStages;
+// Tiles in flight per decode wave of the mixed launch: with three, the step of 75 rows and a chunk takes
+// 2370 us instead of 2364, 70B-shaped 1338 instead of 1327; with four 2383 and 1398.
+constexpr int kSharedRing = 2;
+constexpr bool kSharedWholeRows = true;
 // Wave priority of the tile workgroups.  At equal priority the compute unit serves the older
 // waves first, and the decode waves - launched first, never short of a load to issue - kept
 // the tile waves' few loads waiting: a tile workgroup took 162 us beside them instead of 38 us
@@ -188,11 +190,11 @@ template <int DT, int kPagesPerTile>
 __global__ __launch_bounds__(64 * kSharedWaves, 2) void mixed_attn_kernel(const MixedArgs a)
 {
     static_assert(kSharedWaves == kPrefillWavesShared, "both kinds of workgroup have the launch's size");
-    static_assert(kPrefillLdsBytes >= kSharedWaves * kVTileBytes, "the LDS is shared by the two bodies");
+    static_assert(kPrefillLdsBytes >= kSharedWaves * tile_lds_bytes(kSharedWholeRows), "the LDS is shared by the two bodies");
     __shared__ __align__(16) char lds[kPrefillLdsBytes];
     const int wg = blockIdx.x;
     if (wg < a.n_decode_wgs)
-        decode_attn_body<DT, kPagesPerTile, kSharedWaves, kSharedRing>(
+        decode_attn_body<DT, kPagesPerTile, kSharedWaves, kSharedRing, kSharedWholeRows>(
             lds, wg / a.head_groups, wg % a.head_groups, a.out, a.q, a.pages, a.kv_indices, a.items, a.wg_ptr,
             a.dec_part_o, a.dec_part_ml, a.dec_max_slots, a.n_qo_heads, a.n_kv_heads, a.page_shift,
             a.scale_log2, nullptr, nullptr, a.rope);
