@@ -94,6 +94,7 @@ _SIGNATURES = {
                                                c_int64, c_int32, c_int32, c_int32, c_int32, c_int32,
                                                c_float, c_int32, c_void_p, c_int32, c_void_p]),
     "dskv_decode_step": (c_int32, [POINTER(DecodeStep)] + [c_void_p] * 6),
+    "dskv_decode_layers": (c_int32, [POINTER(DecodeStep), c_int32] + [c_void_p] * 5 + [c_int64, c_void_p]),
     "dskv_prefill_plan_bound": (c_int64, [c_int32, c_int64]),
     "dskv_prefill_plan": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32, c_int32,
                                     c_void_p, c_int64, POINTER(c_int32), POINTER(c_int32),
@@ -114,6 +115,7 @@ _SIGNATURES = {
                                   c_int32, c_int32, c_void_p]),
     "dskv_mixed_step_supported": (c_int32, [c_int32, c_int32, c_int32, c_int32, c_float, c_int32]),
     "dskv_mixed_step": (c_int32, [POINTER(MixedStep)] + [c_void_p] * 6),
+    "dskv_mixed_layers": (c_int32, [POINTER(MixedStep), c_int32] + [c_void_p] * 5 + [c_int64, c_void_p]),
     "dskv_apply_rope": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                   c_int32, c_int32, c_int32, c_int32, c_int32, c_float, c_int32,
                                   c_void_p]),

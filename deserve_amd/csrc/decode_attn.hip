@@ -1077,6 +1077,27 @@ extern "C" int dskv_decode_step(const dskv_decode_step_t *step, void *out, const
                             step->merge_counters, step->n_merge_counters);
 }
 
+// All layers of a step whose q, k and v are there at once.  A call from Python costs a layer 13-16 us of host
+// time, more than the GPU needs where requests are few: a step of 16 layers over 1 request of 1777 tokens
+// 293 -> 219 us, over three prompts of 17 to 203 tokens 355-375 -> 306 us (both the GPU's time now).
+extern "C" int dskv_decode_layers(const dskv_decode_step_t *step, int32_t n_layers, void *out, const void *q,
+                                  const void *k_new, const void *v_new, void *pages, int64_t pages_layer_bytes,
+                                  void *stream)
+{
+    using namespace dskv;
+    DSKV_REQUIRE(step && n_layers >= 0 && step->batch >= 0, "decode_layers: bad arguments");
+    const int64_t elt = step->dtype == DSKV_F32 ? 4 : 2;
+    const int64_t q_bytes = (int64_t)step->batch * step->n_qo_heads * step->head_dim * elt;
+    const int64_t kv_bytes = (int64_t)step->batch * step->n_kv_heads * step->head_dim * elt;
+    auto at = [](const void *p, int64_t bytes) { return p ? (const char *)p + bytes : nullptr; };
+    for (int64_t l = 0; l < n_layers; l++) {
+        const int rc = dskv_decode_step(step, (void *)at(out, l * q_bytes), at(q, l * q_bytes), at(k_new, l * kv_bytes),
+                                        at(v_new, l * kv_bytes), (void *)at(pages, l * pages_layer_bytes), stream);
+        if (rc) return rc;
+    }
+    return 0;
+}
+
 // ---------------------------------------------------------------------------
 // The entry point that allocates nothing: the partial results live in a
 // file-scope device array instead of a caller workspace.

@@ -899,3 +899,20 @@ extern "C" int dskv_mixed_step(const dskv_mixed_step_t *step, void *out, const v
                            s.plan_dev, s.info, s.workspace, s.workspace_bytes, s.batch, s.nnz, s.n_qo_heads,
                            s.n_kv_heads, s.head_dim, s.page_size, s.sm_scale, s.causal, s.dtype, s.rope_table, stream);
 }
+
+extern "C" int dskv_mixed_layers(const dskv_mixed_step_t *step, int32_t n_layers, void *out, const void *q,
+                                 const void *k_new, const void *v_new, void *pages, int64_t pages_layer_bytes,
+                                 void *stream)
+{
+    using namespace dskv;
+    DSKV_REQUIRE(step && n_layers >= 0 && step->nnz >= 0, "mixed_layers: bad arguments");
+    const int64_t q_bytes = (int64_t)step->nnz * step->n_qo_heads * step->head_dim * 2;
+    const int64_t kv_bytes = (int64_t)step->nnz * step->n_kv_heads * step->head_dim * 2;
+    auto at = [](const void *p, int64_t bytes) { return p ? (const char *)p + bytes : nullptr; };
+    for (int64_t l = 0; l < n_layers; l++) {
+        const int rc = dskv_mixed_step(step, (void *)at(out, l * q_bytes), at(q, l * q_bytes), at(k_new, l * kv_bytes),
+                                       at(v_new, l * kv_bytes), (void *)at(pages, l * pages_layer_bytes), stream);
+        if (rc) return rc;
+    }
+    return 0;
+}

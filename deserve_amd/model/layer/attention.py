@@ -9,9 +9,10 @@ from typing import Optional
 
 import torch
 
+from deserve_amd.kvcache.paged.page_pool import PagePool
 from deserve_amd.model.context.flash import FlashDecodeCtx, FlashForwardCtx, FlashPrefillCtx
-from deserve_amd.paged_ops import (append_paged_kv_cache, apply_rope,
-                                   rope_append_paged_kv_cache)
+from deserve_amd.paged_ops import (BatchDecodeWithPagedKVCacheWrapper, BatchPrefillWithPagedKVCacheWrapper,
+                                   append_paged_kv_cache, apply_rope, rope_append_paged_kv_cache)
 
 
 class PagedAttentionCore:
@@ -32,6 +33,40 @@ class PagedAttentionCore:
             return self._paged_forward(xq, xk, xv, ctx, out)
         with torch.inference_mode():
             return self._paged_forward(xq, xk, xv, ctx, out)
+
+    def layers_forward(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ctx: FlashForwardCtx,
+                       out: torch.Tensor) -> bool:
+        """paged_forward for the layers ctx.layer_id .. of q, k, v and out, stacked: (L, tokens, heads, head_dim)
+        each, launched by one call to the library - layer by layer from here a step of one request costs the
+        host 13 us a layer, as long as the GPU works on it.  False, and nothing done, where the layers are not
+        plain stacks for the launches that append as they attend; ctx.layer_id counts on as it would."""
+        if q.dtype is torch.float32 or q.dim() != 4:     # no such launches: not worth looking further
+            return False
+        n, first, pool = q.shape[0], ctx.layer_id, ctx.page_pool
+        decode = type(ctx) is FlashDecodeCtx
+        if not decode and type(ctx) is not FlashPrefillCtx:
+            return False
+        wrapper = ctx.decode_wrapper if decode else ctx.prefill_wrapper
+        kind = BatchDecodeWithPagedKVCacheWrapper if decode else BatchPrefillWithPagedKVCacheWrapper
+        if type(wrapper) is not kind or "forward" in vars(wrapper) or \
+                getattr(pool.get_layered_pages, "__func__", None) is not PagePool.get_layered_pages or \
+                not 0 <= first <= pool.pages.shape[0] - n:
+            return False
+        pages = pool.pages[first: first + n]
+        with torch.inference_mode():
+            if decode:
+                taken = self.fuse_decode_append and k.shape[1] == ctx.bsz and wrapper.forward_layers(
+                    q, pages, out, k, v, ctx.offsets if self.use_rope else None, self.rope_theta)
+            else:
+                if self.use_rope and not self.fuse_rope_append or not wrapper.fused_append_supported(q.dtype):
+                    return False
+                table = ctx.rope_table(q.shape[1], self.head_dim, self.rope_theta) if self.use_rope else None
+                taken = wrapper.forward_layers(q, pages, out, k, v, table)
+                if taken and table is not None:
+                    ctx.rope_layer = first + n - 1     # the layer that would have asked for it last
+        if taken:
+            ctx.layer_id = first + n
+        return taken
 
     def _rows(self, x: torch.Tensor, heads: int) -> torch.Tensor:
         """x as (tokens, heads, head_dim)."""

@@ -179,6 +179,15 @@ class _PagedWrapper:
             raise ValueError(f"the block tables name page {self._max_page_id}, the pool has "
                              f"{paged_kv_data.shape[0]} pages")
 
+    def _stacks_fit(self, layers: int, rows: int, dtype: torch.dtype, q: torch.Tensor, pages: torch.Tensor,
+                    out: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
+        """Whether the stacks over `layers` layers are what forward takes layer by layer."""
+        kv = (layers, rows, self._hkv, self._d)
+        return (q.shape == (layers, rows, self._hq, self._d) and out.shape == q.shape and k.shape == kv and v.shape == kv
+                and pages.dim() == 6 and pages.shape[0] == layers and pages.shape[2:] == (2, self._p, self._hkv, self._d)
+                and self._max_page_id < pages.shape[1]
+                and all(t.dtype == dtype and t.is_cuda and t.is_contiguous() for t in (q, pages, out, k, v)))
+
     def end_forward(self) -> None:
         self._planned = False
 
@@ -308,6 +317,39 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
             return False
         return _decode_append_supported(self._hq, self._hkv, self._d, self._p, _lib.dtype_code(dtype))
 
+    def _step_table(self, rope_offsets: torch.Tensor, rope_theta: float, device: torch.device) -> int:
+        """Address of the step's cosines and sines, built at the first call after begin_forward."""
+        key = (rope_offsets.data_ptr(), float(rope_theta))
+        if self._rope_key != key:
+            if rope_offsets.dtype != torch.int32 or rope_offsets.numel() != self._batch:
+                raise ValueError(f"rope_offsets must be {self._batch} int32 positions")
+            table = torch.empty((self._batch, self._d), dtype=torch.float32, device=device)
+            _lib.check(_lib.lib().dskv_rope_table(table.data_ptr(), rope_offsets.data_ptr(),
+                                                  self._batch, self._d, rope_theta,
+                                                  _lib.current_stream()), "rope table")
+            self._rope_table, self._rope_key = table, key
+        return self._rope_table.data_ptr()
+
+    def forward_layers(self, q: torch.Tensor, pages: torch.Tensor, out: torch.Tensor, k_append: torch.Tensor,
+                       v_append: torch.Tensor, rope_offsets: Optional[torch.Tensor], rope_theta: float) -> bool:
+        """forward(q[l], pages[l], out=out[l], k_append=k_append[l], v_append=v_append[l], ...) for all layers l in
+        one call to the library.  False, and nothing done, for anything but plain contiguous stacks
+        that forward takes: the caller then goes layer by layer (and meets forward's error, if there is one)."""
+        n, dtype = q.shape[0], q.dtype
+        if not self._planned or self._empty_requests or not self.fused_append_supported(dtype) or \
+                not self._stacks_fit(n, self._batch, dtype, q, pages, out, k_append, v_append):
+            return False
+        if rope_offsets is not None and (rope_offsets.dtype != torch.int32 or rope_offsets.numel() != self._batch):
+            return False
+        step = _lib.DecodeStep.from_buffer_copy(self._step)
+        step.rope_table = None if rope_offsets is None else self._step_table(rope_offsets, rope_theta, q.device)
+        step.dtype, step.sm_scale = _lib.dtype_code(dtype), 1.0 / math.sqrt(self._d)
+        rc = _lib.lib().dskv_decode_layers(ctypes.byref(step), n, out.data_ptr(), q.data_ptr(), k_append.data_ptr(),
+                                           v_append.data_ptr(), pages.data_ptr(),
+                                           pages.stride(0) * pages.element_size(), _lib.current_stream())
+        _lib.check(rc, "decode forward")
+        return True
+
     def forward(self, q: torch.Tensor, paged_kv_data: torch.Tensor,
                 sm_scale: Optional[float] = None, *, phases: int = 3,
                 out: Optional[torch.Tensor] = None, k_append: Optional[torch.Tensor] = None,
@@ -351,16 +393,7 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
                     k_append.dtype != dtype or v_append.dtype != dtype:
                 raise ValueError(f"k_append / v_append must be {want} of q's dtype")
             if rope_offsets is not None:
-                key = (rope_offsets.data_ptr(), float(rope_theta))
-                if self._rope_key != key:
-                    if rope_offsets.dtype != torch.int32 or rope_offsets.numel() != self._batch:
-                        raise ValueError(f"rope_offsets must be {self._batch} int32 positions")
-                    table = torch.empty((self._batch, self._d), dtype=torch.float32, device=q.device)
-                    _lib.check(_lib.lib().dskv_rope_table(table.data_ptr(), rope_offsets.data_ptr(),
-                                                          self._batch, self._d, rope_theta,
-                                                          _lib.current_stream()), "rope table")
-                    self._rope_table, self._rope_key = table, key
-                table = self._rope_table.data_ptr()
+                table = self._step_table(rope_offsets, rope_theta, q.device)
         if phases == 3:
             step = _lib.DecodeStep.from_buffer_copy(self._step)    # calls from several threads do not share it
             step.rope_table, step.dtype, step.sm_scale = table, _lib.dtype_code(dtype), scale
@@ -512,6 +545,26 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
             return False
         scale = 1.0 / math.sqrt(self._d) if sm_scale is None else sm_scale
         return _mixed_step_supported(self._hq, self._hkv, self._d, self._p, scale, _lib.dtype_code(dtype))
+
+    def forward_layers(self, q: torch.Tensor, pages: torch.Tensor, out: torch.Tensor, k_append: torch.Tensor,
+                       v_append: torch.Tensor, rope_table: Optional[torch.Tensor]) -> bool:
+        """As the decode wrapper's."""
+        n, dtype = q.shape[0], q.dtype
+        if not self._planned or not self.fused_append_supported(dtype) or \
+                not self._stacks_fit(n, self._nnz, dtype, q, pages, out, k_append, v_append):
+            return False
+        if rope_table is not None and (rope_table.shape != (self._nnz, self._d) or rope_table.dtype != torch.float32 or
+                                       not rope_table.is_contiguous()):
+            return False
+        step = _lib.MixedStep.from_buffer_copy(self._step)
+        step.rope_table = None if rope_table is None else rope_table.data_ptr()
+        step.num_pages, step.causal = pages.shape[1], 1
+        step.dtype, step.sm_scale = _lib.dtype_code(dtype), 1.0 / math.sqrt(self._d)
+        rc = _lib.lib().dskv_mixed_layers(ctypes.byref(step), n, out.data_ptr(), q.data_ptr(), k_append.data_ptr(),
+                                          v_append.data_ptr(), pages.data_ptr(),
+                                          pages.stride(0) * pages.element_size(), _lib.current_stream())
+        _lib.check(rc, "prefill forward")
+        return True
 
     def forward(self, q: torch.Tensor, paged_kv_data: torch.Tensor, causal: bool = True,
                 sm_scale: Optional[float] = None, *, out: Optional[torch.Tensor] = None,

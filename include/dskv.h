@@ -241,6 +241,13 @@ typedef struct dskv_decode_step {
 } dskv_decode_step_t;
 int dskv_decode_step(const dskv_decode_step_t *step, void *out, const void *q, const void *k_new,
                      const void *v_new, void *pages_layer, void *stream);
+/*
+ * dskv_decode_step for n_layers layers one after the other, layer l's out, q, k_new and v_new directly behind
+ * layer l - 1's and its pages pages_layer_bytes behind them; k_new and v_new may be null as there.  The
+ * layers before the first one that is refused or fails have been enqueued.
+ */
+int dskv_decode_layers(const dskv_decode_step_t *step, int32_t n_layers, void *out, const void *q,
+                       const void *k_new, const void *v_new, void *pages, int64_t pages_layer_bytes, void *stream);
 
 /*
  * Paged prefill attention with the end-aligned causal mask.  Replaces
@@ -379,6 +386,9 @@ int dskv_mixed_step_supported(int32_t n_qo_heads, int32_t n_kv_heads, int32_t he
                               int32_t page_size, float sm_scale, int32_t dtype);
 int dskv_mixed_step(const dskv_mixed_step_t *step, void *out, const void *q, const void *k_new,
                     const void *v_new, void *pages_layer, void *stream);
+/* dskv_mixed_step for n_layers layers, laid out as dskv_decode_layers takes them. */
+int dskv_mixed_layers(const dskv_mixed_step_t *step, int32_t n_layers, void *out, const void *q, const void *k_new,
+                      const void *v_new, void *pages, int64_t pages_layer_bytes, void *stream);
 
 /*
  * Rotary embedding, adjacent-pair convention.  Replaces the call site

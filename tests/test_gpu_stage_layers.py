@@ -1,0 +1,64 @@
+"""A stage whose layers run in one call to the library, against the same layers called one by one: the
+same bits in the result and the pages, the same layer count; what is not a plain stack goes layer
+by layer, and a pool with too few layers is refused as it is there."""
+import pytest
+import torch
+
+from deserve_amd.execution.exec import BatchDecode, BatchPrefill
+from deserve_amd.stage import KVStage
+from deserve_amd.synthetic import make_mixed_workload
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = {
+    "one_request": ([70], [], []),
+    "decode": ([33, 600, 1, 16], [], []),
+    "prompts": ([], [0, 40], [17, 5]),
+    "shared_launch": ([30 + 40 * i for i in range(14)], [20], [12]),
+}
+
+
+def _run(shape, dtype, rope, together, q_of=lambda q: q, first=0, out_layers=3):
+    wl = make_mixed_workload("t", *SHAPES[shape], 3, 16, 4, 128, 8, dtype, seed=5)
+    stage = KVStage(wl.args, use_rope=rope)
+    if not together:
+        stage.core.layers_forward = lambda *a: False
+    kind = BatchPrefill if SHAPES[shape][2] else BatchDecode
+    batch = kind(None, stage, wl.tasks, wl.caches)
+    batch.prepare()
+    ctx = batch.prefill_ctx if SHAPES[shape][2] else batch.decode_ctx
+    ctx.layer_id = first
+    out = stage.forward((q_of(wl.q)[:out_layers], wl.k[:out_layers], wl.v[:out_layers]), ctx)
+    torch.cuda.synchronize()
+    return out, wl.pool.pages, ctx.layer_id
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_layers_in_one_call_match_layers_one_by_one(shape, rope, dtype):
+    print("[case] stage layers", shape, rope, dtype, flush=True)
+    for kw in ({}, {"first": 1, "out_layers": 2}):
+        got, want = _run(shape, dtype, rope, True, **kw), _run(shape, dtype, rope, False, **kw)
+        assert got[2] == want[2] == 3
+        for a, b in zip(got[:2], want[:2]):
+            assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+def test_stacks_that_are_not_plain_go_layer_by_layer():
+    print("[case] stage layers, strided q", flush=True)
+    strided = lambda q: q.transpose(0, 1).contiguous().transpose(0, 1)
+    flat = lambda q: q.reshape(q.shape[0], q.shape[1], -1)
+    want = _run("decode", torch.bfloat16, True, False)
+    for q_of in (strided, flat):
+        got = _run("decode", torch.bfloat16, True, True, q_of)
+        assert torch.equal(got[0].view(torch.int16), want[0].view(torch.int16))
+        assert torch.equal(got[1].view(torch.int16), want[1].view(torch.int16))
+
+
+@pytest.mark.parametrize("shape", ["decode", "prompts"])
+def test_more_layers_than_the_pool_has_are_refused(shape):
+    print("[case] stage layers beyond the pool", shape, flush=True)
+    for together in (True, False):
+        with pytest.raises(IndexError):
+            _run(shape, torch.bfloat16, True, together, first=1)
