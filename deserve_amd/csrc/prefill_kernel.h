@@ -358,9 +358,11 @@ __device__ __forceinline__ void prefill_attn_body(
 #pragma unroll
         for (int ct = 0; ct < kColTiles; ct++) {
             asm volatile("" : "+v"(xs[buf][ct]));   // (re)defined here: the selects cannot leave the branch
+            int seen = limit[ct] - 4 * h - t;   // tokens of the lane's half that the column sees
+            asm volatile("" : "+v"(seen));      // the sixteen comparisons hold no registers outside the branch
 #pragma unroll
             for (int v = 0; v < 16; v++)
-                if (t + 8 * (v >> 2) + 4 * h + (v & 3) >= limit[ct]) xs[buf][ct][v] = kNegBig;
+                if (8 * (v >> 2) + (v & 3) >= seen) xs[buf][ct][v] = kNegBig;
         }
     };
     // Column maximum of the block in xs[buf], and whether the running maximum has to be
