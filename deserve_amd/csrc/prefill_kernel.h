@@ -27,20 +27,18 @@ constexpr int kTileWords = 6;                       // plan entry: request, firs
 // region) fall on 16 different 16-byte bank groups each.
 constexpr int kRegionBytes = 1088;
 constexpr int kStageBytes = (kBlock / 4) * kRegionBytes;
-// The running maximum of a column is only raised when a block exceeds it by more
-// than this (log2 domain): probabilities stay below 2^8, the accumulators are
-// rescaled a handful of times per query instead of once per block.
-constexpr float kRescaleSlack = 8.f;
+// The running maximum of a column is only raised when a block's probabilities under it sum to more
+// than this in a lane (half of the block's tokens): the accumulators are rescaled a handful of times per
+// query instead of once per block, and blocks that need no raise (nearly all) need no maximum: with the
+// board at its power cap every instruction costs time.  With a maximum per block (17 of 85 vector instructions) 16
+// chunks of 512 tokens took 11245 us in 16 layers, now 10957; a chunk of 512 over 4096 946, now 933.
+constexpr float kMostProbability = 256.f;
 #ifndef DSKV_PREFILL_KPREFETCH
 #define DSKV_PREFILL_KPREFETCH 1   // K operands of the next iteration read before its barrier (direct path)
 #endif
 #ifndef DSKV_PREFILL_KREADS_FIRST
 #define DSKV_PREFILL_KREADS_FIRST 0
 #endif
-#ifndef DSKV_PREFILL_SUM_ON_MFMA
-#define DSKV_PREFILL_SUM_ON_MFMA 0
-#endif
-constexpr bool kSumOnMfma = DSKV_PREFILL_SUM_ON_MFMA;   // row sums of P by the matrix pipeline
 
 // Lane roles of the 32x32x16 MFMA, with h = lane / 32 and r = lane % 32:
 //   A operand: row r, k = 8h .. 8h+7.   B operand: column r, k = 8h .. 8h+7.
@@ -174,28 +172,18 @@ __device__ __forceinline__ void prefill_attn_body(
     // scaled masked score (kNegBig * scale_log2).
     float m_run[kColTiles];
     f32x16 acc[kColTiles][4];     // O^T: dims 32*dt + 8i + 4h + j of column r in acc[ct][dt][4i + j]
-    // Row sums of P, optionally on the matrix pipeline: ones(32 x tokens) . P^T - every
-    // register of a lane then holds the sum of its column r over the tokens multiplied so
-    // far.  It takes 16 additions per block off the vector pipeline and adds two MFMAs;
-    // measured on MI355X the kernel takes the same time either way, so the default keeps the
-    // sums on the vector pipeline (fewer registers, less matrix work).
-    f32x16 l_acc[kColTiles];
-    float l_run[kColTiles];       // the same sums kept by the vector pipeline (kSumOnMfma off)
-    u32x4 pb[kColTiles][2];       // packed probabilities of the previous block, per k-step
+    float l_run[kColTiles];       // row sums of P, of the lane's half of the tokens
+    u32x4 pb[2][kColTiles][2];    // packed probabilities of this block and the one before, per k-step
 #pragma unroll
     for (int ct = 0; ct < kColTiles; ct++) {
         m_run[ct] = 0.5f * kNegBig * scale_log2;
         l_run[ct] = 0.f;
 #pragma unroll
-        for (int v = 0; v < 16; v++) l_acc[ct][v] = 0.f;
-#pragma unroll
         for (int dt = 0; dt < 4; dt++)
 #pragma unroll
             for (int v = 0; v < 16; v++) acc[ct][dt][v] = 0.f;
-        pb[ct][0] = pb[ct][1] = u32x4{0, 0, 0, 0};
+        pb[1][ct][0] = pb[1][ct][1] = u32x4{0, 0, 0, 0};   // P(-1)
     }
-    const uint32_t one2 = E::pack2(1.f, 1.f);
-    const u32x4 ones = {one2, one2, one2, one2};
 
     // A tile cut into parts: every part leaves (max, sum, unnormalised O) of its rows in the
     // workspace (O blocks of all slots, then their (max, sum) pairs); a part that sees nothing
@@ -365,25 +353,54 @@ __device__ __forceinline__ void prefill_attn_body(
                 if (8 * (v >> 2) + (v & 3) >= seen) xs[buf][ct][v] = kNegBig;
         }
     };
-    // Column maximum of the block in xs[buf], and whether the running maximum has to be
-    // raised before the block's exponentials.
-    float m_blk[kColTiles];
-    bool raise = false;
-    auto block_max = [&](int buf) {
-        raise = false;
+    // P of the block in xs[buf] under the running maximum, packed; returns whether a lane's sum is too large
+    // for that maximum (then P is to be taken again under a higher one), which infinities are, too.
+    auto probabilities = [&](int buf, float(&p_sum)[kColTiles]) {
+        bool over = false;
+#pragma unroll
+        for (int ct = 0; ct < kColTiles; ct++) {
+            float p[16];
+            p_sum[ct] = 0.f;
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                p[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(xs[buf][ct][v], scale_log2, -m_run[ct]));
+                p_sum[ct] += p[v];
+            }
+            over |= p_sum[ct] > kMostProbability;
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++)
+                pb[buf][ct][ks] = u32x4{E::pack2(p[8 * ks], p[8 * ks + 1]), E::pack2(p[8 * ks + 2], p[8 * ks + 3]),
+                                        E::pack2(p[8 * ks + 4], p[8 * ks + 5]), E::pack2(p[8 * ks + 6], p[8 * ks + 7])};
+        }
+        return over;
+    };
+    // Raises the running maximum to the block's in xs[buf] and brings what was computed under the old one
+    // (accumulators, row sum, the block before's P, still to be multiplied) to the new scale.
+    auto raise_maximum = [&](int buf) {
 #pragma unroll
         for (int ct = 0; ct < kColTiles; ct++) {
             const f32x16 &xc = xs[buf][ct];
-            // scale_log2 > 0: the maximum can be taken before scaling.  A chain of
-            // three-input maxima: 8 instructions for 16 values.
+            // scale_log2 > 0: the maximum can be taken before scaling
             float m = fmaxf(fmaxf(xc[0], xc[1]), xc[2]);
 #pragma unroll
             for (int v = 3; v < 15; v += 2) m = fmaxf(fmaxf(m, xc[v]), xc[v + 1]);
             m = fmaxf(m, xc[15]);
             float other = m;
             swap_halves32(m, other);
-            m_blk[ct] = fmaxf(m, other) * scale_log2;
-            raise |= m_blk[ct] > m_run[ct] + kRescaleSlack;
+            const float m_new = fmaxf(m_run[ct], fmaxf(m, other) * scale_log2);
+            const float alpha = __builtin_amdgcn_exp2f(m_run[ct] - m_new);
+            m_run[ct] = m_new;
+            l_run[ct] *= alpha;
+#pragma unroll
+            for (int dt = 0; dt < 4; dt++) acc[ct][dt] *= alpha;
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+                for (int w = 0; w < 4; w++) {
+                    float lo, hi;
+                    E::unpack2(pb[buf ^ 1][ct][ks][w], lo, hi);
+                    pb[buf ^ 1][ct][ks][w] = E::pack2(lo * alpha, hi * alpha);
+                }
         }
     };
 
@@ -452,7 +469,6 @@ __device__ __forceinline__ void prefill_attn_body(
         read_k_operands(k_stage[0], kKPrefetch ? 1 : 0);
         scores(0, kKPrefetch ? 1 : 0);
         if ((blk_begin + 1) * kBlock > w_mask_from) mask_scores(blk_begin, 0);
-        block_max(0);
         if (kKPrefetch) read_k_operands(k_stage[1], 0);   // K(blk_begin + 1) for the first iteration
     }
     // V operand: token 16 ks + 8 hi + 4 h + (c >> 2) = row c >> 2 of region 4 ks + 2 hi + h;
@@ -493,43 +509,15 @@ __device__ __forceinline__ void prefill_attn_body(
             else prepare_rows(m + 4, pg[phase], desc[phase]);
             return;
         }
-        if (__builtin_amdgcn_ballot_w64(raise) != 0) {
-            // rare: raise the maximum and bring what was computed under the old
-            // one (accumulators, row sum, the pending P(m-1)) to the new scale
-#pragma unroll
-            for (int ct = 0; ct < kColTiles; ct++) {
-                const float m_new = fmaxf(m_run[ct], m_blk[ct]);
-                const float alpha = __builtin_amdgcn_exp2f(m_run[ct] - m_new);
-                m_run[ct] = m_new;
-                if (kSumOnMfma) l_acc[ct] *= alpha;
-                else l_run[ct] *= alpha;
-#pragma unroll
-                for (int dt = 0; dt < 4; dt++) acc[ct][dt] *= alpha;
-#pragma unroll
-                for (int ks = 0; ks < 2; ks++)
-#pragma unroll
-                    for (int w = 0; w < 4; w++) {
-                        float lo, hi;
-                        E::unpack2(pb[ct][ks][w], lo, hi);
-                        pb[ct][ks][w] = E::pack2(lo * alpha, hi * alpha);
-                    }
-            }
-        }
         // The rest of the iteration is two straight-line halves, each an MFMA
-        // strand with independent vector work in its shadow:
+        // strand with independent vector and LDS work in its shadow:
         //   S(m+1) = K(m+1).Q^T     |  P(m) = exp2(S(m) * scale - max), packed; row sum;
         //                           |  V(m-1) operands from LDS
-        //   O += P(m-1).V(m-1)      |  maximum of S(m+1)
-        // with the masking of S(m+1), where needed, between them.  A masked score
+        //   O += P(m-1).V(m-1)      |  K(m+2) operands from LDS
+        // with, where needed, the raise of the maximum and the masking of S(m+1) between them.  A masked score
         // is kNegBig and the maximum never drops below its start value, so masked
         // probabilities come out as exp2(-huge) = 0 without a select.
         const int cur = phase & 1, nxt = cur ^ 1;   // xs[cur] = S(m), xs[nxt] receives S(m+1)
-        u32x4 pb_prev[kColTiles][2];
-#pragma unroll
-        for (int ct = 0; ct < kColTiles; ct++) {
-            pb_prev[ct][0] = pb[ct][0];
-            pb_prev[ct][1] = pb[ct][1];
-        }
         // V operand: the transposing read hands each block of 16 lanes four tokens
         // of 16 consecutive dims, lane i of the block supplying the address of dims
         // 4*(i%4) .. +3 of the block's token i/4
@@ -549,22 +537,19 @@ __device__ __forceinline__ void prefill_attn_body(
                 va[dt][ks] = u32x4{a_lo.x, a_lo.y, a_hi.x, a_hi.y};
             }
         scores(nxt, kKPrefetch ? (phase & 1) : 0);
+        float p_sum[kColTiles];
+        const bool over = probabilities(cur, p_sum);
+        // keeps P(m) in this half (it is only consumed by the next iteration)
 #pragma unroll
-        for (int ct = 0; ct < kColTiles; ct++) {
-            float p[16], p_sum = 0.f;
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                p[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(xs[cur][ct][v], scale_log2, -m_run[ct]));
-                if (!kSumOnMfma) p_sum += p[v];
-            }
-            if (!kSumOnMfma) l_run[ct] += p_sum;
-#pragma unroll
-            for (int ks = 0; ks < 2; ks++)
-                pb[ct][ks] = u32x4{E::pack2(p[8 * ks], p[8 * ks + 1]), E::pack2(p[8 * ks + 2], p[8 * ks + 3]),
-                                   E::pack2(p[8 * ks + 4], p[8 * ks + 5]), E::pack2(p[8 * ks + 6], p[8 * ks + 7])};
-            // keeps P(m) in this half (it is only consumed by the next iteration)
-            asm volatile("" ::"v"(pb[ct][0]), "v"(pb[ct][1]), "v"(l_run[ct]));
+        for (int ct = 0; ct < kColTiles; ct++)
+            asm volatile("" ::"v"(pb[cur][ct][0]), "v"(pb[cur][ct][1]), "v"(p_sum[ct]));
+        if (__builtin_amdgcn_ballot_w64(over) != 0) {   // rare
+            raise_maximum(cur);
+            __builtin_amdgcn_sched_barrier(0);   // one after the other: side by side they spill
+            probabilities(cur, p_sum);
         }
+#pragma unroll
+        for (int ct = 0; ct < kColTiles; ct++) l_run[ct] += p_sum[ct];
         if ((m + 2) * kBlock > w_mask_from) mask_scores(m + 1, nxt);   // wave-uniform
 
 #pragma unroll
@@ -573,22 +558,13 @@ __device__ __forceinline__ void prefill_attn_body(
             for (int ks = 0; ks < 2; ks++)
 #pragma unroll
                 for (int ct = 0; ct < kColTiles; ct++)
-                    acc[ct][dt] = E::mfma_32x32(va[dt][ks], pb_prev[ct][ks], acc[ct][dt]);
-        if (kSumOnMfma)
-#pragma unroll
-            for (int ks = 0; ks < 2; ks++)
-#pragma unroll
-                for (int ct = 0; ct < kColTiles; ct++)
-                    l_acc[ct] = E::mfma_32x32(ones, pb_prev[ct][ks], l_acc[ct]);
+                    acc[ct][dt] = E::mfma_32x32(va[dt][ks], pb[nxt][ct][ks], acc[ct][dt]);   // P(m-1): the other buffer
         if (kKPrefetch) {
             read_k_operands(k_stage[(phase + 2) & 3], (phase + 1) & 1);   // K(m+2), published by this iteration's barrier
             prepare_rows(m + 5, pg[(phase + 1) & 3], desc[(phase + 1) & 3]);
         } else {
             prepare_rows(m + 4, pg[phase], desc[phase]);   // for the loads of the next iterations
         }
-        block_max(nxt);
-#pragma unroll
-        for (int ct = 0; ct < kColTiles; ct++) asm volatile("" ::"v"(m_blk[ct]));
     };
     for (int m = blk_begin; m <= n_blocks; m += 4) {
         iteration(m, 0, even);
@@ -625,12 +601,9 @@ __device__ __forceinline__ void prefill_attn_body(
     };
 #pragma unroll
     for (int ct = 0; ct < kColTiles; ct++) {
-        float l = l_acc[ct][0];   // summed over all tokens by the MFMA (both lane halves)
-        if (!kSumOnMfma) {
-            float l_other = l_run[ct];
-            swap_halves32(l_run[ct], l_other);
-            l = l_run[ct] + l_other;
-        }
+        float l_other = l_run[ct];
+        swap_halves32(l_run[ct], l_other);
+        const float l = l_run[ct] + l_other;
         char *const mine = rows_lds + r * kRowsOutPitch;
         if (partial) {   // (max, sum, unnormalised O) of the row into its slot, 64 dims at a time
             const int slot = (qrow[ct] - q0) * tile_parts + split, qh = kvh * group + c_head[ct];   // from first_slot
