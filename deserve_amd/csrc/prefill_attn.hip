@@ -190,8 +190,8 @@ template <int DT, int kPagesPerTile>
 __global__ __launch_bounds__(64 * kSharedWaves, 2) void mixed_attn_kernel(const MixedArgs a)
 {
     static_assert(kSharedWaves == kPrefillWavesShared, "both kinds of workgroup have the launch's size");
-    static_assert(kPrefillLdsBytes >= kSharedWaves * tile_lds_bytes(kSharedWholeRows), "the LDS is shared by the two bodies");
-    __shared__ __align__(16) char lds[kPrefillLdsBytes];
+    static_assert(prefill_lds_bytes(kSharedWaves) >= kSharedWaves * tile_lds_bytes(kSharedWholeRows), "the LDS is shared by the two bodies");
+    __shared__ __align__(16) char lds[prefill_lds_bytes(kSharedWaves)];
     const int wg = blockIdx.x;
     if (wg < a.n_decode_wgs)
         decode_attn_body<DT, kPagesPerTile, kSharedWaves, kSharedRing, kSharedWholeRows>(

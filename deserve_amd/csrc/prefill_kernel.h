@@ -43,18 +43,22 @@ constexpr float kMostProbability = 256.f;
 // Lane roles of the 32x32x16 MFMA, with h = lane / 32 and r = lane % 32:
 //   A operand: row r, k = 8h .. 8h+7.   B operand: column r, k = 8h .. 8h+7.
 //   C/D: column r, rows 8i + 4h + j in register 4i + j (i, j = 0..3).
-// LDS of one workgroup: four stages of K rows, then four of V rows.
-constexpr int kPrefillLdsBytes = 8 * kStageBytes;
-// ... and, at the end, 256 bytes of each of a wave's columns (16 bytes of padding between them)
-constexpr int kRowsOutPitch = 256 + 16;
-constexpr int kRowsOutBytes = 32 * kRowsOutPitch;
+// LDS of one workgroup: four stages of K rows, then four of V rows; at the start, 256 bytes of sixteen of each
+// wave's columns from V's third stage on (beyond the stages where there are eight waves: such a
+// workgroup has its compute unit to itself), at the end of all of them (16 bytes of padding between them).
+constexpr int kRowPitch = 256 + 16;
+constexpr int kQRowsBytes = 16 * kRowPitch, kRowsOutBytes = 32 * kRowPitch;
+constexpr int prefill_lds_bytes(int waves)
+{
+    return 6 * kStageBytes + (waves * kQRowsBytes > 2 * kStageBytes ? waves * kQRowsBytes : 2 * kStageBytes);
+}
 struct LdsStages {
     char *base;
     __device__ __forceinline__ char *operator[](int i) const { return base + i * kStageBytes; }
 };
 
 // The kernel's body for workgroup `wg` of kWaves waves (a tile of kWaves * 32 / group query
-// rows of one kv head); `lds`: kPrefillLdsBytes of the workgroup's LDS.  A function, so that
+// rows of one kv head); `lds`: prefill_lds_bytes(kWaves) of the workgroup's LDS.  A function, so that
 // one launch can hold workgroups of this kind next to workgroups of another.
 //   kStreamOut: the rows leave past the L2 (non-temporal stores), which is the launch's K/V's.  Beside
 //     decode workgroups, whose own K/V stream past it, the partials of a chunk in two parts (14.5 MB)
@@ -102,13 +106,17 @@ __device__ __forceinline__ void prefill_attn_body(
     const bool partial = part_word >= 0;
     const int split = part_word & 0xff, tile_parts = part_word >> 8;
     const int first_slot = entry[5];
-    const int q_begin = qo_indptr[b];
-    const int n_b = qo_indptr[b + 1] - q_begin;
-    const int n_pages = kv_indptr[b + 1] - kv_indptr[b];
-    const int kv_len = n_pages > 0 ? ((n_pages - 1) << page_shift) + kv_last[b] : 0;
+    // (all requested before the first is looked at: the chain plan -> request -> pages -> rows is what a
+    // workgroup's start lasts)
+    const const_i32_ptr qo_at = as_const(qo_indptr) + b, kv_at = as_const(kv_indptr) + b;
+    const int q_begin = qo_at[0], q_next = qo_at[1], page_begin = kv_at[0], page_next = kv_at[1];
+    const int last_page_len = as_const(kv_last)[b];
+    __builtin_amdgcn_sched_barrier(0);
+    const int n_b = q_next - q_begin, n_pages = page_next - page_begin;
+    const int kv_len = n_pages > 0 ? ((n_pages - 1) << page_shift) + last_page_len : 0;
     // tokens this workgroup may look at end here: the request's end, or the end of its part
     const int kv_cap = min(kv_len, kv_cap_blocks < (1 << 25) ? kv_cap_blocks * kBlock : kv_len);
-    const_i32_ptr page_ids = as_const(kv_indices) + kv_indptr[b];
+    const_i32_ptr page_ids = as_const(kv_indices) + page_begin;
     const int row_bytes = n_kv_heads * kHeadDim * 2;
     const int half_bytes = row_bytes << page_shift;
     const long page_bytes = 2L * half_bytes;
@@ -118,7 +126,6 @@ __device__ __forceinline__ void prefill_attn_body(
     const int wq0 = q0 + wave * pos_per_wave;
     int qrow[kColTiles], c_head[kColTiles], limit[kColTiles];   // limit: kv tokens the column may see
     bool live[kColTiles];
-    u32x4 qreg[kColTiles][8];     // dims 16*ks + 8h .. +7 of the column's query
 #pragma unroll
     for (int ct = 0; ct < kColTiles; ct++) {
         const int col = 32 * ct + r;
@@ -128,33 +135,72 @@ __device__ __forceinline__ void prefill_attn_body(
         live[ct] = c_pos < pos_per_wave && qrow[ct] < n_b;
         const int lim = causal ? kv_len - n_b + qrow[ct] + 1 : kv_len;
         limit[ct] = live[ct] ? min(max(lim, 0), kv_cap) : 0;
-        const uint16_t *qrow_p =
-            q + ((long)(q_begin + qrow[ct]) * n_qo_heads + (long)kvh * group + c_head[ct]) * kHeadDim + h * 8;
+    }
+    // The wave's q rows, whole: lane (g, c) holds chunk c of column 4 j + g, and (rope: cos | sin by query row)
+    // the cosines and sines of its four dim pairs.  Loaded as the operand they become, an instruction took 32 bytes
+    // of each of 32 rows, and the address path was busy with a workgroup's before it took the first K and V: three
+    // short prompts 323 us in 16 layers, now 313, a chunk of 512 over 4096 918, now 908.
+    // q is rotated here: a row is loaded by one workgroup per kv head and part, so this costs a workgroup 16 more
+    // loads and the rotation at its start and saves the launch that read
+    // and wrote all of q: for 8192 rows of 32 heads 39 us for rotating q and k and appending
+    // against 15 us for the append that is left, 5.8 against 4.4 for 512 rows.
+    struct QRows {
+        u32x4 q[8];
+        f32x4 cs[8], sn[8];
+    };
+    auto load_q = [&](int ct, QRows &rows) {
+        // a column without a row takes the tile's first: it is not stored
+        const int row = q_begin + (live[ct] ? qrow[ct] : q0), at = row * n_qo_heads + kvh * group + (live[ct] ? c_head[ct] : 0);
+        int from[8], tab_row[8];
 #pragma unroll
-        for (int ks = 0; ks < 8; ks++) {
-            u32x4 z = {0, 0, 0, 0};
-            qreg[ct][ks] = live[ct] ? *reinterpret_cast<const u32x4 *>(qrow_p + ks * 16) : z;
+        for (int j = 0; j < 8; j++) from[j] = __shfl(at, 4 * j + g);
+#pragma unroll
+        for (int j = 0; j < 8; j++) rows.q[j] = *reinterpret_cast<const u32x4 *>(q + (long)from[j] * kHeadDim + c * 8);
+        if (!rope) return;
+#pragma unroll
+        for (int j = 0; j < 8; j++) tab_row[j] = __shfl(row, 4 * j + g);
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const float *tab = rope + (long)tab_row[j] * kHeadDim + c * 4;
+            rows.cs[j] = *reinterpret_cast<const f32x4 *>(tab);
+            rows.sn[j] = *reinterpret_cast<const f32x4 *>(tab + kHeadDim / 2);
         }
-        // q rotated as it is loaded, by the row's cosines and sines (rope: cos | sin by query row).
-        // A row is loaded by one workgroup per kv head and part, so this costs a workgroup 16 more
-        // loads and the rotation at its start (1-2 us of a launch) and saves the launch that read
-        // and wrote all of q: for 8192 rows of 32 heads 39 us for rotating q and k and appending
-        // against 15 us for the append that is left, 5.8 against 4.4 for 512 rows.  (Behind the
-        // requests for the first blocks of K and V it took as long.)
-        if (rope) {
-            const float *tab = rope + (long)(q_begin + (live[ct] ? qrow[ct] : 0)) * kHeadDim + h * 4;
+    };
+    u32x4 qreg[kColTiles][8];     // the B operand: dims 16*ks + 8h .. +7 of the column's query
+    // ... through LDS, sixteen columns at a time, in a stretch of the wave's own that is zero afterwards: V(-1) lies
+    // there, which is multiplied by P(-1) = 0
+    char *const q_lds = v_stage[2] + wave * kQRowsBytes;
+    static_assert(prefill_lds_bytes(4) == 8 * kStageBytes && 4 * kQRowsBytes == 2 * kStageBytes, "four stretches fill two stages");
+    auto finish_q = [&](int ct, QRows &rows) {
+        if (rope)
 #pragma unroll
-            for (int ks = 0; ks < 8; ks++) {   // dims 16 ks + 8 h .. +7 = pairs 8 ks + 4 h .. +3
-                const f32x4 c4 = *reinterpret_cast<const f32x4 *>(tab + ks * 8);
-                const f32x4 s4 = *reinterpret_cast<const f32x4 *>(tab + kHeadDim / 2 + ks * 8);
+            for (int j = 0; j < 8; j++) {
+                const f32x4 c4 = rows.cs[j], s4 = rows.sn[j];
                 const float cs[4] = {c4[0], c4[1], c4[2], c4[3]}, sn[4] = {s4[0], s4[1], s4[2], s4[3]};
                 float f[8];
-                Chunk<DT>::unpack(qreg[ct][ks], f);
+                Chunk<DT>::unpack(rows.q[j], f);
                 rope_rotate<4>(f, cs, sn);
-                qreg[ct][ks] = Chunk<DT>::pack(f);
+                rows.q[j] = Chunk<DT>::pack(f);
             }
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                *reinterpret_cast<u32x4 *>(q_lds + (4 * j + g) * kRowPitch + c * 16) = rows.q[4 * p + j];
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            if (r >> 4 == p)
+#pragma unroll
+                for (int ks = 0; ks < 8; ks++)
+                    qreg[ct][ks] = *reinterpret_cast<const u32x4 *>(q_lds + c * kRowPitch + (2 * ks + h) * 16);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
         }
-    }
+#pragma unroll
+        for (int i = 0; i < 4; i++) *reinterpret_cast<u32x4 *>(q_lds + (i * 64 + lane) * 16) = u32x4{0, 0, 0, 0};
+        static_assert(kQRowsBytes == (4 * 64 + 16) * 16, "");
+        if (lane < 16) *reinterpret_cast<u32x4 *>(q_lds + (4 * 64 + lane) * 16) = u32x4{0, 0, 0, 0};
+    };
     // Token ranges from scalars only: they steer loops, barriers and page lookups
     // and must be uniform for the compiler too.  The workgroup walks [0, t_end);
     // a wave computes on [0, w_end) and masks from w_mask_from on.
@@ -430,31 +476,47 @@ __device__ __forceinline__ void prefill_attn_body(
     };
     RowSet even, odd;
     {
-        const u32x4 z = {0, 0, 0, 0};
-        u32x4 zero[kRowGroups];
-#pragma unroll
-        for (int i = 0; i < kRowGroups; i++) zero[i] = z;
-        store_rows(v_stage[3], zero);   // V(-1): multiplied by P(-1) = 0, must be finite
         // the walk starts at block blk_begin, a multiple of four: block j still lives in stage j % 4
+        QRows rows;
+        load_q(0, rows);
+        auto finish_all_q = [&]() {
+            finish_q(0, rows);
+#pragma unroll
+            for (int ct = 1; ct < kColTiles; ct++) {
+                load_q(ct, rows);
+                finish_q(ct, rows);
+            }
+        };
         if (kRowsSharePage) {
+            int ahead[2][kRowGroups];   // pages of blocks 4 and 5
 #pragma unroll
             for (int blk = 0; blk < 4; blk++) lookup_pages(blk_begin + blk, pg[blk]);
+#pragma unroll
+            for (int blk = 0; blk < 2; blk++) lookup_pages(blk_begin + 4 + blk, ahead[blk]);
+            __builtin_amdgcn_sched_barrier(0);   // all six requested before the first is waited for
+#pragma unroll
+            for (int i = 0; i < kRowGroups; i++)   // (their sign extension otherwise waits for each of them above)
+                asm volatile("" : "+s"(pg[0][i]), "+s"(pg[1][i]), "+s"(pg[2][i]), "+s"(pg[3][i]), "+s"(ahead[0][i]),
+                             "+s"(ahead[1][i]));
 #pragma unroll
             for (int blk = 0; blk < 4; blk++) prepare_rows(blk_begin + blk, pg[blk], desc[blk]);
 #pragma unroll
             for (int blk = 0; blk < (kKPrefetch ? 4 : 3); blk++) load_direct(desc[blk].k, k_stage[blk]);
 #pragma unroll
             for (int blk = 0; blk < 2; blk++) load_direct(desc[blk].v, v_stage[blk]);
-            lookup_pages(blk_begin + 4, pg[0]);
-            if (kKPrefetch) {   // one block further ahead: block 4's descriptors now, block 5's page
-                prepare_rows(blk_begin + 4, pg[0], desc[0]);
-                lookup_pages(blk_begin + 5, pg[1]);
+            finish_all_q();
+#pragma unroll
+            for (int i = 0; i < kRowGroups; i++) {
+                pg[0][i] = ahead[0][i];
+                if (kKPrefetch) pg[1][i] = ahead[1][i];
             }
-            DSKV_WAIT_VMEM(0);
+            if (kKPrefetch) prepare_rows(blk_begin + 4, pg[0], desc[0]);   // one block further ahead: block 4's descriptors now
+            DSKV_WAIT_VMEM(2 * kRowGroups);   // everything but V(0) and V(1), which iterations 1 and 2 multiply
         } else {
             u32x4 first_k[2][kRowGroups], first_v[2][kRowGroups];
 #pragma unroll
             for (int blk = 0; blk < 2; blk++) load_rows(blk_begin + blk, first_k[blk], first_v[blk]);
+            finish_all_q();
 #pragma unroll
             for (int blk = 0; blk < 2; blk++) {
                 store_rows(k_stage[blk], first_k[blk]);
@@ -464,7 +526,13 @@ __device__ __forceinline__ void prefill_attn_body(
             load_rows(blk_begin + 3, odd.k, odd.v);
         }
     }
-    __syncthreads();
+    if (kRowsSharePage) {   // (a bare barrier: with the fences of __syncthreads V would be waited for, too)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    } else {
+        __syncthreads();
+    }
     if (w_end > 0) {
         read_k_operands(k_stage[0], kKPrefetch ? 1 : 0);
         scores(0, kKPrefetch ? 1 : 0);
@@ -582,7 +650,7 @@ __device__ __forceinline__ void prefill_attn_body(
     // chunk of 512 tokens in four parts (16 layers) 944 -> 920.
     __syncthreads();   // the stages have been read by everybody
     char *const rows_lds = lds_base + wave * kRowsOutBytes;
-    static_assert(kWaves * kRowsOutBytes <= kPrefillLdsBytes, "a stretch per wave");
+    static_assert(kWaves * kRowsOutBytes <= prefill_lds_bytes(kWaves), "a stretch per wave");
     // 256 bytes of every column from rows_lds to base + row * row_bytes + at, `row` being the lane's own
     // column's row there (negative: none); any lane may hold any column's bytes
     auto store_columns = [&](char *base, int row, int row_bytes, int at) {
@@ -591,7 +659,7 @@ __device__ __forceinline__ void prefill_attn_body(
 #pragma unroll
         for (int j = 0; j < 8; j++) {
             const int col = 4 * j + g, to = __shfl(row, col);
-            const u32x4 w = *reinterpret_cast<const u32x4 *>(rows_lds + col * kRowsOutPitch + c * 16);
+            const u32x4 w = *reinterpret_cast<const u32x4 *>(rows_lds + col * kRowPitch + c * 16);
             if (to < 0) continue;
             u32x4 *const dst = reinterpret_cast<u32x4 *>(base + (long)to * row_bytes + at + c * 16);
             if (kStreamOut) __builtin_nontemporal_store(w, dst);
@@ -604,7 +672,7 @@ __device__ __forceinline__ void prefill_attn_body(
         float l_other = l_run[ct];
         swap_halves32(l_run[ct], l_other);
         const float l = l_run[ct] + l_other;
-        char *const mine = rows_lds + r * kRowsOutPitch;
+        char *const mine = rows_lds + r * kRowPitch;
         if (partial) {   // (max, sum, unnormalised O) of the row into its slot, 64 dims at a time
             const int slot = (qrow[ct] - q0) * tile_parts + split, qh = kvh * group + c_head[ct];   // from first_slot
             const bool held = live[ct] && first_slot + (long)slot < max_slots;   // never beyond the workspace
@@ -649,7 +717,7 @@ __global__ __launch_bounds__(64 * kPrefillWaves, DSKV_PREFILL_MIN_WAVES) void pr
     int n_kv_heads, int page_shift, float scale_log2, int causal,
     float *__restrict__ part_o, float *__restrict__ part_ml, int max_slots, const float *__restrict__ rope)
 {
-    __shared__ __align__(16) char lds[kPrefillLdsBytes];
+    __shared__ __align__(16) char lds[prefill_lds_bytes(kPrefillWaves)];
     prefill_attn_body<DT, kRowsSharePage, kPrefillWaves, false>(
         lds, (int)blockIdx.x, out, q, qo_indptr, pages, kv_indices, kv_indptr, kv_last, tile_info,
         n_qo_heads, n_kv_heads, page_shift, scale_log2, causal, part_o, part_ml, max_slots, rope);
