@@ -53,9 +53,12 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // alone.  `wide`: eight waves per (row, head), for rows cut into dozens of parts.  Defined
 // beside the decode attention kernels, which write such partials.
 // row_map (may be null): request r's output row is row_map[r] instead of r.
+// some_in_many: some rows may be in more than eight parts (a decode batch of fewer requests than shares; what a
+// captured launch is known by decides it, not the number of items).
 int launch_partials_merge(void *out, const float *part_o, const float *part_ml,
                           const int32_t *row_parts, const int32_t *row_map, int max_slots, int rows,
-                          int n_qo_heads, int head_dim, int dtype, bool wide, hipStream_t stream);
+                          int n_qo_heads, int head_dim, int dtype, bool wide, hipStream_t stream,
+                          bool some_in_many = false);
 
 // The split-KV decode path for requests that are rows of a ragged batch (the one-row
 // requests of a prefill batch): request i has `len` kv tokens, its block table starts at

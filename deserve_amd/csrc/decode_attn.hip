@@ -939,7 +939,7 @@ static int decode_attn_impl(void *out, const void *q, const void *pages_layer,
         // many parts per request (long requests, small batch): eight waves share a merge
         const bool wide = n_items > kWideMergeParts * (int64_t)batch;
         return launch_partials_merge(out, part_o, part_ml, req_parts, row_map, (int)max_slots, batch,
-                                     n_qo_heads, head_dim, dtype, wide, s);
+                                     n_qo_heads, head_dim, dtype, wide, s, batch < n_workgroups);
     }
     return 0;
 }
@@ -958,20 +958,26 @@ int decode_rows_attn(void *out, const void *q, const void *pages_layer,
 
 int launch_partials_merge(void *out, const float *part_o, const float *part_ml,
                           const int32_t *row_parts, const int32_t *row_map, int max_slots, int rows,
-                          int n_qo_heads, int head_dim, int dtype, bool wide, hipStream_t s)
+                          int n_qo_heads, int head_dim, int dtype, bool wide, hipStream_t s, bool some_in_many)
 {
     // rows in a few parts, 16-bit output, head_dim 128: a workgroup per (row, eight heads) that
     // requests all parts at once - half the time of a wave per (row, head) on the 512 rows of a
     // chunk; 4.9 us on a decode batch's 64 requests in 317 parts is about what any launch that
     // reads what the launch before it wrote takes
     if (!wide && head_dim == kHeadDim && dtype != DSKV_F32) {
-        const dim3 grid((unsigned)rows, (unsigned)((n_qo_heads + kMergeHeads - 1) / kMergeHeads));
-        if (dtype == DSKV_BF16)
-            hipLaunchKernelGGL((merge_parts_kernel<DSKV_BF16>), grid, dim3(kMergeThreads), 0, s,
-                               (uint16_t *)out, part_o, part_ml, row_parts, row_map, max_slots, n_qo_heads);
-        else
-            hipLaunchKernelGGL((merge_parts_kernel<DSKV_F16>), grid, dim3(kMergeThreads), 0, s,
-                               (uint16_t *)out, part_o, part_ml, row_parts, row_map, max_slots, n_qo_heads);
+        const int heads = some_in_many ? kMergeHeadsMany : kMergeHeads;
+        const dim3 grid((unsigned)rows, (unsigned)((n_qo_heads + heads - 1) / heads));
+#define DSKV_LAUNCH_PARTS(DT, MANY)                                                                     \
+    hipLaunchKernelGGL((merge_parts_kernel<DT, MANY>), grid, dim3(kMergeThreads), 0, s, (uint16_t *)out, \
+                       part_o, part_ml, row_parts, row_map, max_slots, n_qo_heads)
+        if (dtype == DSKV_BF16) {
+            if (some_in_many) DSKV_LAUNCH_PARTS(DSKV_BF16, true);
+            else DSKV_LAUNCH_PARTS(DSKV_BF16, false);
+        } else {
+            if (some_in_many) DSKV_LAUNCH_PARTS(DSKV_F16, true);
+            else DSKV_LAUNCH_PARTS(DSKV_F16, false);
+        }
+#undef DSKV_LAUNCH_PARTS
         DSKV_LAUNCH_CHECK("merge_parts_kernel");
         return 0;
     }
