@@ -399,29 +399,24 @@ __device__ __forceinline__ void prefill_attn_body(
                 if (8 * (v >> 2) + (v & 3) >= seen) xs[buf][ct][v] = kNegBig;
         }
     };
-    // P of the block in xs[buf] under the running maximum, packed; returns whether a lane's sum is too large
-    // for that maximum (then P is to be taken again under a higher one), which infinities are, too.
-    auto probabilities = [&](int buf, float(&p_sum)[kColTiles]) {
-        bool over = false;
+    // P of k-step ks (the lane's 8 tokens of it) of the block in xs[buf] under the running maximum, packed, and
+    // its sum.  A sum too large for that maximum - infinities are, too - asks for P to be taken again under a higher one.
+    auto probabilities = [&](int buf, int ks, float(&p_sum)[kColTiles]) {
 #pragma unroll
         for (int ct = 0; ct < kColTiles; ct++) {
-            float p[16];
-            p_sum[ct] = 0.f;
+            float p[8];
 #pragma unroll
-            for (int v = 0; v < 16; v++) {
-                p[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(xs[buf][ct][v], scale_log2, -m_run[ct]));
-                p_sum[ct] += p[v];
+            for (int v = 0; v < 8; v++) {
+                p[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(xs[buf][ct][8 * ks + v], scale_log2, -m_run[ct]));
+                p_sum[ct] = ks == 0 && v == 0 ? p[v] : p_sum[ct] + p[v];
             }
-            over |= p_sum[ct] > kMostProbability;
-#pragma unroll
-            for (int ks = 0; ks < 2; ks++)
-                pb[buf][ct][ks] = u32x4{E::pack2(p[8 * ks], p[8 * ks + 1]), E::pack2(p[8 * ks + 2], p[8 * ks + 3]),
-                                        E::pack2(p[8 * ks + 4], p[8 * ks + 5]), E::pack2(p[8 * ks + 6], p[8 * ks + 7])};
+            pb[buf][ct][ks] = u32x4{E::pack2(p[0], p[1]), E::pack2(p[2], p[3]), E::pack2(p[4], p[5]), E::pack2(p[6], p[7])};
+            // keeps them in their half (they are only consumed by the next iteration)
+            asm volatile("" ::"v"(pb[buf][ct][ks]), "v"(p_sum[ct]));
         }
-        return over;
     };
     // Raises the running maximum to the block's in xs[buf] and brings what was computed under the old one
-    // (accumulators, row sum, the block before's P, still to be multiplied) to the new scale.
+    // (accumulators, row sum) to the new scale.
     auto raise_maximum = [&](int buf) {
 #pragma unroll
         for (int ct = 0; ct < kColTiles; ct++) {
@@ -439,14 +434,6 @@ __device__ __forceinline__ void prefill_attn_body(
             l_run[ct] *= alpha;
 #pragma unroll
             for (int dt = 0; dt < 4; dt++) acc[ct][dt] *= alpha;
-#pragma unroll
-            for (int ks = 0; ks < 2; ks++)
-#pragma unroll
-                for (int w = 0; w < 4; w++) {
-                    float lo, hi;
-                    E::unpack2(pb[buf ^ 1][ct][ks][w], lo, hi);
-                    pb[buf ^ 1][ct][ks][w] = E::pack2(lo * alpha, hi * alpha);
-                }
         }
     };
 
@@ -579,10 +566,12 @@ __device__ __forceinline__ void prefill_attn_body(
         }
         // The rest of the iteration is two straight-line halves, each an MFMA
         // strand with independent vector and LDS work in its shadow:
-        //   S(m+1) = K(m+1).Q^T     |  P(m) = exp2(S(m) * scale - max), packed; row sum;
-        //                           |  V(m-1) operands from LDS
-        //   O += P(m-1).V(m-1)      |  K(m+2) operands from LDS
-        // with, where needed, the raise of the maximum and the masking of S(m+1) between them.  A masked score
+        //   S(m+1) = K(m+1).Q^T     |  half of P(m) = exp2(S(m) * scale - max), packed; V(m-1) operands from LDS
+        //   O += P(m-1).V(m-1)      |  the other half; row sum; K(m+2) operands from LDS
+        // with, where needed, the masking of S(m+1) between them and the raise of the maximum behind them.  (The
+        // waves of a unit go through the halves together: with all of P(m) in the first, that one was bound by the
+        // exponentials and the other by the matrix pipeline.  Three short prompts 312 -> 307 us in 16 layers, a chunk of
+        // 512 942 -> 933, 16 chunks 11579 -> 11431.)  A masked score
         // is kNegBig and the maximum never drops below its start value, so masked
         // probabilities come out as exp2(-huge) = 0 without a select.
         const int cur = phase & 1, nxt = cur ^ 1;   // xs[cur] = S(m), xs[nxt] receives S(m+1)
@@ -606,18 +595,7 @@ __device__ __forceinline__ void prefill_attn_body(
             }
         scores(nxt, kKPrefetch ? (phase & 1) : 0);
         float p_sum[kColTiles];
-        const bool over = probabilities(cur, p_sum);
-        // keeps P(m) in this half (it is only consumed by the next iteration)
-#pragma unroll
-        for (int ct = 0; ct < kColTiles; ct++)
-            asm volatile("" ::"v"(pb[cur][ct][0]), "v"(pb[cur][ct][1]), "v"(p_sum[ct]));
-        if (__builtin_amdgcn_ballot_w64(over) != 0) {   // rare
-            raise_maximum(cur);
-            __builtin_amdgcn_sched_barrier(0);   // one after the other: side by side they spill
-            probabilities(cur, p_sum);
-        }
-#pragma unroll
-        for (int ct = 0; ct < kColTiles; ct++) l_run[ct] += p_sum[ct];
+        probabilities(cur, 0, p_sum);
         if ((m + 2) * kBlock > w_mask_from) mask_scores(m + 1, nxt);   // wave-uniform
 
 #pragma unroll
@@ -627,12 +605,21 @@ __device__ __forceinline__ void prefill_attn_body(
 #pragma unroll
                 for (int ct = 0; ct < kColTiles; ct++)
                     acc[ct][dt] = E::mfma_32x32(va[dt][ks], pb[nxt][ct][ks], acc[ct][dt]);   // P(m-1): the other buffer
-        if (kKPrefetch) {
-            read_k_operands(k_stage[(phase + 2) & 3], (phase + 1) & 1);   // K(m+2), published by this iteration's barrier
-            prepare_rows(m + 5, pg[(phase + 1) & 3], desc[(phase + 1) & 3]);
-        } else {
-            prepare_rows(m + 4, pg[phase], desc[phase]);   // for the loads of the next iterations
+        if (kKPrefetch) read_k_operands(k_stage[(phase + 2) & 3], (phase + 1) & 1);   // K(m+2), published by this iteration's barrier
+        probabilities(cur, 1, p_sum);
+        if (kKPrefetch) prepare_rows(m + 5, pg[(phase + 1) & 3], desc[(phase + 1) & 3]);
+        else prepare_rows(m + 4, pg[phase], desc[phase]);   // for the loads of the next iterations
+        bool over = false;
+#pragma unroll
+        for (int ct = 0; ct < kColTiles; ct++) over |= p_sum[ct] > kMostProbability;
+        if (__builtin_amdgcn_ballot_w64(over) != 0) {   // rare
+            raise_maximum(cur);
+            __builtin_amdgcn_sched_barrier(0);   // one after the other: side by side they spill
+            probabilities(cur, 0, p_sum);
+            probabilities(cur, 1, p_sum);
         }
+#pragma unroll
+        for (int ct = 0; ct < kColTiles; ct++) l_run[ct] += p_sum[ct];
     };
     for (int m = blk_begin; m <= n_blocks; m += 4) {
         iteration(m, 0, even);
