@@ -612,7 +612,7 @@ __device__ __forceinline__ void prefill_attn_body(
         bool over = false;
 #pragma unroll
         for (int ct = 0; ct < kColTiles; ct++) over |= p_sum[ct] > kMostProbability;
-        if (__builtin_amdgcn_ballot_w64(over) != 0) {   // rare
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(over) != 0, 0)) {   // rare
             raise_maximum(cur);
             __builtin_amdgcn_sched_barrier(0);   // one after the other: side by side they spill
             probabilities(cur, 0, p_sum);
