@@ -31,9 +31,9 @@
 #include "kv_tile.h"
 #include "decode_kernel.h"
 
-#include <vector>
-
 #include <algorithm>
+#include <atomic>
+#include <vector>
 
 #include "prefill_kernel.h"
 
@@ -203,7 +203,7 @@ __global__ __launch_bounds__(64 * kSharedWaves, 2) void mixed_attn_kernel(const 
         prefill_attn_body<DT, true, kPrefillWavesShared, true>(
             lds, wg - a.n_decode_wgs, a.out, a.q, a.qo_indptr, a.pages, a.kv_indices, a.kv_indptr, a.kv_last,
             a.tile_info, a.n_qo_heads, a.n_kv_heads, a.page_shift, a.scale_log2, a.causal,
-            a.tile_part_o, a.tile_part_ml, a.tile_max_slots, a.rope);
+            a.tile_part_o, a.tile_part_ml, a.tile_max_slots, a.rope, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
     }
 }
 
@@ -589,7 +589,8 @@ static int prefill_attn_impl(void *out, const void *q, const int32_t *qo_indptr,
                              void *workspace, int64_t workspace_bytes, int32_t batch, int32_t nnz,
                              int32_t n_qo_heads, int32_t n_kv_heads, int32_t head_dim,
                              int32_t page_size, float sm_scale, int32_t causal, int32_t dtype,
-                             void *stream, bool some_rows_elsewhere, const float *rope_table = nullptr)
+                             void *stream, bool some_rows_elsewhere, const float *rope_table = nullptr,
+                             const AppendRows &append = AppendRows{})
 {
     DSKV_REQUIRE(batch >= 0 && nnz >= 0 && n_tiles >= 0, "prefill_attn: negative sizes");
     if (batch == 0 || nnz == 0) return 0;
@@ -634,18 +635,19 @@ static int prefill_attn_impl(void *out, const void *q, const int32_t *qo_indptr,
         dim3 grid((unsigned)n_tiles * (unsigned)n_kv_heads);
         dim3 block(64 * kPrefillWaves);
         const int shift = ilog2(page_size);
-#define DSKV_LAUNCH_PREFILL(DT, SHARE)                                                          \
-    hipLaunchKernelGGL((prefill_attn_mfma_kernel<DT, SHARE>), grid, block, 0, s, (uint16_t *)out, \
-                       (const uint16_t *)q, qo_indptr, (const char *)pages_layer,               \
-                       kv_page_indices, kv_page_indptr, kv_last_page_len, plan_dev,             \
-                       n_qo_heads, n_kv_heads, shift, scale_log2, causal, part_o, part_ml,     \
-                       (int)max_slots, rope_table)
+        const PrefillArgs args = {append, (uint16_t *)out, (const uint16_t *)q, qo_indptr, (const char *)pages_layer,
+                                  kv_page_indices, kv_page_indptr, kv_last_page_len, plan_dev, n_qo_heads, n_kv_heads,
+                                  shift, scale_log2, causal, part_o, part_ml, (int)max_slots, rope_table};
+#define DSKV_LAUNCH_PREFILL(DT, SHARE, APPENDS) \
+    hipLaunchKernelGGL((prefill_attn_mfma_kernel<DT, SHARE, APPENDS>), grid, block, 0, s, args)
         if (dtype == DSKV_BF16) {
-            if (page_size >= 4) DSKV_LAUNCH_PREFILL(DSKV_BF16, true);
-            else DSKV_LAUNCH_PREFILL(DSKV_BF16, false);
+            if (append.k) DSKV_LAUNCH_PREFILL(DSKV_BF16, true, true);
+            else if (page_size >= 4) DSKV_LAUNCH_PREFILL(DSKV_BF16, true, false);
+            else DSKV_LAUNCH_PREFILL(DSKV_BF16, false, false);
         } else {
-            if (page_size >= 4) DSKV_LAUNCH_PREFILL(DSKV_F16, true);
-            else DSKV_LAUNCH_PREFILL(DSKV_F16, false);
+            if (append.k) DSKV_LAUNCH_PREFILL(DSKV_F16, true, true);
+            else if (page_size >= 4) DSKV_LAUNCH_PREFILL(DSKV_F16, true, false);
+            else DSKV_LAUNCH_PREFILL(DSKV_F16, false, false);
         }
 #undef DSKV_LAUNCH_PREFILL
         DSKV_LAUNCH_CHECK("prefill_attn_mfma_kernel");
@@ -808,7 +810,8 @@ static int mixed_attn_impl(void *out, const void *q, const int32_t *qo_indptr, c
                            const dskv_mixed_plan_t *info, void *workspace, int64_t workspace_bytes,
                            int32_t batch, int32_t nnz, int32_t n_qo_heads, int32_t n_kv_heads,
                            int32_t head_dim, int32_t page_size, float sm_scale, int32_t causal,
-                           int32_t dtype, const float *rope_table, void *stream)
+                           int32_t dtype, const float *rope_table, void *stream,
+                           const AppendRows &append = AppendRows{})
 {
     DSKV_REQUIRE(info, "mixed_attn: null plan info");
     DSKV_REQUIRE(info->n_decode_rows >= 0 && info->n_tile_rows >= 0 && info->n_tiles >= 0 &&
@@ -824,7 +827,7 @@ static int mixed_attn_impl(void *out, const void *q, const int32_t *qo_indptr, c
         return prefill_attn_impl(out, q, qo_indptr, pages_layer, kv_page_indices, kv_page_indptr,
                                  kv_last_page_len, plan_dev, info->n_tiles, info->n_splits, workspace,
                                  workspace_bytes, batch, nnz, n_qo_heads, n_kv_heads, head_dim,
-                                 page_size, sm_scale, causal, dtype, stream, false, rope_table);
+                                 page_size, sm_scale, causal, dtype, stream, false, rope_table, append);
     DSKV_REQUIRE(plan_dev, "mixed_attn: missing plan");
     DSKV_REQUIRE(info->n_decode_rows + info->n_tile_rows == nnz && info->n_decode_rows <= batch,
                  "mixed_attn: the plan covers %d + %d rows, the batch has %d", info->n_decode_rows,
@@ -881,38 +884,100 @@ extern "C" int dskv_mixed_step_supported(int32_t n_qo_heads, int32_t n_kv_heads,
            prefill_mfma_path(dtype, head_dim, n_qo_heads, n_kv_heads, sm_scale * 1.4426950408889634f);
 }
 
-extern "C" int dskv_mixed_step(const dskv_mixed_step_t *step, void *out, const void *q, const void *k_new,
-                               const void *v_new, void *pages_layer, void *stream)
+namespace dskv {
+
+// Whether a step's attention launch appends the step's rows itself: tiles only (decode workgroups beside
+// them, or a decode pass in front, would need theirs before), loaded straight into LDS, few enough
+// tokens for the first tiles' workgroups.  Rows have to be whole cache lines: see append_rows.h.
+static bool tiles_append(const dskv_mixed_step_t &s, const void *k, const void *v, const void *pages_layer, AppendRows &a)
+{
+    if (s.page_size < 4 || s.info->n_decode_rows > 0 || s.info->n_tiles <= 0 || s.batch > kAppendMaxBatch ||
+        s.n_kv_heads > kAppendFlags || ((uintptr_t)pages_layer % 256) || (((uintptr_t)k | (uintptr_t)v) % 16))
+        return false;
+    a.n_tiles = std::min(s.info->n_tiles, kAppendFlags / s.n_kv_heads);
+    a.tokens = (s.nnz + a.n_tiles - 1) / a.n_tiles;
+    return a.tokens <= kAppendMaxTokens;
+}
+
+static int mixed_step(const dskv_mixed_step_t &s, void *out, const void *q, const void *k_new, const void *v_new,
+                      void *pages_layer, uint32_t *flags, int32_t polls, void *stream)
+{
+    AppendRows append{};
+    if (s.batch > 0 && s.nnz > 0) {
+        DSKV_REQUIRE(pages_layer && k_new && v_new && s.qo_indptr && s.kv_page_indices && s.kv_page_indptr &&
+                         s.kv_last_page_len, "append: null pointer argument");
+        DSKV_REQUIRE(s.num_pages > 0, "append: num_pages must be positive, got %d", s.num_pages);
+        if (flags && tiles_append(s, k_new, v_new, pages_layer, append)) {
+            static std::atomic<uint32_t> launches{0};
+            while (!(append.launch = launches.fetch_add(1, std::memory_order_relaxed) + 1)) {}   // 0: a fresh buffer's
+            append.k = (const uint16_t *)k_new;
+            append.v = (const uint16_t *)v_new;
+            append.flags = flags;
+            append.nnz = s.nnz;
+            append.batch = s.batch;
+            append.num_pages = s.num_pages;
+            append.polls = polls;
+        }
+    }
+    if (!append.k) {
+        const int rc = launch_append(pages_layer, s.num_pages, k_new, v_new, s.qo_indptr, s.kv_page_indices,
+                                     s.kv_page_indptr, s.kv_last_page_len, s.batch, s.nnz, s.page_size, s.n_kv_heads,
+                                     s.head_dim, 2, s.rope_table, s.dtype, (hipStream_t)stream);
+        if (rc) return rc;
+    }
+    return mixed_attn_impl(out, q, s.qo_indptr, pages_layer, s.kv_page_indices, s.kv_page_indptr, s.kv_last_page_len,
+                           s.plan_dev, s.info, s.workspace, s.workspace_bytes, s.batch, s.nnz, s.n_qo_heads,
+                           s.n_kv_heads, s.head_dim, s.page_size, s.sm_scale, s.causal, s.dtype, s.rope_table, stream,
+                           append);
+}
+
+}  // namespace dskv
+
+extern "C" int64_t dskv_append_flags(void) { return dskv::kAppendFlags; }
+
+extern "C" int dskv_mixed_layers_flagged(const dskv_mixed_step_t *step, uint32_t *append_flags, int64_t n_append_flags,
+                                         int32_t polls, int32_t n_layers, void *out, const void *q, const void *k_new,
+                                         const void *v_new, void *pages, int64_t pages_layer_bytes, void *stream)
 {
     using namespace dskv;
-    DSKV_REQUIRE(step, "mixed_step: null step");
+    DSKV_REQUIRE(step && n_layers >= 0 && step->nnz >= 0 && n_append_flags >= 0, "mixed_layers: bad arguments");
+    if (n_layers == 0) return 0;
     const dskv_mixed_step_t &s = *step;
     DSKV_REQUIRE(dskv_mixed_step_supported(s.n_qo_heads, s.n_kv_heads, s.head_dim, s.page_size, s.sm_scale, s.dtype),
                  "mixed_step: shape, scale or type outside the 16-bit kernels (see dskv_mixed_step_supported)");
     DSKV_REQUIRE(s.info, "mixed_step: null plan info");
     DSKV_REQUIRE((uintptr_t)s.rope_table % 16 == 0, "mixed_step: the table must be 16-byte aligned");
-    int rc = launch_append(pages_layer, s.num_pages, k_new, v_new, s.qo_indptr, s.kv_page_indices, s.kv_page_indptr,
-                           s.kv_last_page_len, s.batch, s.nnz, s.page_size, s.n_kv_heads, s.head_dim, 2,
-                           s.rope_table, s.dtype, (hipStream_t)stream);
-    if (rc) return rc;
-    return mixed_attn_impl(out, q, s.qo_indptr, pages_layer, s.kv_page_indices, s.kv_page_indptr, s.kv_last_page_len,
-                           s.plan_dev, s.info, s.workspace, s.workspace_bytes, s.batch, s.nnz, s.n_qo_heads,
-                           s.n_kv_heads, s.head_dim, s.page_size, s.sm_scale, s.causal, s.dtype, s.rope_table, stream);
+    DSKV_REQUIRE(polls >= 0 && (uintptr_t)append_flags % 4 == 0, "mixed_layers: bad flags");
+    // A captured launch would raise its flags with the same number in every replay, and find them raised
+    if (append_flags) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (n_append_flags < kAppendFlags || hipStreamIsCapturing((hipStream_t)stream, &capture) != hipSuccess ||
+            capture != hipStreamCaptureStatusNone) {
+            (void)hipGetLastError();
+            append_flags = nullptr;
+        }
+    }
+    const int64_t q_bytes = (int64_t)s.nnz * s.n_qo_heads * s.head_dim * 2;
+    const int64_t kv_bytes = (int64_t)s.nnz * s.n_kv_heads * s.head_dim * 2;
+    auto at = [](const void *p, int64_t bytes) { return p ? (const char *)p + bytes : nullptr; };
+    for (int64_t l = 0; l < n_layers; l++) {
+        const int rc = mixed_step(s, (void *)at(out, l * q_bytes), at(q, l * q_bytes), at(k_new, l * kv_bytes),
+                                  at(v_new, l * kv_bytes), (void *)at(pages, l * pages_layer_bytes), append_flags,
+                                  polls > 0 ? polls : kAppendPolls, stream);
+        if (rc) return rc;
+    }
+    return 0;
 }
 
 extern "C" int dskv_mixed_layers(const dskv_mixed_step_t *step, int32_t n_layers, void *out, const void *q,
                                  const void *k_new, const void *v_new, void *pages, int64_t pages_layer_bytes,
                                  void *stream)
 {
-    using namespace dskv;
-    DSKV_REQUIRE(step && n_layers >= 0 && step->nnz >= 0, "mixed_layers: bad arguments");
-    const int64_t q_bytes = (int64_t)step->nnz * step->n_qo_heads * step->head_dim * 2;
-    const int64_t kv_bytes = (int64_t)step->nnz * step->n_kv_heads * step->head_dim * 2;
-    auto at = [](const void *p, int64_t bytes) { return p ? (const char *)p + bytes : nullptr; };
-    for (int64_t l = 0; l < n_layers; l++) {
-        const int rc = dskv_mixed_step(step, (void *)at(out, l * q_bytes), at(q, l * q_bytes), at(k_new, l * kv_bytes),
-                                       at(v_new, l * kv_bytes), (void *)at(pages, l * pages_layer_bytes), stream);
-        if (rc) return rc;
-    }
-    return 0;
+    return dskv_mixed_layers_flagged(step, nullptr, 0, 0, n_layers, out, q, k_new, v_new, pages, pages_layer_bytes, stream);
+}
+
+extern "C" int dskv_mixed_step(const dskv_mixed_step_t *step, void *out, const void *q, const void *k_new,
+                               const void *v_new, void *pages_layer, void *stream)
+{
+    return dskv_mixed_layers(step, 1, out, q, k_new, v_new, pages_layer, 0, stream);
 }

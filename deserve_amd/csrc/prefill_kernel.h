@@ -4,6 +4,7 @@
 // workgroups share their compute units with decode workgroups.
 #pragma once
 
+#include "append_rows.h"
 #include "kv_tile.h"
 #include "rope_math.h"
 
@@ -65,14 +66,33 @@ struct LdsStages {
 //     pushed the chunk's K/V out of it: 75 decode rows and the chunk 2638 -> 2471 us a step (16
 //     layers), 70B-shaped 1527 -> 1410.  A launch of tiles only loses (a chunk of 512 in four parts 938
 //     -> 955): its merge pass then reads the partials from farther away.
-template <int DT, bool kRowsSharePage, int kWaves, bool kStreamOut>
-__device__ __forceinline__ void prefill_attn_body(
+//   kAppends: the launch appends the step's rows (append_rows.h); false is returned, and nothing stored, if others'
+//     did not come in time: append_for_tile, then call again with rows_there.
+struct PrefillArgs {
+    AppendRows append;   // at the front: read through the kernel's argument segment
+    uint16_t *out;
+    const uint16_t *q;
+    const int32_t *qo_indptr;
+    const char *pages;
+    const int32_t *kv_indices, *kv_indptr, *kv_last, *tile_info;
+    int n_qo_heads, n_kv_heads, page_shift;
+    float scale_log2;
+    int causal;
+    float *part_o, *part_ml;
+    int max_slots;
+    const float *rope;
+};
+typedef const __attribute__((address_space(4))) PrefillArgs *const_prefill_ptr;
+
+template <int DT, bool kRowsSharePage, int kWaves, bool kStreamOut, bool kAppends = false>
+__device__ __forceinline__ bool prefill_attn_body(
     char *lds_base, int wg, uint16_t *__restrict__ out, const uint16_t *__restrict__ q,
     const int32_t *__restrict__ qo_indptr, const char *__restrict__ pages,
     const int32_t *__restrict__ kv_indices, const int32_t *__restrict__ kv_indptr,
     const int32_t *__restrict__ kv_last, const int32_t *__restrict__ tile_info, int n_qo_heads,
     int n_kv_heads, int page_shift, float scale_log2, int causal,
-    float *__restrict__ part_o, float *__restrict__ part_ml, int max_slots, const float *__restrict__ rope)
+    float *__restrict__ part_o, float *__restrict__ part_ml, int max_slots, const float *__restrict__ rope,
+    int wave, bool rows_there = true)
 {
     typedef Elt<DT> E;
     constexpr int kRowsPerWave = kBlock / kWaves;   // rows of a block one wave loads
@@ -80,8 +100,7 @@ __device__ __forceinline__ void prefill_attn_body(
     static_assert(kRowsPerWave % 4 == 0 && kRowGroups >= 1, "a wave loads whole groups of 4 rows");
     const LdsStages k_stage{lds_base}, v_stage{lds_base + 4 * kStageBytes};
 
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
+    const int lane = kAppends ? lane_id() : threadIdx.x & 63;
     const int g = lane >> 4;     // row group / chunk roles of the K/V row movement
     const int c = lane & 15;
     const int h = lane >> 5;     // MFMA roles
@@ -240,6 +259,29 @@ __device__ __forceinline__ void prefill_attn_body(
         ml[0] = m;
         ml[1] = l;
     };
+    // The workgroup's share of the rows that the launch appends (rows_there: it has been written before).
+    AppendShare<DT, kWaves> share;
+    const const_append_ptr append = (const_append_ptr)__builtin_amdgcn_kernarg_segment_ptr();
+    auto append_request_share = [&]() {
+        if (kAppends) share.request(append, tile, kvh, n_kv_heads, wave, qo_indptr, kv_indptr, kv_last);
+    };
+    auto append_look_up = [&]() {
+        if (kAppends) share.look_up(append, wave, kv_indices, page_shift, rope);
+    };
+    auto append_store = [&]() {
+        if (kAppends) share.store(append, pages, page_shift, row_bytes, kvh, rope != nullptr);
+    };
+    auto raise_flag = [&]() {   // when all waves' stores have been acknowledged
+        const_append_ptr a = (const_append_ptr)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(a));
+        if (wave == 0 && tile < a->n_tiles && lane_id() == 0)
+            __hip_atomic_store(a->flags + (long)tile * n_kv_heads + kvh, a->launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    auto raise_when_stored = [&]() {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        raise_flag();
+    };
     // No kv token of this part visible to any row of the tile: the output rows are zero
     // (or the part is empty).  Uniform over the workgroup, and before the first barrier.
     if (t_end <= t_first) {
@@ -259,8 +301,28 @@ __device__ __forceinline__ void prefill_attn_body(
 #pragma unroll
             for (int i = 0; i < 16; i++) *reinterpret_cast<u32x2 *>(o + 8 * i) = u32x2{0, 0};
         }
-        return;
+        if (kAppends && !rows_there) {   // others may wait for its share
+            append_request_share();
+            append_look_up();
+            append_store();
+            raise_when_stored();
+        }
+        return true;
     }
+
+    // Blocks that end behind new_from hold rows that this launch appends: they are requested when the
+    // flags of the workgroups that append them have been seen.
+    int new_from = kAppends && !rows_there && t_end > kv_len - n_b ? kv_len - n_b : 0x7fffffff;
+    bool in_time = true;
+    int *const late = reinterpret_cast<int *>(lds_base + prefill_lds_bytes(kWaves));
+    auto await_new_rows = [&]() {
+        const_append_ptr a = (const_append_ptr)__builtin_amdgcn_kernarg_segment_ptr();
+        const int tokens = a->tokens;
+        in_time = rows_are_there(a, (q_begin + max(t_first - new_from, 0)) / tokens,
+                                 (q_begin + min(t_end - new_from, n_b) - 1) / tokens, kvh, n_kv_heads);
+        new_from = 0x7fffffff;
+    };
+    if (kAppends && wave == 0) *late = 0;
 
     // This wave's share of the K (or V) rows of block blk: rows wave*kRowsPerWave .. +kRowsPerWave,
     // in groups of four (one region each).  Rows at or past t_end arrive as zeros (their
@@ -462,9 +524,11 @@ __device__ __forceinline__ void prefill_attn_body(
         u32x4 k[kRowGroups], v[kRowGroups];   // rows on their way to LDS (register path)
     };
     RowSet even, odd;
+    bool raise_later = false;
     {
         // the walk starts at block blk_begin, a multiple of four: block j still lives in stage j % 4
         QRows rows;
+        if (kAppends && !rows_there) append_request_share();
         load_q(0, rows);
         auto finish_all_q = [&]() {
             finish_q(0, rows);
@@ -487,11 +551,23 @@ __device__ __forceinline__ void prefill_attn_body(
                              "+s"(ahead[1][i]));
 #pragma unroll
             for (int blk = 0; blk < 4; blk++) prepare_rows(blk_begin + blk, pg[blk], desc[blk]);
+            // a walk that requests new rows within its first four iterations waits for them first; the others append
+            // beside their first loads
+            const bool appends = kAppends && !rows_there, new_first = kAppends && (blk_begin + 8) * kBlock > new_from;
+            if (new_first) {
+                append_look_up();
+                append_store();
+                raise_when_stored();
+                await_new_rows();
+            }
 #pragma unroll
             for (int blk = 0; blk < (kKPrefetch ? 4 : 3); blk++) load_direct(desc[blk].k, k_stage[blk]);
 #pragma unroll
             for (int blk = 0; blk < 2; blk++) load_direct(desc[blk].v, v_stage[blk]);
+            raise_later = appends && !new_first;
+            if (raise_later) append_look_up();
             finish_all_q();
+            if (raise_later) append_store();
 #pragma unroll
             for (int i = 0; i < kRowGroups; i++) {
                 pg[0][i] = ahead[0][i];
@@ -621,11 +697,28 @@ __device__ __forceinline__ void prefill_attn_body(
 #pragma unroll
         for (int ct = 0; ct < kColTiles; ct++) l_run[ct] += p_sum[ct];
     };
-    for (int m = blk_begin; m <= n_blocks; m += 4) {
-        iteration(m, 0, even);
-        iteration(m + 1, 1, odd);
-        iteration(m + 2, 2, even);
-        iteration(m + 3, 3, odd);
+    // The four iterations from m on request blocks up to m + 7.  The walk is cut where they would first meet a
+    // new row, so that the loop itself has nothing to look at.
+    for (int m = blk_begin;;) {
+        int end = n_blocks + 1;
+        const bool raise_now = kAppends && raise_later, wait_now = kAppends && !raise_now && new_from < 0x7fffffff;
+        // The share's stores are older than the loads that three waits of `iteration` leave on their way:
+        // behind the barriers of the first four iterations they have been acknowledged for all waves.
+        if (raise_now) end = min(end, m + 4);
+        if (wait_now) end = min(end, m + max(new_from / kBlock - 8 - m + 4, 0) / 4 * 4);
+        for (; m < end; m += 4) {
+            iteration(m, 0, even);
+            iteration(m + 1, 1, odd);
+            iteration(m + 2, 2, even);
+            iteration(m + 3, 3, odd);
+        }
+        if (!kAppends) break;
+        if (raise_now) {
+            raise_flag();
+            raise_later = false;
+        }
+        if (m > n_blocks) break;
+        if (wait_now) await_new_rows();
     }
     if (kRowsSharePage) DSKV_WAIT_VMEM(0);   // nothing of this wave may still be on its way into LDS
 #undef DSKV_WAIT_VMEM
@@ -635,7 +728,9 @@ __device__ __forceinline__ void prefill_attn_body(
     // 16 bytes (of the 16-bit output) or 32 (of a partial) of each.  Laid out by column, 16 lanes
     // store 256 consecutive bytes: the launch of three short prompts 17.5 -> 15.3 us, the step of a
     // chunk of 512 tokens in four parts (16 layers) 944 -> 920.
+    if (kAppends && !in_time) *late = 1;
     __syncthreads();   // the stages have been read by everybody
+    if (kAppends && __builtin_amdgcn_readfirstlane(*late)) return false;
     char *const rows_lds = lds_base + wave * kRowsOutBytes;
     static_assert(kWaves * kRowsOutBytes <= prefill_lds_bytes(kWaves), "a stretch per wave");
     // 256 bytes of every column from rows_lds to base + row * row_bytes + at, `row` being the lane's own
@@ -690,24 +785,49 @@ __device__ __forceinline__ void prefill_attn_body(
         store_columns(reinterpret_cast<char *>(out + ((long)(q_begin + q0) * n_qo_heads + (long)kvh * group) * kHeadDim),
                       live[ct] ? (qrow[ct] - q0) * n_qo_heads + c_head[ct] : -1, kHeadDim * 2, 0);
     }
+    return true;
+}
+
+// A tile whose new rows did not come in time: its workgroup appends its request's rows of its kv head itself.
+template <int DT, int kWaves>
+__device__ __forceinline__ void append_for_tile(const_prefill_ptr a, int wg, int wave)
+{
+    asm volatile("" : "+s"(a));
+    const int n_kv_heads = a->n_kv_heads, b = a->tile_info[(long)(wg / n_kv_heads) * kTileWords];
+    const int q_begin = a->qo_indptr[b], n_b = a->qo_indptr[b + 1] - q_begin;
+    const int page_begin = a->kv_indptr[b];   // it has pages: the tile has walked them
+    const long kv_len = ((long)(a->kv_indptr[b + 1] - page_begin - 1) << a->page_shift) + a->kv_last[b];
+    append_request<DT, kWaves>(a->append.k, a->append.v, a->append.num_pages, q_begin, n_b, kv_len, a->pages,
+                               a->kv_indices + page_begin, wg % n_kv_heads, n_kv_heads, a->page_shift, a->rope, wave);
 }
 
 #ifndef DSKV_PREFILL_MIN_WAVES
 #define DSKV_PREFILL_MIN_WAVES 1
 #endif
-template <int DT, bool kRowsSharePage>
-__global__ __launch_bounds__(64 * kPrefillWaves, DSKV_PREFILL_MIN_WAVES) void prefill_attn_mfma_kernel(
-    uint16_t *__restrict__ out, const uint16_t *__restrict__ q,
-    const int32_t *__restrict__ qo_indptr, const char *__restrict__ pages,
-    const int32_t *__restrict__ kv_indices, const int32_t *__restrict__ kv_indptr,
-    const int32_t *__restrict__ kv_last, const int32_t *__restrict__ tile_info, int n_qo_heads,
-    int n_kv_heads, int page_shift, float scale_log2, int causal,
-    float *__restrict__ part_o, float *__restrict__ part_ml, int max_slots, const float *__restrict__ rope)
+template <int DT, bool kRowsSharePage, bool kAppends>
+__global__ __launch_bounds__(64 * kPrefillWaves, DSKV_PREFILL_MIN_WAVES) void prefill_attn_mfma_kernel(const PrefillArgs a)
 {
-    __shared__ __align__(16) char lds[prefill_lds_bytes(kPrefillWaves)];
-    prefill_attn_body<DT, kRowsSharePage, kPrefillWaves, false>(
-        lds, (int)blockIdx.x, out, q, qo_indptr, pages, kv_indices, kv_indptr, kv_last, tile_info,
-        n_qo_heads, n_kv_heads, page_shift, scale_log2, causal, part_o, part_ml, max_slots, rope);
+    static_assert(kRowsSharePage || !kAppends, "the register path's rows are in their pages before");
+    __shared__ __align__(16) char lds[prefill_lds_bytes(kPrefillWaves) + (kAppends ? 16 : 0)];
+    int wg = blockIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (!kAppends) {
+        prefill_attn_body<DT, kRowsSharePage, kPrefillWaves, false>(
+            lds, wg, a.out, a.q, a.qo_indptr, a.pages, a.kv_indices, a.kv_indptr, a.kv_last, a.tile_info, a.n_qo_heads,
+            a.n_kv_heads, a.page_shift, a.scale_log2, a.causal, a.part_o, a.part_ml, a.max_slots, a.rope, wave);
+        return;
+    }
+    // Every walk reads the arguments anew: nothing is kept in registers for a second one, which hardly ever comes.
+    for (bool rows_there = false;; rows_there = true) {
+        const_prefill_ptr p = (const_prefill_ptr)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(p), "+s"(wg));
+        if (prefill_attn_body<DT, kRowsSharePage, kPrefillWaves, false, kAppends>(
+                lds, wg, p->out, p->q, p->qo_indptr, p->pages, p->kv_indices, p->kv_indptr, p->kv_last, p->tile_info,
+                p->n_qo_heads, p->n_kv_heads, p->page_shift, p->scale_log2, p->causal, p->part_o, p->part_ml, p->max_slots,
+                p->rope, wave, rows_there))
+            return;
+        append_for_tile<DT, kPrefillWaves>(p, wg, wave);
+    }
 }
 
 }  // namespace dskv

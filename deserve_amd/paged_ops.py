@@ -121,6 +121,7 @@ class _PagedWrapper:
         self._planned = False
         self._rope_table, self._rope_key = None, None
         self._counters = None
+        self._flags = None
         self._max_page_id = -1
         self._empty_requests = []
 
@@ -461,12 +462,20 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
 
     def _bind_step(self) -> None:
         """What all layers of the planned step share, for dskv_mixed_step."""
+        device = self._tiles.device
+        if self._flags is None and not (device.type == "cuda" and torch.cuda.is_current_stream_capturing()):
+            # the appending workgroups' flags, kept for good: every launch has a number of its own
+            self._flags = torch.zeros((_lib.lib().dskv_append_flags(),), dtype=torch.int32, device=device)
         self._step = _lib.MixedStep(
             self._qo_indptr.data_ptr(), self._indices.data_ptr(), self._indptr.data_ptr(), self._last.data_ptr(),
             self._tiles.data_ptr(), ctypes.pointer(self._info), self._workspace.data_ptr(),
             self._workspace.numel() * self._workspace.element_size(), None, 0, self._batch, self._nnz, self._hq,
             self._hkv, self._d, self._p)
         self._planned = True
+
+    def _flag_words(self):
+        """Address and number of the appending workgroups' flags."""
+        return (None, 0) if self._flags is None else (self._flags.data_ptr(), self._flags.numel())
 
     def _check_and_bound(self, h_qo: torch.Tensor, h_kv: torch.Tensor, h_last: torch.Tensor,
                          indices: torch.Tensor, indices_host: Optional[torch.Tensor]):
@@ -560,9 +569,10 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
         step.rope_table = None if rope_table is None else rope_table.data_ptr()
         step.num_pages, step.causal = pages.shape[1], 1
         step.dtype, step.sm_scale = _lib.dtype_code(dtype), 1.0 / math.sqrt(self._d)
-        rc = _lib.lib().dskv_mixed_layers(ctypes.byref(step), n, out.data_ptr(), q.data_ptr(), k_append.data_ptr(),
-                                          v_append.data_ptr(), pages.data_ptr(),
-                                          pages.stride(0) * pages.element_size(), _lib.current_stream())
+        rc = _lib.lib().dskv_mixed_layers_flagged(
+            ctypes.byref(step), *self._flag_words(), 0, n, out.data_ptr(), q.data_ptr(),
+            k_append.data_ptr(), v_append.data_ptr(), pages.data_ptr(), pages.stride(0) * pages.element_size(),
+            _lib.current_stream())
         _lib.check(rc, "prefill forward")
         return True
 
@@ -603,8 +613,9 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
             step.rope_table = None if rope_table is None else rope_table.data_ptr()
             step.num_pages, step.causal = paged_kv_data.shape[0], int(causal)
             step.dtype, step.sm_scale = _lib.dtype_code(dtype), scale
-            rc = _lib.lib().dskv_mixed_step(ctypes.byref(step), out.data_ptr(), q.data_ptr(), k_append.data_ptr(),
-                                            v_append.data_ptr(), paged_kv_data.data_ptr(), _lib.current_stream())
+            rc = _lib.lib().dskv_mixed_layers_flagged(
+                ctypes.byref(step), *self._flag_words(), 0, 1, out.data_ptr(), q.data_ptr(),
+                k_append.data_ptr(), v_append.data_ptr(), paged_kv_data.data_ptr(), 0, _lib.current_stream())
             _lib.check(rc, "prefill forward")
             return out
         rc = _lib.lib().dskv_mixed_attn(

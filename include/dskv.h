@@ -389,6 +389,20 @@ int dskv_mixed_step(const dskv_mixed_step_t *step, void *out, const void *q, con
 /* dskv_mixed_step for n_layers layers, laid out as dskv_decode_layers takes them. */
 int dskv_mixed_layers(const dskv_mixed_step_t *step, int32_t n_layers, void *out, const void *q, const void *k_new,
                       const void *v_new, void *pages, int64_t pages_layer_bytes, void *stream);
+/*
+ * The same with dskv_append_flags() words (device, zero before the first call that is given them), which let the
+ * attention launch append the step's rows itself, without a launch in front of it: a plan of tiles only, at most
+ * 32 new tokens for each of its first entries, fewer than 64 requests, pages of at least 4 tokens, pages and
+ * layers of them at multiples of 256 bytes, a stream that is not being captured; elsewhere, and with
+ * append_flags null or fewer words, it is dskv_mixed_layers.  Pages and output have the same bits either way.
+ * polls: how often a query tile looks for rows that other workgroups append before it appends them itself (0:
+ * the library's number).  Calls on several streams may share the words: their launches then append
+ * some rows twice.
+ */
+int64_t dskv_append_flags(void);
+int dskv_mixed_layers_flagged(const dskv_mixed_step_t *step, uint32_t *append_flags, int64_t n_append_flags,
+                              int32_t polls, int32_t n_layers, void *out, const void *q, const void *k_new,
+                              const void *v_new, void *pages, int64_t pages_layer_bytes, void *stream);
 
 /*
  * Rotary embedding, adjacent-pair convention.  Replaces the call site

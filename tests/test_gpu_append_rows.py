@@ -1,0 +1,104 @@
+"""The prefill launch whose tiles append the step's rows themselves, against the same step with the append as a
+launch of its own: the same bits in pages and result.  Edges: the first new row at the ends of 32-token
+blocks and of the four blocks between two waits, no prior context, parts that end before the new rows or
+hold nothing else, one and two rounds of tokens per wave, empty shares, 63 requests, groups and head counts that
+leave waves idle, pages of 4 tokens; and what keeps the launch in front: pages of 2 tokens, too many tokens, 64
+requests, decode rows beside, a pool that is not at a multiple of 256 bytes, a captured stream.  With one
+look at the flags only, tiles append for themselves."""
+import ctypes
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from deserve_amd import _lib
+from kvutil import make_scenario, to_torch
+
+pytestmark = pytest.mark.gpu
+
+AUTO, SHARED = _lib.ROUTE_AUTO, _lib.ROUTE_SHARED_LAUNCH
+CASES = {   # kv_lens, qo_lens, page, Hq, Hkv, dtype, route, whether the tiles append
+    "block_edges": ([31 + 5, 32 + 33, 33 + 1, 95 + 70, 96 + 2, 128 + 31, 129 + 3], [5, 33, 1, 70, 2, 31, 3], 16, 32, 8, "bf16", AUTO, True),
+    "prompts_page4": ([17, 203, 1], [17, 203, 1], 4, 16, 4, "f16", AUTO, False),
+    "short_prompts_page4": ([17, 3, 1, 30], [17, 3, 1, 30], 4, 32, 8, "f16", AUTO, True),
+    "chunk": ([4096 + 512], [512], 16, 32, 8, "bf16", AUTO, True),
+    "two_rounds": ([1500 + 901], [901], 8, 32, 8, "bf16", AUTO, True),
+    "parts": ([1700, 2300], [129, 40], 16, 32, 8, "bf16", AUTO, True),
+    "part_of_new_rows_only": ([1100], [600], 8, 64, 8, "bf16", AUTO, True),
+    "many_tokens": ([2300, 333], [2211, 70], 16, 8, 2, "bf16", AUTO, False),
+    "kv17": ([50, 20], [20, 3], 16, 17, 17, "f16", AUTO, True),
+    "one_kv_head_group7": ([333, 70], [40, 9], 32, 7, 1, "bf16", AUTO, True),
+    "63_requests": ([20 + i for i in range(63)], [2] * 62 + [9], 8, 32, 8, "bf16", AUTO, True),
+    "64_requests": ([20 + i for i in range(64)], [2] * 63 + [20], 16, 32, 8, "bf16", AUTO, False),
+    "no_rows_between": ([700, 40, 9, 350], [30, 0, 9, 50], 16, 32, 8, "bf16", AUTO, True),
+    "shared": ([700, 1, 33, 250, 64], [130, 1, 1, 1, 30], 16, 64, 8, "bf16", SHARED, False),
+    "page2": ([150, 9], [33, 2], 2, 40, 2, "f16", AUTO, False),
+}
+
+
+def _setup(case):
+    from deserve_amd.paged_ops import BatchPrefillWithPagedKVCacheWrapper, rope_table
+
+    kv, qo, P, Hq, Hkv, dtype, route, _ = CASES[case]
+    sc = make_scenario(63, kv_lens=kv, qo_lens=qo, P=P, Hq=Hq, Hkv=Hkv, D=128, dtype=dtype)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a, np.int32)).cuda()
+    indptr = dev(sc.qo_indptr)
+    w = BatchPrefillWithPagedKVCacheWrapper(torch.empty(64 << 20, dtype=torch.uint8, device="cuda"))
+    w.begin_forward(indptr, dev(sc.kv_page_indptr), dev(sc.kv_page_indices), dev(sc.kv_last_page_lens), Hq, Hkv, 128, P,
+                    route_one_row_requests=route)
+    q, k, v = (to_torch(a, dtype) for a in (sc.q, sc.k, sc.v))
+    table = rope_table(indptr, dev(sc.kv_lens - sc.qo_lens), q.shape[0], 128, 5e5)
+    return w, q, k, v, to_torch(sc.pages, dtype), table
+
+
+def _call(w, q, k, v, pages, table, flags, polls):
+    step = _lib.MixedStep.from_buffer_copy(w._step)
+    step.rope_table = None if table is None else table.data_ptr()
+    step.num_pages, step.causal, step.dtype, step.sm_scale = pages.shape[0], 1, _lib.dtype_code(q.dtype), 1 / math.sqrt(128)
+    out = torch.full_like(q, float("nan"))
+    _lib.check(_lib.lib().dskv_mixed_layers_flagged(
+        ctypes.byref(step), None if flags is None else flags.data_ptr(), 0 if flags is None else flags.numel(), polls, 1,
+        out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), pages.data_ptr(), 0, _lib.current_stream()), "step")
+    return out
+
+
+def _bits(t):
+    return t.view(torch.int16)
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_same_bits_as_an_append_in_front(case):
+    print("[case] append rows", case, *CASES[case], flush=True)
+    w, q, k, v, fresh, table = _setup(case)
+    for tab in (table, None):
+        want_pages = fresh.clone()
+        want = _call(w, q, k, v, want_pages, tab, None, 0)
+        assert bool(torch.isfinite(want.float()).all())
+        for polls in (0, 0, 1, 1, 0):      # the flags of the call before are there, too
+            pages = fresh.clone()
+            got = _call(w, q, k, v, pages, tab, w._flags, polls)
+            torch.cuda.synchronize()
+            assert torch.equal(_bits(pages), _bits(want_pages)) and torch.equal(_bits(got), _bits(want)), polls
+    assert bool(w._flags.any()) == CASES[case][-1]
+
+
+def test_a_pool_between_cache_lines_and_a_captured_stream():
+    print("[case] append rows, odd pool and capture", flush=True)
+    w, q, k, v, fresh, table = _setup("block_edges")
+    want_pages = fresh.clone()
+    want = _call(w, q, k, v, want_pages, table, None, 0)
+    odd = torch.empty(fresh.numel() + 8, dtype=fresh.dtype, device="cuda")[8:].view(fresh.shape)
+    odd.copy_(fresh)
+    got = _call(w, q, k, v, odd, table, w._flags, 0)
+    assert torch.equal(_bits(odd), _bits(want_pages)) and torch.equal(_bits(got), _bits(want))
+    pages = fresh.clone()
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.graph(graph, stream=side):
+        got = _call(w, q, k, v, pages, table, w._flags, 0)
+    for _ in range(3):
+        pages.copy_(fresh)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(_bits(pages), _bits(want_pages)) and torch.equal(_bits(got), _bits(want))
