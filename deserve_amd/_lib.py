@@ -25,7 +25,7 @@ class MixedPlanInfo(ctypes.Structure):
     """dskv_mixed_plan_t of include/dskv.h."""
     _fields_ = [("n_tiles", c_int32), ("n_splits", c_int32), ("n_tile_rows", c_int32),
                 ("n_decode_rows", c_int32), ("n_decode_items", c_int32), ("n_decode_workgroups", c_int32),
-                ("layout", c_int32), ("reserved", c_int32), ("plan_words", c_int64), ("decode_plan_at", c_int64), ("row_map_at", c_int64),
+                ("layout", c_int32), ("new_rows_late", c_int32), ("plan_words", c_int64), ("decode_plan_at", c_int64), ("row_map_at", c_int64),
                 ("tile_workspace_bytes", c_int64),
                 ("decode_workspace_bytes", c_int64)]
 

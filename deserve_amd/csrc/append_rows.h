@@ -3,9 +3,10 @@
 // a tile looks at the flags of the rows that it needs before it requests the first block that holds one.
 //
 // What it saves is a launch in front of the attention (4.8 us for 512 tokens, most of it the start, the chain
-// token -> request -> page -> store and the end of a launch): a chunk of 512 over 4096 904 -> 880 us in 16 layers,
-// three short prompts 307 -> 304.  Workgroups that do nothing but append were tried first: one of eight waves and 250
-// registers fills its compute unit, so they ran in front of tiles and not beside them, and gained nothing.  With
+// token -> request -> page -> store and the end of a launch): a chunk of 512 over 4096 904 -> 880 us in 16 layers.
+// Workgroups that do nothing but append were tried first: one of eight waves and 250 registers fills its compute
+// unit, so they ran in front of tiles and not beside them, and gained nothing; in the launch that tiles share
+// with decode workgroups the loop of the tiles lost more (2341 -> 2395 us).  With
 // more than kAppendMaxTokens a workgroup (16 chunks of 512) the launch in front stays: it moves bytes then, 14.7 us
 // of 700 a layer, and a tile would start that much later.
 //
@@ -28,6 +29,10 @@ namespace dskv {
 constexpr int kAppendFlags = 256;        // flags, at most: one per appending workgroup
 constexpr int kAppendMaxTokens = 32;     // tokens of such a workgroup, at most: two for each lane half of eight waves
 constexpr int kAppendMaxBatch = 63;      // requests, at most: a token's is found with one load and a ballot
+// 32-token blocks that every walk has in front of its first new row, at least: a flag is raised four blocks into
+// the walk of its workgroup.  Walks that begin with new rows - prompts - only wait: three short prompts took 358 us in
+// 16 layers, 305 with the launch in front.
+constexpr int kAppendAheadBlocks = 12;
 constexpr int kAppendPolls = 256;        // looks at a flag (about 0.4 us each) before a tile appends itself
 
 struct AppendRows {

@@ -519,6 +519,14 @@ extern "C" int dskv_mixed_plan_typed(const int32_t *qo_indptr_host, const int32_
                         layout != DSKV_LAYOUT_SHARED);
     if (rc) return rc;
     info->tile_workspace_bytes = (info->tile_workspace_bytes + 255) / 256 * 256;
+    // whether every walk that meets new rows has kAppendAheadBlocks in front of them (tiles_append)
+    info->new_rows_late = info->n_tiles > 0;
+    for (int32_t i = 0; i < info->n_tiles && info->new_rows_late; i++) {
+        const int32_t *e = plan_host + (int64_t)i * kTileWords;
+        const int64_t prior = (int64_t)kv_len[e[0]] - (qo_indptr_host[e[0] + 1] - qo_indptr_host[e[0]]);
+        const bool meets = e[3] == kWholeRange || (int64_t)e[3] * kBlock > prior;
+        if (meets && ((int64_t)e[2] + kAppendAheadBlocks) * kBlock > prior) info->new_rows_late = 0;
+    }
     info->n_tile_rows = (int32_t)n_tile_rows;
     int64_t at = (tile_words + 3) / 4 * 4;
     info->plan_words = tile_words;
@@ -887,11 +895,11 @@ extern "C" int dskv_mixed_step_supported(int32_t n_qo_heads, int32_t n_kv_heads,
 namespace dskv {
 
 // Whether a step's attention launch appends the step's rows itself: tiles only (decode workgroups beside
-// them, or a decode pass in front, would need theirs before), loaded straight into LDS, few enough
-// tokens for the first tiles' workgroups.  Rows have to be whole cache lines: see append_rows.h.
+// them, or a decode pass in front, would need theirs before), loaded straight into LDS, which meet new rows
+// late, and few enough tokens for the first tiles' workgroups.  Rows have to be whole cache lines: see append_rows.h.
 static bool tiles_append(const dskv_mixed_step_t &s, const void *k, const void *v, const void *pages_layer, AppendRows &a)
 {
-    if (s.page_size < 4 || s.info->n_decode_rows > 0 || s.info->n_tiles <= 0 || s.batch > kAppendMaxBatch ||
+    if (!s.info->new_rows_late || s.page_size < 4 || s.info->n_decode_rows > 0 || s.info->n_tiles <= 0 || s.batch > kAppendMaxBatch ||
         s.n_kv_heads > kAppendFlags || ((uintptr_t)pages_layer % 256) || (((uintptr_t)k | (uintptr_t)v) % 16))
         return false;
     a.n_tiles = std::min(s.info->n_tiles, kAppendFlags / s.n_kv_heads);

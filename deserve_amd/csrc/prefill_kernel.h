@@ -551,20 +551,13 @@ __device__ __forceinline__ bool prefill_attn_body(
                              "+s"(ahead[1][i]));
 #pragma unroll
             for (int blk = 0; blk < 4; blk++) prepare_rows(blk_begin + blk, pg[blk], desc[blk]);
-            // a walk that requests new rows within its first four iterations waits for them first; the others append
-            // beside their first loads
-            const bool appends = kAppends && !rows_there, new_first = kAppends && (blk_begin + 8) * kBlock > new_from;
-            if (new_first) {
-                append_look_up();
-                append_store();
-                raise_when_stored();
-                await_new_rows();
-            }
+            // (a plan whose walks begin with new rows is not launched this way: see kAppendAheadBlocks)
+            if (kAppends && (blk_begin + 8) * kBlock > new_from) await_new_rows();
 #pragma unroll
             for (int blk = 0; blk < (kKPrefetch ? 4 : 3); blk++) load_direct(desc[blk].k, k_stage[blk]);
 #pragma unroll
             for (int blk = 0; blk < 2; blk++) load_direct(desc[blk].v, v_stage[blk]);
-            raise_later = appends && !new_first;
+            raise_later = kAppends && !rows_there;
             if (raise_later) append_look_up();
             finish_all_q();
             if (raise_later) append_store();

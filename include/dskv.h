@@ -339,7 +339,8 @@ typedef struct dskv_mixed_plan {
     int32_t n_tile_rows;              /* query rows computed by the tile pass */
     int32_t n_decode_rows;            /* one-row requests computed by the decode pass */
     int32_t n_decode_items, n_decode_workgroups;
-    int32_t layout, reserved;
+    int32_t layout;
+    int32_t new_rows_late;            /* every tile entry that sees new rows walks 12 blocks of 32 tokens before them */
     int64_t plan_words;
     int64_t decode_plan_at, row_map_at;
     int64_t tile_workspace_bytes, decode_workspace_bytes;
@@ -391,8 +392,8 @@ int dskv_mixed_layers(const dskv_mixed_step_t *step, int32_t n_layers, void *out
                       const void *v_new, void *pages, int64_t pages_layer_bytes, void *stream);
 /*
  * The same with dskv_append_flags() words (device, zero before the first call that is given them), which let the
- * attention launch append the step's rows itself, without a launch in front of it: a plan of tiles only, at most
- * 32 new tokens for each of its first entries, fewer than 64 requests, pages of at least 4 tokens, pages and
+ * attention launch append the step's rows itself, without a launch in front of it: a plan of tiles only
+ * with new_rows_late, at most 32 new tokens for each of its first entries, fewer than 64 requests, pages of at least 4 tokens, pages and
  * layers of them at multiples of 256 bytes, a stream that is not being captured; elsewhere, and with
  * append_flags null or fewer words, it is dskv_mixed_layers.  Pages and output have the same bits either way.
  * polls: how often a query tile looks for rows that other workgroups append before it appends them itself (0:

@@ -1,10 +1,10 @@
 """The prefill launch whose tiles append the step's rows themselves, against the same step with the append as a
 launch of its own: the same bits in pages and result.  Edges: the first new row at the ends of 32-token
-blocks and of the four blocks between two waits, no prior context, parts that end before the new rows or
-hold nothing else, one and two rounds of tokens per wave, empty shares, 63 requests, groups and head counts that
-leave waves idle, pages of 4 tokens; and what keeps the launch in front: pages of 2 tokens, too many tokens, 64
-requests, decode rows beside, a pool that is not at a multiple of 256 bytes, a captured stream.  With one
-look at the flags only, tiles append for themselves."""
+blocks and of the four blocks between two waits, parts, one and two rounds of tokens per wave, empty shares, 63
+requests, groups and head counts that leave waves idle, pages of 4 tokens; and what keeps the launch in front:
+new rows within a walk's first twelve blocks, pages of 2 tokens, too many tokens, 64 requests, decode rows
+beside, a pool that is not at a multiple of 256 bytes, a captured stream.  With one look at the flags only,
+tiles append for themselves."""
 import ctypes
 import math
 
@@ -18,22 +18,27 @@ from kvutil import make_scenario, to_torch
 pytestmark = pytest.mark.gpu
 
 AUTO, SHARED = _lib.ROUTE_AUTO, _lib.ROUTE_SHARED_LAUNCH
+def _over(prior, new):   # (kv_lens, qo_lens)
+    return [p + n for p, n in zip(prior, new)], list(new)
+
+
 CASES = {   # kv_lens, qo_lens, page, Hq, Hkv, dtype, route, whether the tiles append
-    "block_edges": ([31 + 5, 32 + 33, 33 + 1, 95 + 70, 96 + 2, 128 + 31, 129 + 3], [5, 33, 1, 70, 2, 31, 3], 16, 32, 8, "bf16", AUTO, True),
-    "prompts_page4": ([17, 203, 1], [17, 203, 1], 4, 16, 4, "f16", AUTO, False),
-    "short_prompts_page4": ([17, 3, 1, 30], [17, 3, 1, 30], 4, 32, 8, "f16", AUTO, True),
-    "chunk": ([4096 + 512], [512], 16, 32, 8, "bf16", AUTO, True),
-    "two_rounds": ([1500 + 901], [901], 8, 32, 8, "bf16", AUTO, True),
-    "parts": ([1700, 2300], [129, 40], 16, 32, 8, "bf16", AUTO, True),
-    "part_of_new_rows_only": ([1100], [600], 8, 64, 8, "bf16", AUTO, True),
-    "many_tokens": ([2300, 333], [2211, 70], 16, 8, 2, "bf16", AUTO, False),
-    "kv17": ([50, 20], [20, 3], 16, 17, 17, "f16", AUTO, True),
-    "one_kv_head_group7": ([333, 70], [40, 9], 32, 7, 1, "bf16", AUTO, True),
-    "63_requests": ([20 + i for i in range(63)], [2] * 62 + [9], 8, 32, 8, "bf16", AUTO, True),
-    "64_requests": ([20 + i for i in range(64)], [2] * 63 + [20], 16, 32, 8, "bf16", AUTO, False),
-    "no_rows_between": ([700, 40, 9, 350], [30, 0, 9, 50], 16, 32, 8, "bf16", AUTO, True),
-    "shared": ([700, 1, 33, 250, 64], [130, 1, 1, 1, 30], 16, 64, 8, "bf16", SHARED, False),
-    "page2": ([150, 9], [33, 2], 2, 40, 2, "f16", AUTO, False),
+    "block_edges": (*_over([384, 385, 415, 416, 447, 480, 511], [5, 33, 1, 70, 2, 31, 3]), 16, 32, 8, "bf16", AUTO, True),
+    "page4": (*_over([400, 390], [50, 9]), 4, 16, 4, "f16", AUTO, True),
+    "too_near": (*_over([383, 500], [30, 20]), 16, 32, 8, "bf16", AUTO, False),
+    "prompts": ([17, 203, 1], [17, 203, 1], 4, 32, 8, "f16", AUTO, False),
+    "chunk": (*_over([4096], [512]), 16, 32, 8, "bf16", AUTO, True),
+    "two_rounds": (*_over([3000], [901]), 8, 32, 8, "bf16", AUTO, True),
+    "parts": (*_over([1700, 2360], [60, 40]), 16, 32, 8, "bf16", AUTO, True),
+    "part_of_new_rows_only": (*_over([1100], [600]), 8, 32, 8, "bf16", AUTO, False),
+    "many_tokens": (*_over([2300, 400], [2211, 70]), 16, 8, 2, "bf16", AUTO, False),
+    "kv17": (*_over([400, 450], [20, 3]), 16, 17, 17, "f16", AUTO, True),
+    "one_kv_head_group7": (*_over([400, 450], [40, 9]), 32, 7, 1, "bf16", AUTO, True),
+    "63_requests": (*_over([400 + 3 * i for i in range(63)], [2] * 62 + [9]), 8, 32, 8, "bf16", AUTO, True),
+    "64_requests": (*_over([400 + i for i in range(64)], [2] * 63 + [20]), 16, 32, 8, "bf16", AUTO, False),
+    "no_rows_between": (*_over([700, 40, 400, 390], [30, 0, 9, 50]), 16, 32, 8, "bf16", AUTO, True),
+    "shared": (*_over([600, 0, 32, 249, 400], [130, 1, 1, 1, 30]), 16, 64, 8, "bf16", SHARED, False),
+    "page2": (*_over([500, 400], [33, 2]), 2, 40, 2, "f16", AUTO, False),
 }
 
 
