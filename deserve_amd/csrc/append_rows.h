@@ -82,11 +82,14 @@ struct AppendShare {
     int q_i, p_i, l_i;             // lane i: entry i of qo_indptr, kv_indptr, kv_last
     long pos[kRounds], page[kRounds];   // page -1: no row of this lane's
     int begin, end;
-    bool mine;
+    bool mine, found;
 
-    // the rows, and what tells their requests
+    // the rows, and what tells their requests - or, where that is the tile's own (tokens q_begin .. + n_b of the batch,
+    // n_pages of the table from page_begin on, kv_len tokens), the pages and the angles at once
     __device__ __forceinline__ void request(const_append_ptr a, int tile, int kvh, int n_kv_heads, int wave,
-                                            const int32_t *qo_indptr, const int32_t *kv_indptr, const int32_t *kv_last)
+                                            const int32_t *qo_indptr, const int32_t *kv_indptr, const int32_t *kv_last,
+                                            int q_begin, int n_b, int page_begin, int kv_len, const int32_t *kv_indices,
+                                            int page_shift, const float *rope)
     {
         asm volatile("" : "+s"(a));
         mine = tile < a->n_tiles;
@@ -94,9 +97,18 @@ struct AppendShare {
         const int lane = lane_id(), nnz = a->nnz, batch = a->batch;
         begin = tile * a->tokens;
         end = min(begin + a->tokens, nnz);
-        q_i = qo_indptr[min(lane, batch)];
-        p_i = kv_indptr[min(lane, batch)];
-        l_i = kv_last[min(lane, batch - 1)];
+        found = begin >= q_begin && end <= q_begin + n_b;
+        if (found) {
+#pragma unroll
+            for (int i = 0; i < kRounds; i++) {
+                const int t = begin + (i * kWaves + wave) * 2 + (lane >> 5);
+                find(i, t, q_begin, n_b, page_begin, kv_len, lane, kv_indices, page_shift, rope);
+            }
+        } else {
+            q_i = qo_indptr[min(lane, batch)];
+            p_i = kv_indptr[min(lane, batch)];
+            l_i = kv_last[min(lane, batch - 1)];
+        }
         const uint16_t *const from = lane & 16 ? a->v : a->k;
 #pragma unroll
         for (int i = 0; i < kRounds; i++) {
@@ -108,7 +120,7 @@ struct AppendShare {
     __device__ __forceinline__ void look_up(const_append_ptr a, int wave, const int32_t *kv_indices, int page_shift,
                                             const float *rope)
     {
-        if (!mine) return;
+        if (!mine || found) return;
         asm volatile("" : "+s"(a));
         const int lane = lane_id(), batch = a->batch;
 #pragma unroll
@@ -121,15 +133,21 @@ struct AppendShare {
             const int first = __shfl(q_i, b), n_b = __shfl(q_i, b + 1) - first;
             const int page_begin = __shfl(p_i, b), n_pages = __shfl(p_i, b + 1) - page_begin, last = __shfl(l_i, b);
             const long kv_len = n_pages > 0 ? ((long)(n_pages - 1) << page_shift) + last : 0;
-            pos[i] = kv_len - n_b + (t - first);
-            page[i] = -1;   // metadata that does not cover the token: touched by nobody
-            if (t < end && t >= first && pos[i] >= 0 && pos[i] < kv_len) {
-                page[i] = kv_indices[page_begin + (pos[i] >> page_shift)];
-                if (rope) {
-                    const float *tab = rope + (long)t * kHeadDim + (lane & 15) * 4;   // dims 8 * chunk .. + 7: 4 pairs
-                    cs[i] = *reinterpret_cast<const f32x4 *>(tab);
-                    sn[i] = *reinterpret_cast<const f32x4 *>(tab + kHeadDim / 2);
-                }
+            find(i, t, first, n_b, page_begin, kv_len, lane, kv_indices, page_shift, rope);
+        }
+    }
+    // the page and the angles of round i's token t, of the request of tokens first .. + n_b
+    __device__ __forceinline__ void find(int i, int t, int first, int n_b, int page_begin, long kv_len, int lane,
+                                         const int32_t *kv_indices, int page_shift, const float *rope)
+    {
+        pos[i] = kv_len - n_b + (t - first);
+        page[i] = -1;   // metadata that does not cover the token: touched by nobody
+        if (t < end && t >= first && pos[i] >= 0 && pos[i] < kv_len) {
+            page[i] = kv_indices[page_begin + (pos[i] >> page_shift)];
+            if (rope) {
+                const float *tab = rope + (long)t * kHeadDim + (lane & 15) * 4;   // dims 8 * chunk .. + 7: 4 pairs
+                cs[i] = *reinterpret_cast<const f32x4 *>(tab);
+                sn[i] = *reinterpret_cast<const f32x4 *>(tab + kHeadDim / 2);
             }
         }
     }

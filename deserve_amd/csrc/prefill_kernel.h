@@ -263,7 +263,9 @@ __device__ __forceinline__ bool prefill_attn_body(
     AppendShare<DT, kWaves> share;
     const const_append_ptr append = (const_append_ptr)__builtin_amdgcn_kernarg_segment_ptr();
     auto append_request_share = [&]() {
-        if (kAppends) share.request(append, tile, kvh, n_kv_heads, wave, qo_indptr, kv_indptr, kv_last);
+        if (kAppends)
+            share.request(append, tile, kvh, n_kv_heads, wave, qo_indptr, kv_indptr, kv_last, q_begin, n_b, page_begin,
+                          kv_len, kv_indices, page_shift, rope);
     };
     auto append_look_up = [&]() {
         if (kAppends) share.look_up(append, wave, kv_indices, page_shift, rope);
