@@ -60,7 +60,7 @@ class KVStage:
         dim = self.core.dim
         result = torch.empty((q.shape[0], q[0].numel() // dim, dim), dtype=q.dtype, device=q.device)
         stacked = result.view(q.shape[0], -1, self.core.n_local_heads, self.core.head_dim)
-        if self._whole_core() and self.core.layers_forward(q, k, v, ctx, stacked):
+        if q.dtype is not torch.float32 and self._whole_core() and self.core.layers_forward(q, k, v, ctx, stacked):
             return result
         outs = stacked.unbind(0)
         qs, ks, vs = q.unbind(0), k.unbind(0), v.unbind(0)
