@@ -17,6 +17,7 @@ CSRC_DIR = os.path.join(_HERE, "csrc")
 
 F32, F16, BF16 = 0, 1, 2
 ROUTE_OFF, ROUTE_AUTO, ROUTE_TWO_LAUNCHES, ROUTE_SHARED_LAUNCH = 0, 1, 2, 3
+APPEND_ODD_LATE = 1 << 30     # DSKV_APPEND_ODD_LATE of include/dskv.h
 LAYOUT_SEPARATE, LAYOUT_SHARED = 0, 1
 ABI_VERSION = 3          # DSKV_ABI_VERSION of the include/dskv.h these signatures were written against
 

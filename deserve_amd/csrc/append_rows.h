@@ -11,14 +11,14 @@
 // of 700 a layer, and a tile would start that much later.
 //
 // Rows that another compute unit reads in the same launch: they are stored with device scope (written
-// through the L2 of the XCD), and a flag is raised when all its stores are acknowledged.  The readers'
-// loads are ordinary ones: no cache can hold the line of a new row before, since the caches are clean of
-// other launches' stores when a launch starts, rows are whole lines (256 bytes at a multiple of 256),
-// and nobody reads them ahead of the flag.
+// through the L2 of the XCD), a flag is raised when all its stores are acknowledged, and blocks that hold
+// new rows are loaded with device scope, too, when the flags have been seen.  So no line that an L2 has held from before
+// is met, whoever brought it there - another stream's kernel that copies whole pages, for one.
 //
 // No order in which workgroups start is relied on: a wait is bounded, and a tile that has looked `polls` times in
-// vain finishes its walk, writes the rows that it needs itself - the same bytes to the same place - and
-// walks again.
+// vain ends its walk there, before it requests a block with a new row, writes the rows that it needs itself - the
+// same bytes to the same place - and walks again, with ordinary loads: its own stores have gone through
+// the L1 and L2 that it reads through (rows are whole lines, 256 bytes at a multiple of 256).
 #pragma once
 
 #include "kv_tile.h"
@@ -26,7 +26,7 @@
 
 namespace dskv {
 
-constexpr int kAppendFlags = 256;        // flags, at most: one per appending workgroup
+constexpr int kAppendFlags = 256;        // flags, at most: one per appending workgroup; behind them the count of second walks
 constexpr int kAppendMaxTokens = 32;     // tokens of such a workgroup, at most: two for each lane half of eight waves
 constexpr int kAppendMaxBatch = 63;      // requests, at most: a token's is found with one load and a ballot
 // 32-token blocks that every walk has in front of its first new row, at least: a flag is raised four blocks into
@@ -40,7 +40,8 @@ struct AppendRows {
     uint32_t *flags;           // word tile * Hkv + kv head, raised by writing `launch` to it
     uint32_t launch;           // a number no earlier launch with these flags had
     int n_tiles, tokens;       // plan entries that append; tokens of each
-    int nnz, batch, num_pages, polls;
+    int nnz, batch, num_pages;
+    int polls[2];              // looks at a flag of plan entries of even and of odd number
 };
 typedef const __attribute__((address_space(4))) AppendRows *const_append_ptr;
 
@@ -169,14 +170,15 @@ struct AppendShare {
     }
 };
 
-// Whether entries first .. last have raised their flags for kv head kvh, after up to `polls` looks.
+// Whether entries first .. last have raised their flags for kv head kvh, after as many looks as plan entry `tile` has.
 // Called with a tile's registers full: the arguments are read where they are needed.
-__device__ __forceinline__ bool rows_are_there(const_append_ptr a, int first, int last, int kvh, int n_kv_heads)
+__device__ __forceinline__ bool rows_are_there(const_append_ptr a, int tile, int first, int last, int kvh, int n_kv_heads)
 {
     asm volatile("" : "+s"(a));
     uint32_t *const flags = a->flags;
     const uint32_t launch = a->launch;
-    const int polls = a->polls, lane = lane_id();
+    const int polls = a->polls[tile & 1];
+    const int lane = lane_id();
     for (int f = first; f <= last; f += 64) {
         bool there = false;
         for (int i = 0; i < polls && !there; i++) {

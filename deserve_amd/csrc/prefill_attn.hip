@@ -924,7 +924,8 @@ static int mixed_step(const dskv_mixed_step_t &s, void *out, const void *q, cons
             append.nnz = s.nnz;
             append.batch = s.batch;
             append.num_pages = s.num_pages;
-            append.polls = polls;
+            append.polls[0] = polls & ~DSKV_APPEND_ODD_LATE;
+            append.polls[1] = polls & DSKV_APPEND_ODD_LATE ? 0 : polls;
         }
     }
     if (!append.k) {
@@ -941,7 +942,7 @@ static int mixed_step(const dskv_mixed_step_t &s, void *out, const void *q, cons
 
 }  // namespace dskv
 
-extern "C" int64_t dskv_append_flags(void) { return dskv::kAppendFlags; }
+extern "C" int64_t dskv_append_flags(void) { return dskv::kAppendFlags + 1; }
 
 extern "C" int dskv_mixed_layers_flagged(const dskv_mixed_step_t *step, uint32_t *append_flags, int64_t n_append_flags,
                                          int32_t polls, int32_t n_layers, void *out, const void *q, const void *k_new,
@@ -959,7 +960,7 @@ extern "C" int dskv_mixed_layers_flagged(const dskv_mixed_step_t *step, uint32_t
     // A captured launch would raise its flags with the same number in every replay, and find them raised
     if (append_flags) {
         hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        if (n_append_flags < kAppendFlags || hipStreamIsCapturing((hipStream_t)stream, &capture) != hipSuccess ||
+        if (n_append_flags < dskv_append_flags() || hipStreamIsCapturing((hipStream_t)stream, &capture) != hipSuccess ||
             capture != hipStreamCaptureStatusNone) {
             (void)hipGetLastError();
             append_flags = nullptr;
@@ -971,7 +972,7 @@ extern "C" int dskv_mixed_layers_flagged(const dskv_mixed_step_t *step, uint32_t
     for (int64_t l = 0; l < n_layers; l++) {
         const int rc = mixed_step(s, (void *)at(out, l * q_bytes), at(q, l * q_bytes), at(k_new, l * kv_bytes),
                                   at(v_new, l * kv_bytes), (void *)at(pages, l * pages_layer_bytes), append_flags,
-                                  polls > 0 ? polls : kAppendPolls, stream);
+                                  polls & ~DSKV_APPEND_ODD_LATE ? polls : polls | kAppendPolls, stream);
         if (rc) return rc;
     }
     return 0;

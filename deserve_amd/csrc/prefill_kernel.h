@@ -66,8 +66,8 @@ struct LdsStages {
 //     pushed the chunk's K/V out of it: 75 decode rows and the chunk 2638 -> 2471 us a step (16
 //     layers), 70B-shaped 1527 -> 1410.  A launch of tiles only loses (a chunk of 512 in four parts 938
 //     -> 955): its merge pass then reads the partials from farther away.
-//   kAppends: the launch appends the step's rows (append_rows.h); false is returned, and nothing stored, if others'
-//     did not come in time: append_for_tile, then call again with rows_there.
+//   kAppends: the launch appends the step's rows (append_rows.h); false is returned if others' did not come in
+//     time, with no output stored and no block requested that holds one: append_for_tile, then again with rows_there.
 struct PrefillArgs {
     AppendRows append;   // at the front: read through the kernel's argument segment
     uint16_t *out;
@@ -312,17 +312,25 @@ __device__ __forceinline__ bool prefill_attn_body(
         return true;
     }
 
+    // A walk whose first requests would hold new rows: a plan with one is not launched this way
+    // (kAppendAheadBlocks), but the lengths that count are the device's.
+    if (kAppends && !rows_there && t_end > kv_len - n_b && (blk_begin + 8) * kBlock > kv_len - n_b) return false;
+
     // Blocks that end behind new_from hold rows that this launch appends: they are requested when the
-    // flags of the workgroups that append them have been seen.
+    // flags of the workgroups that append them have been seen by every wave, and never before.
     int new_from = kAppends && !rows_there && t_end > kv_len - n_b ? kv_len - n_b : 0x7fffffff;
-    bool in_time = true;
     int *const late = reinterpret_cast<int *>(lds_base + prefill_lds_bytes(kWaves));
-    auto await_new_rows = [&]() {
+    auto await_new_rows = [&]() {   // whether some wave looked in vain
         const_append_ptr a = (const_append_ptr)__builtin_amdgcn_kernarg_segment_ptr();
         const int tokens = a->tokens;
-        in_time = rows_are_there(a, (q_begin + max(t_first - new_from, 0)) / tokens,
-                                 (q_begin + min(t_end - new_from, n_b) - 1) / tokens, kvh, n_kv_heads);
+        const bool in_time = rows_are_there(a, tile, (q_begin + max(t_first - new_from, 0)) / tokens,
+                                            (q_begin + min(t_end - new_from, n_b) - 1) / tokens, kvh, n_kv_heads);
         new_from = 0x7fffffff;
+        if (!in_time) *late = 1;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (bare, as the loop's barriers)
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        return __builtin_amdgcn_readfirstlane(*late) != 0;
     };
     if (kAppends && wave == 0) *late = 0;
 
@@ -384,18 +392,26 @@ __device__ __forceinline__ bool prefill_attn_body(
     // for ALL of these loads (it cannot tell which region a read touches), which would undo
     // requesting them three iterations early.  What it does not know it does not wait for:
     // the waits for these loads are the explicit ones below.
+    // with_new_rows: with device scope, past the XCD's L2 - whoever has read a new row's line too early, nobody here
+    // meets that reading.
     // M0 is on the clobber list (the compiler reserves it, sets it itself before the few
     // instructions that read it, and must not assume that such a setting survives this one).
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-    auto load_direct = [&](const u32x4(&rows)[kRowGroups], char *stage) {
+    auto load_direct = [&](const u32x4(&rows)[kRowGroups], char *stage, bool with_new_rows = false) {   // (a literal)
 #pragma unroll
         for (int i = 0; i < kRowGroups; i++) {
             const uint32_t lds_addr = (uint32_t)(uintptr_t)(lds_ptr)region_of(stage, i);
-            asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                         :
-                         : "s"(lds_addr), "v"(direct_off), "s"(rows[i])
-                         : "memory", "m0");
+            if (with_new_rows)
+                asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen sc1 lds"
+                             :
+                             : "s"(lds_addr), "v"(direct_off), "s"(rows[i])
+                             : "memory", "m0");
+            else
+                asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                             :
+                             : "s"(lds_addr), "v"(direct_off), "s"(rows[i])
+                             : "memory", "m0");
         }
     };
 #pragma clang diagnostic pop
@@ -553,8 +569,6 @@ __device__ __forceinline__ bool prefill_attn_body(
                              "+s"(ahead[1][i]));
 #pragma unroll
             for (int blk = 0; blk < 4; blk++) prepare_rows(blk_begin + blk, pg[blk], desc[blk]);
-            // (a plan whose walks begin with new rows is not launched this way: see kAppendAheadBlocks)
-            if (kAppends && (blk_begin + 8) * kBlock > new_from) await_new_rows();
 #pragma unroll
             for (int blk = 0; blk < (kKPrefetch ? 4 : 3); blk++) load_direct(desc[blk].k, k_stage[blk]);
 #pragma unroll
@@ -600,7 +614,7 @@ __device__ __forceinline__ bool prefill_attn_body(
     // V operand: token 16 ks + 8 hi + 4 h + (c >> 2) = row c >> 2 of region 4 ks + 2 hi + h;
     // bytes 64 dt + 32 (g & 1) + 8 (c & 3) of its row = half (c & 1) of chunk 4 dt + 2 (g & 1) + ((c & 3) >> 1)
     const int v_lane_off = h * kRegionBytes + (2 * (g & 1) + ((c & 3) >> 1)) * 64 + (c >> 2) * 16 + (c & 1) * 8;
-    auto iteration = [&](int m, int phase, RowSet &rows) {   // phase = m % 4, a literal at each call
+    auto iteration = [&](int m, int phase, RowSet &rows, bool with_new_rows) {   // the last and phase = m % 4 are literals at each call
         if (kRowsSharePage) {
             // this wave's rows of K(m+1) have landed; then the bare barrier: with the fences of
             // __syncthreads the compiler waits for EVERY load into LDS still on its way, which
@@ -619,8 +633,8 @@ __device__ __forceinline__ bool prefill_attn_body(
         }
         if (kRowsSharePage && kKPrefetch) {
             lookup_pages(m + 6, pg[(phase + 2) & 3]);
-            load_direct(desc[phase].k, k_stage[phase]);                       // K(m+4) over K(m), read in iteration m-2
-            load_direct(desc[(phase + 2) & 3].v, v_stage[(phase + 2) & 3]);   // V(m+2)
+            load_direct(desc[phase].k, k_stage[phase], with_new_rows);                       // K(m+4) over K(m), read in iteration m-2
+            load_direct(desc[(phase + 2) & 3].v, v_stage[(phase + 2) & 3], with_new_rows);   // V(m+2)
         } else if (kRowsSharePage) {
             lookup_pages(m + 5, pg[(phase + 1) & 3]);
             load_direct(desc[(phase + 3) & 3].k, k_stage[(phase + 3) & 3]);   // K(m+3)
@@ -693,7 +707,9 @@ __device__ __forceinline__ bool prefill_attn_body(
         for (int ct = 0; ct < kColTiles; ct++) l_run[ct] += p_sum[ct];
     };
     // The four iterations from m on request blocks up to m + 7.  The walk is cut where they would first meet a
-    // new row, so that the loop itself has nothing to look at.
+    // new row, so that the loop itself has nothing to look at; what is behind the cut is a loop of its own, with
+    // device scope (a chunk of 512 over 4096 takes the same 880 us either way; with a scalar branch at each load
+    // of one loop 889).
     for (int m = blk_begin;;) {
         int end = n_blocks + 1;
         const bool raise_now = kAppends && raise_later, wait_now = kAppends && !raise_now && new_from < 0x7fffffff;
@@ -702,10 +718,10 @@ __device__ __forceinline__ bool prefill_attn_body(
         if (raise_now) end = min(end, m + 4);
         if (wait_now) end = min(end, m + max(new_from / kBlock - 8 - m + 4, 0) / 4 * 4);
         for (; m < end; m += 4) {
-            iteration(m, 0, even);
-            iteration(m + 1, 1, odd);
-            iteration(m + 2, 2, even);
-            iteration(m + 3, 3, odd);
+            iteration(m, 0, even, false);
+            iteration(m + 1, 1, odd, false);
+            iteration(m + 2, 2, even, false);
+            iteration(m + 3, 3, odd, false);
         }
         if (!kAppends) break;
         if (raise_now) {
@@ -713,7 +729,16 @@ __device__ __forceinline__ bool prefill_attn_body(
             raise_later = false;
         }
         if (m > n_blocks) break;
-        if (wait_now) await_new_rows();
+        if (wait_now) {
+            if (await_new_rows()) break;
+            for (; m <= n_blocks; m += 4) {
+                iteration(m, 0, even, true);
+                iteration(m + 1, 1, odd, true);
+                iteration(m + 2, 2, even, true);
+                iteration(m + 3, 3, odd, true);
+            }
+            break;
+        }
     }
     if (kRowsSharePage) DSKV_WAIT_VMEM(0);   // nothing of this wave may still be on its way into LDS
 #undef DSKV_WAIT_VMEM
@@ -723,7 +748,6 @@ __device__ __forceinline__ bool prefill_attn_body(
     // 16 bytes (of the 16-bit output) or 32 (of a partial) of each.  Laid out by column, 16 lanes
     // store 256 consecutive bytes: the launch of three short prompts 17.5 -> 15.3 us, the step of a
     // chunk of 512 tokens in four parts (16 layers) 944 -> 920.
-    if (kAppends && !in_time) *late = 1;
     __syncthreads();   // the stages have been read by everybody
     if (kAppends && __builtin_amdgcn_readfirstlane(*late)) return false;
     char *const rows_lds = lds_base + wave * kRowsOutBytes;
@@ -783,17 +807,29 @@ __device__ __forceinline__ bool prefill_attn_body(
     return true;
 }
 
-// A tile whose new rows did not come in time: its workgroup appends its request's rows of its kv head itself.
+// A walk that ended before a block with new rows: its workgroup leaves its share of the launch's rows, in case the
+// walk had not come to that, and appends all of its request's of its kv head.
 template <int DT, int kWaves>
 __device__ __forceinline__ void append_for_tile(const_prefill_ptr a, int wg, int wave)
 {
     asm volatile("" : "+s"(a));
-    const int n_kv_heads = a->n_kv_heads, b = a->tile_info[(long)(wg / n_kv_heads) * kTileWords];
+    const const_append_ptr append = (const_append_ptr)a;
+    const int n_kv_heads = a->n_kv_heads, page_shift = a->page_shift, tile = wg / n_kv_heads, kvh = wg % n_kv_heads;
+    const int b = a->tile_info[(long)tile * kTileWords];
     const int q_begin = a->qo_indptr[b], n_b = a->qo_indptr[b + 1] - q_begin;
-    const int page_begin = a->kv_indptr[b];   // it has pages: the tile has walked them
-    const long kv_len = ((long)(a->kv_indptr[b + 1] - page_begin - 1) << a->page_shift) + a->kv_last[b];
+    const int page_begin = a->kv_indptr[b];   // it has pages: the tile sees tokens
+    const int kv_len = ((a->kv_indptr[b + 1] - page_begin - 1) << page_shift) + a->kv_last[b];
+    AppendShare<DT, kWaves> share;
+    share.request(append, tile, kvh, n_kv_heads, wave, a->qo_indptr, a->kv_indptr, a->kv_last, q_begin, n_b, page_begin,
+                  kv_len, a->kv_indices, page_shift, a->rope);
+    share.look_up(append, wave, a->kv_indices, page_shift, a->rope);
+    share.store(append, a->pages, page_shift, n_kv_heads * kHeadDim * 2, kvh, a->rope != nullptr);
     append_request<DT, kWaves>(a->append.k, a->append.v, a->append.num_pages, q_begin, n_b, kv_len, a->pages,
-                               a->kv_indices + page_begin, wg % n_kv_heads, n_kv_heads, a->page_shift, a->rope, wave);
+                               a->kv_indices + page_begin, kvh, n_kv_heads, page_shift, a->rope, wave);
+    if (wave > 0 || lane_id() > 0) return;
+    __hip_atomic_fetch_add(a->append.flags + kAppendFlags, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tile < a->append.n_tiles)
+        __hip_atomic_store(a->append.flags + (long)tile * n_kv_heads + kvh, a->append.launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 #ifndef DSKV_PREFILL_MIN_WAVES

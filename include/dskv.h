@@ -397,9 +397,13 @@ int dskv_mixed_layers(const dskv_mixed_step_t *step, int32_t n_layers, void *out
  * layers of them at multiples of 256 bytes, a stream that is not being captured; elsewhere, and with
  * append_flags null or fewer words, it is dskv_mixed_layers.  Pages and output have the same bits either way.
  * polls: how often a query tile looks for rows that other workgroups append before it appends them itself (0:
- * the library's number).  Calls on several streams may share the words: their launches then append
- * some rows twice.
+ * the library's number, about 100 us of looking); with DSKV_APPEND_ODD_LATE added, every other plan entry does not look
+ * at all, so that a test meets both kinds of tile.  The last word counts the walks that began again for it.
+ * Calls on several streams may share the words; a tile that misses its flag because the other call's
+ * number overwrote it looks in vain for that long, appends its request's rows once more and walks its context
+ * twice.
  */
+#define DSKV_APPEND_ODD_LATE (1 << 30)
 int64_t dskv_append_flags(void);
 int dskv_mixed_layers_flagged(const dskv_mixed_step_t *step, uint32_t *append_flags, int64_t n_append_flags,
                               int32_t polls, int32_t n_layers, void *out, const void *q, const void *k_new,

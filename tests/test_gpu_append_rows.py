@@ -3,8 +3,8 @@ launch of its own: the same bits in pages and result.  Edges: the first new row 
 blocks and of the four blocks between two waits, parts, one and two rounds of tokens per wave, empty shares, 63
 requests, groups and head counts that leave waves idle, pages of 4 tokens; and what keeps the launch in front:
 new rows within a walk's first twelve blocks, pages of 2 tokens, too many tokens, 64 requests, decode rows
-beside, a pool that is not at a multiple of 256 bytes, a captured stream.  With one look at the flags only,
-tiles append for themselves."""
+beside, a pool that is not at a multiple of 256 bytes, a captured stream.  Tiles that find no flag raised -
+every other plan entry does not look - append for themselves and walk again, beside tiles that wait."""
 import ctypes
 import math
 
@@ -27,6 +27,7 @@ CASES = {   # kv_lens, qo_lens, page, Hq, Hkv, dtype, route, whether the tiles a
     "page4": (*_over([400, 390], [50, 9]), 4, 16, 4, "f16", AUTO, True),
     "too_near": (*_over([383, 500], [30, 20]), 16, 32, 8, "bf16", AUTO, False),
     "prompts": ([17, 203, 1], [17, 203, 1], 4, 32, 8, "f16", AUTO, False),
+    "short_prompts": ([17, 30, 9], [17, 30, 9], 4, 32, 8, "f16", AUTO, False),
     "chunk": (*_over([4096], [512]), 16, 32, 8, "bf16", AUTO, True),
     "two_rounds": (*_over([3000], [901]), 8, 32, 8, "bf16", AUTO, True),
     "parts": (*_over([1700, 2360], [60, 40]), 16, 32, 8, "bf16", AUTO, True),
@@ -86,6 +87,46 @@ def test_same_bits_as_an_append_in_front(case):
             torch.cuda.synchronize()
             assert torch.equal(_bits(pages), _bits(want_pages)) and torch.equal(_bits(got), _bits(want)), polls
     assert bool(w._flags.any()) == CASES[case][-1]
+
+
+@pytest.mark.parametrize("case", [c for c in CASES if CASES[c][-1]])
+def test_tiles_that_do_not_look_beside_tiles_that_wait(case):
+    """The last word of the flags counts the second walks: one for each workgroup of an odd plan entry that
+    meets new rows, none for the others."""
+    print("[case] append rows, odd entries late", case, *CASES[case], flush=True)
+    w, q, k, v, fresh, table = _setup(case)
+    kv, qo, _, _, Hkv = CASES[case][:5]
+    entries = w._tiles.cpu().numpy()[: 6 * w._n_tiles].reshape(-1, 6)
+    meet = np.array([32 * int(e[3]) > kv[e[0]] - qo[e[0]] for e in entries])   # (whole walks end far beyond)
+    want_pages = fresh.clone()
+    want = _call(w, q, k, v, want_pages, table, None, 0)
+    for polls in (_lib.APPEND_ODD_LATE, _lib.APPEND_ODD_LATE, _lib.APPEND_ODD_LATE | 1):
+        pages, before = fresh.clone(), int(w._flags[-1])
+        got = _call(w, q, k, v, pages, table, w._flags, polls)
+        torch.cuda.synchronize()
+        assert torch.equal(_bits(pages), _bits(want_pages)) and torch.equal(_bits(got), _bits(want)), polls
+        walks = int(w._flags[-1]) - before
+        assert walks >= Hkv * int(meet[1::2].sum())
+        if polls == _lib.APPEND_ODD_LATE:
+            assert walks == Hkv * int(meet[1::2].sum())
+    assert meet[1::2].any()
+
+
+@pytest.mark.parametrize("case", ["too_near", "short_prompts", "part_of_new_rows_only"])
+def test_walks_that_begin_with_new_rows_although_the_plan_says_late(case):
+    """The lengths that count are the device's: such a walk leaves its share and appends for itself."""
+    print("[case] append rows, not late", case, *CASES[case], flush=True)
+    w, q, k, v, fresh, table = _setup(case)
+    want_pages = fresh.clone()
+    want = _call(w, q, k, v, want_pages, table, None, 0)
+    assert not w._info.new_rows_late
+    w._info.new_rows_late = 1
+    pages = fresh.clone()
+    got = _call(w, q, k, v, pages, table, w._flags, 0)
+    torch.cuda.synchronize()
+    assert torch.equal(_bits(pages), _bits(want_pages)) and torch.equal(_bits(got), _bits(want))
+    # eight blocks are requested before the first look: 383 tokens of context are more
+    assert bool(w._flags[-1]) == (case != "too_near")
 
 
 def test_a_pool_between_cache_lines_and_a_captured_stream():
