@@ -118,6 +118,7 @@ _SIGNATURES = {
     "dskv_mixed_step": (c_int32, [POINTER(MixedStep)] + [c_void_p] * 6),
     "dskv_mixed_layers": (c_int32, [POINTER(MixedStep), c_int32] + [c_void_p] * 5 + [c_int64, c_void_p]),
     "dskv_append_flags": (c_int64, []),
+    "dskv_new_rows_apart": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int32]),
     "dskv_mixed_layers_flagged": (c_int32, [POINTER(MixedStep), c_void_p, c_int64, c_int32, c_int32] + [c_void_p] * 5 +
                                   [c_int64, c_void_p]),
     "dskv_apply_rope": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,

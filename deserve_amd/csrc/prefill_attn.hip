@@ -33,6 +33,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <new>
 #include <vector>
 
 #include "prefill_kernel.h"
@@ -941,6 +942,52 @@ static int mixed_step(const dskv_mixed_step_t &s, void *out, const void *q, cons
 }
 
 }  // namespace dskv
+
+// A batch's pages that take new rows are few; every other entry of the tables passes a filter of 8192 bits first.
+extern "C" int dskv_new_rows_apart(const int32_t *qo_indptr_host, const int32_t *kv_page_indptr_host,
+                                   const int32_t *kv_last_page_len_host, const int32_t *kv_page_indices_host,
+                                   int32_t batch, int32_t page_size)
+{
+    using namespace dskv;
+    if (batch <= 0) return 1;
+    if (!qo_indptr_host || !kv_page_indptr_host || !kv_last_page_len_host || !kv_page_indices_host || page_size <= 0) return 0;
+    // entries [first, end) of request b's table take its new rows
+    auto first_new = [&](int32_t b, int64_t end) {
+        const int64_t n_b = (int64_t)qo_indptr_host[b + 1] - qo_indptr_host[b];
+        if (n_b <= 0) return end;
+        const int64_t prior = (end - 1) * page_size + kv_last_page_len_host[b] - n_b;
+        return std::min(end, std::max<int64_t>(prior, 0) / page_size);
+    };
+    try {
+        std::vector<int32_t> taking;
+        for (int pass = 0; pass < 2; pass++) {
+            uint64_t filter[128] = {};
+            for (const int32_t id : taking) filter[(uint32_t)id / 64 % 128] |= 1ull << ((uint32_t)id % 64);
+            for (int32_t b = 0; b < batch; b++) {
+                const int32_t *table = kv_page_indices_host + kv_page_indptr_host[b];
+                const int64_t end = (int64_t)kv_page_indptr_host[b + 1] - kv_page_indptr_host[b];
+                if (end <= 0) continue;
+                const int64_t first = first_new(b, end);
+                if (pass == 0) {
+                    taking.insert(taking.end(), table + first, table + end);
+                    continue;
+                }
+                for (int64_t i = 0; i < first; i++) {
+                    const uint32_t id = (uint32_t)table[i];
+                    if ((filter[id / 64 % 128] >> (id % 64) & 1) && std::binary_search(taking.begin(), taking.end(), table[i]))
+                        return 0;
+                }
+            }
+            if (pass == 0) {
+                std::sort(taking.begin(), taking.end());
+                if (std::adjacent_find(taking.begin(), taking.end()) != taking.end()) return 0;
+            }
+        }
+    } catch (const std::bad_alloc &) {
+        return 0;
+    }
+    return 1;
+}
 
 extern "C" int64_t dskv_append_flags(void) { return dskv::kAppendFlags + 1; }
 

@@ -124,6 +124,7 @@ class _PagedWrapper:
         self._flags = None
         self._max_page_id = -1
         self._empty_requests = []
+        self._ids: Optional[np.ndarray] = None      # entries of the block tables, from their check to the plan
 
     def _shape_args(self, num_qo_heads: int, num_kv_heads: int, head_dim: int, page_size: int,
                     data_type=None) -> None:
@@ -139,11 +140,11 @@ class _PagedWrapper:
         return src.to(torch.int32).contiguous()
 
     def _check_block_tables(self, h_indptr: torch.Tensor, indices: torch.Tensor,
-                            indices_host: Optional[torch.Tensor], h_last: torch.Tensor) -> None:
+                            indices_host: Optional[torch.Tensor], h_last: torch.Tensor) -> np.ndarray:
         """The kernels index the pool by block-table entries: refuse, on the host, tables that
         are shorter than indptr says or hold a negative id, last-page lengths that are missing
         or outside [1, page_size], and remember the largest id so that forward() can refuse a
-        pool that does not have that page."""
+        pool that does not have that page.  Returns the ids that are used, on the host."""
         ptr = h_indptr.numpy()
         batch = ptr.shape[0] - 1
         used = int(ptr[-1]) if batch > 0 else 0
@@ -168,6 +169,7 @@ class _PagedWrapper:
             if lo < 0:
                 raise ValueError(f"negative page id {lo} in the block tables")
             self._max_page_id = hi
+        return ids
 
     def _check_pool(self, paged_kv_data: torch.Tensor, dtype: torch.dtype) -> None:
         want, shape = (2, self._p, self._hkv, self._d), paged_kv_data.shape
@@ -485,7 +487,7 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
             raise ValueError("qo_indptr must start at 0 and not decrease")
         if h_kv.shape[0] != h_qo.shape[0]:
             raise ValueError("qo_indptr and paged_kv_indptr disagree about the batch")
-        self._check_block_tables(h_kv, indices, indices_host, h_last)
+        self._ids = self._check_block_tables(h_kv, indices, indices_host, h_last)
         nnz = int(h_qo[-1]) if batch > 0 else 0
         total_tokens = int(h_kv[-1]) * self._p if batch > 0 else 0
         return int(_lib.lib().dskv_mixed_plan_bound(batch, nnz, total_tokens))
@@ -507,6 +509,10 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
             _lib.check(rc, "prefill begin_forward")
             if info.tile_workspace_bytes + info.decode_workspace_bytes <= ws_bytes:
                 break
+        ids, self._ids = self._ids, None
+        if info.new_rows_late and (ids is None or not _lib.lib().dskv_new_rows_apart(
+                h_qo.data_ptr(), h_kv.data_ptr(), h_last.data_ptr(), ids.ctypes.data, batch, self._p)):
+            info.new_rows_late = 0      # a tile waits for its own request's rows only
         self._batch, self._nnz = batch, (int(h_qo[-1]) if batch > 0 else 0)
         self._info = info
         self._n_tiles, self._n_splits = info.n_tiles, info.n_splits
@@ -582,7 +588,7 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
                 rope_table: Optional[torch.Tensor] = None, **_ignored) -> torch.Tensor:
         """out: optional result tensor (contiguous, q's shape and dtype); every row is written.
         k_append, v_append (nnz, Hkv, D): the step's tokens, not yet in the pages - the call
-        appends them first (see fused_append_supported).
+        appends them, as if before anything else (see fused_append_supported).
         rope_table (with k_append / v_append): rope_table() of their positions; q and k_append are
         then taken unrotated, k_append is rotated on its way into the pages and q as the attention
         loads it."""

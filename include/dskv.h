@@ -395,7 +395,10 @@ int dskv_mixed_layers(const dskv_mixed_step_t *step, int32_t n_layers, void *out
  * attention launch append the step's rows itself, without a launch in front of it: a plan of tiles only
  * with new_rows_late, at most 32 new tokens for each of its first entries, fewer than 64 requests, pages of at least 4 tokens, pages and
  * layers of them at multiples of 256 bytes, a stream that is not being captured; elsewhere, and with
- * append_flags null or fewer words, it is dskv_mixed_layers.  Pages and output have the same bits either way.
+ * append_flags null or fewer words, it is dskv_mixed_layers.  Pages and output have the same bits either way, provided
+ * that no page that takes new rows is named twice in the step's tables: a tile waits for its own request's
+ * rows only.  dskv_new_rows_apart tells from the host's arrays (1: none is); where it returns 0, clear
+ * info->new_rows_late.
  * polls: how often a query tile looks for rows that other workgroups append before it appends them itself (0:
  * the library's number, about 100 us of looking); with DSKV_APPEND_ODD_LATE added, every other plan entry does not look
  * at all, so that a test meets both kinds of tile.  The last word counts the walks that began again for it.
@@ -404,6 +407,9 @@ int dskv_mixed_layers(const dskv_mixed_step_t *step, int32_t n_layers, void *out
  * twice.
  */
 #define DSKV_APPEND_ODD_LATE (1 << 30)
+int dskv_new_rows_apart(const int32_t *qo_indptr_host, const int32_t *kv_page_indptr_host,
+                        const int32_t *kv_last_page_len_host, const int32_t *kv_page_indices_host,
+                        int32_t batch, int32_t page_size);
 int64_t dskv_append_flags(void);
 int dskv_mixed_layers_flagged(const dskv_mixed_step_t *step, uint32_t *append_flags, int64_t n_append_flags,
                               int32_t polls, int32_t n_layers, void *out, const void *q, const void *k_new,

@@ -129,6 +129,31 @@ def test_walks_that_begin_with_new_rows_although_the_plan_says_late(case):
     assert bool(w._flags[-1]) == (case != "too_near")
 
 
+def test_one_sequence_handed_in_as_two_requests():
+    """The second request attends to rows that the first one appends."""
+    from deserve_amd.paged_ops import BatchPrefillWithPagedKVCacheWrapper
+
+    print("[case] append rows, one sequence as two requests", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    dev = lambda a: torch.tensor(a, dtype=torch.int32, device="cuda")
+    table = torch.randperm(60, generator=g, device="cuda").int()
+    w = BatchPrefillWithPagedKVCacheWrapper(torch.empty(64 << 20, dtype=torch.uint8, device="cuda"))
+    w.begin_forward(dev([0, 60, 100]), dev([0, 48, 98]), torch.cat([table[:48], table[:50]]), dev([8, 16]), 32, 8, 128, 16)
+    q, k, v, fresh = rand(100, 32, 128), rand(100, 8, 128), rand(100, 8, 128), rand(60, 2, 16, 8, 128)
+    want_pages, pages = fresh.clone(), fresh.clone()
+    want = _call(w, q, k, v, want_pages, None, None, 0)
+    got = w.forward(q, pages, k_append=k, v_append=v)
+    torch.cuda.synchronize()
+    assert not bool(w._flags.any())
+    assert torch.equal(_bits(pages), _bits(want_pages)) and torch.equal(_bits(got), _bits(want))
+    one = BatchPrefillWithPagedKVCacheWrapper(torch.empty(64 << 20, dtype=torch.uint8, device="cuda"))
+    one.begin_forward(dev([0, 100]), dev([0, 50]), table[:50], dev([16]), 32, 8, 128, 16)
+    whole = one.forward(q, fresh.clone(), k_append=k, v_append=v)
+    # the same sums in another order: two roundings to bf16 of values below 1
+    assert float((whole.float() - got.float()).abs().max()) <= 2 * 2.0 ** -8
+
+
 def test_a_pool_between_cache_lines_and_a_captured_stream():
     print("[case] append rows, odd pool and capture", flush=True)
     w, q, k, v, fresh, table = _setup("block_edges")
