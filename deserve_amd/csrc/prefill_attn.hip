@@ -898,8 +898,16 @@ namespace dskv {
 // Whether a step's attention launch appends the step's rows itself: tiles only (decode workgroups beside
 // them, or a decode pass in front, would need theirs before), loaded straight into LDS, which meet new rows
 // late, and few enough tokens for the first tiles' workgroups.  Rows have to be whole cache lines: see append_rows.h.
-static bool tiles_append(const dskv_mixed_step_t &s, const void *k, const void *v, const void *pages_layer, AppendRows &a)
+// Results and partials that lie where the new rows do are written when the rows have been read by a launch before.
+static bool tiles_append(const dskv_mixed_step_t &s, const void *out, const void *k, const void *v, const void *pages_layer,
+                         AppendRows &a)
 {
+    const uintptr_t out_bytes = (uintptr_t)s.nnz * s.n_qo_heads * s.head_dim * 2;
+    const uintptr_t kv_bytes = (uintptr_t)s.nnz * s.n_kv_heads * s.head_dim * 2;
+    for (const void *rows : {k, v}) {
+        const uintptr_t at = (uintptr_t)rows, o = (uintptr_t)out, w = (uintptr_t)s.workspace;
+        if ((at < o + out_bytes && o < at + kv_bytes) || (at < w + s.workspace_bytes && w < at + kv_bytes)) return false;
+    }
     if (!s.info->new_rows_late || s.page_size < 4 || s.info->n_decode_rows > 0 || s.info->n_tiles <= 0 || s.batch > kAppendMaxBatch ||
         s.n_kv_heads > kAppendFlags || ((uintptr_t)pages_layer % 256) || (((uintptr_t)k | (uintptr_t)v) % 16))
         return false;
@@ -916,7 +924,7 @@ static int mixed_step(const dskv_mixed_step_t &s, void *out, const void *q, cons
         DSKV_REQUIRE(pages_layer && k_new && v_new && s.qo_indptr && s.kv_page_indices && s.kv_page_indptr &&
                          s.kv_last_page_len, "append: null pointer argument");
         DSKV_REQUIRE(s.num_pages > 0, "append: num_pages must be positive, got %d", s.num_pages);
-        if (flags && tiles_append(s, k_new, v_new, pages_layer, append)) {
+        if (flags && tiles_append(s, out, k_new, v_new, pages_layer, append)) {
             static std::atomic<uint32_t> launches{0};
             while (!(append.launch = launches.fetch_add(1, std::memory_order_relaxed) + 1)) {}   // 0: a fresh buffer's
             append.k = (const uint16_t *)k_new;

@@ -154,6 +154,21 @@ def test_one_sequence_handed_in_as_two_requests():
     assert float((whole.float() - got.float()).abs().max()) <= 2 * 2.0 ** -8
 
 
+@pytest.mark.parametrize("where", ["k", "v", "workspace"])
+def test_a_result_or_partials_that_lie_where_the_new_rows_do(where):
+    """The new rows have been read before they are overwritten."""
+    print("[case] append rows, overlapping", where, flush=True)
+    w, q, k, v, fresh, table = _setup("kv17")
+    want_pages, pages = fresh.clone(), fresh.clone()
+    want = _call(w, q, k, v, want_pages, table, None, 0)
+    if where == "workspace":
+        v = w._workspace[: v.numel() * 2].view(v.dtype).view(v.shape).copy_(v)
+    got = w.forward(q, pages, out={"k": k, "v": v}.get(where), k_append=k, v_append=v, rope_table=table)
+    torch.cuda.synchronize()
+    assert not bool(w._flags.any())
+    assert torch.equal(_bits(pages), _bits(want_pages)) and torch.equal(_bits(got), _bits(want))
+
+
 def test_a_pool_between_cache_lines_and_a_captured_stream():
     print("[case] append rows, odd pool and capture", flush=True)
     w, q, k, v, fresh, table = _setup("block_edges")
