@@ -37,8 +37,8 @@ constexpr int kAppendPolls = 256;        // looks at a flag (about 0.4 us each) 
 
 struct AppendRows {
     const uint16_t *k, *v;     // (nnz, Hkv, D) new rows; null: they are in the pages already
-    uint32_t *flags;           // word tile * Hkv + kv head, raised by writing `launch` to it
-    uint32_t launch;           // a number no earlier launch with these flags had
+    uint64_t *flags;           // flag tile * Hkv + kv head, raised by writing `launch` to it
+    uint64_t launch;           // a number no earlier launch of the process had
     int n_tiles, tokens;       // plan entries that append; tokens of each
     int nnz, batch, num_pages;
     int polls[2];              // looks at a flag of plan entries of even and of odd number
@@ -175,8 +175,8 @@ struct AppendShare {
 __device__ __forceinline__ bool rows_are_there(const_append_ptr a, int tile, int first, int last, int kvh, int n_kv_heads)
 {
     asm volatile("" : "+s"(a));
-    uint32_t *const flags = a->flags;
-    const uint32_t launch = a->launch;
+    uint64_t *const flags = a->flags;
+    const uint64_t launch = a->launch;
     const int polls = a->polls[tile & 1];
     const int lane = lane_id();
     for (int f = first; f <= last; f += 64) {

@@ -917,7 +917,7 @@ static bool tiles_append(const dskv_mixed_step_t &s, const void *out, const void
 }
 
 static int mixed_step(const dskv_mixed_step_t &s, void *out, const void *q, const void *k_new, const void *v_new,
-                      void *pages_layer, uint32_t *flags, int32_t polls, void *stream)
+                      void *pages_layer, uint64_t *flags, int32_t polls, void *stream)
 {
     AppendRows append{};
     if (s.batch > 0 && s.nnz > 0) {
@@ -925,8 +925,8 @@ static int mixed_step(const dskv_mixed_step_t &s, void *out, const void *q, cons
                          s.kv_last_page_len, "append: null pointer argument");
         DSKV_REQUIRE(s.num_pages > 0, "append: num_pages must be positive, got %d", s.num_pages);
         if (flags && tiles_append(s, out, k_new, v_new, pages_layer, append)) {
-            static std::atomic<uint32_t> launches{0};
-            while (!(append.launch = launches.fetch_add(1, std::memory_order_relaxed) + 1)) {}   // 0: a fresh buffer's
+            static std::atomic<uint64_t> launches{0};
+            append.launch = launches.fetch_add(1, std::memory_order_relaxed) + 1;   // 0: a fresh buffer's
             append.k = (const uint16_t *)k_new;
             append.v = (const uint16_t *)v_new;
             append.flags = flags;
@@ -997,7 +997,7 @@ extern "C" int dskv_new_rows_apart(const int32_t *qo_indptr_host, const int32_t 
     return 1;
 }
 
-extern "C" int64_t dskv_append_flags(void) { return dskv::kAppendFlags + 1; }
+extern "C" int64_t dskv_append_flags(void) { return 2 * (dskv::kAppendFlags + 1); }
 
 extern "C" int dskv_mixed_layers_flagged(const dskv_mixed_step_t *step, uint32_t *append_flags, int64_t n_append_flags,
                                          int32_t polls, int32_t n_layers, void *out, const void *q, const void *k_new,
@@ -1015,7 +1015,7 @@ extern "C" int dskv_mixed_layers_flagged(const dskv_mixed_step_t *step, uint32_t
     // A captured launch would raise its flags with the same number in every replay, and find them raised
     if (append_flags) {
         hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        if (n_append_flags < dskv_append_flags() || hipStreamIsCapturing((hipStream_t)stream, &capture) != hipSuccess ||
+        if (n_append_flags < dskv_append_flags() || (uintptr_t)append_flags % 8 || hipStreamIsCapturing((hipStream_t)stream, &capture) != hipSuccess ||
             capture != hipStreamCaptureStatusNone) {
             (void)hipGetLastError();
             append_flags = nullptr;
@@ -1026,7 +1026,7 @@ extern "C" int dskv_mixed_layers_flagged(const dskv_mixed_step_t *step, uint32_t
     auto at = [](const void *p, int64_t bytes) { return p ? (const char *)p + bytes : nullptr; };
     for (int64_t l = 0; l < n_layers; l++) {
         const int rc = mixed_step(s, (void *)at(out, l * q_bytes), at(q, l * q_bytes), at(k_new, l * kv_bytes),
-                                  at(v_new, l * kv_bytes), (void *)at(pages, l * pages_layer_bytes), append_flags,
+                                  at(v_new, l * kv_bytes), (void *)at(pages, l * pages_layer_bytes), (uint64_t *)append_flags,
                                   polls & ~DSKV_APPEND_ODD_LATE ? polls : polls | kAppendPolls, stream);
         if (rc) return rc;
     }

@@ -827,7 +827,7 @@ __device__ __forceinline__ void append_for_tile(const_prefill_ptr a, int wg, int
     append_request<DT, kWaves>(a->append.k, a->append.v, a->append.num_pages, q_begin, n_b, kv_len, a->pages,
                                a->kv_indices + page_begin, kvh, n_kv_heads, page_shift, a->rope, wave);
     if (wave > 0 || lane_id() > 0) return;
-    __hip_atomic_fetch_add(a->append.flags + kAppendFlags, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_fetch_add(a->append.flags + kAppendFlags, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (tile < a->append.n_tiles)
         __hip_atomic_store(a->append.flags + (long)tile * n_kv_heads + kvh, a->append.launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }

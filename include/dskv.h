@@ -395,13 +395,14 @@ int dskv_mixed_layers(const dskv_mixed_step_t *step, int32_t n_layers, void *out
  * attention launch append the step's rows itself, without a launch in front of it: a plan of tiles only
  * with new_rows_late, at most 32 new tokens for each of its first entries, fewer than 64 requests, pages of at least 4 tokens, pages and
  * layers of them at multiples of 256 bytes, a stream that is not being captured; elsewhere, and with
- * append_flags null or fewer words, it is dskv_mixed_layers.  Pages and output have the same bits either way, provided
+ * append_flags null, not 8-byte aligned or of fewer words, it is dskv_mixed_layers.  Pages and output have the same bits either way, provided
  * that no page that takes new rows is named twice in the step's tables: a tile waits for its own request's
  * rows only.  dskv_new_rows_apart tells from the host's arrays (1: none is); where it returns 0, clear
  * info->new_rows_late.
  * polls: how often a query tile looks for rows that other workgroups append before it appends them itself (0:
  * the library's number, about 100 us of looking); with DSKV_APPEND_ODD_LATE added, every other plan entry does not look
- * at all, so that a test meets both kinds of tile.  The last word counts the walks that began again for it.
+ * at all, so that a test meets both kinds of tile.  The last eight bytes count the walks that began again
+ * for it, the others hold 64-bit numbers of launches.
  * Calls on several streams may share the words; a tile that misses its flag because the other call's
  * number overwrote it looks in vain for that long, appends its request's rows once more and walks its context
  * twice.

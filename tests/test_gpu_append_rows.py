@@ -73,6 +73,10 @@ def _bits(t):
     return t.view(torch.int16)
 
 
+def _numbers(w):
+    return w._flags.view(torch.int64).tolist()
+
+
 @pytest.mark.parametrize("case", CASES)
 def test_same_bits_as_an_append_in_front(case):
     print("[case] append rows", case, *CASES[case], flush=True)
@@ -89,9 +93,26 @@ def test_same_bits_as_an_append_in_front(case):
     assert bool(w._flags.any()) == CASES[case][-1]
 
 
+def test_flags_are_64_bit_numbers_of_launches():
+    """They do not come round: each launch's is the one before's plus one, in words of its own."""
+    print("[case] append rows, numbers of launches", flush=True)
+    w, q, k, v, fresh, table = _setup("block_edges")
+    seen = []
+    for _ in range(3):
+        _call(w, q, k, v, fresh, table, w._flags, 0)
+        raised = {n for n in _numbers(w)[:-1] if n}
+        assert len(raised) == 1
+        seen.append(raised.pop())
+    assert seen == [seen[0], seen[0] + 1, seen[0] + 2] and 0 < seen[0] < 1 << 32
+    odd = torch.zeros(w._flags.numel() + 1, dtype=torch.int32, device="cuda")[1:]
+    _call(w, q, k, v, fresh, table, odd, 0)
+    _call(w, q, k, v, fresh, table, odd[1:], 0)      # too few
+    assert not bool(odd.any())
+
+
 @pytest.mark.parametrize("case", [c for c in CASES if CASES[c][-1]])
 def test_tiles_that_do_not_look_beside_tiles_that_wait(case):
-    """The last word of the flags counts the second walks: one for each workgroup of an odd plan entry that
+    """The last number of the flags counts the second walks: one for each workgroup of an odd plan entry that
     meets new rows, none for the others."""
     print("[case] append rows, odd entries late", case, *CASES[case], flush=True)
     w, q, k, v, fresh, table = _setup(case)
@@ -101,11 +122,11 @@ def test_tiles_that_do_not_look_beside_tiles_that_wait(case):
     want_pages = fresh.clone()
     want = _call(w, q, k, v, want_pages, table, None, 0)
     for polls in (_lib.APPEND_ODD_LATE, _lib.APPEND_ODD_LATE, _lib.APPEND_ODD_LATE | 1):
-        pages, before = fresh.clone(), int(w._flags[-1])
+        pages, before = fresh.clone(), _numbers(w)[-1]
         got = _call(w, q, k, v, pages, table, w._flags, polls)
         torch.cuda.synchronize()
         assert torch.equal(_bits(pages), _bits(want_pages)) and torch.equal(_bits(got), _bits(want)), polls
-        walks = int(w._flags[-1]) - before
+        walks = _numbers(w)[-1] - before
         assert walks >= Hkv * int(meet[1::2].sum())
         if polls == _lib.APPEND_ODD_LATE:
             assert walks == Hkv * int(meet[1::2].sum())
@@ -126,7 +147,7 @@ def test_walks_that_begin_with_new_rows_although_the_plan_says_late(case):
     torch.cuda.synchronize()
     assert torch.equal(_bits(pages), _bits(want_pages)) and torch.equal(_bits(got), _bits(want))
     # eight blocks are requested before the first look: 383 tokens of context are more
-    assert bool(w._flags[-1]) == (case != "too_near")
+    assert bool(_numbers(w)[-1]) == (case != "too_near")
 
 
 def test_one_sequence_handed_in_as_two_requests():
