@@ -39,8 +39,11 @@ class PagedAttentionCore:
         """paged_forward for the layers ctx.layer_id .. of q, k, v and out, stacked: (L, tokens, heads, head_dim)
         each, launched by one call to the library - layer by layer from here a step of one request costs the
         host 13 us a layer, as long as the GPU works on it.  False, and nothing done, where the layers are not
-        plain stacks for the launches that append as they attend; ctx.layer_id counts on as it would."""
-        if q.dtype is torch.float32 or q.dim() != 4:     # no such launches: not worth looking further
+        plain stacks for the launches that append as they attend (fp32 has none), or a method that a layer
+        goes through has been replaced, on an object or its class: it is called for every layer then.
+        ctx.layer_id counts on as it would."""
+        if q.dtype is torch.float32 or q.dim() != 4 or _core_methods() != _CORE_METHODS or \
+                not _CORE_METHODS.keys().isdisjoint(vars(self)):
             return False
         n, first, pool = q.shape[0], ctx.layer_id, ctx.page_pool
         decode = type(ctx) is FlashDecodeCtx
@@ -48,8 +51,8 @@ class PagedAttentionCore:
             return False
         wrapper = ctx.decode_wrapper if decode else ctx.prefill_wrapper
         kind = BatchDecodeWithPagedKVCacheWrapper if decode else BatchPrefillWithPagedKVCacheWrapper
-        if type(wrapper) is not kind or "forward" in vars(wrapper) or \
-                getattr(pool.get_layered_pages, "__func__", None) is not PagePool.get_layered_pages or \
+        if type(wrapper) is not kind or "forward" in vars(wrapper) or kind.forward is not _WRAPPER_FORWARD[kind] or \
+                getattr(pool.get_layered_pages, "__func__", None) is not _LAYERED_PAGES or \
                 not 0 <= first <= pool.pages.shape[0] - n:
             return False
         pages = pool.pages[first: first + n]
@@ -113,3 +116,15 @@ class PagedAttentionCore:
         else:
             raise TypeError(f"unsupported forward context {type(ctx).__name__}")
         return out.view(-1, self.dim)
+
+
+def _core_methods() -> dict:
+    """What paged_forward goes through."""
+    core = vars(PagedAttentionCore)
+    return {name: core.get(name) for name in ("paged_forward", "_paged_forward", "_rows")}
+
+
+# as they are here: see layers_forward
+_CORE_METHODS = _core_methods()
+_WRAPPER_FORWARD = {kind: kind.forward for kind in (BatchDecodeWithPagedKVCacheWrapper, BatchPrefillWithPagedKVCacheWrapper)}
+_LAYERED_PAGES = PagePool.get_layered_pages

@@ -37,10 +37,6 @@ class KVStage:
         self.core = PagedAttentionCore(model_args.n_heads, n_kv, model_args.dim // model_args.n_heads,
                                        model_args.rope_theta, use_rope)
 
-    def _whole_core(self) -> bool:
-        """Whether no method of the core has been replaced, so that its layers may run in one call."""
-        return type(self.core) is PagedAttentionCore and not {"paged_forward", "_paged_forward"} & vars(self.core).keys()
-
     def forward(self, xs: Tuple[torch.Tensor, torch.Tensor, torch.Tensor],
                 ctx: FlashForwardCtx) -> torch.Tensor:
         """xs = (q, k, v) stacked per layer: (L, nnz, Hq, D), (L, nnz, Hkv, D) x2.
@@ -60,7 +56,7 @@ class KVStage:
         dim = self.core.dim
         result = torch.empty((q.shape[0], q[0].numel() // dim, dim), dtype=q.dtype, device=q.device)
         stacked = result.view(q.shape[0], -1, self.core.n_local_heads, self.core.head_dim)
-        if q.dtype is not torch.float32 and self._whole_core() and self.core.layers_forward(q, k, v, ctx, stacked):
+        if type(self.core) is PagedAttentionCore and self.core.layers_forward(q, k, v, ctx, stacked):
             return result
         outs = stacked.unbind(0)
         qs, ks, vs = q.unbind(0), k.unbind(0), v.unbind(0)
