@@ -1,9 +1,11 @@
-"""A stage whose layers run in one call to the library, against the same layers called one by one: the
-same bits in the result and the pages, the same layer count; what is not a plain stack goes layer
-by layer, and a pool with too few layers is refused as it is there."""
+"""A stage whose layers run in one call to the library, against the same layers called one by one (chunks with
+their append as a launch in front): the same bits in the result and the pages, the same layer count.  What is
+not a plain stack goes layer by layer, fp32 layers too, and a pool with too few layers is refused as it is there.
+"""
 import pytest
 import torch
 
+from deserve_amd import _lib
 from deserve_amd.execution.exec import BatchDecode, BatchPrefill
 from deserve_amd.stage import KVStage
 from deserve_amd.synthetic import make_mixed_workload
@@ -14,23 +16,35 @@ SHAPES = {
     "one_request": ([70], [], []),
     "decode": ([33, 600, 1, 16], [], []),
     "prompts": ([], [0, 40], [17, 5]),
+    "chunks": ([], [500, 430], [30, 20]),      # whose launches append the rows themselves
     "shared_launch": ([30 + 40 * i for i in range(14)], [20], [12]),
 }
 
 
 def _run(shape, dtype, rope, together, q_of=lambda q: q, first=0, out_layers=3):
+    """(result, pages, layer id, what layers_forward answered, whether flags were raised)."""
     wl = make_mixed_workload("t", *SHAPES[shape], 3, 16, 4, 128, 8, dtype, seed=5)
     stage = KVStage(wl.args, use_rope=rope)
-    if not together:
-        stage.core.layers_forward = lambda *a: False
+    answers, layers_forward = [], stage.core.layers_forward
+
+    def asked(*a):
+        answers.append(layers_forward(*a) if together else False)
+        return answers[-1]
+
+    stage.core.layers_forward = asked
     kind = BatchPrefill if SHAPES[shape][2] else BatchDecode
     batch = kind(None, stage, wl.tasks, wl.caches)
     batch.prepare()
     ctx = batch.prefill_ctx if SHAPES[shape][2] else batch.decode_ctx
+    flags = None
+    if SHAPES[shape][2]:
+        assert bool(ctx.prefill_wrapper._info.new_rows_late) == (shape == "chunks")
+        flags = torch.zeros(_lib.lib().dskv_append_flags(), dtype=torch.int32, device="cuda") if together else None
+        ctx.prefill_wrapper._flags = flags      # none: the append is a launch in front
     ctx.layer_id = first
     out = stage.forward((q_of(wl.q)[:out_layers], wl.k[:out_layers], wl.v[:out_layers]), ctx)
     torch.cuda.synchronize()
-    return out, wl.pool.pages, ctx.layer_id
+    return out, wl.pool.pages, ctx.layer_id, answers, flags is not None and bool(flags.any())
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
@@ -41,6 +55,8 @@ def test_layers_in_one_call_match_layers_one_by_one(shape, rope, dtype):
     for kw in ({}, {"first": 1, "out_layers": 2}):
         got, want = _run(shape, dtype, rope, True, **kw), _run(shape, dtype, rope, False, **kw)
         assert got[2] == want[2] == 3
+        assert got[3] == [dtype is not torch.float32]
+        assert got[4] == (shape == "chunks" and dtype is not torch.float32)
         for a, b in zip(got[:2], want[:2]):
             assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
 
@@ -52,6 +68,7 @@ def test_stacks_that_are_not_plain_go_layer_by_layer():
     want = _run("decode", torch.bfloat16, True, False)
     for q_of in (strided, flat):
         got = _run("decode", torch.bfloat16, True, True, q_of)
+        assert got[3] == [False]
         assert torch.equal(got[0].view(torch.int16), want[0].view(torch.int16))
         assert torch.equal(got[1].view(torch.int16), want[1].view(torch.int16))
 
