@@ -962,8 +962,9 @@ int launch_partials_merge(void *out, const float *part_o, const float *part_ml,
 {
     // rows in a few parts, 16-bit output, head_dim 128: a workgroup per (row, eight heads) that
     // requests all parts at once - half the time of a wave per (row, head) on the 512 rows of a
-    // chunk; 4.9 us on a decode batch's 64 requests in 317 parts is about what any launch that
-    // reads what the launch before it wrote takes
+    // chunk; 4.7 us on a decode batch's 64 requests in 317 parts is about what any launch that
+    // reads what the launch before it wrote takes.  Where some rows may be in more than eight parts: a workgroup per
+    // (row, two heads), whose four groups of threads take a quarter of such a row's parts each (merge_kernel.h).
     if (!wide && head_dim == kHeadDim && dtype != DSKV_F32) {
         const int heads = some_in_many ? kMergeHeadsMany : kMergeHeads;
         const dim3 grid((unsigned)rows, (unsigned)((n_qo_heads + heads - 1) / heads));

@@ -63,9 +63,12 @@ def _call(w, q, k, v, pages, table, flags, polls):
     step.rope_table = None if table is None else table.data_ptr()
     step.num_pages, step.causal, step.dtype, step.sm_scale = pages.shape[0], 1, _lib.dtype_code(q.dtype), 1 / math.sqrt(128)
     out = torch.full_like(q, float("nan"))
+    if flags is None:
+        _lib.check(_lib.lib().dskv_mixed_step(ctypes.byref(step), out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                                              pages.data_ptr(), _lib.current_stream()), "step")
+        return out
     _lib.check(_lib.lib().dskv_mixed_layers_flagged(
-        ctypes.byref(step), None if flags is None else flags.data_ptr(), 0 if flags is None else flags.numel(), polls, 1,
-        out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), pages.data_ptr(), 0, _lib.current_stream()), "step")
+        ctypes.byref(step), flags.data_ptr(), flags.numel(), polls, 1, out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), pages.data_ptr(), 0, _lib.current_stream()), "step")
     return out
 
 

@@ -1,7 +1,7 @@
 """The merge pass of rows in parts: a workgroup per (row, eight heads), a thread per four dims.  Sizes
-at its edges: rows in two to eight parts (each requested in one go), in 9, 16, 17 and 33 (sixteen at a
-time, remainders), rows without parts beside them, head counts that do not fill a workgroup or
-need several, both element types."""
+at its edges: rows in two to eight parts (each requested in one go), in 9, 16, 17 and 33 (a workgroup for every two
+heads, whose four groups of threads take a quarter each: quarters of unequal length, more than eight in one),
+rows without parts beside them, head counts that do not fill a workgroup or need several, both element types."""
 import numpy as np
 import pytest
 import torch

@@ -2,6 +2,8 @@
 their append as a launch in front): the same bits in the result and the pages, the same layer count.  What is
 not a plain stack goes layer by layer, fp32 layers too, and a pool with too few layers is refused as it is there.
 """
+import ctypes
+
 import pytest
 import torch
 
@@ -79,3 +81,33 @@ def test_more_layers_than_the_pool_has_are_refused(shape):
     for together in (True, False):
         with pytest.raises(IndexError):
             _run(shape, torch.bfloat16, True, together, first=1)
+
+
+@pytest.mark.parametrize("entry", ["mixed", "decode_fp32"])
+def test_the_librarys_calls_for_layers_match_its_calls_for_one(entry):
+    print("[case] stage layers, C entries", entry, flush=True)
+    wl = make_mixed_workload("t", *SHAPES["shared_launch" if entry == "mixed" else "decode"], 3, 16, 4, 128, 8,
+                             torch.bfloat16 if entry == "mixed" else torch.float32, seed=5)
+    batch = (BatchPrefill if entry == "mixed" else BatchDecode)(None, KVStage(wl.args, use_rope=False), wl.tasks, wl.caches)
+    batch.prepare()
+    lib, pages, stream = _lib.lib(), wl.pool.pages, _lib.current_stream()
+    ptrs = lambda *ts: [t.data_ptr() for t in ts]
+    if entry == "mixed":
+        step = _lib.MixedStep.from_buffer_copy(batch.prefill_ctx.prefill_wrapper._step)
+        step.num_pages, step.causal, step.dtype, step.sm_scale = pages.shape[1], 1, _lib.BF16, 0.1
+        one, all_layers, rows = lib.dskv_mixed_step, lib.dskv_mixed_layers, lambda l: ptrs(wl.k[l], wl.v[l])
+    else:
+        step = _lib.DecodeStep.from_buffer_copy(batch.decode_ctx.decode_wrapper._step)
+        step.dtype, step.sm_scale = _lib.F32, 0.1
+        one, all_layers, rows = lib.dskv_decode_step, lib.dskv_decode_layers, lambda l: [None, None]   # in the pages
+    fresh, want, got = pages.clone(), torch.zeros_like(wl.q), torch.zeros_like(wl.q)
+    for l in range(3):
+        _lib.check(one(ctypes.byref(step), *ptrs(want[l], wl.q[l]), *rows(l), pages[l].data_ptr(), stream), "one")
+    want_pages = pages.clone()
+    pages.copy_(fresh)
+    _lib.check(all_layers(ctypes.byref(step), 3, *ptrs(got, wl.q), *rows(slice(None)), pages.data_ptr(),
+                          pages.stride(0) * pages.element_size(), stream), "layers")
+    torch.cuda.synchronize()
+    assert bool(torch.isfinite(want).all()) and bool(want.any())
+    assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+    assert torch.equal(pages.view(torch.uint8), want_pages.view(torch.uint8))
