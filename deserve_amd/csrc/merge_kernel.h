@@ -70,7 +70,7 @@ __device__ __forceinline__ void merge_dims(uint16_t *__restrict__ dst, const flo
 //
 // kMany (a decode batch of fewer requests than shares: some may be in more than kMergeFewParts parts): such a row gets a workgroup
 // for two heads, in which four groups of threads take a quarter of the parts each, requested in one trip up to
-// 32 parts: those 128 requests 11.0 -> 7.2 us, 2415 -> 2367 us a step of 10 layers; the other rows' surplus
+// 32 parts: those 128 requests 10.9 -> 6.9 us a launch, 2406 -> 2368 us a step of 10 layers; the other rows' surplus
 // workgroups return at once (64 requests: 4.7 us either way).  A batch of many rows, none of which can have so many
 // parts (tiles), is launched without them: 512 rows of a chunk 7.1 against 7.7 us.
 constexpr int kMergeHeads = 8, kMergeHeadsMany = 2, kMergeFewParts = 8;
