@@ -43,7 +43,7 @@ class PagedAttentionCore:
         goes through has been replaced, on an object or its class: it is called for every layer then.
         ctx.layer_id counts on as it would."""
         if q.dtype is torch.float32 or q.dim() != 4 or _core_methods() != _CORE_METHODS or \
-                not _CORE_METHODS.keys().isdisjoint(vars(self)):
+                not _CORE_NAMES.isdisjoint(vars(self)):
             return False
         n, first, pool = q.shape[0], ctx.layer_id, ctx.page_pool
         decode = type(ctx) is FlashDecodeCtx
@@ -118,13 +118,13 @@ class PagedAttentionCore:
         return out.view(-1, self.dim)
 
 
-def _core_methods() -> dict:
+def _core_methods() -> tuple:
     """What paged_forward goes through."""
-    core = vars(PagedAttentionCore)
-    return {name: core.get(name) for name in ("paged_forward", "_paged_forward", "_rows")}
+    return PagedAttentionCore.paged_forward, PagedAttentionCore._paged_forward, PagedAttentionCore._rows
 
 
 # as they are here: see layers_forward
+_CORE_NAMES = {"paged_forward", "_paged_forward", "_rows"}
 _CORE_METHODS = _core_methods()
 _WRAPPER_FORWARD = {kind: kind.forward for kind in (BatchDecodeWithPagedKVCacheWrapper, BatchPrefillWithPagedKVCacheWrapper)}
 _LAYERED_PAGES = PagePool.get_layered_pages
