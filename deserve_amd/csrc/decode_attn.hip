@@ -618,6 +618,43 @@ static bool gqa_splitting_pays(int64_t tiles, int64_t longest, int batch, int n_
     return work <= 2048 && pairs <= most_pairs;
 }
 
+// Shares of a batch whose tiles are split over the waves of workgroups (splitting_pays), as the global tile at which each
+// ends, at most `most` of them.  Uncut, requests lie whole in a share, several of them as long as they fit into `cap`
+// tiles; cut, longer ones get shares of their own.
+static int64_t lay_out_shares(const std::vector<int64_t> &tiles, int64_t cap, bool cut, std::vector<int64_t> *ends)
+{
+    int64_t at = 0, filled = 0, shares = 0;
+    auto end_share = [&](int64_t end) {
+        shares++;
+        if (ends) ends->push_back(end);
+    };
+    for (const int64_t n : tiles) {
+        if (n == 0) continue;
+        if (filled && filled + n > cap) {
+            end_share(at);
+            filled = 0;
+        }
+        const int64_t parts = cut ? (n + cap - 1) / cap : 1;
+        if (parts > 1)
+            for (int64_t p = 1; p <= parts; p++) end_share(at + n * p / parts);
+        else
+            filled += n;
+        at += n;
+    }
+    if (filled) end_share(at);
+    return shares;
+}
+// The smallest cap (at least lo) with which they are at most `most`.
+static int64_t smallest_cap(const std::vector<int64_t> &tiles, int64_t lo, int64_t hi, int64_t most, bool cut)
+{
+    while (lo < hi) {
+        const int64_t mid = (lo + hi) / 2;
+        if (lay_out_shares(tiles, mid, cut, nullptr) <= most) hi = mid;
+        else lo = mid + 1;
+    }
+    return lo;
+}
+
 // The planner proper.  reqs[i]: tokens, start of the block table and q / output row of
 // request i (row i itself for a decode batch).
 int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, int32_t n_kv_heads,
@@ -635,8 +672,7 @@ int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, i
     }
     // Share count: one per CU unless told otherwise, fewer when there is so little work that a
     // share would drop below a few tiles.  Batches for which splitting pays get so few that the
-    // attention runs as one workgroup per (share, kv head), shares of six tiles at least: one request
-    // of 112 tiles takes 13.1 us in 18 shares (14.0 in 28), three of 13 tiles 10.7 in 9 (13.0 in 4).
+    // attention runs as one workgroup per (share, kv head).
     // The launcher knows that form by the number of workgroups (decode_splits_tokens), so a plan for
     // the other one is filled up with workgroups that have nothing to do where it would pass for it.
     // (the generic kernel's forms likewise: gqa_splits_tokens)
@@ -649,10 +685,29 @@ int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, i
                             ? splitting_pays(total_tiles, longest, batch, n_kv_heads, n_qo_heads / n_kv_heads, merges_itself)
                             : gqa_splitting_pays(total_tiles, longest, batch, n_kv_heads, head_dim));
     int64_t wgs = own_rule ? default_workgroups() : target_workgroups;
-    if (split && head_dim == kHeadDim)
+    const bool few_shares = split && mfma_path(dtype, head_dim, n_qo_heads, n_kv_heads);
+    if (few_shares)
+        wgs /= n_kv_heads;
+    else if (split && head_dim == kHeadDim)
         wgs = std::min<int64_t>(wgs / n_kv_heads, std::max<int64_t>(1, total_tiles / kSplitTilesPerShare));
     wgs = std::min<int64_t>(wgs, kMaxWorkgroups);
-    wgs = std::min<int64_t>(wgs, std::max<int64_t>(1, total_tiles / kMinTilesPerWorkgroup));
+    if (!few_shares) wgs = std::min<int64_t>(wgs, std::max<int64_t>(1, total_tiles / kMinTilesPerWorkgroup));
+    // In such a batch a share is one round of its waves (a tile each) as long as there are shares for it, and a
+    // request is not cut where two rounds of whole ones do, since merging costs more than a round.  Layers in a replayed graph,
+    // us, 8 kv heads: one request of 16 tiles whole 7.1 / cut 7.4-7.6, of 19 tiles 8.8 / 7.5, of 26 10.5 / 7.6; of 112
+    // tiles in 14 shares 9.2 / in 18 of six tiles 10.0; 8 requests of 7 tiles whole 6.1 / in equal shares 7.7; 16 of 13
+    // tiles 8.4 / 8.8; 32 of 4-13 tiles 9.1 / 10.6.  Where the rounds become many, equal shares count for more.
+    std::vector<int64_t> ends;
+    if (few_shares && total_tiles > 0) {
+        const int64_t most = wgs, even = (total_tiles + most - 1) / most;
+        const int64_t whole = smallest_cap(tiles, std::max<int64_t>(longest, kSplitWaves), std::max<int64_t>(total_tiles, kSplitWaves), most, false);
+        const int64_t cut = smallest_cap(tiles, std::max<int64_t>(even, kSplitWaves), std::max<int64_t>(total_tiles, kSplitWaves), most, true);
+        auto rounds = [](int64_t n) { return (n + kSplitWaves - 1) / kSplitWaves; };
+        const bool uncut = rounds(whole) <= rounds(cut) + 1;
+        if (uncut || rounds(cut) == 1) wgs = lay_out_shares(tiles, uncut ? whole : cut, !uncut, &ends);
+    } else if (few_shares) {
+        wgs = 1;
+    }
     int64_t launched = wgs;
     if (own_rule && two_forms && !split) launched = std::max<int64_t>(wgs, default_workgroups() / n_kv_heads + 1);
 
@@ -663,7 +718,7 @@ int plan_decode_rows(const DecodeRow *reqs, int32_t batch, int32_t n_qo_heads, i
     std::vector<int32_t> wg_ptr(1, 0), req(2 * (size_t)batch, 0);
     int32_t n_slots = 0;
     int64_t w = 0, g0 = 0, share_begin = 0;       // current workgroup, global tile index, its share's first
-    auto share_end = [&](int64_t wg) { return (wg + 1) * total_tiles / wgs; };
+    auto share_end = [&](int64_t wg) { return ends.empty() ? (wg + 1) * total_tiles / wgs : ends[wg]; };
     for (int b = 0; b < batch; b++) {
         const int64_t len = reqs[b].len;
         if (tiles[b] == 0) {
@@ -855,12 +910,14 @@ static int decode_attn_impl(void *out, const void *q, const void *pages_layer,
             // (a request in dozens of parts: one workgroup takes longer over them than the launch of the
             // eight-wave merge, 35.7 against 16.9 us for 250 parts, 16.0 against 13.0 for 62)
             merged = merge_counters && phases == 3 && n_items <= kWideMergeParts * (int64_t)batch;
-            const SplitArgs args = {(uint16_t *)out, (const uint16_t *)q, (const char *)pages_layer, kv_page_indices,
-                                    items, wg_ptr, part_o, part_ml, (int)max_slots, n_qo_heads, n_kv_heads, shift,
-                                    scale_log2, (const uint16_t *)k_new, (const uint16_t *)v_new, rope_table,
+            // (a plan's slots are fewer than two per share)
+            const int split_slots = (int)std::min<int64_t>(max_slots, 2 * (int64_t)n_workgroups);
+            const SplitArgs args = {(const char *)pages_layer, kv_page_indices, items, wg_ptr, (const uint16_t *)q, rope_table,
+                                    (const uint16_t *)k_new, (const uint16_t *)v_new, n_qo_heads, n_kv_heads,
+                                    n_qo_heads / n_kv_heads, shift, scale_log2, split_slots, part_o, part_ml,
                                     merged && n_items > batch ? merge_counters : nullptr,
-                                    (int)std::min<int64_t>(n_merge_counters, 1 << 30), n_workgroups};
-            const dim3 grid((unsigned)split_launch_workgroups(n_workgroups, n_kv_heads)), block(64 * kSplitWaves);
+                                    (int)std::min<int64_t>(n_merge_counters, 1 << 30), 0, (uint16_t *)out};
+            const dim3 grid((unsigned)n_workgroups, (unsigned)n_kv_heads), block(64 * kSplitWaves);
 #define DSKV_LAUNCH_SPLIT(DT, COVER) \
     hipLaunchKernelGGL((decode_attn_split_kernel<DT, COVER>), grid, block, 0, s, args)
             if (dtype == DSKV_BF16) {

@@ -4,12 +4,16 @@
 //
 // What bounds it: latency.  A step over 7 MB of K/V (one request of 1777 tokens) needs 1 us of
 // HBM time; what lasts is the chain plan -> page id -> tile -> result and everything that hangs
-// behind it.  With workgroups of one wave per kv head (decode_kernel.h) that request is cut into
+// behind it, and in that chain the instructions: a wave that depends on itself issues one every five to ten cycles
+// and fetches most of them for the first time, so everything that is executed once counts.  With
+// workgroups of one wave per kv head (decode_kernel.h) that request is cut into
 // 28 parts of four tiles, walked one after the other, and merged by a second launch that takes
 // nearly as long (14.5 + 11.3 us by rocprofv3; 20.5 us per layer in a replayed graph).  Here a wave
-// walks one tile or two, eight waves meet in LDS, the request has 18 parts, and the part that
-// finishes last merges them in the same launch: 13.1 us.  8 requests of 512 tokens: 19.3 -> 13.0 us,
-// 8 of 300-1100: 24.3 -> 14.7, 24 of 64-2048: 35 -> 28.
+// walks one tile or two, eight waves meet in LDS, and the part that
+// finishes last merges the request's parts in the same launch: 9.2 us a layer in a replayed graph, 8 requests
+// of 512 tokens 9.2, 8 of 300-1100 11.3, 24 of 64-2048 23.0, 32 of 60-200 9.1 (13.1, 12.9, 15.1, 25.6 and 14.4 while
+// the code in front of the first tile and behind the last one was three times as long and shares were cut
+// without regard to the requests).
 //
 // A wave owns a slice of the share's tile stream, which may cross requests: the pieces it
 // computes are whole items (it writes them itself), or the two ends of items that reach into its
@@ -24,7 +28,6 @@ constexpr int kSplitWaves = 8;
 // K by whole rows (TileRegs): all waves request their tiles at once, at the start, and the address path is
 // through with the requests sooner: 8 requests of 300-1100, 16 layers replayed, 277.1 -> 270.4 us.
 constexpr bool kSplitWholeRows = true;
-constexpr int kSplitRing = 2;        // tiles in flight per wave: a wave rarely has more
 // The planner's rule, measured there: tiles of a batch at most (one kv head: at least), tiles of a
 // share at least, and parts of one request that make a batch lopsided.
 constexpr int kSplitMaxTiles = 2560, kSplitMinTilesOneHead = 5000, kSplitTilesPerShare = 6, kLopsidedParts = 64;
@@ -48,30 +51,40 @@ struct SplitShared {
 // The parts of a cut request are merged by whoever finishes last: every part stores its
 // partial, waits until the stores are acknowledged and counts itself in; the one that completes
 // the count reads all parts and writes the output row.  No fence is involved: partials are
-// stored and read as relaxed atomics of device scope (written through, and read past the L2 of
-// the XCD), so nothing else in the caches has to be written back or dropped - release / acquire
-// fences write back the whole L2.  The counter is set back to zero by the last one, ready for
-// the next launch.
-__device__ __forceinline__ void put2(float *p, f32x2 v)
-{
-    __hip_atomic_store(reinterpret_cast<uint64_t *>(p), __builtin_bit_cast(uint64_t, v), __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ f32x2 get2(const float *p)
-{
-    return __builtin_bit_cast(f32x2, __hip_atomic_load(reinterpret_cast<const uint64_t *>(p), __ATOMIC_RELAXED,
-                                                       __HIP_MEMORY_SCOPE_AGENT));
-}
-__device__ __forceinline__ void put4(float *p, f32x4 v)
-{
-    put2(p, f32x2{v[0], v[1]});
-    put2(p + 2, f32x2{v[2], v[3]});
-}
-__device__ __forceinline__ f32x4 get4(const float *p)
-{
-    const f32x2 a = get2(p), b = get2(p + 2);
-    return f32x4{a.x, a.y, b.x, b.y};
-}
+// stored and read with device scope (written through, and read past the L2 of the XCD), so nothing
+// else in the caches has to be written back or dropped - release / acquire fences write back the whole
+// L2.  The counter is set back to zero by the last one, ready for the next launch.
+// (Counting in at the start instead, the last one to start waiting for words that are zero between launches to be
+// written, saves the acknowledgement and the counter's trip, and costs the looking and the zeros: the request
+// of 1777 tokens 9.92 against 10.03 us, two of 1000-3000 with 64 heads 14.4 against 13.1, and the code is longer.)
+constexpr int kCoherent = 16;   // cache policy of the buffer instructions: device scope (sc1)
+struct Partials {
+    __amdgpu_buffer_rsrc_t o, ml;     // the slots' O rows, and their (maximum, sum)
+    int o_bytes, ml_bytes;            // of a slot
+    __device__ __forceinline__ Partials(const float *part_o, const float *part_ml, int slots, int n_qo_heads)
+    {
+        o_bytes = n_qo_heads * kHeadDim * 4;
+        ml_bytes = n_qo_heads * 8;
+        o = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(part_o), 0, slots * o_bytes, kBufferFlags);
+        ml = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(part_ml), 0, slots * ml_bytes, kBufferFlags);
+    }
+    __device__ __forceinline__ void put_o(int slot, int at, f32x4 v) const
+    {
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), o, at * 4, slot * o_bytes, kCoherent);
+    }
+    __device__ __forceinline__ void put_ml(int slot, int qh, f32x2 v) const
+    {
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), ml, qh * 8, slot * ml_bytes, kCoherent);
+    }
+    __device__ __forceinline__ f32x4 get_o(int slot, int at) const
+    {
+        return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(o, at * 4, slot * o_bytes, kCoherent));
+    }
+    __device__ __forceinline__ f32x2 get_ml(int slot, int qh) const
+    {
+        return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(ml, qh * 8, slot * ml_bytes, kCoherent));
+    }
+};
 // Counts one part in; to be called by one lane.  True for the part that completes the set.
 __device__ __forceinline__ bool arrive_last(uint32_t *counter, int parts)
 {
@@ -83,8 +96,7 @@ __device__ __forceinline__ bool arrive_last(uint32_t *counter, int parts)
 // Dims d0 .. d0 + 3 of q head qh merged over `parts` consecutive slots, kAtOnce of them requested
 // per trip to memory under a running maximum: their sum under maximum m, l the sum of weights.
 template <int kAtOnce>
-__device__ __forceinline__ f32x4 merge_slots(float *part_o, float *part_ml, int first, int parts,
-                                             int n_qo_heads, int qh, int d0, float &m, float &l)
+__device__ __forceinline__ f32x4 merge_slots(const Partials &at, int first, int parts, int qh, int d0, float &m, float &l)
 {
     m = kNegBig;
     l = 0.f;
@@ -94,9 +106,9 @@ __device__ __forceinline__ f32x4 merge_slots(float *part_o, float *part_ml, int 
         f32x2 ml[kAtOnce];   // (maximum, sum)
 #pragma unroll
         for (int i = 0; i < kAtOnce; i++) {
-            const long slot = first + min(i0 + i, parts - 1);   // past the last: it again, weight zero
-            ml[i] = get2(part_ml + (slot * n_qo_heads + qh) * 2);
-            o[i] = get4(part_o + (slot * n_qo_heads + qh) * kHeadDim + d0);
+            const int slot = first + min(i0 + i, parts - 1);   // past the last: it again, weight zero
+            ml[i] = at.get_ml(slot, qh);
+            o[i] = at.get_o(slot, qh * kHeadDim + d0);
         }
         float m_new = m;
 #pragma unroll
@@ -115,90 +127,92 @@ __device__ __forceinline__ f32x4 merge_slots(float *part_o, float *part_ml, int 
     return acc;
 }
 
+// Two cache lines, what the first loads need in front (they come by scalar loads, a line at a time).
 struct SplitArgs {
-    uint16_t *out;
-    const uint16_t *q;
     const char *pages;
     const int32_t *kv_indices;
     const Item *items;
     const int32_t *wg_ptr;
-    float *part_o, *part_ml;
-    int max_slots, n_qo_heads, n_kv_heads, page_shift;
-    float scale_log2;
-    const uint16_t *k_new, *v_new;   // null: the newest tokens are in the pages already
+    const uint16_t *q;
     const float *rope;               // null: q and k_new are not to be rotated
+    const uint16_t *k_new, *v_new;   // null: the newest tokens are in the pages already
+    int n_qo_heads, n_kv_heads, group, page_shift;
+    float scale_log2;
+    int max_slots;
+    float *part_o, *part_ml;
     uint32_t *counters;              // one zeroed word per (partial slot, kv head); null: a merge launch follows
-    int n_counters, n_shares;
+    int n_counters;
+    int unused;
+    uint16_t *out;
 };
+static_assert(sizeof(SplitArgs) == 128, "");
+typedef const __attribute__((address_space(4))) SplitArgs *const_args_ptr;
+typedef int32_t i32x8 __attribute__((ext_vector_type(8), aligned(4)));
+typedef const __attribute__((address_space(4))) i32x8 *const_i32x8_ptr;
 
 // A workgroup fills its compute unit's LDS, so what counts is that the workgroups spread evenly: ids go
 // round the 8 XCDs, and without gaps in them no XCD gets more than its 32, whatever the number of
 // heads.  (The heads of a share need not meet on an XCD: they read other bytes of the same pages.)
+//
+// What keeps the path through it short: no division (a share and a head are grid coordinates; an item's heads are
+// dealt to whole waves), an item's words in one load, both first pages in one trip, q turned by a lane per chunk instead of by
+// every lane for its operand (45 instead of 180 instructions), operands of a tile requested from LDS together, nothing issued
+// for tiles that are not there, arguments read anew behind the loop instead of spilled, pieces that meet
+// requested together.  All that: the request of 1777 tokens, in 18 parts, 13.1 -> 10.9 us a layer, 4 of 60 tokens 9.6 -> 6.3.
 template <int DT, int kPagesPerTile>
 __global__ __launch_bounds__(64 * kSplitWaves) void decode_attn_split_kernel(const SplitArgs a)
 {
     typedef Elt<DT> E;
     constexpr bool kPageCoversTile = kPagesPerTile == 1, kWholeRows = kSplitWholeRows;
     __shared__ __align__(16) SplitShared sh;
-    const int share = (int)blockIdx.x % a.n_shares, kvh = (int)blockIdx.x / a.n_shares;
+    const int share = (int)blockIdx.x, kvh = (int)blockIdx.y;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int g = lane >> 4, c = lane & 15;
-    const int group = a.n_qo_heads / a.n_kv_heads;
+    const int group = a.group;
     const const_i32_ptr item_words = as_const(reinterpret_cast<const int32_t *>(a.items));
-    const const_i32_ptr indices_c = as_const(a.kv_indices);
     const int item_begin = as_const(a.wg_ptr)[share], item_end = as_const(a.wg_ptr)[share + 1];
     if (item_begin >= item_end) return;
 
     // ---- this wave's slice of the share's tiles, and the items it meets
-    auto tiles_of = [](int begin, int end) { return (end - begin + kTile - 1) / kTile; };
-    const const_i32_ptr last_words = item_words + (long)(item_end - 1) * kItemWords;
-    const int total = last_words[7] + tiles_of(last_words[1], last_words[2]);
-    const int lo = total * wave / kSplitWaves, hi = total * (wave + 1) / kSplitWaves;   // tiles of the share
-    int first_item = item_end, end_item = item_begin;
-    for (int idx = item_begin; idx < item_end; idx++) {
-        const const_i32_ptr w = item_words + (long)idx * kItemWords;
-        const int at = w[7], n = tiles_of(w[1], w[2]);
-        if (n == 0) {
-            // a request without tokens: a row of zeros
-            if (wave == 0)
-                for (int i = lane * 8; i < group * kHeadDim; i += 64 * 8)
-                    *reinterpret_cast<u32x4 *>(a.out + ((long)w[0] * a.n_qo_heads + (long)kvh * group) * kHeadDim + i) =
-                        u32x4{0, 0, 0, 0};
-        } else if (at < hi && at + n > lo) {
-            first_item = min(first_item, idx);
-            end_item = idx + 1;
-        }
-    }
+    struct Words {
+        int row, begin, end, slot, page_begin, tail, parts, at;
+    };
+    auto words_of = [&](int idx) {   // (one load of eight words, not a few of two when they are needed)
+        const i32x8 w = *reinterpret_cast<const_i32x8_ptr>(item_words + (long)idx * kItemWords);
+        return Words{w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7]};
+    };
+    auto tiles_of = [](int begin, int end) { return (int)((unsigned)(end - begin + kTile - 1) / kTile); };
+    const Words head_item = words_of(item_begin), tail_item = words_of(item_end - 1);   // (requested together)
+    const int total = tail_item.at + tiles_of(tail_item.begin, tail_item.end);
+    const int lo = (int)((unsigned)(total * wave) / kSplitWaves), hi = (int)((unsigned)(total * (wave + 1)) / kSplitWaves);
+    // the first item whose tiles end behind lo, if they begin before hi
+    Words w0 = head_item;
+    int first_item = item_begin;
+    while (w0.at + tiles_of(w0.begin, w0.end) <= lo && first_item < item_end - 1) w0 = words_of(++first_item);
     struct Piece {
         int b, tok_begin, tok_end, slot, page_begin;
         bool tail;        // holds the request's newest token
         bool starts, ends;   // the item starts / ends in this wave's slice
         int at;           // the item's first tile within the share
     };
-    auto load_piece = [&](int idx) {
-        const const_i32_ptr w = item_words + (long)idx * kItemWords;
-        const int begin = w[1], end = w[2], at = w[7];
+    auto piece_of = [&](const Words &w) {   // (of an item with tiles in the slice, or without tiles: without any then)
         Piece p;
-        p.b = w[0];
-        p.tok_begin = max(begin, begin + (lo - at) * kTile);
-        p.tok_end = min(end, begin + (hi - at) * kTile);
-        p.slot = w[3];
-        p.page_begin = w[4];
-        p.starts = at >= lo;
-        p.ends = p.tok_end == end;
-        p.tail = w[5] && p.ends;
-        if (p.tok_end <= p.tok_begin) {   // not this wave's, or without tokens
-            p.tok_end = p.tok_begin;
-            p.tail = false;
-        }
-        p.at = at;
+        p.b = w.row;
+        p.tok_begin = w.begin + max(lo - w.at, 0) * kTile;
+        p.tok_end = min(w.end, w.begin + (hi - w.at) * kTile);
+        p.slot = w.slot;
+        p.page_begin = w.page_begin;
+        p.starts = w.at >= lo;
+        p.ends = p.tok_end == w.end;
+        p.tail = w.tail && p.ends;
+        p.at = w.at;
         return p;
     };
 
     KvView kv;
     kv.pages = a.pages;
-    kv.page_ids = indices_c;
+    kv.page_ids = as_const(a.kv_indices);
     kv.page_shift = a.page_shift;
     kv.row_bytes = a.n_kv_heads * kHeadDim * 2;
     kv.half_bytes = kv.row_bytes << a.page_shift;
@@ -207,53 +221,60 @@ __global__ __launch_bounds__(64 * kSplitWaves) void decode_attn_split_kernel(con
     char *tile_lds = sh.tiles + wave * tile_lds_bytes(kSplitWholeRows);
     uint32_t *new_k = sh.new_row[wave][0], *new_v = sh.new_row[wave][1];
 
-    // ---- what a piece needs besides its tiles: the q rows as the B operand of the score MFMAs
-    // (zero beyond the group), their cosines and sines, and the new token's rows (lanes 0-15: K,
-    // 16-31: V; lanes 0-15 also the cosines and sines of their chunk).
+    // ---- what a piece needs besides its tiles: lane i has chunk i % 16 (8 dims) of q rows i / 16 and i / 16 + 4 (past
+    // the group: some chunk), the cosines and sines of the chunk, and of the new token's rows (K in lanes 0-15, V in
+    // lanes 16-31) the same chunk.
     struct Raw {
-        u32x4 q[4], fresh;
-        f32x4 cs[4], sn[4], fresh_cs, fresh_sn;
+        u32x4 q[2], fresh;
+        f32x4 cs, sn;
+        int page;         // of the new token
     };
     auto request = [&](const Piece &p, Raw &r) {
-        const uint16_t *qrow = a.q + ((long)p.b * a.n_qo_heads + (long)kvh * group + c) * kHeadDim + g * 8;
-        const u32x4 z = {0, 0, 0, 0};
-#pragma unroll
-        for (int kk = 0; kk < 4; kk++) r.q[kk] = c < group ? *reinterpret_cast<const u32x4 *>(qrow + kk * 32) : z;
-        const float *tab = a.rope + (long)p.b * kHeadDim;
-        if (a.rope) {   // dims 32*kk + 8*g .. +7
-#pragma unroll
-            for (int kk = 0; kk < 4; kk++) {
-                r.cs[kk] = *reinterpret_cast<const f32x4 *>(tab + g * 4 + kk * 16);
-                r.sn[kk] = *reinterpret_cast<const f32x4 *>(tab + kHeadDim / 2 + g * 4 + kk * 16);
-            }
+        const uint16_t *rows = a.q + ((long)p.b * a.n_qo_heads + kvh * group) * kHeadDim;
+        r.q[0] = *reinterpret_cast<const u32x4 *>(rows + min(lane, group * 16 - 1) * 8);
+        if (group > 4) r.q[1] = *reinterpret_cast<const u32x4 *>(rows + min(64 + lane, group * 16 - 1) * 8);
+        if (a.rope) {
+            const float *tab = a.rope + (long)p.b * kHeadDim + c * 4;
+            r.cs = *reinterpret_cast<const f32x4 *>(tab);
+            r.sn = *reinterpret_cast<const f32x4 *>(tab + kHeadDim / 2);
         }
-        r.fresh = z;
-        if (a.k_new && p.tail && lane < 32) {
-            const long src = ((long)p.b * a.n_kv_heads + kvh) * kHeadDim + c * 8;
-            r.fresh = *reinterpret_cast<const u32x4 *>((lane < 16 ? a.k_new : a.v_new) + src);
-            if (a.rope && lane < 16) {
-                r.fresh_cs = *reinterpret_cast<const f32x4 *>(tab + c * 4);
-                r.fresh_sn = *reinterpret_cast<const f32x4 *>(tab + kHeadDim / 2 + c * 4);
-            }
+        if (a.k_new && p.tail) {
+            r.page = as_const(a.kv_indices)[p.page_begin + ((p.tok_end - 1) >> a.page_shift)];
+            const long src = ((long)p.b * a.n_kv_heads + kvh) * kHeadDim;
+            r.fresh = *reinterpret_cast<const u32x4 *>((lane < 16 ? a.k_new + src : a.v_new + src) + c * 8);
         }
     };
-    auto rotate = [&](u32x4 chunk, const f32x4 &cs, const f32x4 &sn) {
-        const float c4[4] = {cs[0], cs[1], cs[2], cs[3]}, s4[4] = {sn[0], sn[1], sn[2], sn[3]};
+    auto rotate = [&](u32x4 chunk, const Raw &r) {
+        const float c4[4] = {r.cs[0], r.cs[1], r.cs[2], r.cs[3]}, s4[4] = {r.sn[0], r.sn[1], r.sn[2], r.sn[3]};
         float f[8];
         Chunk<DT>::unpack(chunk, f);
         rope_rotate<4>(f, c4, s4);
         return Chunk<DT>::pack(f);
     };
+    // The q rows as the B operand of the score MFMAs, through the wave's V tile; columns past the group repeat
+    // the last row (nobody reads their results).
+    auto operand_of = [&](const Raw &r, u32x4 (&qreg)[4]) {
+        char *rows = tile_lds;
+        __builtin_amdgcn_wave_barrier();
+        *reinterpret_cast<u32x4 *>(rows + g * kVPitch + c * 16) = a.rope ? rotate(r.q[0], r) : r.q[0];
+        if (group > 4) *reinterpret_cast<u32x4 *>(rows + (4 + g) * kVPitch + c * 16) = a.rope ? rotate(r.q[1], r) : r.q[1];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const char *mine = rows + min(c, group - 1) * kVPitch + g * 16;
+#pragma unroll
+        for (int kk = 0; kk < 4; kk++) qreg[kk] = *reinterpret_cast<const u32x4 *>(mine + kk * 64);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
     // Writes the new token's rows into their page slot, and into LDS, from where the tile that
     // holds them takes them: nobody waits for the page to have them.
     auto place_new_row = [&](const Piece &p, const Raw &r) {
         const int tok = p.tok_end - 1;
-        const long page = indices_c[p.page_begin + (tok >> a.page_shift)];
-        char *row = const_cast<char *>(a.pages) + page * kv.page_bytes +
+        char *row = const_cast<char *>(a.pages) + (long)r.page * kv.page_bytes +
                     (long)(tok & ((1 << a.page_shift) - 1)) * kv.row_bytes + kv.head_off + c * 16;
         if (lane < 32) {
             u32x4 chunk = r.fresh;
-            if (a.rope && lane < 16) chunk = rotate(chunk, r.fresh_cs, r.fresh_sn);
+            if (a.rope && lane < 16) chunk = rotate(chunk, r);
             *reinterpret_cast<u32x4 *>(row + (lane < 16 ? 0 : kv.half_bytes)) = chunk;
             *reinterpret_cast<u32x4 *>((lane < 16 ? new_k : new_v) + c * 4) = chunk;
         }
@@ -261,83 +282,101 @@ __global__ __launch_bounds__(64 * kSplitWaves) void decode_attn_split_kernel(con
         __builtin_amdgcn_wave_barrier();
     };
 
-    // ---- load side: runs ahead of the compute side through the wave's pieces
-    int next_item = first_item, t = 0, t_end = 0, t_pad_end = 0;
-    long page[2] = {0, 0};
-    auto settle = [&]() {
-        while (t >= t_pad_end && next_item < end_item) {
-            const Piece p = load_piece(next_item++);
-            t = p.tok_begin;
-            t_end = p.tok_end;
-            t_pad_end = t + (tiles_of(t, t_end) + kSplitRing - 1) / kSplitRing * kSplitRing * kTile;
-            kv.page_ids = indices_c + p.page_begin;
-        }
-        if (t >= t_pad_end) t_end = 0;   // exhausted: every further tile is empty and reads no block table
-        if (kPagesPerTile >= 1)
-#pragma unroll
-            for (int j = 0; j < kPagesPerTile; j++)
-                page[j] = t_end > 0 ? kv.page_ids[page_slot_of(kv, t + (j << kv.page_shift), t_end)] : 0;
-    };
-    auto load_next = [&](TileRegs &r) {
-        if (kPageCoversTile) {
-            load_kv_tile_in_page<kLoadStreaming, kWholeRows>(kv, page[0], t, t_end, g, c, r);
-        } else if (kPagesPerTile == 2) {
-            load_kv_tile_small_pages<2, kLoadStreaming, kWholeRows>(kv, page, t, t_end, g, c, r);
-        } else {
-            load_kv_tile<false, kLoadStreaming, kWholeRows>(kv, t, t_end, g, c, r);
-        }
-        t += kTile;
-        settle();
-    };
-
     if (lane == 0) {
         sh.owner[wave] = -1;
         sh.meet_row[wave] = -1;
     }
-    if (first_item < end_item) {
-        Piece piece = load_piece(first_item);
+    if (lo < hi) {
+        // ---- load side: runs ahead of the compute side through the wave's pieces
+        Piece piece = piece_of(w0);
+        int left = hi - lo, t, t_end, next_item = first_item + 1;   // tiles that are not requested yet; the next of them
+        auto enter = [&](const Piece &p) {
+            t = p.tok_begin;
+            t_end = p.tok_end;
+            kv.page_ids = as_const(a.kv_indices) + p.page_begin;
+        };
+        auto look_up = [&](int tok, long (&pg)[2]) {
+#pragma unroll
+            for (int j = 0; j < kPagesPerTile; j++) pg[j] = kv.page_ids[page_slot_of(kv, tok + (j << kv.page_shift), t_end)];
+        };
+        auto load_tile = [&](TileRegs &r, const long (&pg)[2]) {
+            if (kPageCoversTile) {
+                load_kv_tile_in_page<kLoadStreaming, kWholeRows>(kv, pg[0], t, t_end, g, c, r);
+            } else if (kPagesPerTile == 2) {
+                load_kv_tile_small_pages<2, kLoadStreaming, kWholeRows>(kv, pg, t, t_end, g, c, r);
+            } else {
+                load_kv_tile<false, kLoadStreaming, kWholeRows>(kv, t, t_end, g, c, r);
+            }
+            t += kTile;
+            left--;
+            while (left > 0 && t >= t_end) enter(piece_of(words_of(next_item++)));   // (items without tokens are stepped over)
+        };
+        // Two tiles are in flight; the second passes to the first's registers when that one is done with, so that
+        // there is one copy of the code.
+        enter(piece);
+        long page[2] = {0, 0}, page_after[2] = {0, 0};
+        look_up(t, page);
+        const bool both = t + kTile < t_end;
+        if (both) look_up(t + kTile, page_after);
         Raw raw;
         request(piece, raw);
-        settle();
-        TileRegs ring[kSplitRing];
-#pragma unroll
-        for (int s = 0; s < kSplitRing; s++) load_next(ring[s]);
+        TileRegs now, after;
+        load_tile(now, page);
+        auto load_after = [&]() {
+            if (left <= 0) return;
+            load_tile(after, page_after);
+            if (left > 0) look_up(t, page_after);
+        };
+        if (left > 0 && !both) look_up(t, page_after);
+        load_after();
 
-        for (int idx = first_item; idx < end_item; idx++) {
+        int idx = first_item, computed_tiles = 0;
+        while (true) {
             u32x4 qreg[4];
-#pragma unroll
-            for (int kk = 0; kk < 4; kk++) {
-                qreg[kk] = raw.q[kk];
-                if (a.rope) qreg[kk] = rotate(raw.q[kk], raw.cs[kk], raw.sn[kk]);
-            }
+            operand_of(raw, qreg);
             const bool fresh = a.k_new && piece.tail;
             if (fresh) place_new_row(piece, raw);
-            const Piece next = load_piece(min(idx + 1, end_item - 1));
-            if (idx + 1 < end_item) request(next, raw);
+            // the wave's next piece, if there is one
+            computed_tiles += tiles_of(piece.tok_begin, piece.tok_end);
+            const bool more = computed_tiles < hi - lo;
+            Piece next = piece;
+            if (more) {
+                do next = piece_of(words_of(++idx));
+                while (next.tok_end <= next.tok_begin);   // (without tokens)
+                request(next, raw);
+            }
 
             f32x4 acc[8];
 #pragma unroll
             for (int dt = 0; dt < 8; dt++) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
             float m_run = kNegBig, l_run = 0.f;
+            const bool own_maximum = piece.slot < 0 && piece.tok_end - piece.tok_begin > kTile;
             auto compute_tile = [&](int t0, TileRegs &r) {
                 const int end = piece.tok_end;
                 if (fresh && t0 + kTile >= end) {
                     // the newest token is this tile's row nr, and the page may not have it yet
                     const int nr = end - 1 - t0;
 #pragma unroll
-                    for (int kk = 0; kk < 4; kk++) {
-                        if (kWholeRows && g + 4 * kk == nr) r.k[kk] = *reinterpret_cast<const u32x4 *>(new_k + c * 4);
-                        if (!kWholeRows && c == nr) r.k[kk] = *reinterpret_cast<const u32x4 *>(new_k + kk * 16 + g * 4);
-                    }
-#pragma unroll
                     for (int i = 0; i < 4; i++)
+                    {
+                        if (kWholeRows && g + 4 * i == nr) r.k[i] = *reinterpret_cast<const u32x4 *>(new_k + c * 4);
+                        if (!kWholeRows && c == nr) r.k[i] = *reinterpret_cast<const u32x4 *>(new_k + i * 16 + g * 4);
                         if (g + 4 * i == nr) r.v[i] = *reinterpret_cast<const u32x4 *>(new_v + c * 4);
+                    }
                 }
+                // all twelve operands are requested before the first is waited for
                 if (kWholeRows) stage_k_tile(tile_lds, r, g, c);
+                stage_v_tile<kPageCoversTile>(tile_lds, r, t0, end, g, c);
+                u32x4 ka[4];
+                u32x2 va[8];
+#pragma unroll
+                for (int kk = 0; kk < 4; kk++) ka[kk] = kWholeRows ? read_k_operand(tile_lds, kk, g, c) : r.k[kk];
+#pragma unroll
+                for (int dt = 0; dt < 8; dt++) va[dt] = read_v_operand(tile_lds, dt, g, c);
+                __builtin_amdgcn_sched_barrier(0);
                 f32x4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int kk = 0; kk < 4; kk++)
-                    s = E::mfma_k32(kWholeRows ? read_k_operand(tile_lds, kk, g, c) : r.k[kk], qreg[kk], s);
+                for (int kk = 0; kk < 4; kk++) s = E::mfma_k32(ka[kk], qreg[kk], s);
                 const bool ragged = t0 + kTile > end;
                 float x[4];
 #pragma unroll
@@ -345,173 +384,220 @@ __global__ __launch_bounds__(64 * kSplitWaves) void decode_attn_split_kernel(con
                     x[j] = s[j] * a.scale_log2;
                     if (ragged && t0 + 4 * g + j >= end) x[j] = kNegBig;
                 }
-                stage_v_tile<kPageCoversTile>(tile_lds, r, t0, end, g, c);
-                const float m_new = fmaxf(m_run, quad_rows_max(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]))));
+                const float m_tile = quad_rows_max(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])));
+                const float m_new = fmaxf(m_run, m_tile);
+                const float m_of_p = own_maximum ? m_tile : m_new;
                 const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-                m_run = m_new;
                 float p[4], p_sum = 0.f;
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
-                    p[j] = x[j] > kNegBig ? __builtin_amdgcn_exp2f(x[j] - m_new) : 0.f;
+                    p[j] = x[j] > kNegBig ? __builtin_amdgcn_exp2f(x[j] - m_of_p) : 0.f;
                     p_sum += p[j];
                 }
-                l_run = l_run * alpha + p_sum;
+                m_run = m_new;
                 const u32x2 pb = {E::pack2(p[0], p[1]), E::pack2(p[2], p[3])};
+                if (own_maximum) {
+                    // A request that lies whole in the share, where a wave may have more tiles than in shares that cut
+                    // it: P under the tile's own maximum, brought to the common one in fp32.  The largest
+                    // probability of every tile is then exactly 1 in 16 bits, however many a wave has (under the running
+                    // maximum two tiles a wave instead of one put the error against 64 bits up by 1.5 to 3 %).
+                    const float beta = __builtin_amdgcn_exp2f(m_tile - m_new);
+                    l_run = l_run * alpha + p_sum * beta;
+                    f32x4 o[8];
 #pragma unroll
-                for (int dt = 0; dt < 8; dt++)
-                    acc[dt] = E::mfma_k16(read_v_operand(tile_lds, dt, g, c), pb, acc[dt] * alpha);
+                    for (int dt = 0; dt < 8; dt++) o[dt] = E::mfma_k16(va[dt], pb, f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+                    for (int dt = 0; dt < 8; dt++) acc[dt] = acc[dt] * alpha + o[dt] * beta;
+                } else {
+                    l_run = l_run * alpha + p_sum;
+#pragma unroll
+                    for (int dt = 0; dt < 8; dt++) acc[dt] = E::mfma_k16(va[dt], pb, acc[dt] * alpha);
+                }
                 __builtin_amdgcn_wave_barrier();
             };
-            const int pad_end = piece.tok_begin +
-                                (tiles_of(piece.tok_begin, piece.tok_end) + kSplitRing - 1) / kSplitRing * kSplitRing * kTile;
-            for (int t0 = piece.tok_begin; t0 < pad_end; t0 += kSplitRing * kTile) {
-#pragma unroll
-                for (int s = 0; s < kSplitRing; s++) {
-                    if (t0 + s * kTile < piece.tok_end) compute_tile(t0 + s * kTile, ring[s]);
-                    __builtin_amdgcn_sched_barrier(0);
-                    load_next(ring[s]);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
+            for (int t0 = piece.tok_begin;;) {
+                compute_tile(t0, now);
+                t0 += kTile;
+                now = after;
+                load_after();
+                if (t0 >= piece.tok_end) break;
             }
             l_run = quad_rows_sum(l_run);
-            if (piece.tok_end > piece.tok_begin) {
-                if (piece.starts && piece.ends) {   // a whole item
-                    if (c < group) {
-                        const int qh = kvh * group + c;
-                        if (piece.slot < 0) {
-                            const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
-                            uint16_t *o = a.out + ((long)piece.b * a.n_qo_heads + qh) * kHeadDim + 4 * g;
+            const bool whole = piece.starts && piece.ends;
+            if (whole && piece.slot < 0) {
+                if (c < group) {
+                    const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
+                    uint16_t *o = a.out + ((long)piece.b * a.n_qo_heads + kvh * group + c) * kHeadDim + 4 * g;
 #pragma unroll
-                            for (int dt = 0; dt < 8; dt++)
-                                *reinterpret_cast<u32x2 *>(o + dt * 16) =
-                                    u32x2{E::pack2(acc[dt][0] * inv, acc[dt][1] * inv),
-                                          E::pack2(acc[dt][2] * inv, acc[dt][3] * inv)};
-                        } else if (piece.slot < a.max_slots) {   // a slot beyond the workspace is never written
-                            const long at = (long)piece.slot * a.n_qo_heads + qh;
+                    for (int dt = 0; dt < 8; dt++)
+                        *reinterpret_cast<u32x2 *>(o + dt * 16) =
+                            u32x2{E::pack2(acc[dt][0] * inv, acc[dt][1] * inv), E::pack2(acc[dt][2] * inv, acc[dt][3] * inv)};
+                }
+            } else if (whole) {
+                // a part of a cut request that no other wave of the share has tiles of; a slot beyond the workspace is
+                // never written
+                const Partials to(a.part_o, a.part_ml, a.max_slots, a.n_qo_heads);
+                if (c < group && piece.slot < a.max_slots) {
+                    const int qh = kvh * group + c;
 #pragma unroll
-                            for (int dt = 0; dt < 8; dt++) put4(a.part_o + at * kHeadDim + dt * 16 + 4 * g, acc[dt]);
-                            if (g == 0) put2(a.part_ml + at * 2, f32x2{m_run, l_run});
-                        }
-                    }
-                } else {   // one end of an item that other waves share
-                    const int place = piece.starts ? 1 : 0;
-                    if (c < group) {
-                        float *o = sh.o[wave][place] + c * kHeadDim + 4 * g;
+                    for (int dt = 0; dt < 8; dt++) to.put_o(piece.slot, qh * kHeadDim + 4 * g + dt * 16, acc[dt]);
+                    if (g == 0) to.put_ml(piece.slot, qh, f32x2{m_run, l_run});
+                }
+            } else {
+                // one end of an item that other waves share
+                const int place = piece.starts ? 1 : 0;
+                if (c < group) {
+                    float *o = sh.o[wave][place] + c * kHeadDim + 4 * g;
 #pragma unroll
-                        for (int dt = 0; dt < 8; dt++) *reinterpret_cast<f32x4 *>(o + dt * 16) = acc[dt];
-                        if (g == 0) {
-                            sh.ml[wave][place][c][0] = m_run;
-                            sh.ml[wave][place][c][1] = l_run;
-                        }
-                    }
-                    if (lane == 0) {
-                        if (piece.starts) {
-                            sh.meet_row[wave] = piece.b;
-                            sh.meet_slot[wave] = piece.slot;
-                        } else {
-                            // the wave whose slice holds the item's first tile
-                            int o = wave - 1;
-                            while (total * o / kSplitWaves > piece.at) o--;
-                            sh.owner[wave] = o;
-                        }
+                    for (int dt = 0; dt < 8; dt++) *reinterpret_cast<f32x4 *>(o + dt * 16) = acc[dt];
+                    if (g == 0) *reinterpret_cast<f32x2 *>(sh.ml[wave][place][c]) = f32x2{m_run, l_run};
+                }
+                // the wave whose slice holds the item's first tile: the last one to begin at it or before
+                const int holder = __builtin_popcountll(__builtin_amdgcn_ballot_w64(
+                                       lane < kSplitWaves && (int)((unsigned)(total * lane) / kSplitWaves) <= piece.at)) - 1;
+                if (lane == 0) {
+                    if (piece.starts) {
+                        sh.meet_row[wave] = piece.b;
+                        sh.meet_slot[wave] = piece.slot;
+                    } else {
+                        sh.owner[wave] = holder;
                     }
                 }
             }
+            if (!more) break;
             piece = next;
         }
     }
-
-    // ---- the items that meet: a thread owns four values
+    // requests without tokens: rows of zeros
+    if (wave == kSplitWaves - 1 && (item_end - item_begin > 1 || total == 0))
+        for (int i = item_begin; i < item_end; i++) {
+            const const_i32_ptr w = item_words + (long)i * kItemWords;
+            if (w[1] < w[2]) continue;
+            uint16_t *row = a.out + ((long)w[0] * a.n_qo_heads + kvh * group) * kHeadDim;
+            for (int at = lane * 8; at < group * kHeadDim; at += 64 * 8) *reinterpret_cast<u32x4 *>(row + at) = u32x4{0, 0, 0, 0};
+        }
+    // ---- behind the barrier a thread owns four dims of a head, and an item's heads are dealt to whole waves, two
+    // each: `side` items are worked on side by side.  (Arguments and items are read anew from here on: held through
+    // the loop, they are spilled.)
     __syncthreads();
-    const int per_item = group * (kHeadDim / 4), side_by_side = 64 * kSplitWaves / per_item;
-    const int mine = (int)threadIdx.x / per_item, idx4 = (int)threadIdx.x % per_item;
-    const int head = idx4 / (kHeadDim / 4), qh = kvh * group + head, d0 = idx4 % (kHeadDim / 4) * 4;
-    if (mine < side_by_side) {
-        for (int e = mine; e < kSplitWaves; e += side_by_side) {
-            const int row = sh.meet_row[e], slot = sh.meet_slot[e];
-            if (row < 0) continue;
-            float m_all = sh.ml[e][1][head][0];
-            for (int w = e + 1; w < kSplitWaves; w++)
-                if (sh.owner[w] == e) m_all = fmaxf(m_all, sh.ml[w][0][head][0]);
-            f32x4 sum = {0.f, 0.f, 0.f, 0.f};
-            float l_all = 0.f;
-            for (int w = e; w < kSplitWaves; w++) {
-                if (w > e && sh.owner[w] != e) continue;
-                const int place = w == e ? 1 : 0;
-                const float weight = __builtin_amdgcn_exp2f(sh.ml[w][place][head][0] - m_all);
-                l_all += weight * sh.ml[w][place][head][1];
-                sum += weight * *reinterpret_cast<const f32x4 *>(sh.o[w][place] + head * kHeadDim + d0);
-            }
-            if (slot < 0) {
-                const float inv = l_all > 0.f ? 1.f / l_all : 0.f;
-                *reinterpret_cast<u32x2 *>(a.out + ((long)row * a.n_qo_heads + qh) * kHeadDim + d0) =
-                    u32x2{E::pack2(sum[0] * inv, sum[1] * inv), E::pack2(sum[2] * inv, sum[3] * inv)};
-            } else if (slot < a.max_slots) {
-                const long at = (long)slot * a.n_qo_heads + qh;
-                put4(a.part_o + at * kHeadDim + d0, sum);
-                if (d0 == 0) put2(a.part_ml + at * 2, f32x2{m_all, l_all});
-            }
+    const_args_ptr late = (const_args_ptr)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(late));
+    const int waves_per_item = (group + 1) / 2;
+    const int side_shift = waves_per_item >= 3 ? 1 : 4 - waves_per_item, side = 1 << side_shift;
+    const int mine = waves_per_item == 3 ? wave / 3 : wave >> (3 - side_shift);
+    const int head = (wave - mine * waves_per_item) * 2 + (lane >> 5), d0 = (lane & 31) * 4;
+    const bool works = mine < side && head < group;
+    const int qh = kvh * group + head;
+    const Partials parts_at(late->part_o, late->part_ml, late->max_slots, late->n_qo_heads);
+    auto put_row = [&](int row, f32x4 sum, float l) {
+        const float inv = l > 0.f ? 1.f / l : 0.f;
+        *reinterpret_cast<u32x2 *>(late->out + ((long)row * late->n_qo_heads + qh) * kHeadDim + d0) =
+            u32x2{E::pack2(sum[0] * inv, sum[1] * inv), E::pack2(sum[2] * inv, sum[3] * inv)};
+    };
+
+    // ---- the items that meet
+    const int in_wave = lane & (kSplitWaves - 1);
+    const int owner = sh.owner[in_wave];
+    uint32_t meetings = (uint32_t)__builtin_amdgcn_ballot_w64(sh.meet_row[in_wave] >= 0) & ((1 << kSplitWaves) - 1);
+    for (int n = 0; meetings; n++, meetings &= meetings - 1) {
+        if ((n & (side - 1)) != mine) continue;
+        const int e = __builtin_ctz(meetings);
+        const uint32_t from = (uint32_t)__builtin_amdgcn_ballot_w64(owner == e) & ((1 << kSplitWaves) - 1);
+        const int row = __builtin_amdgcn_readfirstlane(sh.meet_row[e]), slot = __builtin_amdgcn_readfirstlane(sh.meet_slot[e]);
+        // all waves' pieces are requested at once; waves that hold no piece of the item have its first, weighing nothing
+        f32x4 o[kSplitWaves];
+        f32x2 ml[kSplitWaves];
+        const int h = min(head, group - 1);
+#pragma unroll
+        for (int w = 0; w < kSplitWaves; w++) {
+            const bool in = from >> w & 1;
+            const int from_wave = in ? w : e, place = in ? 0 : 1;
+            o[w] = *reinterpret_cast<const f32x4 *>(sh.o[from_wave][place] + h * kHeadDim + d0);
+            ml[w] = *reinterpret_cast<const f32x2 *>(sh.ml[from_wave][place][h]);
+            if (!in && w != e) ml[w].x = 2.f * kNegBig;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        float m_all = ml[0].x;
+#pragma unroll
+        for (int w = 1; w < kSplitWaves; w++) m_all = fmaxf(m_all, ml[w].x);
+        f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+        float l_all = 0.f;
+#pragma unroll
+        for (int w = 0; w < kSplitWaves; w++) {
+            const float weight = __builtin_amdgcn_exp2f(ml[w].x - m_all);
+            l_all += weight * ml[w].y;
+            sum += weight * o[w];
+        }
+        if (!works) continue;
+        if (slot < 0) {
+            put_row(row, sum, l_all);
+        } else if (slot < late->max_slots) {
+            parts_at.put_o(slot, qh * kHeadDim + d0, sum);
+            if (d0 == 0) parts_at.put_ml(slot, qh, f32x2{m_all, l_all});
         }
     }
 
     // ---- the parts of cut requests.  Only the first and the last item of a share can be parts
     // (the shares' boundaries cut); both are counted in, and merged, side by side.
-    if (!a.counters) return;
+    if (!late->counters) return;
+    struct Set {
+        int row, first, parts, counter;
+        bool cut;
+    };
+    const const_i32_ptr late_words = as_const(reinterpret_cast<const int32_t *>(late->items));
+    auto set_of = [&](int idx) {
+        const i32x8 w = *reinterpret_cast<const_i32x8_ptr>(late_words + (long)idx * kItemWords);
+        Set s;
+        s.row = w[0];
+        s.first = w[6] >> kPartsBits;
+        s.parts = w[6] & ((1 << kPartsBits) - 1);
+        s.counter = s.first * late->n_kv_heads + kvh;
+        s.cut = (w[3] >= 0) & (s.parts > 0) & (s.first + s.parts <= late->max_slots) & (s.counter < late->n_counters);
+        return s;
+    };
+    Set sets[2] = {set_of(item_begin), set_of(item_end - 1)};
+    sets[1].cut &= item_end - 1 != item_begin;
+    if (!sets[0].cut && !sets[1].cut) return;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the partials are where other XCDs see them
-    int row[2], first[2], parts[2];
-    bool cut[2];
-#pragma unroll
-    for (int k = 0; k < 2; k++) {
-        const const_i32_ptr w = item_words + (long)(k ? item_end - 1 : item_begin) * kItemWords;
-        row[k] = w[0];
-        first[k] = w[6] >> kPartsBits;
-        parts[k] = w[6] & ((1 << kPartsBits) - 1);
-        cut[k] = w[3] >= 0 && parts[k] > 0 && first[k] + parts[k] <= a.max_slots &&
-                 (long)first[k] * a.n_kv_heads + kvh < a.n_counters && !(k && item_end - 1 == item_begin);
+    __syncthreads();
+    if (wave < 2 && lane == 0) {
+        const Set &s = wave ? sets[1] : sets[0];
+        sh.last[wave] = s.cut && arrive_last(late->counters + s.counter, s.parts);
     }
-    if (!cut[0] && !cut[1]) return;
     __syncthreads();
-    if (wave < 2 && lane == 0)
-        sh.last[wave] = cut[wave] && arrive_last(a.counters + (long)first[wave] * a.n_kv_heads + kvh, parts[wave]);
-    __syncthreads();
-    const bool last[2] = {sh.last[0] != 0, sh.last[1] != 0};
+    const bool last[2] = {__builtin_amdgcn_readfirstlane(sh.last[0]) != 0, __builtin_amdgcn_readfirstlane(sh.last[1]) != 0};
     if (!last[0] && !last[1]) return;
     asm volatile("" ::: "memory");
-    // A set's parts are merged in `runs`, one per group of per_item threads where there are enough
-    // of those, and the runs in LDS.  How a set is cut into runs depends on its parts alone: the
-    // sums are in the same order whoever comes last and whatever else it merges.
-    const int each = last[0] && last[1] ? side_by_side / 2 : side_by_side;   // groups of threads per set
+    // A set's parts are merged in `runs`, one per `mine` where there are enough, and the runs in LDS.  How a
+    // set is cut into runs depends on its parts alone: the sums are in the same order whoever merges and
+    // whatever else it merges.
+    const int each = last[0] && last[1] ? side >> 1 : side;   // per set
     const int k = last[0] && mine < each ? 0 : 1, me = last[0] && last[1] ? mine - k * each : mine;
-    const int runs = min(side_by_side, (parts[k] + 3) / 4);
-    const bool works = mine < side_by_side && me < each;
-    float *o_lds = sh.o[0][0] + (long)k * side_by_side * per_item * 4, *ml_lds = sh.ml[k][0][0];
-    static_assert(sizeof(sh.o) >= 2 * 64 * kSplitWaves * 16 && sizeof(sh.ml[0]) >= 16 * 8, "a place per thread and set");
-    if (works)
-        for (int r = me; r < runs; r += each) {
-            const int p0 = parts[k] * r / runs, p1 = parts[k] * (r + 1) / runs;
+    const int set_parts = k ? sets[1].parts : sets[0].parts, set_first = k ? sets[1].first : sets[0].first;
+    const int set_row = k ? sets[1].row : sets[0].row;
+    const int per_run = max(4, (set_parts + side - 1) >> side_shift);
+    const bool merges = works && me < each;
+    float *o_lds = sh.o[0][0] + k * side * group * kHeadDim, *ml_lds = sh.ml[0][0][0] + k * side * group * 2;
+    static_assert(sizeof(sh.o) >= 2 * 8 * 2 * kHeadDim * 4 && sizeof(sh.ml) >= 2 * 16 * 8, "a place per run and set");
+    if (merges)
+        for (int r = me; r * per_run < set_parts; r += each) {
+            const int at = set_first + r * per_run, n = min(per_run, set_parts - r * per_run);
             float m, l;
-            const f32x4 o =
-                p1 - p0 <= 4 ? merge_slots<4>(a.part_o, a.part_ml, first[k] + p0, p1 - p0, a.n_qo_heads, qh, d0, m, l)
-                             : merge_slots<8>(a.part_o, a.part_ml, first[k] + p0, p1 - p0, a.n_qo_heads, qh, d0, m, l);
-            *reinterpret_cast<f32x4 *>(o_lds + (r * per_item + idx4) * 4) = o;
-            if (d0 == 0) {
-                ml_lds[(r * group + head) * 2] = m;
-                ml_lds[(r * group + head) * 2 + 1] = l;
-            }
+            const f32x4 o = n <= 4 ? merge_slots<4>(parts_at, at, n, qh, d0, m, l) : merge_slots<8>(parts_at, at, n, qh, d0, m, l);
+            *reinterpret_cast<f32x4 *>(o_lds + (r * group + head) * kHeadDim + d0) = o;
+            if (d0 == 0) *reinterpret_cast<f32x2 *>(ml_lds + (r * group + head) * 2) = f32x2{m, l};
         }
     __syncthreads();
-    if (works && me == 0) {
+    if (merges && me == 0) {
         float m_all = kNegBig, l_all = 0.f;
-        for (int r = 0; r < runs; r++) m_all = fmaxf(m_all, ml_lds[(r * group + head) * 2]);
+        for (int r = 0; r * per_run < set_parts; r++) m_all = fmaxf(m_all, ml_lds[(r * group + head) * 2]);
         f32x4 sum = {0.f, 0.f, 0.f, 0.f};
-        for (int r = 0; r < runs; r++) {
+        for (int r = 0; r * per_run < set_parts; r++) {
             const float weight = __builtin_amdgcn_exp2f(ml_lds[(r * group + head) * 2] - m_all);
             l_all += weight * ml_lds[(r * group + head) * 2 + 1];
-            sum += weight * *reinterpret_cast<const f32x4 *>(o_lds + (r * per_item + idx4) * 4);
+            sum += weight * *reinterpret_cast<const f32x4 *>(o_lds + (r * group + head) * kHeadDim + d0);
         }
-        const float inv = l_all > 0.f ? 1.f / l_all : 0.f;
-        *reinterpret_cast<u32x2 *>(a.out + ((long)row[k] * a.n_qo_heads + qh) * kHeadDim + d0) =
-            u32x2{E::pack2(sum[0] * inv, sum[1] * inv), E::pack2(sum[2] * inv, sum[3] * inv)};
+        put_row(set_row, sum, l_all);
     }
 }
 
