@@ -8,7 +8,7 @@ from __future__ import annotations
 import ctypes
 import os
 import subprocess
-from ctypes import POINTER, c_char_p, c_float, c_int32, c_int64, c_void_p
+from ctypes import POINTER, c_char_p, c_float, c_int16, c_int32, c_int64, c_void_p
 from typing import Optional
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -26,7 +26,7 @@ class MixedPlanInfo(ctypes.Structure):
     """dskv_mixed_plan_t of include/dskv.h."""
     _fields_ = [("n_tiles", c_int32), ("n_splits", c_int32), ("n_tile_rows", c_int32),
                 ("n_decode_rows", c_int32), ("n_decode_items", c_int32), ("n_decode_workgroups", c_int32),
-                ("layout", c_int32), ("new_rows_late", c_int32), ("plan_words", c_int64), ("decode_plan_at", c_int64), ("row_map_at", c_int64),
+                ("layout", c_int32), ("new_rows_late", c_int16), ("tile_workgroups", c_int16), ("plan_words", c_int64), ("decode_plan_at", c_int64), ("row_map_at", c_int64),
                 ("tile_workspace_bytes", c_int64),
                 ("decode_workspace_bytes", c_int64)]
 

@@ -37,6 +37,7 @@
 #include <vector>
 
 #include "prefill_kernel.h"
+#include "prefill_short_kernel.h"
 
 namespace dskv {
 
@@ -256,6 +257,42 @@ namespace dskv {
 // row is computed by the decode kernel).  Plan: the tile entries (kTileWords each), then, if
 // any tile is cut into parts, two words per query row of the batch (first partial slot,
 // number of parts; 0 parts = the row needs no merge).
+static bool prefill_mfma_path(int dtype, int head_dim, int n_qo_heads, int n_kv_heads, float scale_log2)
+{
+    // the MFMA kernel takes maxima before scaling: it needs a positive, sane scale
+    return (dtype == DSKV_BF16 || dtype == DSKV_F16) && head_dim == kHeadDim && n_kv_heads > 0 &&
+           n_qo_heads / n_kv_heads <= kWaveCols && scale_log2 > 1e-6f && scale_log2 < 1e6f;
+}
+
+// Tiles of few and short walks (prefill_short_kernel.h): in quarters or halves, or as they are.
+// A quarter is for a launch whose quarters with rows have a compute unit each: 16 more would be a second turn of all
+// (bf16, 8 kv heads, groups of 4, us a layer, as they are -> quarters -> halves: 8 prompts of 64, 256 quarters:
+// 15.1 -> 10.2 -> 12.3; 8 of 128, 512 quarters: 19.5 -> 19.5 -> 16.5; 16 of 128, 512 halves: 24.9 -> 33.0 -> 29.7).
+// A workgroup has 256 keys in LDS and waits for memory anew for the next ones, a tile's ring does not; with half the
+// waves for the keys it has lost what it gained by the second time (a prompt of 256 tokens: 18.9 -> 13.8 -> 16.9; of
+// 512: 24.8 -> 20.3 -> 25.0), and the other pays for the second time only where it has columns enough to use the matrix
+// pipeline for (128 tokens behind 300: 22.3 -> 18.3, 32 behind 400: 21.4 -> 21.5, 16 behind 500: 19.4 -> 20.7).
+constexpr int64_t kShortKeys = kShortRoundTokens, kShortTwiceKeys = 2 * kShortRoundTokens;
+static int short_walk_workgroups(const int32_t *qo_indptr_host, const int32_t *kv_len_host, const int32_t *plan_host,
+                                 int32_t n_tiles, int32_t n_qo_heads, int32_t n_kv_heads)
+{
+    const int rows = prefill_rows_per_tile(n_qo_heads, n_kv_heads, kPrefillWaves), quarter = rows / 4;
+    int64_t quarters = 0, halves = 0;
+    bool once = true;
+    if (n_tiles == 0 || n_tiles > compute_units()) return 0;
+    for (int32_t i = 0; i < n_tiles; i++) {
+        const int32_t *e = plan_host + (int64_t)i * kTileWords;
+        const int64_t n_b = (int64_t)qo_indptr_host[e[0] + 1] - qo_indptr_host[e[0]];
+        const int64_t live = std::min<int64_t>(rows, n_b - e[1]), keys = kv_len_host[e[0]] - n_b + e[1] + live;
+        if (keys > (n_b > rows / 2 ? kShortTwiceKeys : kShortKeys)) return 0;
+        once = once && keys <= kShortKeys;
+        quarters += (live + quarter - 1) / quarter;
+        halves += (live + 2 * quarter - 1) / (2 * quarter);
+    }
+    if (quarters * n_kv_heads <= compute_units()) return 4;
+    return once && halves * n_kv_heads <= compute_units() ? 2 : 0;
+}
+
 static int plan_tiles(const int32_t *qo_indptr_host, const int32_t *kv_len_host, const char *skip,
                       int32_t batch, int32_t n_qo_heads, int32_t n_kv_heads, int32_t head_dim,
                       int32_t target_workgroups, int32_t *plan_host, int64_t capacity_words,
@@ -529,6 +566,9 @@ extern "C" int dskv_mixed_plan_typed(const int32_t *qo_indptr_host, const int32_
         if (meets && ((int64_t)e[2] + kAppendAheadBlocks) * kBlock > prior) info->new_rows_late = 0;
     }
     info->n_tile_rows = (int32_t)n_tile_rows;
+    if (rows.empty() && target_workgroups == 0 && info->n_splits == 1 && !info->new_rows_late && page_size >= 8 &&
+        is_pow2(page_size) && prefill_mfma_path(dtype, head_dim, n_qo_heads, n_kv_heads, 1.f))
+        info->tile_workgroups = short_walk_workgroups(qo_indptr_host, kv_len.data(), plan_host, info->n_tiles, n_qo_heads, n_kv_heads);
     int64_t at = (tile_words + 3) / 4 * 4;
     info->plan_words = tile_words;
     if (rows.empty()) return 0;
@@ -582,13 +622,6 @@ static int launch_parts_merge(void *out, const float *part_o, const float *part_
                               const int32_t *row_parts, int32_t nnz, int64_t max_slots,
                               int32_t n_qo_heads, int32_t dtype, hipStream_t s);
 
-static bool prefill_mfma_path(int dtype, int head_dim, int n_qo_heads, int n_kv_heads, float scale_log2)
-{
-    // the MFMA kernel takes maxima before scaling: it needs a positive, sane scale
-    return (dtype == DSKV_BF16 || dtype == DSKV_F16) && head_dim == kHeadDim && n_kv_heads > 0 &&
-           n_qo_heads / n_kv_heads <= kWaveCols && scale_log2 > 1e-6f && scale_log2 < 1e6f;
-}
-
 // some_rows_elsewhere: the tiles do not cover all nnz rows of the batch (the others are the
 // decode kernel's); an MFMA-path call with n_tiles == 0 then has nothing to do.
 static int prefill_attn_impl(void *out, const void *q, const int32_t *qo_indptr,
@@ -599,7 +632,7 @@ static int prefill_attn_impl(void *out, const void *q, const int32_t *qo_indptr,
                              int32_t n_qo_heads, int32_t n_kv_heads, int32_t head_dim,
                              int32_t page_size, float sm_scale, int32_t causal, int32_t dtype,
                              void *stream, bool some_rows_elsewhere, const float *rope_table = nullptr,
-                             const AppendRows &append = AppendRows{})
+                             const AppendRows &append = AppendRows{}, int tile_workgroups = 0)
 {
     DSKV_REQUIRE(batch >= 0 && nnz >= 0 && n_tiles >= 0, "prefill_attn: negative sizes");
     if (batch == 0 || nnz == 0) return 0;
@@ -644,6 +677,32 @@ static int prefill_attn_impl(void *out, const void *q, const int32_t *qo_indptr,
         dim3 grid((unsigned)n_tiles * (unsigned)n_kv_heads);
         dim3 block(64 * kPrefillWaves);
         const int shift = ilog2(page_size);
+        // (the plan's choice; a launch that appends new rows does so in the kernel of long walks)
+        if ((tile_workgroups == 2 || tile_workgroups == 4) && !append.k && n_splits == 1 && page_size >= 8 && n_tiles <= 65535) {
+            const int group = n_qo_heads / n_kv_heads;
+            const ShortArgs short_args = {plan_dev, qo_indptr, kv_page_indptr, kv_last_page_len, kv_page_indices,
+                                          (const char *)pages_layer, (const uint16_t *)q, rope_table, (uint16_t *)out,
+                                          n_tiles, n_qo_heads, n_kv_heads, group, 65536 / group + 1, shift, causal, scale_log2};
+#define DSKV_LAUNCH_SHORT_W(DT, W, ROWS)                                                                         \
+    hipLaunchKernelGGL((prefill_short_kernel<DT, W, ROWS>), dim3((unsigned)n_kv_heads, (unsigned)n_tiles, kPrefillWaves / W), \
+                       dim3(64 * kShortWaves), 0, s, short_args)
+#define DSKV_LAUNCH_SHORT(DT, ROWS)                                       \
+    do {                                                                  \
+        if (tile_workgroups == 4) DSKV_LAUNCH_SHORT_W(DT, 2, ROWS);       \
+        else DSKV_LAUNCH_SHORT_W(DT, 4, ROWS);                            \
+    } while (0)
+            if (dtype == DSKV_BF16) {
+                if (page_size >= 16) DSKV_LAUNCH_SHORT(DSKV_BF16, 16);
+                else DSKV_LAUNCH_SHORT(DSKV_BF16, 8);
+            } else {
+                if (page_size >= 16) DSKV_LAUNCH_SHORT(DSKV_F16, 16);
+                else DSKV_LAUNCH_SHORT(DSKV_F16, 8);
+            }
+#undef DSKV_LAUNCH_SHORT
+#undef DSKV_LAUNCH_SHORT_W
+            DSKV_LAUNCH_CHECK("prefill_short_kernel");
+            return 0;
+        }
         const PrefillArgs args = {append, (uint16_t *)out, (const uint16_t *)q, qo_indptr, (const char *)pages_layer,
                                   kv_page_indices, kv_page_indptr, kv_last_page_len, plan_dev, n_qo_heads, n_kv_heads,
                                   shift, scale_log2, causal, part_o, part_ml, (int)max_slots, rope_table};
@@ -836,7 +895,8 @@ static int mixed_attn_impl(void *out, const void *q, const int32_t *qo_indptr, c
         return prefill_attn_impl(out, q, qo_indptr, pages_layer, kv_page_indices, kv_page_indptr,
                                  kv_last_page_len, plan_dev, info->n_tiles, info->n_splits, workspace,
                                  workspace_bytes, batch, nnz, n_qo_heads, n_kv_heads, head_dim,
-                                 page_size, sm_scale, causal, dtype, stream, false, rope_table, append);
+                                 page_size, sm_scale, causal, dtype, stream, false, rope_table, append,
+                                 info->tile_workgroups);
     DSKV_REQUIRE(plan_dev, "mixed_attn: missing plan");
     DSKV_REQUIRE(info->n_decode_rows + info->n_tile_rows == nnz && info->n_decode_rows <= batch,
                  "mixed_attn: the plan covers %d + %d rows, the batch has %d", info->n_decode_rows,
