@@ -34,6 +34,7 @@
 #include <algorithm>
 #include <atomic>
 #include <new>
+#include <numeric>
 #include <vector>
 
 #include "prefill_kernel.h"
@@ -228,6 +229,16 @@ constexpr int kMinSharedLaunchRows = 12;
 // ... and when, run as tiles (one live row per tile), they would be most of the launch's work:
 // a tile is priced at its 32-token blocks plus this much for its start and end.
 constexpr int kTileFixedCostBlocks = 16;
+// ... or if a launch of tiles had a walk longer than 3/2 of those of the shared one's tiles and this many blocks more.
+constexpr int kLongWalkBlocks = 16;
+// A dozen rows and more stay with the tiles where these have a compute unit each, walk at most kFewBlocks and at most
+// kFewerBlocks more than the shared launch's tiles (8 kv heads, us a layer, shared -> tiles: 23 rows of 282 beside 5
+// tokens behind 366 21.9 -> 17.3, 29 of 465 beside 78 behind 253 25.3 -> 22.3, groups of 8, 29 of 69 to 276 beside 14 behind
+// 549 25.7 -> 19.9; 12 blocks against 1: 15.2 -> 17.1).
+constexpr int kFewBlocks = 32, kFewerBlocks = 8;
+// (a shared launch's tile counts this much more where there are many: four of 350 to 980 beside eight of 100 to 230,
+// groups of 8, 31.8 as tiles and 36.9 shared)
+constexpr int kSharedTileOverheadBlocks = 8;
 
 static int compute_units()
 {
@@ -533,29 +544,90 @@ extern "C" int dskv_mixed_plan_typed(const int32_t *qo_indptr_host, const int32_
             tile_cost += (keys + kBlock - 1) / kBlock + kTileFixedCostBlocks;
         }
     }
-    int layout = DSKV_LAYOUT_SEPARATE;
+    // How long a launch of tiles lasts that does not fill the chip: as long as its longest walk.  A few rows of long
+    // context are such walks (of 343 blocks beside two prompts), cut into parts or not, where the shared launch spreads
+    // them over all compute units; and as tiles they use up the parts that the chunks' tiles would be cut into.
+    // Microseconds a layer, all as tiles -> shared (8 kv heads, groups of 4): one row of 900 tokens beside a prompt of 40
+    // 25.7 -> 17.4, of 10000 beside three of 67 53.3 -> 22.7; four of 3000 beside two chunks of 512 behind 500 69 -> 42,
+    // eleven of 150 beside a chunk of 512 behind 3000 88 -> 55; groups of 8, two of 10000 beside three of 67
+    // 91 -> 29.  It loses where the walks are no longer than its own tiles' (two of 3000 beside a chunk of 512 behind 3000,
+    // 44 blocks against 56: 54 -> 61; groups of 8, two of 3000 beside 200 behind 1000, 44 against 32: 40 -> 43; six of
+    // 1100 to 1700 beside two of 47, 28 against 9: 26.7 -> 30.5), hence 3/2 of them and kLongWalkBlocks.  And where the kernel
+    // of short walks takes all rows it loses however many rows there are (twelve of 50 beside three of 30:
+    // 9.2 -> 14.9, sixteen of 55, groups of 8: 10.3 -> 16.4).
+    auto plan_all = [&](int layout, int64_t *words) {
+        const bool shared = layout == DSKV_LAYOUT_SHARED;
+        return plan_tiles(qo_indptr_host, kv_len.data(), rows.empty() ? nullptr : routed.data(), batch, n_qo_heads, n_kv_heads,
+                          head_dim, target_workgroups, plan_host, capacity_words, &info->n_tiles, &info->n_splits, words,
+                          &info->tile_workspace_bytes, shared ? kPrefillWavesShared : kPrefillWaves,
+                          /* the tiles of a shared launch run beside decode workgroups for its whole length */ !shared);
+    };
+    // blocks of the plan's longest walk; spread: no less than what a compute unit gets of all of them
+    auto walk_of_plan = [&](int waves, bool spread) {
+        const int64_t tile_rows = prefill_rows_per_tile(n_qo_heads, n_kv_heads, waves);
+        int64_t longest = 0, total = 0;
+        for (int32_t i = 0; i < info->n_tiles; i++) {
+            const int32_t *e = plan_host + (int64_t)i * kTileWords;
+            const int64_t n_b = (int64_t)qo_indptr_host[e[0] + 1] - qo_indptr_host[e[0]];
+            const int64_t keys = kv_len[e[0]] - n_b + std::min<int64_t>(e[1] + tile_rows, n_b);
+            const int64_t blocks = std::max<int64_t>(std::min<int64_t>(e[3], (keys + kBlock - 1) / kBlock) - e[2], 0);
+            longest = std::max(longest, blocks);
+            total += blocks + kSharedTileOverheadBlocks;
+        }
+        return spread ? std::max(longest, total * n_kv_heads / compute_units()) : longest;
+    };
+    auto short_walks = [&] {
+        if (target_workgroups != 0 || info->n_splits != 1 || page_size < 8 || !is_pow2(page_size) ||
+            !prefill_mfma_path(dtype, head_dim, n_qo_heads, n_kv_heads, 1.f))
+            return 0;
+        return short_walk_workgroups(qo_indptr_host, kv_len.data(), plan_host, info->n_tiles, n_qo_heads, n_kv_heads);
+    };
+    int layout = DSKV_LAYOUT_SEPARATE, rc = 0;
+    int64_t tile_words = 0;
+    bool planned = false;
     if (!rows.empty() && n_tile_rows > 0) {
-        const bool can_share = page_size >= 4;
-        if (route_one_row_requests == DSKV_ROUTE_SHARED_LAUNCH ||
-            (route_one_row_requests == DSKV_ROUTE_AUTO && (int64_t)rows.size() >= kMinSharedLaunchRows &&
-             decode_cost >= tile_cost))
+        const bool can_share = page_size >= 4, choose = route_one_row_requests == DSKV_ROUTE_AUTO;
+        const bool most = choose && (int64_t)rows.size() >= kMinSharedLaunchRows && decode_cost >= tile_cost;
+        // (a caller with less room than any plan may need keeps the form that it has room for)
+        const bool weighs = choose && target_workgroups == 0 && prefill_mfma_path(dtype, head_dim, n_qo_heads, n_kv_heads, 1.f) &&
+                            capacity_words >= dskv_mixed_plan_bound(batch, qo_indptr_host[batch],
+                                                                    std::accumulate(kv_len.begin(), kv_len.end(), int64_t(0)));
+        // (only a launch that gives every tile a compute unit may be better than most rows shared)
+        const bool may_fit = weighs &&
+                             ((int64_t)rows.size() + (n_tile_rows + rows_per_tile - 1) / rows_per_tile) * n_kv_heads <= compute_units();
+        if (route_one_row_requests == DSKV_ROUTE_SHARED_LAUNCH || (most && !may_fit))
             layout = can_share ? DSKV_LAYOUT_SHARED : DSKV_LAYOUT_SEPARATE;
         if (layout != DSKV_LAYOUT_SHARED && route_one_row_requests != DSKV_ROUTE_TWO_LAUNCHES) {
-            // not worth it, or not possible: everything as tiles
-            rows.clear();
-            std::fill(routed.begin(), routed.end(), 0);
-            n_tile_rows = qo_indptr_host[batch];
+            // everything as tiles, and a look at whether that is the better form where sharing is possible
+            const std::vector<DecodeRow> decode_rows = std::move(rows);
+            const std::vector<char> decode_routed = routed;
+            const int64_t chunk_rows = n_tile_rows;
+            auto take_rows_out = [&](bool out) {
+                if (out) rows = decode_rows, routed = decode_routed;
+                else rows.clear(), std::fill(routed.begin(), routed.end(), 0);
+            };
+            take_rows_out(false);
+            if ((rc = plan_all(layout, &tile_words))) return rc;
+            planned = true;
+            const int64_t walk = walk_of_plan(kPrefillWaves, false);
+            const bool few = (int64_t)info->n_tiles * n_kv_heads <= compute_units() && walk <= kFewBlocks;
+            bool shared = can_share && weighs && (most || walk > kLongWalkBlocks) && !short_walks();
+            if (shared) {
+                take_rows_out(true);
+                if ((rc = plan_all(DSKV_LAYOUT_SHARED, &tile_words))) return rc;
+                shared = most ? !few || walk > walk_of_plan(kPrefillWavesShared, false) + kFewerBlocks
+                              : 2 * (walk - kLongWalkBlocks) >= 3 * walk_of_plan(kPrefillWavesShared, true);
+                if (!shared) {
+                    take_rows_out(false);
+                    if ((rc = plan_all(layout, &tile_words))) return rc;
+                }
+            }
+            if (shared) layout = DSKV_LAYOUT_SHARED;
+            n_tile_rows = shared ? chunk_rows : qo_indptr_host[batch];
         }
     }
     info->layout = layout;
-    const int waves = layout == DSKV_LAYOUT_SHARED ? kPrefillWavesShared : kPrefillWaves;
-    int64_t tile_words = 0;
-    int rc = plan_tiles(qo_indptr_host, kv_len.data(), rows.empty() ? nullptr : routed.data(), batch,
-                        n_qo_heads, n_kv_heads, head_dim, target_workgroups, plan_host, capacity_words,
-                        &info->n_tiles, &info->n_splits, &tile_words, &info->tile_workspace_bytes, waves,
-                        /* the tiles of a shared launch run beside decode workgroups for its whole length */
-                        layout != DSKV_LAYOUT_SHARED);
-    if (rc) return rc;
+    if (!planned && (rc = plan_all(layout, &tile_words))) return rc;
     info->tile_workspace_bytes = (info->tile_workspace_bytes + 255) / 256 * 256;
     // whether every walk that meets new rows has kAppendAheadBlocks in front of them (tiles_append)
     info->new_rows_late = info->n_tiles > 0;
@@ -566,15 +638,14 @@ extern "C" int dskv_mixed_plan_typed(const int32_t *qo_indptr_host, const int32_
         if (meets && ((int64_t)e[2] + kAppendAheadBlocks) * kBlock > prior) info->new_rows_late = 0;
     }
     info->n_tile_rows = (int32_t)n_tile_rows;
-    if (rows.empty() && target_workgroups == 0 && info->n_splits == 1 && !info->new_rows_late && page_size >= 8 &&
-        is_pow2(page_size) && prefill_mfma_path(dtype, head_dim, n_qo_heads, n_kv_heads, 1.f))
-        info->tile_workgroups = short_walk_workgroups(qo_indptr_host, kv_len.data(), plan_host, info->n_tiles, n_qo_heads, n_kv_heads);
+    if (rows.empty() && !info->new_rows_late) info->tile_workgroups = short_walks();
     int64_t at = (tile_words + 3) / 4 * 4;
     info->plan_words = tile_words;
     if (rows.empty()) return 0;
     info->decode_plan_at = at;
     int64_t decode_words = 0;
     if (at > capacity_words) at = capacity_words;   // the decode planner then reports the shortage
+    std::fill(plan_host + tile_words, plan_host + std::max(at, tile_words), 0);   // (words of a plan made before)
     // shared launch: one decode workgroup (a share x a group of four kv heads) per compute unit
     int32_t decode_target = target_workgroups;
     if (layout == DSKV_LAYOUT_SHARED) {

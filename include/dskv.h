@@ -310,12 +310,13 @@ int dskv_prefill_attn(void *out, const void *q, const int32_t *qo_indptr, const 
  * dskv_prefill_plan / dskv_prefill_attn.  fp32 data is computed by the generic kernel,
  * whatever the plan routed.
  * With DSKV_ROUTE_AUTO a batch of one-row requests only runs the decode pass alone; a batch
- * of both kinds runs as ONE launch (DSKV_LAYOUT_SHARED: pages of at least 4 tokens, at least
+ * of both kinds runs as ONE launch (DSKV_LAYOUT_SHARED: pages of at least 4 tokens; at least
  * 12 one-row requests, which as query tiles of their own would be at least half of the launch's
- * work) in which every compute unit hosts a decode workgroup, which keeps its memory path
+ * work, or - 16-bit types, target_workgroups 0, room for dskv_mixed_plan_bound words - any number of them whose
+ * tiles would walk far longer than the others') in which every compute unit hosts a decode workgroup, which keeps its memory path
  * busy, and tile workgroups beside it, which use its matrix pipeline, followed by one merge
  * pass for both kinds of rows - or, where that launch does not apply or does not pay (a handful
- * of decode rows, a large prefill batch), as tiles only.  The two other modes force a layout
+ * of short decode rows, short walks throughout, a large prefill batch), as tiles only.  The two other modes force a layout
  * (for measurements and tests).
  * The plan (at most dskv_mixed_plan_bound words; upload the first info->plan_words) holds
  * the tile plan (entries, then the rows' parts if a tile is cut), then at word
