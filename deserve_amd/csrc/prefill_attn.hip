@@ -231,11 +231,12 @@ constexpr int kMinSharedLaunchRows = 12;
 constexpr int kTileFixedCostBlocks = 16;
 // ... or if a launch of tiles had a walk longer than 3/2 of those of the shared one's tiles and this many blocks more.
 constexpr int kLongWalkBlocks = 16;
-// A dozen rows and more stay with the tiles where these have a compute unit each, walk at most kFewBlocks and at most
+// A dozen rows and more stay with the tiles where these are whole, have a compute unit each, walk at most kFewBlocks and at most
 // kFewerBlocks more than the shared launch's tiles (8 kv heads, us a layer, shared -> tiles: 23 rows of 282 beside 5
 // tokens behind 366 21.9 -> 17.3, 29 of 465 beside 78 behind 253 25.3 -> 22.3, groups of 8, 29 of 69 to 276 beside 14 behind
-// 549 25.7 -> 19.9; 12 blocks against 1: 15.2 -> 17.1).
-constexpr int kFewBlocks = 32, kFewerBlocks = 8;
+// 549 25.7 -> 19.9, 29 of 204 to 402 beside 66 behind 628 30.6 -> 24.4; 12 blocks against 1: 15.2 -> 17.1, 9 against 1
+// 14.6 -> 15.6; eleven of 150 beside 200 behind 1000, in two parts, 29.6 -> 33.5).
+constexpr int kFewBlocks = 32, kFewerBlocks = 6;
 // (a shared launch's tile counts this much more where there are many: four of 350 to 980 beside eight of 100 to 230,
 // groups of 8, 31.8 as tiles and 36.9 shared)
 constexpr int kSharedTileOverheadBlocks = 8;
@@ -281,9 +282,11 @@ static bool prefill_mfma_path(int dtype, int head_dim, int n_qo_heads, int n_kv_
 // 15.1 -> 10.2 -> 12.3; 8 of 128, 512 quarters: 19.5 -> 19.5 -> 16.5; 16 of 128, 512 halves: 24.9 -> 33.0 -> 29.7).
 // A workgroup has 256 keys in LDS and waits for memory anew for the next ones, a tile's ring does not; with half the
 // waves for the keys it has lost what it gained by the second time (a prompt of 256 tokens: 18.9 -> 13.8 -> 16.9; of
-// 512: 24.8 -> 20.3 -> 25.0), and the other pays for the second time only where it has columns enough to use the matrix
-// pipeline for (128 tokens behind 300: 22.3 -> 18.3, 32 behind 400: 21.4 -> 21.5, 16 behind 500: 19.4 -> 20.7).
-constexpr int64_t kShortKeys = kShortRoundTokens, kShortTwiceKeys = 2 * kShortRoundTokens;
+// 512: 24.8 -> 20.3 -> 25.0), and the other pays for more only where it has columns enough to use the matrix
+// pipeline for (128 tokens behind 300: 22.3 -> 18.3, 32 behind 400: 21.4 -> 21.5, 16 behind 500: 19.4 -> 20.7), and up
+// to the fourth time (64 tokens behind 450 24.4 -> 20.7, behind 900 33.8 -> 30.3; 181 behind 450 27.0 -> 23.0, behind 900, where
+// the tiles would be in two parts, 38.0 -> 33.0; 512 behind 450 34.6 -> 32.1; 64 behind 1500, in three parts, 31.3 -> 43.9).
+constexpr int64_t kShortKeys = kShortRoundTokens, kShortMostKeys = 4 * kShortRoundTokens;
 static int short_walk_workgroups(const int32_t *qo_indptr_host, const int32_t *kv_len_host, const int32_t *plan_host,
                                  int32_t n_tiles, int32_t n_qo_heads, int32_t n_kv_heads)
 {
@@ -293,9 +296,10 @@ static int short_walk_workgroups(const int32_t *qo_indptr_host, const int32_t *k
     if (n_tiles == 0 || n_tiles > compute_units()) return 0;
     for (int32_t i = 0; i < n_tiles; i++) {
         const int32_t *e = plan_host + (int64_t)i * kTileWords;
+        if (e[2] != 0) continue;   // a tile's second part
         const int64_t n_b = (int64_t)qo_indptr_host[e[0] + 1] - qo_indptr_host[e[0]];
         const int64_t live = std::min<int64_t>(rows, n_b - e[1]), keys = kv_len_host[e[0]] - n_b + e[1] + live;
-        if (keys > (n_b > rows / 2 ? kShortTwiceKeys : kShortKeys)) return 0;
+        if (keys > (n_b > rows / 2 ? kShortMostKeys : kShortKeys)) return 0;
         once = once && keys <= kShortKeys;
         quarters += (live + quarter - 1) / quarter;
         halves += (live + 2 * quarter - 1) / (2 * quarter);
@@ -555,10 +559,10 @@ extern "C" int dskv_mixed_plan_typed(const int32_t *qo_indptr_host, const int32_
     // 1100 to 1700 beside two of 47, 28 against 9: 26.7 -> 30.5), hence 3/2 of them and kLongWalkBlocks.  And where the kernel
     // of short walks takes all rows it loses however many rows there are (twelve of 50 beside three of 30:
     // 9.2 -> 14.9, sixteen of 55, groups of 8: 10.3 -> 16.4).
-    auto plan_all = [&](int layout, int64_t *words) {
+    auto plan_all = [&](int layout, int64_t *words, bool in_parts = true) {
         const bool shared = layout == DSKV_LAYOUT_SHARED;
         return plan_tiles(qo_indptr_host, kv_len.data(), rows.empty() ? nullptr : routed.data(), batch, n_qo_heads, n_kv_heads,
-                          head_dim, target_workgroups, plan_host, capacity_words, &info->n_tiles, &info->n_splits, words,
+                          head_dim, in_parts ? target_workgroups : -1, plan_host, capacity_words, &info->n_tiles, &info->n_splits, words,
                           &info->tile_workspace_bytes, shared ? kPrefillWavesShared : kPrefillWaves,
                           /* the tiles of a shared launch run beside decode workgroups for its whole length */ !shared);
     };
@@ -577,7 +581,7 @@ extern "C" int dskv_mixed_plan_typed(const int32_t *qo_indptr_host, const int32_
         return spread ? std::max(longest, total * n_kv_heads / compute_units()) : longest;
     };
     auto short_walks = [&] {
-        if (target_workgroups != 0 || info->n_splits != 1 || page_size < 8 || !is_pow2(page_size) ||
+        if (target_workgroups != 0 || page_size < 8 || !is_pow2(page_size) ||
             !prefill_mfma_path(dtype, head_dim, n_qo_heads, n_kv_heads, 1.f))
             return 0;
         return short_walk_workgroups(qo_indptr_host, kv_len.data(), plan_host, info->n_tiles, n_qo_heads, n_kv_heads);
@@ -610,8 +614,8 @@ extern "C" int dskv_mixed_plan_typed(const int32_t *qo_indptr_host, const int32_
             if ((rc = plan_all(layout, &tile_words))) return rc;
             planned = true;
             const int64_t walk = walk_of_plan(kPrefillWaves, false);
-            const bool few = (int64_t)info->n_tiles * n_kv_heads <= compute_units() && walk <= kFewBlocks;
-            bool shared = can_share && weighs && (most || walk > kLongWalkBlocks) && !short_walks();
+            const bool few = (int64_t)info->n_tiles * n_kv_heads <= compute_units() && info->n_splits == 1 && walk <= kFewBlocks;
+            bool shared = can_share && weighs && (walk > kLongWalkBlocks || (most && !short_walks()));
             if (shared) {
                 take_rows_out(true);
                 if ((rc = plan_all(DSKV_LAYOUT_SHARED, &tile_words))) return rc;
@@ -628,8 +632,11 @@ extern "C" int dskv_mixed_plan_typed(const int32_t *qo_indptr_host, const int32_
     }
     info->layout = layout;
     if (!planned && (rc = plan_all(layout, &tile_words))) return rc;
+    const int tile_workgroups = rows.empty() ? short_walks() : 0;
+    if (tile_workgroups && info->n_splits > 1 && (rc = plan_all(layout, &tile_words, false))) return rc;
     info->tile_workspace_bytes = (info->tile_workspace_bytes + 255) / 256 * 256;
     // whether every walk that meets new rows has kAppendAheadBlocks in front of them (tiles_append)
+    info->tile_workgroups = tile_workgroups;
     info->new_rows_late = info->n_tiles > 0;
     for (int32_t i = 0; i < info->n_tiles && info->new_rows_late; i++) {
         const int32_t *e = plan_host + (int64_t)i * kTileWords;
@@ -638,7 +645,6 @@ extern "C" int dskv_mixed_plan_typed(const int32_t *qo_indptr_host, const int32_
         if (meets && ((int64_t)e[2] + kAppendAheadBlocks) * kBlock > prior) info->new_rows_late = 0;
     }
     info->n_tile_rows = (int32_t)n_tile_rows;
-    if (rows.empty() && !info->new_rows_late) info->tile_workgroups = short_walks();
     int64_t at = (tile_words + 3) / 4 * 4;
     info->plan_words = tile_words;
     if (rows.empty()) return 0;
@@ -748,7 +754,7 @@ static int prefill_attn_impl(void *out, const void *q, const int32_t *qo_indptr,
         dim3 grid((unsigned)n_tiles * (unsigned)n_kv_heads);
         dim3 block(64 * kPrefillWaves);
         const int shift = ilog2(page_size);
-        // (the plan's choice; a launch that appends new rows does so in the kernel of long walks)
+        // (the plan's choice; the rows are appended in front)
         if ((tile_workgroups == 2 || tile_workgroups == 4) && !append.k && n_splits == 1 && page_size >= 8 && n_tiles <= 65535) {
             const int group = n_qo_heads / n_kv_heads;
             const ShortArgs short_args = {plan_dev, qo_indptr, kv_page_indptr, kv_last_page_len, kv_page_indices,
@@ -1039,7 +1045,9 @@ static bool tiles_append(const dskv_mixed_step_t &s, const void *out, const void
         const uintptr_t at = (uintptr_t)rows, o = (uintptr_t)out, w = (uintptr_t)s.workspace;
         if ((at < o + out_bytes && o < at + kv_bytes) || (at < w + s.workspace_bytes && w < at + kv_bytes)) return false;
     }
-    if (!s.info->new_rows_late || s.page_size < 4 || s.info->n_decode_rows > 0 || s.info->n_tiles <= 0 || s.batch > kAppendMaxBatch ||
+    // (short walks are shared instead: 181 tokens behind 456 27.7 us a layer with the append in the launch, 22.9 shared, with
+    // it in front; 512 behind 450 35.8 and 32.0)
+    if (!s.info->new_rows_late || s.info->tile_workgroups || s.page_size < 4 || s.info->n_decode_rows > 0 || s.info->n_tiles <= 0 || s.batch > kAppendMaxBatch ||
         s.n_kv_heads > kAppendFlags || ((uintptr_t)pages_layer % 256) || (((uintptr_t)k | (uintptr_t)v) % 16))
         return false;
     a.n_tiles = std::min(s.info->n_tiles, kAppendFlags / s.n_kv_heads);

@@ -9,7 +9,7 @@
 // 256 keys come into LDS at once, with one wait and one barrier, and the key groups' sums meet in LDS.
 // Measured with the launch that appends the new rows (bf16, 8 kv heads, groups of 4, us a layer, in the kernel of long
 // walks -> here): prompts of 20 tokens 12.0 -> 8.3, of 128 16.2 -> 11.0, of 256 18.9 -> 13.8; three of 17 to 203
-// 17.7 -> 13.6; 64 tokens behind 190 18.6 -> 13.4; 8 prompts of 128 (halves) 19.5 -> 16.5.
+// 17.7 -> 13.6; 64 tokens behind 190 18.6 -> 13.4, behind 450 24.4 -> 20.7; 8 prompts of 128 (halves) 19.5 -> 16.5.
 // The append inside this launch (rows from k and v, K rotated on the way into LDS) was slower than in front of it: 18.7
 // against 13.6 for three prompts, the walk's registers spilled.
 #pragma once

@@ -343,7 +343,8 @@ typedef struct dskv_mixed_plan {
     int32_t layout;
     int16_t new_rows_late;            /* every tile entry that sees new rows walks 12 blocks of 32 tokens before them */
     int16_t tile_workgroups;          /* few short walks (tiles only, none cut, pages of at least 8 tokens): workgroups
-                                         that share a tile's columns, 2 or 4; 0: one walks it (always right) */
+                                         that share a tile's columns, 2 or 4, new rows appended in front; 0: one walks
+                                         it (always right) */
     int64_t plan_words;
     int64_t decode_plan_at, row_map_at;
     int64_t tile_workspace_bytes, decode_workspace_bytes;

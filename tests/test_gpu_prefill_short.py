@@ -20,7 +20,9 @@ CASES = [
     ("one_round", [256, 255], [64, 256], 16, 32, 8, "bf16", 4),
     ("two_rounds", [257, 512, 289], [33, 64, 40], 16, 32, 8, "f16", 4),
     ("long_walk_of_few_columns", [257], [32], 16, 32, 8, "bf16", 0),
-    ("three_rounds", [513], [200], 16, 32, 8, "bf16", 0),
+    ("three_rounds", [513], [200], 16, 32, 8, "bf16", 4),
+    ("four_rounds_behind_tokens", [1024, 769, 60], [40, 64, 60], 8, 32, 8, "bf16", 4),
+    ("four_rounds_group8", [1000], [129], 16, 64, 8, "f16", 4),
     ("as_many_as_units", [128] * 4, [128] * 4, 16, 32, 8, "bf16", 4),
     ("one_more_than_units", [128] * 4 + [2], [128] * 4 + [2], 16, 32, 8, "bf16", 2),
     ("halves", [250] * 3 + [203, 17], [250] * 3 + [203, 17], 8, 32, 8, "f16", 2),
@@ -49,13 +51,26 @@ def test_which_plans_share_their_tiles():
         plan, info = np.zeros(cap, np.int32), _lib.MixedPlanInfo()
         rc = lib.dskv_mixed_plan_typed(qo_indptr.ctypes.data, pages.ctypes.data, last.ctypes.data, len(kv), P, Hq, Hkv, 128,
                                        _lib.BF16, 0, _lib.ROUTE_OFF, plan.ctypes.data, cap, ctypes.byref(info))
-        assert rc == 0 and not info.new_rows_late and info.n_splits == 1, name
+        assert rc == 0 and info.n_splits == 1, name
         assert info.tile_workgroups == workgroups and info.layout == _lib.LAYOUT_SEPARATE, name
         # a caller's own number of workgroups, 32 bits: never
         for target, route, typed in ((512, _lib.ROUTE_OFF, _lib.BF16), (0, _lib.ROUTE_OFF, _lib.F32)):
             assert lib.dskv_mixed_plan_typed(qo_indptr.ctypes.data, pages.ctypes.data, last.ctypes.data, len(kv), P, Hq, Hkv,
                                              128, typed, target, route, plan.ctypes.data, cap, ctypes.byref(info)) == 0
             assert info.tile_workgroups == 0, name
+
+
+def test_a_walk_past_four_rounds_is_cut():
+    lib = _lib.lib()
+    for keys, shared in ((1024, True), (1025, False)):
+        pages = -(-keys // 16)
+        qo, indptr, last = (np.array(a, np.int32) for a in ([0, 200], [0, pages], [keys - 16 * (pages - 1)]))
+        cap = lib.dskv_mixed_plan_bound(1, 200, keys)
+        plan, info = np.zeros(cap, np.int32), _lib.MixedPlanInfo()
+        assert lib.dskv_mixed_plan_typed(qo.ctypes.data, indptr.ctypes.data, last.ctypes.data, 1, 16, 32, 8, 128, _lib.BF16, 0,
+                                         _lib.ROUTE_AUTO, plan.ctypes.data, cap, ctypes.byref(info)) == 0
+        assert info.tile_workgroups == (4 if shared else 0) and info.n_splits == (1 if shared else 2)
+        assert info.tile_workspace_bytes == 0 or not shared
 
 
 @pytest.mark.gpu
