@@ -21,7 +21,8 @@
 // A wave's token is one, so everything between the links is scalar, the page of a power of two a
 // shift, and the common row sets have code without bounds: 104 vector instructions instead of 249 for 8 kv heads
 // with rotation.  Steps of a few prompts lost 0.5 to 0.7 us a layer of their 8 to 14 (3 prompts of 17 to 203: 13.95 ->
-// 13.35; 16 of 16 tokens: 9.3 -> 8.6), 8192 tokens 14.6 -> 13.7 us.
+// 13.35; 16 of 16 tokens: 9.3 -> 8.6).
+// Launches of many rows are bound by memory and take another form (kMany), see there.
 // Nontemporal stores: ordinary ones made a small step 0.1 us a layer faster (the next launch finds some rows in
 // its L2) and a mixed step of 512 tokens 2 us a layer slower (2334 -> 2368 us over 16 layers).
 #include "kv_tile.h"
@@ -48,12 +49,22 @@ struct AppendArgs {
 
 // kChunks: 16-byte chunks of a row set that a lane has in registers, where that is all of them (row sets of
 // 1, 2 or 4 KiB); 0: any row set, up to four in registers, more of them copied after the lookup.
-template <int DT, bool kRotate, int kChunks>
+// kMany: for launches that memory bounds, with more K than kAppendManyBytes (half the waves of a full chip at 2 KiB a row
+// set).  The rows are requested first, then the metadata, and the position and with it the page id are the vector
+// unit's.  That chain is longer (512 tokens 3.2 us instead of 2.8) and lets many waves through faster: 16 x 512
+// tokens of 8 heads, us without / with rotation, 13.1 / 13.0 -> 11.3 / 11.4 (5.9 TB/s).  Launches in a replayed
+// graph, scalar form -> this one: 2048 tokens 4.7 / 4.7 -> 4.4 / 4.5, 4096 7.6 / 7.7 -> 6.7 / 6.9, 16384 25.1 / 24.1 ->
+// 24.5 / 23.6; 16 heads, 1024 tokens 5.1 / 4.7 -> 4.9 / 5.0, 4096 13.4 / 13.3 -> 11.7 / 12.0; 4 heads, 4096 5.1 / 5.2 ->
+// 4.8 / 5.0; 100 requests of 81 tokens 13.8 / 12.7 -> 12.2 / 12.2.  The line lies above the last size at which it still
+// loses somewhere (4 MiB, 16 heads).
+constexpr int64_t kAppendManyBytes = 4 << 20;
+template <int DT, bool kRotate, int kChunks, bool kMany>
 __global__ __launch_bounds__(64 * kAppendWaves) void append_kernel(const AppendArgs a)
 {
     constexpr int kHeld = kChunks ? kChunks : kAppendMaxChunks;
     const int lane = threadIdx.x & 63;
-    const int t = blockIdx.x * kAppendWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = threadIdx.x >> 6;
+    const int t = blockIdx.x * kAppendWaves + (kMany ? wave : __builtin_amdgcn_readfirstlane(wave));
     // (all arguments in one trip)
     asm volatile("" ::"s"(a.pages), "s"(a.k), "s"(a.v), "s"(a.qo_indptr), "s"(a.kv_indices), "s"(a.kv_indptr), "s"(a.kv_last),
                  "s"(a.table), "s"(a.batch), "s"(a.nnz), "s"(a.num_pages), "s"(a.page_size), "s"(a.page_shift));
@@ -65,11 +76,14 @@ __global__ __launch_bounds__(64 * kAppendWaves) void append_kernel(const AppendA
     const int batch = a.batch;
     const bool by_ballot = batch < 64;
     int q_i = 0, p_i = 0, l_i = 0;
-    if (by_ballot) {
-        q_i = a.qo_indptr[min(lane, batch)];
-        p_i = a.kv_indptr[min(lane, batch)];
-        l_i = a.kv_last[min(lane, batch - 1)];
-    }
+    auto request_metadata = [&] {
+        if (by_ballot) {
+            q_i = a.qo_indptr[min(lane, batch)];
+            p_i = a.kv_indptr[min(lane, batch)];
+            l_i = a.kv_last[min(lane, batch - 1)];
+        }
+    };
+    if (!kMany) request_metadata();
     const bool in_regs = kChunks || row_bytes <= kAppendMaxChunks * 64 * 16;
     u32x4 rk[kHeld], rv[kHeld];
     if (in_regs) {
@@ -88,7 +102,8 @@ __global__ __launch_bounds__(64 * kAppendWaves) void append_kernel(const AppendA
         c4 = *reinterpret_cast<const f32x4 *>(tab);
         s4 = *reinterpret_cast<const f32x4 *>(tab + kAppendRotatePairs);
     }
-    asm volatile("" ::: "memory");   // (requested here, not where the branches below have met)
+    if (kMany) request_metadata();
+    else asm volatile("" ::: "memory");   // (requested here, not where the branches below have met)
     auto k_chunk = [&](const u32x4 &raw) {
         if (!kRotate) return raw;
         const float cs[4] = {c4[0], c4[1], c4[2], c4[3]}, sn[4] = {s4[0], s4[1], s4[2], s4[3]};
@@ -181,11 +196,17 @@ int launch_append(void *pages_layer, int32_t num_pages, const void *k, const voi
                                  (dtype == DSKV_BF16 || dtype == DSKV_F16)),
                  "append: rotation by a table takes 16-bit rows of head_dim %d", 2 * kAppendRotatePairs);
     const unsigned grid = (unsigned)((nnz + kAppendWaves - 1) / kAppendWaves);
+    const bool many = nnz * row_bytes > kAppendManyBytes;
     const AppendArgs args = {(char *)pages_layer, (const char *)k, (const char *)v, qo_indptr, kv_page_indices, kv_page_indptr,
                              kv_last_page_len, rope_table, batch, nnz, (int)row_bytes, num_pages, page_size,
                              is_pow2(page_size) ? ilog2(page_size) : -1};
-#define DSKV_LAUNCH_APPEND_CHUNKS(DT, ROTATE, CHUNKS) \
-    hipLaunchKernelGGL((append_kernel<DT, ROTATE, CHUNKS>), dim3(grid), dim3(64 * kAppendWaves), 0, stream, args)
+#define DSKV_LAUNCH_APPEND_FORM(DT, ROTATE, CHUNKS, MANY) \
+    hipLaunchKernelGGL((append_kernel<DT, ROTATE, CHUNKS, MANY>), dim3(grid), dim3(64 * kAppendWaves), 0, stream, args)
+#define DSKV_LAUNCH_APPEND_CHUNKS(DT, ROTATE, CHUNKS)                          \
+    do {                                                                       \
+        if (many) DSKV_LAUNCH_APPEND_FORM(DT, ROTATE, CHUNKS, true);           \
+        else DSKV_LAUNCH_APPEND_FORM(DT, ROTATE, CHUNKS, false);               \
+    } while (0)
 #define DSKV_LAUNCH_APPEND(DT, ROTATE)                                         \
     do {                                                                       \
         if (row_bytes == 1024) DSKV_LAUNCH_APPEND_CHUNKS(DT, ROTATE, 1);       \
@@ -197,6 +218,7 @@ int launch_append(void *pages_layer, int32_t num_pages, const void *k, const voi
     else if (dtype == DSKV_BF16) DSKV_LAUNCH_APPEND(DSKV_BF16, true);
     else DSKV_LAUNCH_APPEND(DSKV_F16, true);
 #undef DSKV_LAUNCH_APPEND_CHUNKS
+#undef DSKV_LAUNCH_APPEND_FORM
 #undef DSKV_LAUNCH_APPEND
     DSKV_LAUNCH_CHECK("append_kernel");
     return 0;
