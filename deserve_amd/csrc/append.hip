@@ -150,7 +150,7 @@ __global__ __launch_bounds__(64 * kAppendWaves) void append_kernel(const AppendA
     const int slot = (int)(pos - (long)nth * a.page_size);
 
     const long half_bytes = (long)a.page_size * row_bytes;
-    char *dst_k = a.pages + page * 2 * half_bytes + (long)slot * row_bytes;
+    char *dst_k = a.pages + (long)page * 2 * half_bytes + (long)slot * row_bytes;
     char *dst_v = dst_k + half_bytes;
     if (in_regs) {
 #pragma unroll
