@@ -100,11 +100,13 @@ static hipError_t link_copy(void *dst, const void *src, int64_t bytes, int64_t p
     const int64_t width = page_bytes >= kRowLow && page_bytes <= kRowHigh ? page_bytes : kRow;
     int64_t done = 0;
     if (bytes >= width && ((uintptr_t)dst | (uintptr_t)src | (uintptr_t)width) % 16 == 0) {
+        // (memory that HIP does not know is no failure, and the note of one would not be told from an error that the
+        // caller's thread has not fetched yet: with one pending nobody asks, and the copy is linear)
         hipPointerAttribute_t at{};
-        const bool pinned = hipPointerGetAttributes(&at, kind == hipMemcpyDeviceToHost ? dst : src) == hipSuccess &&
-                            at.type == hipMemoryTypeHost;
-        (void)hipGetLastError();   // memory that HIP does not know is no failure
-        if (pinned) {
+        const bool clear = hipPeekAtLastError() == hipSuccess;
+        const bool known = clear && hipPointerGetAttributes(&at, kind == hipMemcpyDeviceToHost ? dst : src) == hipSuccess;
+        if (clear && !known) (void)hipGetLastError();
+        if (known && at.type == hipMemoryTypeHost) {
             done = bytes / width * width;
             const hipError_t e = hipMemcpy2DAsync(dst, (size_t)width, src, (size_t)width, (size_t)width,
                                                   (size_t)(bytes / width), kind, s);
