@@ -231,12 +231,6 @@ constexpr int kMinSharedLaunchRows = 12;
 constexpr int kTileFixedCostBlocks = 16;
 // ... or if a launch of tiles had a walk longer than 3/2 of those of the shared one's tiles and this many blocks more.
 constexpr int kLongWalkBlocks = 16;
-// A dozen rows and more stay with the tiles where these are whole, have a compute unit each, walk at most kFewBlocks and at most
-// kFewerBlocks more than the shared launch's tiles (8 kv heads, us a layer, shared -> tiles: 23 rows of 282 beside 5
-// tokens behind 366 21.9 -> 17.3, 29 of 465 beside 78 behind 253 25.3 -> 22.3, groups of 8, 29 of 69 to 276 beside 14 behind
-// 549 25.7 -> 19.9, 29 of 204 to 402 beside 66 behind 628 30.6 -> 24.4; 12 blocks against 1: 15.2 -> 17.1, 9 against 1
-// 14.6 -> 15.6; eleven of 150 beside 200 behind 1000, in two parts, 29.6 -> 33.5).
-constexpr int kFewBlocks = 32, kFewerBlocks = 6;
 // (a shared launch's tile counts this much more where there are many: four of 350 to 980 beside eight of 100 to 230,
 // groups of 8, 31.8 as tiles and 36.9 shared)
 constexpr int kSharedTileOverheadBlocks = 8;
@@ -556,9 +550,13 @@ extern "C" int dskv_mixed_plan_typed(const int32_t *qo_indptr_host, const int32_
     // eleven of 150 beside a chunk of 512 behind 3000 88 -> 55; groups of 8, two of 10000 beside three of 67
     // 91 -> 29.  It loses where the walks are no longer than its own tiles' (two of 3000 beside a chunk of 512 behind 3000,
     // 44 blocks against 56: 54 -> 61; groups of 8, two of 3000 beside 200 behind 1000, 44 against 32: 40 -> 43; six of
-    // 1100 to 1700 beside two of 47, 28 against 9: 26.7 -> 30.5), hence 3/2 of them and kLongWalkBlocks.  And where the kernel
-    // of short walks takes all rows it loses however many rows there are (twelve of 50 beside three of 30:
-    // 9.2 -> 14.9, sixteen of 55, groups of 8: 10.3 -> 16.4).
+    // 1100 to 1700 beside two of 47, 28 against 9: 26.7 -> 30.5), hence 3/2 of them and kLongWalkBlocks.
+    // A dozen rows and more that are most of the work are tiles only where the kernel of short walks takes all of them whole
+    // (twelve of 50 beside three prompts of 30: shared 14.9, tiles 9.2; sixteen of 55, groups of 8: 16.4 and 10.3; in two
+    // parts, eleven of 150 beside 200 behind 1000: 29.6 and 33.5).  Errors against 64 bits are 0.98 of the shared launch's over
+    // 120 such steps (of the rows alone 1.01, of the chunks 0.97).  The kernel of long walks would be faster for some
+    // more (29 rows of 465 beside 78 tokens behind 253: 25.3 and 22.3), but raises its maximum more seldom: errors of the rows
+    // 1.10 of the shared launch's, 1.15 at most.
     auto plan_all = [&](int layout, int64_t *words, bool in_parts = true) {
         const bool shared = layout == DSKV_LAYOUT_SHARED;
         return plan_tiles(qo_indptr_host, kv_len.data(), rows.empty() ? nullptr : routed.data(), batch, n_qo_heads, n_kv_heads,
@@ -614,13 +612,12 @@ extern "C" int dskv_mixed_plan_typed(const int32_t *qo_indptr_host, const int32_
             if ((rc = plan_all(layout, &tile_words))) return rc;
             planned = true;
             const int64_t walk = walk_of_plan(kPrefillWaves, false);
-            const bool few = (int64_t)info->n_tiles * n_kv_heads <= compute_units() && info->n_splits == 1 && walk <= kFewBlocks;
-            bool shared = can_share && weighs && (walk > kLongWalkBlocks || (most && !short_walks()));
+            const bool brief = info->n_splits == 1 && short_walks();
+            bool shared = can_share && weighs && (most ? !brief : walk > kLongWalkBlocks);
             if (shared) {
                 take_rows_out(true);
                 if ((rc = plan_all(DSKV_LAYOUT_SHARED, &tile_words))) return rc;
-                shared = most ? !few || walk > walk_of_plan(kPrefillWavesShared, false) + kFewerBlocks
-                              : 2 * (walk - kLongWalkBlocks) >= 3 * walk_of_plan(kPrefillWavesShared, true);
+                shared = most || 2 * (walk - kLongWalkBlocks) >= 3 * walk_of_plan(kPrefillWavesShared, true);
                 if (!shared) {
                     take_rows_out(false);
                     if ((rc = plan_all(layout, &tile_words))) return rc;

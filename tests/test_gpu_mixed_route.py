@@ -25,7 +25,7 @@ CASES = [
     ("short_rows_short_prompts", [50] * 12 + [30] * 3, [1] * 12 + [30] * 3, 8, 32, 8, "bf16", SEPARATE, 4),
     ("short_rows_halves", [55] * 24 + [34, 34], [1] * 24 + [34, 34], 8, 64, 8, "bf16", SEPARATE, 2),
     ("rows_too_many_for_short", [55] * 40 + [34], [1] * 40 + [34], 8, 32, 8, "bf16", SHARED, 0),
-    ("dozen_beside_as_long_a_chunk", [282] * 14 + [371], [1] * 14 + [5], 8, 32, 8, "bf16", SEPARATE, 0),
+    ("dozen_beside_as_long_a_chunk", [282] * 14 + [371], [1] * 14 + [5], 8, 32, 8, "bf16", SHARED, 0),
     ("dozen_of_longer_rows", [372] * 12 + [18], [1] * 12 + [18], 16, 32, 8, "bf16", SHARED, 0),
     ("page2", [3001, 40], [1, 40], 2, 32, 8, "bf16", SEPARATE, 0),
     ("row_without_tokens", [3001, 0, 40], [1, 1, 40], 16, 32, 8, "bf16", SHARED, 0),
@@ -103,3 +103,21 @@ def test_a_caller_with_little_room_keeps_the_tiles():
         assert lib.dskv_mixed_plan_typed(qo.ctypes.data, pages.ctypes.data, last.ctypes.data, 2, 16, 32, 8, 128, _lib.BF16, 0,
                                          _lib.ROUTE_AUTO, plan.ctypes.data, cap, ctypes.byref(info)) == 0
         assert info.layout == layout and not plan[cap:].any()
+
+
+@pytest.mark.parametrize("group", [4, 8])
+def test_a_dozen_rows_are_tiles_only_where_the_kernel_of_short_walks_takes_them(group):
+    """(the kernel of long walks is further off for them than the shared launch, which they had before there was a choice)"""
+    rng, seen = np.random.default_rng(group), {}
+    for _ in range(400):
+        rows, chunks = int(rng.integers(12, 41)), int(rng.integers(1, 4))
+        kv, qo = rng.integers(2, int(rng.choice([60, 250, 600, 1000])), rows).tolist(), [1] * rows
+        for _ in range(chunks):
+            qo.append(int(rng.integers(2, 300)))
+            kv.append(qo[-1] + int(rng.choice([0, rng.integers(0, 900)])))
+        had = _plan(kv, qo, 16, 8 * group, 8, target=-1)[0].layout      # no choice with a number of workgroups
+        now = _plan(kv, qo, 16, 8 * group, 8)[0]
+        if had == SHARED:
+            assert now.layout == SHARED or now.tile_workgroups, (kv, qo)
+        seen[had, now.layout, bool(now.tile_workgroups)] = True
+    assert (SHARED, SHARED, False) in seen and (SHARED, SEPARATE, True) in seen
