@@ -70,6 +70,8 @@ _SIGNATURES = {
     "dskv_decode_plan_typed": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32, c_int32,
                                          c_int32, c_int32, c_void_p, c_int64, POINTER(c_int32),
                                          POINTER(c_int32), POINTER(c_int64), POINTER(c_int64)]),
+    "dskv_decode_plan_fill": (c_int32, [c_void_p, c_int64, c_int32, c_int32, c_int32, c_int32, POINTER(c_int32),
+                                        POINTER(c_int64)]),
     "dskv_decode_launch": (c_int64, [c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, POINTER(c_int32)]),
     "dskv_decode_attn": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int32,
                                    c_int32, c_void_p, c_int64, c_int32, c_int32, c_int32, c_int32,

@@ -7,7 +7,9 @@ into a graph and replays it: per step the host only rebuilds the CSR metadata
 and the split-KV work list in pinned buffers that never move, copies both to
 device buffers that never move, and replays.  A new batch size (or workgroup
 count) triggers a new capture; the last few captures are kept, so a scheduler that
-alternates between batch sizes replays instead of capturing again.
+alternates between batch sizes replays instead of capturing again.  The workgroup count
+of small 16-bit batches does not follow the requests' lengths (their plans are filled up
+with empty workgroups): a size needs a capture for whole requests and one where some are cut.
 
 Nothing that is captured clears memory with a memset node, and the library
 calls allocate nothing; the outputs of the captured forward live in the graph's

@@ -212,7 +212,8 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
         back, which synchronises.
         plan_buffers: optional staged upload (an object with staging() / upload(words) /
         dev, see model.context.flash.StagedUpload) that receives the work list instead of
-        fresh tensors, for callers that replay captured launches."""
+        fresh tensors, for callers that replay captured launches; with the planner's own number of
+        workgroups a small batch then gets empty ones up to a number that all such batches have."""
         self._shape_args(num_qo_heads, num_kv_heads, head_dim, page_size, data_type)
         self._indptr, self._indices = _i32(indptr), _i32(indices)
         h_indptr = self._host(indptr, indptr_host)
@@ -229,6 +230,8 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
             plan = block.tensor
         words = self._plan_into(plan, cap, h_indptr, h_last, target_workgroups)
         if plan_buffers is not None:
+            if target_workgroups <= 0:
+                words = self._fill_up(plan, cap, words)
             self._plan = plan_buffers.dev
             plan_buffers.upload(max(words, 1))
         else:
@@ -275,6 +278,16 @@ class BatchDecodeWithPagedKVCacheWrapper(_PagedWrapper):
         ptr = h_indptr.numpy()
         self._empty_requests = np.flatnonzero(ptr[1:] <= ptr[:-1])[:4].tolist() if batch > 0 else []
         return int(words.value)
+
+    def _fill_up(self, plan: torch.Tensor, cap: int, words: int) -> int:
+        """The plan with as many workgroups as any batch of the form for small batches has: what a captured
+        launch is known by then does not follow the requests' lengths.  Returns its words."""
+        n_wgs, n_words = ctypes.c_int32(self._n_workgroups), ctypes.c_int64(words)
+        rc = _lib.lib().dskv_decode_plan_fill(plan.data_ptr(), cap, self._hq, self._hkv, self._d, self._plan_dtype,
+                                              ctypes.byref(n_wgs), ctypes.byref(n_words))
+        _lib.check(rc, "decode begin_forward")
+        self._n_workgroups = n_wgs.value
+        return int(n_words.value)
 
     def _few_shares_apply(self, h_indptr: torch.Tensor, h_last: torch.Tensor) -> bool:
         """Whether a batch whose plan does not fit the workspace runs in the few shares of the form for

@@ -120,6 +120,15 @@ int dskv_decode_plan_typed(const int32_t *kv_page_indptr_host, const int32_t *kv
                            int32_t *plan_host, int64_t plan_capacity_words, int32_t *n_items_out,
                            int32_t *n_workgroups_out, int64_t *plan_words_out,
                            int64_t *workspace_bytes_out);
+/*
+ * Fills a plan of dskv_decode_plan_typed up, for callers that replay captured launches, which hold the number of
+ * workgroups: where the attention is one workgroup per (share, kv head), shares without items follow until
+ * there are as many as compute units allow, so that all batches which run in that form have one number, and results
+ * stay as they are, bit for bit.  Other plans stay as they are.  *n_workgroups and *plan_words in: the plan's, out: the filled
+ * one's; dskv_decode_plan_bound words always suffice, a smaller capacity may be DSKV_E_NOMEM with the plan untouched.
+ */
+int dskv_decode_plan_fill(int32_t *plan_host, int64_t plan_capacity_words, int32_t n_qo_heads, int32_t n_kv_heads,
+                          int32_t head_dim, int32_t dtype, int32_t *n_workgroups, int64_t *plan_words);
 
 /*
  * out, q: (batch, n_qo_heads, head_dim) of dtype; pages_layer as for append.
