@@ -509,18 +509,24 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedWrapper):
                    h_last: torch.Tensor, target_workgroups: int, route: bool = True) -> int:
         """Runs the host planner into `plan` (pinned int32, at least cap words); returns the words
         written.  The kv lengths order the tiles longest first and allow parts per tile; when
-        the workspace cannot hold the parts' partials, whole tiles (which need none) are planned,
-        and if it cannot even hold the partials of cut decode rows, nothing is routed."""
+        the workspace cannot hold the partials of the form that the planner chose, rows that were most of the
+        work stay with the decode workgroups beside whole tiles (which leave none), a few rows become tiles like
+        the others, in parts if those fit, and in the end nothing is routed and nothing cut."""
         batch = h_qo.shape[0] - 1
         info = _lib.MixedPlanInfo()
         ws_bytes = self._workspace.numel() * self._workspace.element_size()
         route = int(route)          # True = _lib.ROUTE_AUTO
-        for target, routed in ((target_workgroups, route), (-1, route), (-1, _lib.ROUTE_OFF)):
+        tries = [(target_workgroups, route), (-1, route), (-1, _lib.ROUTE_OFF)]
+        if route == _lib.ROUTE_AUTO and target_workgroups >= 0:
+            tries.insert(2, (target_workgroups, _lib.ROUTE_OFF))
+        for target, routed in tries:
             rc = _lib.lib().dskv_mixed_plan_typed(h_qo.data_ptr(), h_kv.data_ptr(), h_last.data_ptr(), batch,
                                                   self._p, self._hq, self._hkv, self._d, self._plan_dtype, target,
                                                   int(routed), plan.data_ptr(), cap, ctypes.byref(info))
             _lib.check(rc, "prefill begin_forward")
-            if info.tile_workspace_bytes + info.decode_workspace_bytes <= ws_bytes:
+            # (whole tiles only once parts do not fit either)
+            passed_over = len(tries) == 4 and target == -1 and routed == route and info.layout == _lib.LAYOUT_SEPARATE
+            if info.tile_workspace_bytes + info.decode_workspace_bytes <= ws_bytes and not passed_over:
                 break
         ids, self._ids = self._ids, None
         if info.new_rows_late and (ids is None or not _lib.lib().dskv_new_rows_apart(
