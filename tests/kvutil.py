@@ -98,6 +98,48 @@ def max_rel_err_per_request(got: np.ndarray, ref: np.ndarray, row_indptr=None) -
     return worst
 
 
+def attention_bound(sc: Scenario, want: np.ndarray, causal: bool = True) -> np.ndarray:
+    """How far an element of 16-bit attention may be from the fp32 oracle's `want`: with u half a unit in the last place
+    of the element type over its value (8 bits of bf16: 2^-8, 11 of f16: 2^-11), every probability is off by u
+    of itself, so the sum of w_j v_j by u times the sum of w_j |v_j| (the oracle over |V|), and the result is rounded to 16
+    bits, by u of itself; a tenth more for sums in 32 bits, exponentials and second-order terms."""
+    from oracle import c_oracle
+
+    pages = sc.pages.copy()
+    pages[:, 1] = pages[:, 1] & 0x7FFF if sc.dtype == "bf16" else np.abs(pages[:, 1])
+    spread = c_oracle.prefill_attn(sc.q, sc.qo_indptr, pages, sc.kv_page_indices, sc.kv_page_indptr, sc.kv_last_page_lens,
+                                   sc.dtype, causal)
+    return 1.1 * (2.0 ** -8 if sc.dtype == "bf16" else 2.0 ** -11) * (spread + np.abs(want)) + 1e-6
+
+
+def attention_row(sc: Scenario, request: int, row: int, keys: np.ndarray) -> np.ndarray:
+    """The attention of one new row of a request over the given keys of it, in 64 bits: (Hq, D)."""
+    wide = orc.f32_from_bf16_bits if sc.dtype == "bf16" else lambda a: a.astype(np.float32)
+    table = sc.kv_page_indices[sc.kv_page_indptr[request]: sc.kv_page_indptr[request + 1]]
+    kv = wide(sc.pages[table]).astype(np.float64)                         # (pages, 2, P, Hkv, D)
+    k, v = (kv[:, i].reshape(-1, sc.Hkv, sc.D)[keys] for i in (0, 1))
+    q = wide(sc.q[sc.qo_indptr[request] + row]).astype(np.float64).reshape(sc.Hkv, -1, sc.D)
+    s = np.einsum("hgd,khd->hgk", q, k) / np.sqrt(sc.D)
+    w = np.exp(s - s.max(-1, keepdims=True))
+    return np.einsum("hgk,khd->hgd", w / w.sum(-1, keepdims=True), v).reshape(sc.Hq, sc.D)
+
+
+def assert_bound_bites(sc: Scenario, want: np.ndarray, bound: np.ndarray) -> None:
+    """That `bound` lets no request's last row miss a block of 32 keys in the middle, nor - up to 1024 keys: one of more weighs
+    less than all roundings together may - its newest or its oldest key."""
+    for i, (n, new) in enumerate(zip(sc.kv_lens, sc.qo_lens)):
+        if new == 0 or n < max(new, 2):
+            continue
+        at = int(sc.qo_indptr[i + 1]) - 1
+        exact = attention_row(sc, i, int(new) - 1, np.arange(n))
+        assert (np.abs(exact - want[at]) <= 1e-4).all(), i
+        middle = int(n) // 2 // 32 * 32
+        for gone in (np.arange(n - 1, n), np.arange(1), np.arange(middle, min(middle + 32, n))):
+            if len(gone) < n and (len(gone) > 1 or n <= 1024):
+                mutated = attention_row(sc, i, int(new) - 1, np.setdiff1d(np.arange(n), gone))
+                assert (np.abs(mutated - want[at]) > bound[at]).any(), (i, gone[0])
+
+
 # ---- torch <-> storage helpers (GPU tests only)
 def torch_dtype(dtype: str):
     import torch

@@ -8,7 +8,7 @@ import pytest
 import torch
 
 from deserve_amd import _lib
-from kvutil import make_scenario, to_torch
+from kvutil import assert_bound_bites, attention_bound, make_scenario, to_torch
 from oracle import c_oracle
 
 SEPARATE, SHARED = _lib.LAYOUT_SEPARATE, _lib.LAYOUT_SHARED
@@ -62,6 +62,14 @@ def test_which_form_a_mixed_batch_takes(case):
             assert _plan(kv, qo, P, Hq, Hkv, **other)[0].layout == SEPARATE
 
 
+@pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
+def test_the_bound_lets_no_row_miss_a_key(case):
+    name, kv, qo, P, Hq, Hkv, dtype, layout, workgroups = case
+    sc = make_scenario(83, kv_lens=kv, qo_lens=qo, P=P, Hq=Hq, Hkv=Hkv, D=128, dtype=dtype)
+    want = c_oracle.prefill_attn(sc.q, sc.qo_indptr, sc.pages, sc.kv_page_indices, sc.kv_page_indptr, sc.kv_last_page_lens, dtype)
+    assert_bound_bites(sc, want, attention_bound(sc, want))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
 def test_mixed_batches_match_oracle_and_tiles(case):
@@ -84,14 +92,11 @@ def test_mixed_batches_match_oracle_and_tiles(case):
     assert np.isfinite(got).all()
     want = c_oracle.prefill_attn(sc.q, sc.qo_indptr, sc.pages, sc.kv_page_indices, sc.kv_page_indptr,
                                  sc.kv_last_page_lens, dtype, True)
-    for i in range(len(qo)):
-        rows = slice(int(sc.qo_indptr[i]), int(sc.qo_indptr[i + 1]))
-        if qo[i] == 0:
-            continue
-        b = np.asarray(want[rows], np.float32)
-        # a row of P in 16 bits and the result's own rounding: 2^-8 each of values up to the row's largest
-        for a in (got[rows], tiles[rows]):
-            assert np.abs(a - b).max() <= 2e-2 * max(np.abs(b).max(), 1e-3), i
+    bound = attention_bound(sc, want)
+    for form in (got, tiles):
+        off = np.abs(form - want) / bound
+        assert off.max() <= 1, (np.unravel_index(off.argmax(), off.shape), off.max())
+
 
 
 def test_a_caller_with_little_room_keeps_the_tiles():
