@@ -537,33 +537,29 @@ namespace dskv {
 
 // Whether the 16-bit attention of a batch should run as a workgroup per (share, kv head), on
 // few = CUs / n_kv_heads shares, instead of a workgroup per share whose waves are kv heads (at most
-// eight; more heads, more workgroups per share).  Measured with equal, ragged and lopsided batches
-// of 1 to 64 requests at 1 to 160 kv heads (bf16, attention and merge in a replayed graph, us,
-// workgroup per (share, kv head) / the other form; a range is over the batches):
-//   * Eight heads fill a workgroup of the other form, which then wins as soon as memory is the limit:
-//     1200 tiles 23-24 / 24-27, 1800 tiles 30-31 / 30-32, 2550 tiles 38-39 / 36-39 for 1 to 48 requests; 64 and more
-//     from 1200 tiles on 24-25 / 23.  9 to 24 requests are in ten parts and more each, which the merge launch
-//     adds up in two trips: 10 requests of 2550 tiles 38 / 42, 16 39 / 40-42; one of 2000 tiles 33-35 / 35-38, 2250
-//     tiles 36 / 36.  The line: 60 tiles a share, 40 for more than 48 requests, 80 for 9 to 24, 70 for one or two.
-//   * More heads, or fewer than eight that leave waves of the other form idle, lose there later or
-//     not at all where few * n_kv_heads workgroups leave hardly a unit idle: 5 heads, 2000 tiles 23-26 /
-//     23-27; 12 heads, 1706 tiles 40 / 42-44, 2500 tiles 54 / 53-56; 16 heads, 2500 tiles 64 / 69; 64
-//     heads, 625 tiles 64 / 74-80.  Where they do leave units idle: 20 heads (240 workgroups), 1024 tiles
-//     43 / 44-46, 1500 tiles 59 / 54; 96 heads (192), 104 tiles 27-28 / 30-34, 156 tiles 36 / 34-36.
+// eight; more heads, more workgroups per share).  The lines below were drawn where the two forms crossed while the
+// split kernel took half as long again for its first tile and shares were cut without regard to the requests.
+// It is ahead on both sides of every one of them now: they leave some batches to the slower form, whose errors the split
+// one has not been compared with beyond them.  Ragged and equal batches of 1 to 64 requests, groups of four (bf16; append, rotation, attention and merge in a
+// replayed graph, us a layer, workgroup per (share, kv head) / the other form; a range is over the batches):
+//   * Eight heads: 600 tiles 12-15 / 19-22, 1200 tiles 19-22 / 22-27, 1500 tiles 22-25 / 24-29, 1800 tiles 26-28 /
+//     28-33, 2200 tiles 29-32 / 31-36, 2560 tiles 33-37 / 35-40; 64 requests 1500 tiles 22-24 / 24-27.  The line: 60
+//     tiles a share, 40 for more than 48 requests, 80 for 9 to 24, 70 for one or two.
+//   * More heads, or fewer than eight that leave waves of the other form idle: 5 heads, 2560 tiles 24-25 / 28-31; 12 heads,
+//     1700 tiles 36-37 / 44-46, 2500 tiles 48-50 / 56-59; 16 heads, 2500 tiles 62-64 / 78-84; 64 heads in groups of one,
+//     500 tiles 48-52 / 64-77.  Where few * n_kv_heads workgroups leave units idle: 20 heads (240 workgroups), 900 tiles
+//     31-33 / 49-51, 1500 tiles 48-52 / 65-71; 96 heads (192), 110 tiles 22-26 / 32-41, 200 tiles 34-38 / 48-57.
 //     The line: 80 tiles a share, lower by the share of units that idle.
-//   * Groups under four q heads have small partials to merge: up to 15 heads the lines lie a quarter lower
-//     (8 heads in groups of one, 1400 tiles 24 / 22-27, 2000 tiles 31 / 27-34; 12 heads, 2083 tiles 46 / 43-48).
-//   * Up to four heads a request is cut into many parts (few is 64 and more), and merging them costs
-//     more than the walk saves: 4 heads, 375 tiles 12-15 / 12-20, but one request 16 / 14 (87 tiles, which are
-//     no more than 32 parts, 11 / 15), and 750 tiles 15-18 / 13-16 (8 requests, just under the 32 parts of the wide
-//     merge, 15 / 20); 2 heads, 1500 tiles 14-20 / 11-15.
-//   * One head: 256 workgroups of a wave each leave the chip idle: 1500 tiles 14-23 / 11-13, 5000 tiles
-//     17-21 / 18-21, 20480 tiles 36-40 / 47-52.
-//   * Lopsided: one request in dozens of parts beside short ones.  The merge launch gives a row one
-//     workgroup per eight heads: 24 requests, one of 1250 tiles with 8 heads 25 / 58, 2 heads 20 / 48.
-//     (Where requests have more than kWideMergeParts parts on average, that launch gives a row more.)
-//   * Without counters to merge inside the launch (merges_itself) a request pays for the merge launch
-//     as well: 8 heads, 625 tiles 16-22 / 19-24, 937 tiles 20-25 / 22-27, 1250 tiles 23-28 / 23-26.  A third.
+//   * Groups under four q heads, up to 15 heads: the lines lie a quarter lower (8 heads in groups of one, 1400 tiles 22-23 /
+//     25-27, 2000 tiles 28-30 / 30-33; 12 heads, 1700 tiles 35-36 / 40-43, 2000 tiles 39-41 / 44-47).
+//   * Up to four heads a request is cut into many parts (few is 64 and more): 4 heads, 400 tiles 9-10 / 13-15, 1000
+//     tiles 13-14 / 15-19, one request of 192 tiles 9.3 / 13.9, of 300 10.5 / 15.0; 2 heads, 100 tiles 6-8 / 10-12, 1500
+//     tiles 12-14 / 14-17.
+//   * One head: 100 tiles 6-8 / 9-12, 3000 tiles 12-16 / 15-19, 5000 tiles 15-19 / 19-22, 20480 tiles 33-38 / 47-50.
+//   * Lopsided: one request of 1250 tiles beside 23 short ones, 8 heads 24 / 33, 2 heads 16 / 20, 16 heads 38 / 61.
+//     (Where requests have more than kWideMergeParts parts on average, the merge launch gives a row more.)
+//   * Without counters to merge inside the launch (merges_itself) a request pays for the merge launch as well: 8 heads, 600
+//     tiles 14-15 / 19-21, 900 tiles 17-18 / 20-24, 1800 tiles 27-28 / 28-32.  A third.
 static bool splitting_pays(int64_t tiles, int64_t longest, int batch, int n_kv_heads, int group, bool merges_itself)
 {
     const int64_t cus = default_workgroups(), few = cus / n_kv_heads, busy = few * n_kv_heads;
@@ -573,7 +569,7 @@ static bool splitting_pays(int64_t tiles, int64_t longest, int batch, int n_kv_h
     if (longest * cus > kLopsidedParts * tiles && batch + cus <= kWideMergeParts * (int64_t)batch) return true;
     int64_t most;
     if (n_kv_heads <= 2) most = 0;
-    else if (n_kv_heads <= 4) most = batch > 1 ? 2048 / n_kv_heads : kWideMergeParts * kSplitTilesPerShare;
+    else if (n_kv_heads <= 4) most = batch > 1 ? 2048 / n_kv_heads : kSplitMaxTilesOneRequest;
     else if (n_kv_heads != kMaxWaves && 32 * busy >= 31 * cus) most = kSplitMaxTiles;
     else most = (n_kv_heads > kMaxWaves || (batch >= 9 && batch <= 24) ? 80 : batch > 48 ? 40 : batch <= 2 ? 70 : 60) *
                 few * busy / cus;
@@ -618,9 +614,9 @@ static bool gqa_splitting_pays(int64_t tiles, int64_t longest, int batch, int n_
     return work <= 2048 && pairs <= most_pairs;
 }
 
-// Shares of a batch whose tiles are split over the waves of workgroups (splitting_pays), as the global tile at which each
-// ends, at most `most` of them.  Uncut, requests lie whole in a share, several of them as long as they fit into `cap`
-// tiles; cut, longer ones get shares of their own.
+// Shares of a batch whose tiles are split over the waves of workgroups (splitting_pays): how many, and the global tile at
+// which each ends.  Uncut, requests lie whole in a share, several of them as long as they fit into `cap` tiles; cut,
+// longer ones get shares of their own.
 static int64_t lay_out_shares(const std::vector<int64_t> &tiles, int64_t cap, bool cut, std::vector<int64_t> *ends)
 {
     int64_t at = 0, filled = 0, shares = 0;
@@ -948,7 +944,7 @@ static int decode_attn_impl(void *out, const void *q, const void *pages_layer,
                                     (const uint16_t *)k_new, (const uint16_t *)v_new, n_qo_heads, n_kv_heads,
                                     n_qo_heads / n_kv_heads, shift, scale_log2, split_slots, part_o, part_ml,
                                     merged && n_items > batch ? merge_counters : nullptr,
-                                    (int)std::min<int64_t>(n_merge_counters, 1 << 30), 0, (uint16_t *)out};
+                                    (int)std::min<int64_t>(n_merge_counters, 1 << 30), (uint16_t *)out};
             const dim3 grid((unsigned)n_workgroups, (unsigned)n_kv_heads), block(64 * kSplitWaves);
 #define DSKV_LAUNCH_SPLIT(DT, COVER) \
     hipLaunchKernelGGL((decode_attn_split_kernel<DT, COVER>), grid, block, 0, s, args)

@@ -28,9 +28,11 @@ constexpr int kSplitWaves = 8;
 // K by whole rows (TileRegs): all waves request their tiles at once, at the start, and the address path is
 // through with the requests sooner: 8 requests of 300-1100, 16 layers replayed, 277.1 -> 270.4 us.
 constexpr bool kSplitWholeRows = true;
-// The planner's rule, measured there: tiles of a batch at most (one kv head: at least), tiles of a
-// share at least, and parts of one request that make a batch lopsided.
-constexpr int kSplitMaxTiles = 2560, kSplitMinTilesOneHead = 5000, kSplitTilesPerShare = 6, kLopsidedParts = 64;
+// The planner's rules, measured there: tiles of a batch at most (one kv head: at least; one request with three or four heads:
+// at most), and parts of one request that make a batch lopsided.  Tiles of a share at least, for the generic kernel's
+// plans (the 16-bit ones follow the requests).
+constexpr int kSplitMaxTiles = 2560, kSplitMinTilesOneHead = 5000, kSplitMaxTilesOneRequest = 192, kLopsidedParts = 64;
+constexpr int kSplitTilesPerShare = 6;
 constexpr int kSplitMaxGroup = 8;    // q heads per kv head, at most (LDS for the pieces that meet)
 // LDS: the waves' V tiles; two meeting places per wave ([0] a piece that continues an item of an
 // earlier wave, [1] one that a later wave continues) of O and (m, l) per q head; the new token's
@@ -142,7 +144,6 @@ struct SplitArgs {
     float *part_o, *part_ml;
     uint32_t *counters;              // one zeroed word per (partial slot, kv head); null: a merge launch follows
     int n_counters;
-    int unused;
     uint16_t *out;
 };
 static_assert(sizeof(SplitArgs) == 128, "");

@@ -756,7 +756,7 @@ static int prefill_attn_impl(void *out, const void *q, const int32_t *qo_indptr,
             const int group = n_qo_heads / n_kv_heads;
             const ShortArgs short_args = {plan_dev, qo_indptr, kv_page_indptr, kv_last_page_len, kv_page_indices,
                                           (const char *)pages_layer, (const uint16_t *)q, rope_table, (uint16_t *)out,
-                                          n_tiles, n_qo_heads, n_kv_heads, group, 65536 / group + 1, shift, causal, scale_log2};
+                                          n_qo_heads, n_kv_heads, group, 65536 / group + 1, shift, causal, scale_log2};
 #define DSKV_LAUNCH_SHORT_W(DT, W, ROWS)                                                                         \
     hipLaunchKernelGGL((prefill_short_kernel<DT, W, ROWS>), dim3((unsigned)n_kv_heads, (unsigned)n_tiles, kPrefillWaves / W), \
                        dim3(64 * kShortWaves), 0, s, short_args)

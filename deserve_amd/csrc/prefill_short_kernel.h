@@ -44,7 +44,7 @@ struct ShortArgs {
     const uint16_t *q;
     const float *rope;   // cos | sin by query row (q is rotated as it is loaded), or null
     uint16_t *out;
-    int n_tiles, n_qo_heads, n_kv_heads, group;
+    int n_qo_heads, n_kv_heads, group;
     int group_inverse;   // x / group = x * this >> 16 for x < 32
     int page_shift, causal;
     float scale_log2;
