@@ -553,8 +553,8 @@ extern "C" int dskv_mixed_plan_typed(const int32_t *qo_indptr_host, const int32_
     // 1100 to 1700 beside two of 47, 28 against 9: 26.7 -> 30.5), hence 3/2 of them and kLongWalkBlocks.
     // A dozen rows and more that are most of the work are tiles only where the kernel of short walks takes all of them whole
     // (twelve of 50 beside three prompts of 30: shared 14.9, tiles 9.2; sixteen of 55, groups of 8: 16.4 and 10.3; in two
-    // parts, eleven of 150 beside 200 behind 1000: 29.6 and 33.5).  Errors against 64 bits are 0.98 of the shared launch's over
-    // 120 such steps (of the rows alone 1.01, of the chunks 0.97).  The kernel of long walks would be faster for some
+    // parts, eleven of 150 beside 200 behind 1000: 29.6 and 33.5).  Errors against 64 bits are 0.99 of the shared launch's over
+    // 260 such steps, 0.93 to 1.01 (of the rows alone 1.01, 1.03 at most; of the chunks 0.98).  The kernel of long walks would be faster for some
     // more (29 rows of 465 beside 78 tokens behind 253: 25.3 and 22.3), but raises its maximum more seldom: errors of the rows
     // 1.10 of the shared launch's, 1.15 at most.
     auto plan_all = [&](int layout, int64_t *words, bool in_parts = true) {
